@@ -202,3 +202,74 @@ def tolerance(case):
     # 2.3e-3, gradients 2.3e-3 to 2.7e-3, which is what rounding weights and results to bf16 gives;
     # four times that.
     return {"rel": 1e-2}
+
+
+def _visible(case, rows):
+    """Mask of the query positions `rows` against every key position."""
+    i, j = rows[:, None], torch.arange(case["S"], device=rows.device)[None, :]
+    pattern = case["pattern"]
+    if case["family"] == "image":
+        W = case["width"]
+
+        def group(t):  # text chunks of 64 tokens ride with groups 0..7
+            return torch.where(t < TEXT_LEN, t // 64, (t - TEXT_LEN) // W % 2 * 4 + (t - TEXT_LEN) % W % 4)
+
+        scattered = (j < TEXT_LEN) | (group(i) == group(j))
+        if pattern == "scatter":
+            return scattered
+
+        def in_window(query, key):  # 16 rows or columns around the query's patch of 8, inside the grid
+            start = (query // 8 * 8 - 4).clamp(0, W - 16)
+            return (key >= start) & (key < start + 16)
+
+        qi, kj = i - TEXT_LEN, j - TEXT_LEN
+        window = in_window(qi // W, kj // W) & in_window(qi % W, kj % W)
+        return torch.where(i < TEXT_LEN, scattered, (j < TEXT_LEN) | window)
+    causal = j <= i
+    if pattern == "scatter":
+        return causal & (i % case["group_num"] == j % case["group_num"])
+    if pattern == "gather1":
+        G = case["group_num"]
+        return causal & (i // G % G == j // G % G)
+    if pattern == "window":
+        return causal & (j >= i // 64 * 64 - (case["window"] - 64))
+    if pattern == "window_sink":
+        return causal & ((i - j < case["window"]) | (j < case["n_sink"]))
+    G, off = case["group_num"], case["offset"]
+    qb, kb = i // case["block"], j // case["block"]
+    source = (qb + off) % G
+    own = (kb == qb) & ((source == qb % G) | (off != 0))
+    return causal & (((kb < qb) & (kb % G == source)) | own | (j < case["n_sink"]))
+
+
+def exact(case, seed):
+    """The outputs of `run` in float64: dense masked attention, a block of query rows at a time."""
+    state = prepare(case, seed)
+    q, k, v = (x.detach().transpose(1, 2) for x in state["qkv"])  # (B, heads, S, 128)
+    B, H, S, D = q.shape
+    train, ratio, scale = case["mode"] == "train", H // k.shape[1], D ** -0.5
+    out = torch.empty(B, H, S, D, dtype=torch.float64, device=q.device)
+    lse = torch.empty(B, H, S, dtype=torch.float64, device=q.device)
+    dq = torch.empty_like(out)
+    dk, dv = (torch.zeros(k.shape, dtype=torch.float64, device=q.device) for _ in range(2))
+    step = max(64, (1 << 27) // S)
+    for r0 in range(0, S, step):
+        rows = slice(r0, min(S, r0 + step))
+        hidden = ~_visible(case, torch.arange(S, device=q.device)[rows])
+        for b in range(B):
+            for h in range(H):
+                g = h // ratio
+                qr, kh, vh = q[b, h, rows].double(), k[b, g].double(), v[b, g].double()
+                weights = (qr @ kh.T).mul_(scale).masked_fill_(hidden, -torch.inf)
+                lse[b, h, rows] = torch.logsumexp(weights, 1)
+                weights = weights.sub_(lse[b, h, rows, None]).exp_()
+                out[b, h, rows] = weights @ vh
+                if train:
+                    do = state["dout"].transpose(1, 2)[b, h, rows].double()
+                    dv[b, g] += weights.T @ do
+                    ds = (do @ vh.T).sub_((do * out[b, h, rows]).sum(1, keepdim=True)).mul_(weights).mul_(scale)
+                    dq[b, h, rows] = ds @ kh
+                    dk[b, g] += ds.T @ qr
+    if train:
+        return tuple(x.transpose(1, 2) for x in (out, dq, dk, dv))
+    return (out.transpose(1, 2), lse) if case["lse"] else out.transpose(1, 2)
