@@ -47,7 +47,7 @@ int make_request(int domain, int pattern, int B, int S, int H, int Hkv, int arg0
   r->H = H;
   r->Hkv = Hkv;
   r->geom = IntraGeom{S, 1, 64, 16, 8, 0, 1, 1, 64, 0, 0};  // derived fields: geom_finish() in shape_for()
-  r->geom.sink_chunk = 1024;  // backward: set by leading_chunk() once the number of leading keys is known
+  r->geom.sink_chunk = 1024;  // backward: set by set_leading_chunks() once the number of leading keys is known
   if (domain == 0) {
     if (!extended && (pattern == INTRA_LLM_BLOCK_SCATTER || pattern == INTRA_LLM_WINDOW_SINK))
       return fail(INTRA_ERR_INVALID, "unknown LLM pattern id %d (0 scatter, 1 gather1, 4 window)", pattern);
@@ -542,94 +542,97 @@ int run(int domain, const void* q, const void* k, const void* v, void* o, int B,
 
 
 // ------------------------------------------------------------------------------------ backward
-template <class RMAP, int MODE, int HP, bool PARTIAL = false>
-int launch_bwd(const intra::BParams& p, int64_t grid, hipStream_t stream) {
-  if (grid <= 0 || grid > 0x7fffffff) return fail(INTRA_ERR_UNSUPPORTED, "backward needs more than 2^31 workgroups");
-  hipLaunchKernelGGL((intra::intra_bwd_kernel<RMAP, MODE, HP, PARTIAL>), dim3((unsigned)grid), dim3(intra::bwd_waves(MODE) * 64), 0, stream, p);
+template <class RMAP, int MODE, int HP, class LEAD = intra::NoLeadingKeys>
+int launch_bwd(const intra::BParams& p, hipStream_t stream) {
+  const int64_t grid = (int64_t)p.grid.blocks + p.lead.blocks;
+  if (p.grid.blocks <= 0 || p.lead.blocks < 0 || grid > 0x7fffffff) return fail(INTRA_ERR_UNSUPPORTED, "backward needs more than 2^31 workgroups");
+  hipLaunchKernelGGL((intra::intra_bwd_kernel<RMAP, MODE, HP, LEAD>), dim3((unsigned)grid), dim3(intra::bwd_waves(MODE) * 64), 0, stream, p);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return fail(INTRA_ERR_HIP, "kernel launch failed: %s", hipGetErrorString(e));
   return INTRA_OK;
 }
 
-// Grid of one backward launch: per XCD, bundles of pairs x items of a pair (see the kernel).
-int64_t bwd_grid(intra::BParams& p, int64_t pairs) {
-  p.items_per_pair = p.n_rblocks * p.hgroups;
+// Workgroups of a row map with `rows` rows each: per XCD, bundles of pairs x items of a pair (see the
+// kernel).  blocks = -1 if they are too many to number.
+template <class R>
+intra::BwdGrid bwd_grid(const intra::BParams& p, int rows, int hgroups) {
+  intra::BwdGrid g;
+  const int64_t pairs = (int64_t)R::num_sets(p.geom) * p.B * p.Hkv;
+  g.hgroups = hgroups;
+  g.n_rblocks = (R::max_rows(p.geom) + rows - 1) / rows;
+  g.items_per_pair = g.n_rblocks * hgroups;
   const int64_t pairs_per_xcd = (pairs + 7) / 8;
-  const int64_t want = (32 + p.items_per_pair - 1) / p.items_per_pair;  // pairs that fill an XCD's 32 CUs
-  p.bundle = (int)std::max<int64_t>(1, std::min<int64_t>(want, pairs_per_xcd));
-  const int64_t bundles = (pairs_per_xcd + p.bundle - 1) / p.bundle;
-  return 8 * bundles * p.bundle * p.items_per_pair;
+  const int64_t want = (32 + g.items_per_pair - 1) / g.items_per_pair;  // pairs that fill an XCD's 32 CUs
+  g.bundle = (int)std::max<int64_t>(1, std::min<int64_t>(want, pairs_per_xcd));
+  const int64_t bundles = (pairs_per_xcd + g.bundle - 1) / g.bundle;
+  const int64_t blocks = 8 * bundles * g.bundle * g.items_per_pair;
+  g.blocks = blocks > 0x7fffffff ? -1 : (int)blocks;
+  return g;
 }
 
 // dQ of a forward map: row blocks of 256 / hp queries of hp heads; also writes D = rowsum(dO o O)
 template <class MAP>
 int run_bwd_dq(intra::BParams p, int hp, hipStream_t stream) {
   using R = intra::QueryRows<MAP>;
-  const int64_t pairs = (int64_t)R::num_sets(p.geom) * p.B * p.Hkv;
-  p.hgroups = p.ratio / hp;
-  p.n_rblocks = (R::max_rows(p.geom) + 256 / hp - 1) / (256 / hp);
-  const int64_t grid = bwd_grid(p, pairs);
+  p.grid = bwd_grid<R>(p, 256 / hp, p.ratio / hp);
   switch (hp) {
-    case 4: return launch_bwd<R, intra::BWD_DQ, 4>(p, grid, stream);
-    case 2: return launch_bwd<R, intra::BWD_DQ, 2>(p, grid, stream);
-    default: return launch_bwd<R, intra::BWD_DQ, 1>(p, grid, stream);
+    case 4: return launch_bwd<R, intra::BWD_DQ, 4>(p, stream);
+    case 2: return launch_bwd<R, intra::BWD_DQ, 2>(p, stream);
+    default: return launch_bwd<R, intra::BWD_DQ, 1>(p, stream);
   }
 }
 
-// One launch over a key-row map: row blocks of one kv head's keys (32 per wavefront of the mode's
-// workgroups), all query heads of its group streamed past
-template <class R, bool PARTIAL, int MODE>
-int run_bwd_keys_mode(intra::BParams p, hipStream_t stream) {
-  constexpr int rows = intra::bwd_waves(MODE) * 32;
-  const int64_t pairs = (int64_t)R::num_sets(p.geom) * p.B * p.Hkv;
-  p.hgroups = 1;
-  p.n_rblocks = (R::max_rows(p.geom) + rows - 1) / rows;
-  return launch_bwd<R, MODE, 1, PARTIAL>(p, bwd_grid(p, pairs), stream);
-}
-// dK and dV over a key-row map, in one pass
+// dK and dV over a key-row map: row blocks of 128 keys of one kv head, all query heads of its group
+// streamed past.
+constexpr int KEY_ROWS = intra::bwd_waves(intra::BWD_DKV) * 32;
 template <class R>
-int run_bwd_keys(const intra::BParams& p, hipStream_t stream) {
-  return run_bwd_keys_mode<R, false, intra::BWD_DKV>(p, stream);
+int run_bwd_keys(intra::BParams p, hipStream_t stream) {
+  p.grid = bwd_grid<R>(p, KEY_ROWS, 1);
+  return launch_bwd<R, intra::BWD_DKV, 1>(p, stream);
 }
 
-// Queries per workgroup of the pass over the `ns` leading keys (LLM sinks, image text keys): about
-// one workgroup per CU (`cus`: the device's count; the workspace size and the launch have to use the
-// same one), at least 128 queries each, a multiple of 64.
-constexpr int MODEL_CUS = 256;  // host-only walks of the decomposition: any value gives a valid split
-// The workspace is sized for a device of WS_CUS CUs (no device has to be current to ask for the size);
-// a launch splits for min(its device's CUs, WS_CUS), which never needs more chunks than that.
+// Chunks of queries that the pass over the `ns` leading keys (LLM sinks, image text keys) is cut into,
+// and their length, a multiple of 64 and at least 128 (except for the last).  The workspace holds
+// fp32 sums of one result for about one 256-key row block per CU of a device of WS_CUS CUs; dk and
+// dv share that room, so half as many chunks have both.  (Twice the chunks would even out sinks
+// better and cost the text keys of an image twice the partial sums.)
 constexpr int WS_CUS = 320;
-int leading_chunk(int S, int B, int Hkv, int ns, int cus) {
+int workspace_chunks(int S, int B, int Hkv, int ns) {
   const int64_t row_wgs = (int64_t)B * Hkv * ((ns + 255) / 256);
-  int64_t chunks = std::max<int64_t>(1, cus / row_wgs);  // at most one workgroup per CU: no second, thin round
+  int64_t chunks = std::max<int64_t>(1, WS_CUS / row_wgs);
   chunks = std::min<int64_t>(chunks, std::max(1, S / 128));
-  return (int)(64 * ((S + 64 * chunks - 1) / (64 * chunks)));
+  const int64_t chunk = 64 * ((S + 64 * chunks - 1) / (64 * chunks));
+  return (int)((S + chunk - 1) / chunk);
+}
+void set_leading_chunks(IntraGeom& ge, int S, int B, int Hkv, int ns) {
+  const int64_t chunks = std::max(1, workspace_chunks(S, B, Hkv, ns) / 2);
+  ge.ns = ns;
+  ge.sink_chunk = (int)(64 * ((S + 64 * chunks - 1) / (64 * chunks)));
 }
 
-// The rows of dk and dv of the leading keys: partial sums per chunk of queries, then their sum
-// (twice: dk and dv share the partial buffer; everything is ordered by the stream).
-template <class R>
-int run_bwd_leading(const intra::BParams& p, hipStream_t stream) {
-  const int ns = R::max_rows(p.geom), chunks = R::num_sets(p.geom);
+// dK and dV over a key-row map and, in the same launch, over the leading keys LEAD.
+// `longest`: columns of the longest row block of R.
+template <class R, class LEAD>
+int run_bwd_keys_lead(intra::BParams p, int64_t longest, hipStream_t stream) {
+  p.grid = bwd_grid<R>(p, KEY_ROWS, 1);
+  p.lead = bwd_grid<LEAD>(p, KEY_ROWS, 1);
+  p.lead_first = p.geom.sink_chunk > longest;
+  return launch_bwd<R, intra::BWD_DKV, 1, LEAD>(p, stream);
+}
+
+// The leading keys' rows of dk and dv from their partial sums (one chunk: written by the launch itself)
+int run_bwd_lead_reduce(const intra::BParams& p, int ns, hipStream_t stream) {
+  const int chunks = intra::KeyRowsSinks::num_sets(p.geom);
+  if (chunks == 1) return INTRA_OK;
   const int64_t threads = (int64_t)p.B * p.Hkv * ns * 32;
-  const unsigned blocks = (unsigned)((threads + 255) / 256);
-  for (int mode = 0; mode < 2; ++mode) {
-    int rc = mode == 0 ? run_bwd_keys_mode<R, true, intra::BWD_DK>(p, stream)
-                       : run_bwd_keys_mode<R, true, intra::BWD_DV>(p, stream);
-    if (rc) return rc;
-    if (mode == 0)
-      hipLaunchKernelGGL(intra::intra_bwd_sink_reduce, dim3(blocks), dim3(256), 0, stream, p.part, chunks, p.B, p.Hkv,
-                         ns, p.dk, p.dk_bs, p.dk_rs, p.dk_hs);
-    else
-      hipLaunchKernelGGL(intra::intra_bwd_sink_reduce, dim3(blocks), dim3(256), 0, stream, p.part, chunks, p.B, p.Hkv,
-                         ns, p.dv, p.dv_bs, p.dv_rs, p.dv_hs);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return fail(INTRA_ERR_HIP, "kernel launch failed: %s", hipGetErrorString(e));
-  }
+  hipLaunchKernelGGL(intra::intra_bwd_lead_reduce, dim3((unsigned)((threads + 255) / 256), 2), dim3(256), 0, stream, p,
+                     chunks, ns);
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return fail(INTRA_ERR_HIP, "kernel launch failed: %s", hipGetErrorString(e));
   return INTRA_OK;
 }
 
-// keys every query sees, handled by run_bwd_leading
+// keys every (later) query sees
 int leading_keys(const Request& r) {
   if (r.kind == KIND_LLM_BLOCK_SCATTER || r.kind == KIND_LLM_WINDOW_SINK) return std::min(r.geom.ns, r.S);
   if (r.kind == KIND_IMG_SCATTER || r.kind == KIND_IMG_GATHER0) return r.geom.text_len;
@@ -639,13 +642,10 @@ int leading_keys(const Request& r) {
 // floats of workspace: -D = -rowsum(dO o O) and lse * log2(e) per (batch, head, token), then the partial
 // sums of the leading keys
 int64_t bwd_dsum_floats(int B, int S, int H) { return ((int64_t)B * H * S + 3) & ~(int64_t)3; }
-int64_t bwd_workspace_floats(const Request& r, int cus) {
+int64_t bwd_workspace_floats(const Request& r) {
   int64_t n = 2 * bwd_dsum_floats(r.B, r.S, r.H);
   const int ns = leading_keys(r);
-  if (ns > 0) {
-    const int chunk = leading_chunk(r.S, r.B, r.Hkv, ns, cus);
-    n += (int64_t)((r.S + chunk - 1) / chunk) * r.B * r.Hkv * ns * 128;
-  }
+  if (ns > 0) n += (int64_t)workspace_chunks(r.S, r.B, r.Hkv, ns) * r.B * r.Hkv * ns * 128;
   return n;
 }
 
@@ -717,12 +717,9 @@ int run_bwd(int domain, const void* q, const void* k, const void* v, const void*
   if (!shape_for(r, default_hp(H / Hkv), &sh)) return fail(INTRA_ERR_UNSUPPORTED, "no kernel shape for this request");
   p.geom = sh.geom;
   const int ns = leading_keys(r);
-  if (ns > 0) {
-    p.geom.ns = ns;
-    const int cus = cu_count();
-    if (cus <= 0) return fail(INTRA_ERR_HIP, "cannot query the current device: %s", hipGetErrorString(hipGetLastError()));
-    p.geom.sink_chunk = leading_chunk(S, B, Hkv, ns, std::min(cus, WS_CUS));
-  }
+  if (ns > 0) set_leading_chunks(p.geom, S, B, Hkv, ns);
+  p.lead = intra::BwdGrid{};
+  p.lead_first = 0;
   hipStream_t st = static_cast<hipStream_t>(stream);
   switch (sh.map) {
     case MAP_LLM_SCATTER:
@@ -736,21 +733,23 @@ int run_bwd(int domain, const void* q, const void* k, const void* v, const void*
       return run_bwd_keys<intra::KeyRowsOf<MapLlmWindow>>(p, st);
     case MAP_LLM_BLOCK_SCATTER:
       if ((rc = run_bwd_dq<MapLlmBlockScatter>(p, sh.hp, st))) return rc;
-      if ((rc = run_bwd_keys<intra::KeyRowsBlockScatter>(p, st))) return rc;
-      return ns > 0 ? run_bwd_leading<intra::KeyRowsSinks>(p, st) : INTRA_OK;
+      if (ns == 0) return run_bwd_keys<intra::KeyRowsBlockScatter>(p, st);
+      rc = run_bwd_keys_lead<intra::KeyRowsBlockScatter, intra::KeyRowsSinks>(p, intra::KeyRowsBlockScatter::max_rows(p.geom), st);
+      return rc ? rc : run_bwd_lead_reduce(p, ns, st);
     case MAP_LLM_WINDOW_SINK:
       if ((rc = run_bwd_dq<MapLlmWindowSink>(p, sh.hp, st))) return rc;
-      if ((rc = run_bwd_keys<intra::KeyRowsWindowSink>(p, st))) return rc;
-      return ns > 0 ? run_bwd_leading<intra::KeyRowsSinks>(p, st) : INTRA_OK;
+      if (ns == 0) return run_bwd_keys<intra::KeyRowsWindowSink>(p, st);
+      rc = run_bwd_keys_lead<intra::KeyRowsWindowSink, intra::KeyRowsSinks>(p, (int64_t)p.geom.window + KEY_ROWS, st);
+      return rc ? rc : run_bwd_lead_reduce(p, ns, st);
     case MAP_IMG_SCATTER:  // grid keys against their group's queries, text keys against all queries
       if ((rc = run_bwd_dq<MapImgScatter>(p, sh.hp, st))) return rc;
-      if ((rc = run_bwd_keys<intra::KeyRowsImgGroup<false>>(p, st))) return rc;
-      return run_bwd_leading<intra::KeyRowsText>(p, st);
+      rc = run_bwd_keys_lead<intra::KeyRowsImgGroup<false>, intra::KeyRowsText>(p, S / 8, st);
+      return rc ? rc : run_bwd_lead_reduce(p, ns, st);
     case MAP_IMG_GATHER0:  // grid keys against the grid queries around them, plus their group's text queries
       if ((rc = run_bwd_dq<MapImgGather0>(p, sh.hp, st))) return rc;
-      if ((rc = run_bwd_keys<intra::KeyRowsImgWindow>(p, st))) return rc;
+      if ((rc = run_bwd_keys_lead<intra::KeyRowsImgWindow, intra::KeyRowsText>(p, 3 * (intra::KeyRowsImgWindow::RUN + 2) * 64, st))) return rc;
       if ((rc = run_bwd_keys<intra::KeyRowsImgGroup<true>>(p, st))) return rc;
-      return run_bwd_leading<intra::KeyRowsText>(p, st);
+      return run_bwd_lead_reduce(p, ns, st);
     default: return fail(INTRA_ERR_UNSUPPORTED, "backward: no kernels for this pattern");
   }
 }
@@ -783,8 +782,8 @@ float* noalloc_scratch() {
 // Host walk of the backward decomposition: count[q * S + k] += 1 for every (query, key) pair that
 // the dK / dV launches (key-row maps with their `store` rule, then the sink pass) multiply.
 template <class R>
-void bwd_walk(const IntraGeom& ge, uint8_t* count, int rows) {  // rows: keys per row block of the launch
-  const int S = ge.S;
+void bwd_walk(const IntraGeom& ge, uint8_t* count) {
+  const int S = ge.S, rows = KEY_ROWS;
   for (int set = 0; set < R::num_sets(ge); ++set)
     for (int r0 = 0; r0 < R::max_rows(ge); r0 += rows) {
       const R m(ge, set, r0);
@@ -805,16 +804,16 @@ int model_mask_bwd(const Request& r, uint8_t* count) {
   Shape sh;
   if (!shape_for(r, 1, &sh)) return fail(INTRA_ERR_UNSUPPORTED, "no kernel shape for this request");
   switch (sh.map) {
-    case MAP_LLM_SCATTER: bwd_walk<intra::KeyRowsOf<MapLlmScatter>>(sh.geom, count, intra::bwd_waves(intra::BWD_DKV) * 32); break;
-    case MAP_LLM_GATHER1: bwd_walk<intra::KeyRowsOf<MapLlmGather1>>(sh.geom, count, intra::bwd_waves(intra::BWD_DKV) * 32); break;
-    case MAP_LLM_WINDOW: bwd_walk<intra::KeyRowsOf<MapLlmWindow>>(sh.geom, count, intra::bwd_waves(intra::BWD_DKV) * 32); break;
-    case MAP_LLM_BLOCK_SCATTER: bwd_walk<intra::KeyRowsBlockScatter>(sh.geom, count, intra::bwd_waves(intra::BWD_DKV) * 32); break;
-    case MAP_LLM_WINDOW_SINK: bwd_walk<intra::KeyRowsWindowSink>(sh.geom, count, intra::bwd_waves(intra::BWD_DKV) * 32); break;
+    case MAP_LLM_SCATTER: bwd_walk<intra::KeyRowsOf<MapLlmScatter>>(sh.geom, count); break;
+    case MAP_LLM_GATHER1: bwd_walk<intra::KeyRowsOf<MapLlmGather1>>(sh.geom, count); break;
+    case MAP_LLM_WINDOW: bwd_walk<intra::KeyRowsOf<MapLlmWindow>>(sh.geom, count); break;
+    case MAP_LLM_BLOCK_SCATTER: bwd_walk<intra::KeyRowsBlockScatter>(sh.geom, count); break;
+    case MAP_LLM_WINDOW_SINK: bwd_walk<intra::KeyRowsWindowSink>(sh.geom, count); break;
     default: return fail(INTRA_ERR_UNSUPPORTED, "backward: no kernels for this pattern");
   }
   if (leading_keys(r) > 0) {
-    sh.geom.sink_chunk = leading_chunk(r.S, 1, 1, leading_keys(r), MODEL_CUS);
-    bwd_walk<intra::KeyRowsSinks>(sh.geom, count, 256);
+    set_leading_chunks(sh.geom, r.S, 1, 1, leading_keys(r));
+    bwd_walk<intra::KeyRowsSinks>(sh.geom, count);
   }
   return INTRA_OK;
 }
@@ -834,15 +833,14 @@ int model_mask_image_bwd(const Request& r, uint8_t* count) {
   Shape sh;
   if (!shape_for(r, 1, &sh)) return fail(INTRA_ERR_UNSUPPORTED, "no kernel shape for this request");
   IntraGeom ge = sh.geom;
-  ge.ns = ge.text_len;  // the text keys are the leading keys every query sees
-  ge.sink_chunk = leading_chunk(r.S, 1, 1, ge.ns, MODEL_CUS);
+  set_leading_chunks(ge, r.S, 1, 1, ge.text_len);  // the text keys are the leading keys every query sees
   if (r.kind == KIND_IMG_SCATTER) {
-    bwd_walk<intra::KeyRowsImgGroup<false>>(ge, count, intra::bwd_waves(intra::BWD_DKV) * 32);
+    bwd_walk<intra::KeyRowsImgGroup<false>>(ge, count);
   } else {
-    bwd_walk<intra::KeyRowsImgWindow>(ge, count, intra::bwd_waves(intra::BWD_DKV) * 32);
-    bwd_walk<intra::KeyRowsImgGroup<true>>(ge, count, intra::bwd_waves(intra::BWD_DKV) * 32);
+    bwd_walk<intra::KeyRowsImgWindow>(ge, count);
+    bwd_walk<intra::KeyRowsImgGroup<true>>(ge, count);
   }
-  bwd_walk<intra::KeyRowsText>(ge, count, 256);
+  bwd_walk<intra::KeyRowsText>(ge, count);
   return INTRA_OK;
 }
 
@@ -907,7 +905,7 @@ int intra_llm_bwd_noalloc(const void* q, const void* k, const void* v, const voi
   int rc = make_request(0, pattern, B, S, H, Hkv, group_num, window, &r, block, offset, n_sink, true);
   if (rc) return rc;
   if ((rc = bwd_supported(r))) return rc;
-  const int64_t need = bwd_workspace_floats(r, WS_CUS);
+  const int64_t need = bwd_workspace_floats(r);
   if (need > (int64_t)INTRA_NOALLOC_SCRATCH_FLOATS)
     return fail(INTRA_ERR_UNSUPPORTED,
                 "intra_llm_bwd_noalloc: this call needs %lld floats of workspace, the built-in one holds %lld; "
@@ -925,7 +923,7 @@ int64_t intra_llm_bwd_workspace(int B, int S, int H, int Hkv, int pattern, int g
   Request r;
   if (make_request(0, pattern, B, S, H, Hkv, group_num, window, &r, block, offset, n_sink, true)) return -1;
   if (bwd_supported(r)) return -1;
-  return bwd_workspace_floats(r, WS_CUS);
+  return bwd_workspace_floats(r);
 }
 
 int intra_image_bwd(const void* q, const void* k, const void* v, const void* o, const float* lse, const void* dout,
@@ -943,7 +941,7 @@ int64_t intra_image_bwd_workspace(int B, int S, int H, int Hkv, int pattern, int
   g_err[0] = 0;
   Request r;
   if (make_request(1, pattern, B, S, H, Hkv, width, text_len, &r)) return -1;
-  return bwd_workspace_floats(r, WS_CUS);
+  return bwd_workspace_floats(r);
 }
 
 int intra_model_mask_llm_bwd(int pattern, int S, int group_num, int window, int block, int offset, int n_sink,

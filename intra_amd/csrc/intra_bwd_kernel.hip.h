@@ -8,15 +8,17 @@
 //   P = exp(scale * S - lse),  dV = P^T dO,  dP = dO V^T,  dS = P o (dP - D),  D_i = dO_i . O_i,
 //   dQ = scale * dS K,  dK = scale * dS^T Q.
 //
-// One template serves the three results.  A workgroup owns 256 / HP "rows" (queries for dQ, keys
-// for dK and dV; 32 per wavefront, held as MFMA B operands in registers like Q in the forward
-// kernel) and streams the "columns" that see them through LDS in tiles of 64 (K and V rows for
-// dQ, Q and dO rows of every query head of the group for dK / dV) through three slots.  Per 32
+// One template serves the three results, dQ in one launch and dK with dV in another.  A workgroup
+// owns 256 / HP queries or 128 keys ("rows"; 32 per wavefront, held as MFMA B operands in registers
+// like Q in the forward kernel) and streams the "columns" that see them through LDS in tiles of 64
+// (K and V rows for dQ, Q and dO rows of every query head of the group for dK / dV).  Per 32
 // columns a wavefront forms the scores S^T = C1 R1^T and dP^T = C2 R2^T, turns them into the
 // weights (P or dS), packed to bf16 straight from the accumulators, and adds X^T W^T to its
 // accumulators, X being the K, Q or dO tile read with transposing LDS reads - the data flow of
 // the forward kernel without the online softmax.
 #pragma once
+#include <type_traits>
+
 #include "intra_bwd_maps.h"
 #include "intra_kernel.hip.h"
 
@@ -35,16 +37,25 @@ __device__ __forceinline__ void static_for(F&& f) {
   }
 }
 
-enum BwdMode : int { BWD_DQ = 0, BWD_DK = 1, BWD_DV = 2, BWD_DKV = 3 };
+enum BwdMode : int { BWD_DQ = 0, BWD_DKV = 1 };
 constexpr int bwd_waves(int mode) { return mode == BWD_DKV ? 4 : 8; }
+
+// Workgroups of one row map in a launch
+struct BwdGrid {
+  int n_rblocks;       // row blocks per set
+  int hgroups;         // ratio / HP (dQ only)
+  int items_per_pair;  // n_rblocks * hgroups
+  int bundle;          // pairs of one XCD that are worked on together
+  int blocks;          // workgroups, a multiple of 8
+};
 
 struct BParams {
   const uint16_t *q, *k, *v, *o, *dout;  // bf16 (B, S, heads, 128)
   const float* lse;                      // (B, H, S): ln sum exp(scale * q.k) from the forward pass
-  float* dsum;                           // (B, H, S) workspace: -D = -rowsum(dO o O), written by dQ, read by dK
+  float* dsum;                           // (B, H, S) workspace: -D = -rowsum(dO o O), written by dQ, read by dK / dV
   float* l2;                             // (B, H, S) workspace: lse * log2(e), written by dQ, read by dK / dV
   uint16_t *dq, *dk, *dv;
-  float* part;  // partial sums of the sink pass: (chunk, batch, kv head, sink, 128) fp32
+  float* part;  // partial sums of the leading keys, dk then dv: (chunk, batch, kv head, key, 128) fp32
   // element strides: batch, row (token), head
   int64_t q_bs, q_rs, q_hs, k_bs, k_rs, k_hs, v_bs, v_rs, v_hs, o_bs, o_rs, o_hs, do_bs, do_rs, do_hs;
   int64_t dq_bs, dq_rs, dq_hs, dk_bs, dk_rs, dk_hs, dv_bs, dv_rs, dv_hs;
@@ -53,10 +64,9 @@ struct BParams {
   IntraGeom geom;
   float scale;       // softmax scale
   float scale_log2;  // scale * log2(e)
-  int n_rblocks;     // row blocks per set
-  int hgroups;       // ratio / HP (dQ only)
-  int items_per_pair;  // n_rblocks * hgroups
-  int bundle;        // pairs of one XCD that are worked on together
+  BwdGrid grid;      // the launch's row map
+  BwdGrid lead;      // the leading keys that share the launch (blocks == 0: none)
+  int lead_first;    // their workgroups come before the others
 };
 
 constexpr int BWD_SLOT = 2 * FTILE + 512;  // two tiles and 2 x 64 column scalars
@@ -69,20 +79,18 @@ __device__ __forceinline__ void dma_dwords(const void* gsrc, uint32_t lds_addr) 
   asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dword %0, off" : : "v"(gsrc), "s"(lds_addr) : "memory");
 }
 
-// RMAP: row map (intra_bwd_maps.h).  PARTIAL: the results are partial sums over the set's columns,
-// written as fp32 to p.part instead of bf16 to dk / dv (sink pass).
+// The work of one workgroup, number `block` of the grid `g`.  RMAP: row map (intra_bwd_maps.h).
+// PARTIAL: where there are several sets, the results are partial sums over the set's columns, written
+// as fp32 to p.part instead of bf16 to dk / dv (leading keys).
 //
 // MFMA layout (v_mfma_f32_16x16x32_bf16, as in the forward kernel): a block of 32 columns times the
 // wavefront's 32 rows is 2 x 2 tiles [ct][rt] with 4 k-steps; lane (l16 = lane % 16, g4 = lane / 16)
 // holds columns 16*ct + 4*g4 .. +3 of row 16*rt + l16.  The packed weights of a row tile are the B
 // operand of the accumulation, whose 32-column reduction is numbered slot s of lane quarter g4 =
 // column 16*(s/4) + 4*g4 + s%4; the transposing reads of the X tile follow that numbering.
-template <class RMAP, int MODE, int HP, bool PARTIAL = false>
-__global__ __launch_bounds__(bwd_waves(MODE) * 64) void intra_bwd_kernel(const BParams p) {
+template <class RMAP, int MODE, int HP, bool PARTIAL>
+__device__ __forceinline__ void bwd_rows(const BParams& p, const BwdGrid& g, const int block, unsigned char* const smem) {
   constexpr int NW = bwd_waves(MODE);
-  constexpr bool HAS_DP = MODE != BWD_DV;                    // forms dP and dS
-  constexpr bool HAS_V = MODE == BWD_DV || MODE == BWD_DKV;  // accumulates dV (weights P)
-  static_assert(!(MODE == BWD_DKV && PARTIAL), "the partial sums of the sink pass come from the separate modes");
   constexpr bool ROWS_ARE_QUERIES = MODE == BWD_DQ;
   constexpr int POS = ROWS_ARE_QUERIES ? NW * 32 / HP : NW * 32;  // rows per row block (of one head)
 
@@ -90,8 +98,6 @@ __global__ __launch_bounds__(bwd_waves(MODE) * 64) void intra_bwd_kernel(const B
   // its ring is one slot deeper and a tile has two steps to land; the column scalars travel the same
   // way (every wavefront requests those of 16 columns) instead of through registers.
   constexpr bool DEEP = MODE == BWD_DKV;
-  constexpr bool TWO_STAGES = MODE == BWD_DKV || MODE == BWD_DQ;  // P and dS = P * dP formed apart
-  __shared__ __attribute__((aligned(1024))) unsigned char smem[bwd_ring_slots(MODE) * BWD_SLOT];
   const uint32_t lds_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)smem;
 
   const int tid = threadIdx.x;
@@ -106,17 +112,17 @@ __global__ __launch_bounds__(bwd_waves(MODE) * 64) void intra_bwd_kernel(const B
   // `bundle` pairs - as few as fill its 32 CUs - so that the workgroups running together stream the
   // same few megabytes of columns through the XCD's L2; within a bundle the row blocks with the
   // most columns come first (the last query blocks for dQ, the first key blocks for dK / dV).
-  const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
-  const int per_bundle = p.bundle * p.items_per_pair;
+  const int xcd = block & 7, slot = block >> 3;
+  const int per_bundle = g.bundle * g.items_per_pair;
   const int bun = slot / per_bundle, rem = slot - bun * per_bundle;
-  const int heavy = rem / p.bundle;
+  const int heavy = rem / g.bundle;
   const int nbh = p.B * p.Hkv;
-  const int pair = (bun * p.bundle + (rem - heavy * p.bundle)) * 8 + xcd;
+  const int pair = (bun * g.bundle + (rem - heavy * g.bundle)) * 8 + xcd;
   if (pair >= RMAP::num_sets(p.geom) * nbh) return;
   int hg = 0, rblk = heavy;
   if (ROWS_ARE_QUERIES) {
-    hg = heavy % p.hgroups;
-    rblk = p.n_rblocks - 1 - heavy / p.hgroups;
+    hg = heavy % g.hgroups;
+    rblk = g.n_rblocks - 1 - heavy / g.hgroups;
   }
   const int set = pair / nbh;
   const int bh = pair % nbh;
@@ -192,7 +198,7 @@ __global__ __launch_bounds__(bwd_waves(MODE) * 64) void intra_bwd_kernel(const B
 #pragma unroll
     for (int ks = 0; ks < 4; ++ks) {
       r1f[rt][ks] = *reinterpret_cast<const bf16x8*>(a1 + ks * 32);
-      if (HAS_DP) r2f[rt][ks] = *reinterpret_cast<const bf16x8*>(a2 + ks * 32);
+      r2f[rt][ks] = *reinterpret_cast<const bf16x8*>(a2 + ks * 32);
     }
     if (ROWS_ARE_QUERIES) {
       // D = dO . O of the row: this lane's 32 head dims, then the rest from the other three lanes of the row
@@ -334,24 +340,6 @@ __global__ __launch_bounds__(bwd_waves(MODE) * 64) void intra_bwd_kernel(const B
       dma_dwords(p.dsum + (batch * p.ds_bs + hcol * p.ds_hs + pos), lds_base + slot_off + 2 * FTILE + 256);
     }
   };
-  // column scalars of a step (dK / dV): wavefront 0 fetches lse * log2(e) and -D of its 64 columns
-  float sc_l = 0.f, sc_d = 0.f;
-  auto fetch_scalars = [&](const Cursor& cu) {
-    if (!ROWS_ARE_QUERIES && !DEEP && wave == 0) {
-      const int c = im_min(cb + cu.tile * BN + lane, n_cols - 1);
-      const int64_t pos = col_pos(c);
-      const int hcol = kvh * p.ratio + cu.head;
-      sc_l = p.l2[batch * p.ds_bs + hcol * p.ds_hs + pos];
-      if (HAS_DP) sc_d = p.dsum[batch * p.ds_bs + hcol * p.ds_hs + pos];
-    }
-  };
-  auto put_scalars = [&](int slot_off) {
-    if (!ROWS_ARE_QUERIES && !DEEP && wave == 0) {
-      float* sc = reinterpret_cast<float*>(smem + slot_off + 2 * FTILE);
-      sc[lane] = sc_l;
-      sc[64 + lane] = sc_d;
-    }
-  };
   // Three tile slots: while step t works on its tile, the tile of step t+1 has landed (the scores
   // of its first block are formed at the end of step t) and the tile of step t+2 is in flight.
   Cursor cur{ROWS_ARE_QUERIES ? 0 : ntiles - 1, 0};  // step being computed
@@ -361,8 +349,6 @@ __global__ __launch_bounds__(bwd_waves(MODE) * 64) void intra_bwd_kernel(const B
   for (int t = 0; t < (DEEP ? 3 : 2) && t < n_steps; ++t) {
     load_tile(ld, t * BWD_SLOT);
     if (DEEP) load_scalars(ld, t * BWD_SLOT);
-    fetch_scalars(ld);
-    put_scalars(t * BWD_SLOT);
     advance(ld);
   }
   // The deep ring's barriers leave requests in flight.  The row operands are ordinary loads the
@@ -380,13 +366,12 @@ __global__ __launch_bounds__(bwd_waves(MODE) * 64) void intra_bwd_kernel(const B
   for (int t = 0; t < 4; ++t) s_cur[t >> 1][t & 1] = zero4;
   bool have = false;  // s_cur and fr hold what a previous block prepared for the one that comes next
   // One slot is one MFMA; an LDS operand serves two consecutive slots (the two row tiles).
-  constexpr int NFRAG = MODE == BWD_DV ? 16 : MODE == BWD_DKV ? 32 : 24;  // LDS operands per block
-  constexpr int LA = MODE == BWD_DK ? 4 : MODE == BWD_DQ ? 6 : 8;  // operands between the request of one and its use
+  constexpr int NFRAG = MODE == BWD_DKV ? 32 : 24;  // LDS operands per block
+  constexpr int LA = MODE == BWD_DKV ? 8 : 6;       // operands between the request of one and its use
   static_assert(NFRAG % LA == 0, "a block must leave the ring where the next block expects it");
-  // slot of the first weight stage and slots from one stage to the next; BWD_DKV: of the dS stages
-  // (its P stages run in slots 5 .. 15, in front of the dV accumulation)
-  constexpr int WS = MODE == BWD_DV ? 4 : MODE == BWD_DKV ? 22 : 16;
-  constexpr int WSTEP = MODE == BWD_DV ? 1 : MODE == BWD_DKV ? 3 : 2;
+  // slot of the first dS stage and slots from one stage to the next (the P stages run while dP accumulates)
+  constexpr int WS = MODE == BWD_DKV ? 22 : 16;
+  constexpr int WSTEP = MODE == BWD_DKV ? 3 : 2;
   bf16x8 fr[LA];
 #pragma unroll
   for (int i = 0; i < LA; ++i) fr[i] = bf16x8{};
@@ -406,7 +391,6 @@ __global__ __launch_bounds__(bwd_waves(MODE) * 64) void intra_bwd_kernel(const B
       }
     } else if (t + 2 < n_steps) {
       load_tile(ld, slot2);
-      fetch_scalars(ld);
       advance(ld);
     }
 #pragma unroll
@@ -431,12 +415,11 @@ __global__ __launch_bounds__(bwd_waves(MODE) * 64) void intra_bwd_kernel(const B
       } else {
         masked = !block_unmasked(wb, kpre, sb_lo);
       }
-      // Hand-scheduled.  dQ / dK: slots 0-15 dP of this block, 16-31 the scores of the next block,
-      // 32-47 the accumulation; dV: 0-15 scores of the next block, 16-31 the accumulation.  LDS
+      // Hand-scheduled.  dQ: slots 0-15 dP of this block, 16-31 the scores of the next block, 32-47 the
+      // accumulation; dK / dV: dP, the dV accumulation, the next scores, the dK accumulation.  LDS
       // operand f (slots 2f, 2f+1) is requested LA operands earlier into a ring of LA fragments,
-      // across block and step boundaries (both following blocks have landed); the weights of
-      // element pair u are formed in slot WS + WSTEP * u, after dP has drained and before the
-      // accumulation needs them.  sched_barrier keeps the compiler from regrouping the slots.
+      // across block and step boundaries (both following blocks have landed); dS of element pair u is
+      // formed in slot WS + WSTEP * u, after dP has drained and before the accumulation needs it.  sched_barrier keeps the compiler from regrouping the slots.
       auto fetch = [&](int f) {
         const int here = blk * FBLOCK32;  // the block inside the step's slot
         // rows of the block that follows in this order, at tile `which` of its slot
@@ -450,18 +433,12 @@ __global__ __launch_bounds__(bwd_waves(MODE) * 64) void intra_bwd_kernel(const B
           if (f < 32) return vread_b(here, f - 24);          // Q^T: dK accumulation
           return next_rows(1, f - 32);
         }
-        if (MODE == BWD_DV) {
-          if (f < 8) return next_rows(0, f);
-          if (f < 16) return vread_b(here + FTILE, f - 8);
-          return blk == 0 ? kread_b(kb1, 0, f - 16) : kread_b(kb1, FBLOCK32, f - 16);  // the block after the next
-        }
         if (f < 8) return kread_b(kb0, here + FTILE, f);
         if (f < 16) return next_rows(0, f - 8);
         if (f < 24) return vread_b(here, f - 16);
         return next_rows(1, f - 24);
       };
-      const float* sc = DEEP ? reinterpret_cast<const float*>(smem + (sb0 + 128 * blk))
-                             : reinterpret_cast<const float*>(smem + slot0 + 2 * FTILE) + 32 * blk + 4 * g4;
+      const float* sc = reinterpret_cast<const float*>(smem + (sb0 + 128 * blk));
       // scalars of the block that follows in this order
       const float* scn = blk == 0 ? sc + 32 : reinterpret_cast<const float*>(smem + sb1);
       if (!have) {  // first block of a run: nothing was prepared by a previous block
@@ -497,12 +474,11 @@ __global__ __launch_bounds__(bwd_waves(MODE) * 64) void intra_bwd_kernel(const B
       floatx4 dp[2][2], s_next[2][2];
       bf16x8 wp[2];
       bf16x8 wp_p[MODE == BWD_DKV ? 2 : 1];   // BWD_DKV: the weights P (wp holds dS)
-      floatx4 pf[TWO_STAGES ? 2 : 1][2];       // P before rounding, for dS
-      floatx4 l4_[2], d4_[2];  // column scalars of the lane's columns, per column tile
-      // (BWD_DKV keeps them across blocks: a block reads those of the next one in its last slots)
-      floatx4 (&l4)[2] = MODE == BWD_DKV ? l4_keep : l4_;
-      floatx4 (&d4)[2] = MODE == BWD_DKV ? d4_keep : d4_;
-      // weights of pair u = 4 * rt + 2 * ct + h (columns 16 * ct + 4 * g4 + 2 * h, + 1 of row tile rt): P, or dS = P * (dP - D)
+      floatx4 pf[2][2];                        // P before rounding, for dS
+      // BWD_DKV: scalars of the lane's columns, per column tile (a block reads those of the next one in its last slots)
+      floatx4 (&l4)[2] = l4_keep;
+      floatx4 (&d4)[2] = d4_keep;
+      // P of pair u = 4 * rt + 2 * ct + h (columns 16 * ct + 4 * g4 + 2 * h, + 1 of row tile rt)
       auto stage = [&](int u) {
         const int rt = u >> 2, ct = (u >> 1) & 1, h = u & 1;
         float w[2];
@@ -510,28 +486,18 @@ __global__ __launch_bounds__(bwd_waves(MODE) * 64) void intra_bwd_kernel(const B
         for (int v = 0; v < 2; ++v) {
           const int e = 2 * h + v;
           const float l = ROWS_ARE_QUERIES ? L2_row[rt] : l4[ct][e];
-          float x = __builtin_amdgcn_exp2f(__builtin_fmaf(s_cur[ct][rt][e], c2, -l));
-          if (MODE == BWD_DK) x *= dp[ct][rt][e] + d4[ct][e];
-          w[v] = x;
+          w[v] = __builtin_amdgcn_exp2f(__builtin_fmaf(s_cur[ct][rt][e], c2, -l));
         }
-        if (MODE == BWD_DQ) {  // (the P stage: dS follows when dP is there)
-          pf[ct][rt][2 * h] = w[0];
-          pf[ct][rt][2 * h + 1] = w[1];
-          return;
-        }
-        floatx2 f2 = {w[0], w[1]};
-        bf16x2 h2 = __builtin_convertvector(f2, bf16x2);
-        if (MODE == BWD_DKV) {  // (this is the P stage: keep the unrounded values for dS)
-          pf[ct][rt][2 * h] = w[0];
-          pf[ct][rt][2 * h + 1] = w[1];
+        pf[ct][rt][2 * h] = w[0];  // (unrounded, for dS, which follows when dP is there)
+        pf[ct][rt][2 * h + 1] = w[1];
+        if (MODE == BWD_DKV) {
+          floatx2 f2 = {w[0], w[1]};
+          bf16x2 h2 = __builtin_convertvector(f2, bf16x2);
           wp_p[rt][4 * ct + 2 * h] = h2[0];
           wp_p[rt][4 * ct + 2 * h + 1] = h2[1];
-        } else {
-          wp[rt][4 * ct + 2 * h] = h2[0];
-          wp[rt][4 * ct + 2 * h + 1] = h2[1];
         }
       };
-      // dQ and BWD_DKV: dS = P * (dP - D) of pair u; the accumulators of dP start from -D
+      // dS = P * (dP - D) of pair u; the accumulators of dP start from -D
       auto stage_ds = [&](int u) {
         const int rt = u >> 2, ct = (u >> 1) & 1, h = u & 1;
         floatx2 f2 = {pf[ct][rt][2 * h] * dp[ct][rt][2 * h], pf[ct][rt][2 * h + 1] * dp[ct][rt][2 * h + 1]};  // (dP started from -D)
@@ -545,17 +511,14 @@ __global__ __launch_bounds__(bwd_waves(MODE) * 64) void intra_bwd_kernel(const B
         constexpr int i = decltype(slot_c)::value;
         constexpr int f = i >> 1, rt = i & 1;
         const bf16x8 a = fr[f % LA];
-        if (MODE == BWD_DKV) {
-          if (f < 8) dp[f & 1][rt] = mfma(a, r2f[rt][f >> 1], f < 2 ? d4[f & 1] : dp[f & 1][rt]);  // from -D of the tile's columns
-          else if (f < 16) acc_v[f - 8][rt] = mfma(a, wp_p[rt], acc_v[f - 8][rt]);
-          else if (f < 24) s_next[f & 1][rt] = mfma(a, r1f[rt][(f - 16) >> 1], f < 18 ? zero4 : s_next[f & 1][rt]);
+        if constexpr (MODE == BWD_DKV) {
+          if constexpr (f < 8) dp[f & 1][rt] = mfma(a, r2f[rt][f >> 1], f < 2 ? d4[f & 1] : dp[f & 1][rt]);  // from -D of the tile's columns
+          else if constexpr (f < 16) acc_v[f - 8][rt] = mfma(a, wp_p[rt], acc_v[f - 8][rt]);
+          else if constexpr (f < 24) s_next[f & 1][rt] = mfma(a, r1f[rt][(f - 16) >> 1], f < 18 ? zero4 : s_next[f & 1][rt]);
           else acc[f - 24][rt] = mfma(a, wp[rt], acc[f - 24][rt]);
-        } else if (MODE == BWD_DV) {
-          if (f < 8) s_next[f & 1][rt] = mfma(a, r1f[rt][f >> 1], f < 2 ? zero4 : s_next[f & 1][rt]);
-          else acc[f - 8][rt] = mfma(a, wp[rt], acc[f - 8][rt]);
         } else {
-          if (f < 8) dp[f & 1][rt] = mfma(a, r2f[rt][f >> 1], f < 2 ? (ROWS_ARE_QUERIES ? nd_row[rt] : zero4) : dp[f & 1][rt]);  // dQ: from -D of the row
-          else if (f < 16) s_next[f & 1][rt] = mfma(a, r1f[rt][(f - 8) >> 1], f < 10 ? zero4 : s_next[f & 1][rt]);
+          if constexpr (f < 8) dp[f & 1][rt] = mfma(a, r2f[rt][f >> 1], f < 2 ? nd_row[rt] : dp[f & 1][rt]);  // from -D of the row
+          else if constexpr (f < 16) s_next[f & 1][rt] = mfma(a, r1f[rt][(f - 8) >> 1], f < 10 ? zero4 : s_next[f & 1][rt]);
           else acc[f - 16][rt] = mfma(a, wp[rt], acc[f - 16][rt]);
         }
         if (rt == 1) fr[f % LA] = fetch(f + LA);
@@ -567,19 +530,9 @@ __global__ __launch_bounds__(bwd_waves(MODE) * 64) void intra_bwd_kernel(const B
           if (i == 56) d4[1] = *reinterpret_cast<const floatx4*>(scn + 64 + 16);
           if (i >= 5 && i < 16 && (i - 5) % 3 != 2) stage((i - 5) - (i - 5) / 3);  // slots 5, 6, 8, 9, 11, 12, 14, 15
           if (i >= WS && (i - WS) % WSTEP == 0 && (i - WS) / WSTEP < 8) stage_ds((i - WS) / WSTEP);
-        } else {
-        if (!ROWS_ARE_QUERIES) {  // column scalars, four slots ahead of the first weight stage
-          if (i == WS - 4) l4[0] = *reinterpret_cast<const floatx4*>(sc);
-          if (i == WS - 3) l4[1] = *reinterpret_cast<const floatx4*>(sc + 16);
-          if (MODE == BWD_DK && i == WS - 2) d4[0] = *reinterpret_cast<const floatx4*>(sc + 64);
-          if (MODE == BWD_DK && i == WS - 1) d4[1] = *reinterpret_cast<const floatx4*>(sc + 64 + 16);
-        }
-        // dQ: P while dP is formed (the scores are then free for those of the next block), dS behind it
-        if (MODE == BWD_DQ && i < 16 && i % 2 == 0) stage(i / 2);
-        if (i >= WS && (i - WS) % WSTEP == 0 && (i - WS) / WSTEP < 8) {
-          if (MODE == BWD_DQ) stage_ds((i - WS) / WSTEP);
-          else stage((i - WS) / WSTEP);
-        }
+        } else {  // P while dP is formed (the scores are then free for those of the next block), dS behind it
+          if (i < 16 && i % 2 == 0) stage(i / 2);
+          if (i >= WS && (i - WS) % WSTEP == 0 && (i - WS) / WSTEP < 8) stage_ds((i - WS) / WSTEP);
         }
         __builtin_amdgcn_sched_barrier(0);
       });
@@ -587,7 +540,6 @@ __global__ __launch_bounds__(bwd_waves(MODE) * 64) void intra_bwd_kernel(const B
       for (int t4 = 0; t4 < 4; ++t4) s_cur[t4 >> 1][t4 & 1] = s_next[t4 >> 1][t4 & 1];
       have = true;
     }
-    if (t + 2 < n_steps) put_scalars(slot2);
     advance(cur);
     const int ts = slot0;
     slot0 = slot1;
@@ -618,29 +570,33 @@ __global__ __launch_bounds__(bwd_waves(MODE) * 64) void intra_bwd_kernel(const B
 
   // ---------------------------------------------------------------- scale, round, store
   if (!wave_active) return;
-  const float f = MODE == BWD_DV ? 1.f : p.scale;
-  if (PARTIAL) {
-    // fp32 partial sums: part[((set * B + batch) * Hkv + kvh) * n_rows + row][128]
+  if (PARTIAL && RMAP::num_sets(p.geom) > 1) {
+    // fp32 partial sums: part[((set * B + batch) * Hkv + kvh) * n_rows + row][128] of dk, behind all of them those of dv
+    const int64_t all = (int64_t)RMAP::num_sets(p.geom) * nbh * n_rows * 128;
 #pragma unroll
     for (int rt = 0; rt < 2; ++rt)
       if (row_valid[rt]) {
         float* prow = p.part + ((((int64_t)set * p.B + batch) * p.Hkv + kvh) * n_rows + row[rt]) * 128 + 4 * g4;
 #pragma unroll
-        for (int dt = 0; dt < 8; ++dt) *reinterpret_cast<floatx4*>(prow + 16 * dt) = acc[dt][rt] * f;
+        for (int dt = 0; dt < 8; ++dt) {
+          *reinterpret_cast<floatx4*>(prow + 16 * dt) = acc[dt][rt] * p.scale;
+          *reinterpret_cast<floatx4*>(prow + all + 16 * dt) = acc_v[MODE == BWD_DKV ? dt : 0][rt];
+        }
       }
     return;
   }
   // The four lanes of a row hold head dims 4 * g4 .. + 3 of every 16-dim tile; a lane quarter and
   // its neighbour trade 8 bytes per tile pair so that each lane owns the whole 16-byte chunk
   // 4 * m + 2 * (g4 % 2) + g4 / 2 of its row.
+  enum { TO_DQ, TO_DK, TO_DV };
   auto store_rows = [&](const floatx4 (&a)[8][2], int what, float factor) {
 #pragma unroll
     for (int rt = 0; rt < 2; ++rt) {
       const bool keep = row_valid[rt] && map.store((int)rpos[rt]);
       uint16_t* orow;
       const int cofs = (2 * (g4 & 1) + (g4 >> 1)) * 8;
-      if (what == BWD_DQ) orow = p.dq + (batch * p.dq_bs + rpos[rt] * p.dq_rs + hq * p.dq_hs + cofs);
-      else if (what == BWD_DK) orow = p.dk + (batch * p.dk_bs + rpos[rt] * p.dk_rs + kvh * p.dk_hs + cofs);
+      if (what == TO_DQ) orow = p.dq + (batch * p.dq_bs + rpos[rt] * p.dq_rs + hq * p.dq_hs + cofs);
+      else if (what == TO_DK) orow = p.dk + (batch * p.dk_bs + rpos[rt] * p.dk_rs + kvh * p.dk_hs + cofs);
       else orow = p.dv + (batch * p.dv_bs + rpos[rt] * p.dv_rs + kvh * p.dv_hs + cofs);
 #pragma unroll
       for (int m = 0; m < 4; ++m) {
@@ -671,31 +627,65 @@ __global__ __launch_bounds__(bwd_waves(MODE) * 64) void intra_bwd_kernel(const B
     }
   };
   if constexpr (MODE == BWD_DKV) {
-    store_rows(acc, BWD_DK, p.scale);
-    store_rows(acc_v, BWD_DV, 1.f);
+    store_rows(acc, TO_DK, p.scale);
+    store_rows(acc_v, TO_DV, 1.f);
   } else {
-    store_rows(acc, MODE, f);
+    store_rows(acc, TO_DQ, p.scale);
   }
 }
 
-// Adds up the partial sums of the sink pass over the chunks and writes the sink rows of dk or dv:
-// one thread per (batch, kv head, sink, 4 head dims).
-__global__ void intra_bwd_sink_reduce(const float* part, int n_chunks, int B, int Hkv, int ns, uint16_t* out,
-                                      int64_t o_bs, int64_t o_rs, int64_t o_hs) {
+struct NoLeadingKeys {};
+
+// One launch: the workgroups of RMAP and, with LEAD, those of the keys that every (later) query sees
+// (KeyRowsLeading).  The leading keys are few rows with very many columns, whose launch of its own
+// had one thin round of workgroups; here the rest of the GPU works on the other keys meanwhile.  The
+// longer kind of workgroup comes first, so that the short ones fill the last round.  Against two
+// launches of their own, dK (three products) and dV (two) with 8 wavefronts: a training step with 64
+// sinks 551 -> 505 us (window 575, S = 8192, 32 / 8 heads), 870 -> 817 us (block Scatter G = 2,
+// S = 6000), image Scatter 1024^2 at 24 heads 339 -> 327 us.
+template <class RMAP, int MODE, int HP, class LEAD = NoLeadingKeys>
+__global__ __launch_bounds__(bwd_waves(MODE) * 64) void intra_bwd_kernel(const BParams p) {
+  __shared__ __attribute__((aligned(1024))) unsigned char smem[bwd_ring_slots(MODE) * BWD_SLOT];
+  int block = blockIdx.x;
+  if constexpr (!std::is_same_v<LEAD, NoLeadingKeys>) {
+    const int lead_block = block - (p.lead_first ? 0 : p.grid.blocks);
+    if (lead_block >= 0 && lead_block < p.lead.blocks) {
+      bwd_rows<LEAD, MODE, HP, true>(p, p.lead, lead_block, smem);
+      return;
+    }
+    if (p.lead_first) block -= p.lead.blocks;
+  }
+  bwd_rows<RMAP, MODE, HP, false>(p, p.grid, block, smem);
+}
+
+// Adds up the partial sums of the leading keys over the chunks and writes their rows of dk
+// (blockIdx.y == 0) or dv: one thread per (batch, kv head, key, 4 head dims).  Eight chunks are
+// requested before the first is added: a chain of one load per chunk is latency only.
+__global__ void intra_bwd_lead_reduce(const BParams p, int n_chunks, int ns) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int64_t total = (int64_t)B * Hkv * ns * 32;
-  if (i >= total) return;
+  const int64_t rows = (int64_t)p.B * p.Hkv * ns;
+  if (i >= rows * 32) return;
   const int d4 = (int)(i & 31);
-  const int64_t row = i >> 5;  // (batch * Hkv + kvh) * ns + sink
+  const int64_t row = i >> 5;  // (batch * Hkv + kvh) * ns + key
+  const float* part = p.part + ((blockIdx.y ? n_chunks * rows : 0) + row) * 128 + 4 * d4;
   floatx4 s = {0.f, 0.f, 0.f, 0.f};
-  for (int c = 0; c < n_chunks; ++c) s += *reinterpret_cast<const floatx4*>(part + ((int64_t)c * B * Hkv * ns + row) * 128 + 4 * d4);
-  const int sink = (int)(row % ns);
+  int c = 0;
+  for (; c + 8 <= n_chunks; c += 8) {
+    floatx4 v[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) v[k] = *reinterpret_cast<const floatx4*>(part + (c + k) * rows * 128);
+#pragma unroll
+    for (int k = 0; k < 8; ++k) s += v[k];
+  }
+  for (; c < n_chunks; ++c) s += *reinterpret_cast<const floatx4*>(part + c * rows * 128);
+  const int key = (int)(row % ns);
   const int64_t bh = row / ns;
-  const int kvh = (int)(bh % Hkv), batch = (int)(bh / Hkv);
+  const int kvh = (int)(bh % p.Hkv), batch = (int)(bh / p.Hkv);
   floatx2 a = {s[0], s[1]}, b = {s[2], s[3]};
   uint32_t lo = __builtin_bit_cast(uint32_t, __builtin_convertvector(a, bf16x2));
   uint32_t hi = __builtin_bit_cast(uint32_t, __builtin_convertvector(b, bf16x2));
-  uint16_t* o = out + (batch * o_bs + sink * o_rs + kvh * o_hs + 4 * d4);
+  uint16_t* o = blockIdx.y ? p.dv + (batch * p.dv_bs + key * p.dv_rs + kvh * p.dv_hs + 4 * d4)
+                           : p.dk + (batch * p.dk_bs + key * p.dk_rs + kvh * p.dk_hs + 4 * d4);
   *reinterpret_cast<uint2*>(o) = make_uint2(lo, hi);
 }
 

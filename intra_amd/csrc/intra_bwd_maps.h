@@ -5,12 +5,13 @@
 // whose sets number queries and keys alike, the query range of a key follows from the forward
 // map's monotone bounds by bisection (KeyRowsOf).  Block Scatter with a stripe offset and the
 // per-token window have their own inverse maps.  Keys that are sinks are seen by every later
-// query of every set; they are left out of those maps' results (`store`) and get a pass of their
-// own (KeyRowsSinks), split over chunks of queries whose partial sums a small kernel adds up.
+// query of every set; they are left out of those maps' results (`store`) and get row blocks of
+// their own in the same launch (KeyRowsSinks), split over chunks of queries whose partial sums a
+// small kernel adds up.
 //
 // Interface (host and device):
 //   static num_sets(ge), max_rows(ge)      grid size: sets per (batch, kv head), rows of the largest
-//   RowMap(ge, set, r0)                    r0: first row of the row block (rows r0 .. r0+255 at most)
+//   RowMap(ge, set, r0)                    r0: first row of the row block (rows r0 .. r0+255 at most, keys r0 .. r0+127)
 //   n_rows(), n_cols()
 //   row_pos(t), col_pos(c)                 token positions
 //   lo(t), hi(t)                           row t meets the columns lo..hi (and those below kpre())
@@ -172,7 +173,7 @@ struct KeyRowsWindowSink {
 
 // The first ge.ns keys (LLM sinks; the text keys of the image patterns) against the queries of the
 // whole sequence: every later query (CAUSAL) or every query.  set = chunk of ge.sink_chunk queries
-// (chosen by the host so that the pass fills the GPU).  The results are partial sums over the chunk.
+// (leading_chunk on the host).  With several chunks the results are partial sums over the chunk.
 template <bool CAUSAL>
 struct KeyRowsLeading {
   int S, ns, c0, c1;

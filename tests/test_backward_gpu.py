@@ -163,6 +163,14 @@ def test_window_sink_grads(S, kw, B, H, Hkv):
     run_case("llm/window_sink", "window_sink", B, S, H, Hkv, **kw)
 
 
+# The sinks' queries are cut into chunks whose partial sums are added up: one chunk (written without
+# partial sums, by few queries or by many kv heads), more sinks than a row block of 128, and more
+# chunks than the summation requests at once (8), with a remainder.
+@pytest.mark.parametrize("B,S,H,Hkv,n_sink", [(1, 130, 2, 1, 4), (1, 390, 4, 2, 130), (2, 320, 82, 82, 3), (1, 2700, 4, 1, 129)])
+def test_sink_chunks_grads(B, S, H, Hkv, n_sink):
+    run_case("llm/window_sink", "window_sink", B, S, H, Hkv, window=70, n_sink=n_sink)
+
+
 def test_model_setting_at_16k():
     run_case("llm/block_scatter", "block_scatter", 1, 16384, 8, 2, group_num=2, block=256, offset=1, n_sink=64)
     run_case("llm/window_sink", "window_sink", 1, 16384, 8, 2, window=575, n_sink=64)
