@@ -747,7 +747,7 @@ int run_bwd(int domain, const void* q, const void* k, const void* v, const void*
       return rc ? rc : run_bwd_lead_reduce(p, ns, st);
     case MAP_IMG_GATHER0:  // grid keys against the grid queries around them, plus their group's text queries
       if ((rc = run_bwd_dq<MapImgGather0>(p, sh.hp, st))) return rc;
-      if ((rc = run_bwd_keys_lead<intra::KeyRowsImgWindow, intra::KeyRowsText>(p, 3 * (intra::KeyRowsImgWindow::RUN + 2) * 64, st))) return rc;
+      if ((rc = run_bwd_keys_lead<intra::KeyRowsImgWindow, intra::KeyRowsText>(p, 8 * 64, st))) return rc;
       if ((rc = run_bwd_keys<intra::KeyRowsImgGroup<true>>(p, st))) return rc;
       return run_bwd_lead_reduce(p, ns, st);
     default: return fail(INTRA_ERR_UNSUPPORTED, "backward: no kernels for this pattern");

@@ -227,36 +227,58 @@ struct KeyRowsImgGroup {
 
 // Grid keys of image Gather 0 against the grid queries.  Query patch (R, C) sees the grid rows
 // win(R) .. win(R)+15 and columns win(C) .. win(C)+15, so key (r, c) is seen by whole 8x8 query
-// patches: those with win(R) <= r < win(R)+16 and win(C) <= c < win(C)+16 - at most 3 x 3 of them
-// around its own patch, 2 x 2 for a key away from the borders.  A set is a run of up to 4 key
-// patches of one patch row (rows: patch after patch; inside a patch its upper 4 grid rows, then
-// its lower 4, so that a wavefront owns 4 x 8 keys with few query patches between them); its
-// columns are the query patches R-1 .. R+1 x C0-1 .. C0+4 (cut at the borders), 64 queries each,
-// so a block of 32 columns lies inside one query patch and a row meets it entirely or not at all.
+// patches: those with win(R) <= r < win(R)+16 and win(C) <= c < win(C)+16 - 2 x 2 of them away from
+// the borders, and the same ones along 8 grid rows that start half a patch (4 rows) above a patch.
+// A set is one row block of up to 128 keys, its columns are the query patches that see any of them,
+// 64 queries each, so a block of 32 columns lies inside one patch and a row meets all of it or
+// nothing.  Sets, in this order:
+//  * for every s = 1 .. W/8 - 1 and every 16 columns: the 8 grid rows from 8s - 4 on, 32 rows of
+//    the set (a wavefront) being 8 x 4 keys, which all see the same 2 x 2 patches: 2 x 4 patches of
+//    columns, of which a wavefront works on its 4;
+//  * the 4 upper and the 4 lower grid rows, 32 columns of the grid at a time: one patch row of columns.
+// Cutting along patches instead (2 patches of keys, 3 x 4 patches of columns, 6 of them a
+// wavefront's own) streams a quarter more columns, runs of 4 patches half as many again.
 struct KeyRowsImgWindow {
-  int W, T, np, Rk, Ck0, pk, Rlo, Clo, nR, nC;
-  static constexpr int RUN = 4;
-  static IM_HD int runs_per_row(const IntraGeom& ge) { return (ge.width / 8 + RUN - 1) / RUN; }
-  static IM_HD int num_sets(const IntraGeom& ge) { return (ge.width / 8) * runs_per_row(ge); }
-  static IM_HD int max_rows(const IntraGeom& ge) { return 64 * im_min(RUN, ge.width / 8); }
+  int W, T, np, r0, c0, kw, wcols, Rlo, Clo, nR, nC;
+  static IM_HD int mid_runs(const IntraGeom& ge) { return (ge.width + 15) / 16; }
+  static IM_HD int edge_runs(const IntraGeom& ge) { return (ge.width + 31) / 32; }
+  static IM_HD int num_sets(const IntraGeom& ge) { return (ge.width / 8 - 1) * mid_runs(ge) + 2 * edge_runs(ge); }
+  static IM_HD int max_rows(const IntraGeom&) { return 128; }
+  // first and last patch (along either axis) whose window covers grid row / column x
+  static IM_HD int first_patch(int x) { return x <= 15 ? 0 : (x - 4) >> 3; }
+  static IM_HD int last_patch(int x, int W) { return x >= W - 16 ? W / 8 - 1 : (x + 4) >> 3; }
   IM_HD KeyRowsImgWindow(const IntraGeom& ge, int set, int) {
     W = ge.width;
     T = ge.text_len;
     np = W / 8;
-    const int rpr = runs_per_row(ge);
-    Rk = set / rpr;
-    Ck0 = (set - Rk * rpr) * RUN;
-    pk = im_min(RUN, np - Ck0);
-    Rlo = im_max(Rk - 1, 0);
-    Clo = im_max(Ck0 - 1, 0);
-    nR = im_min(Rk + 1, np - 1) - Rlo + 1;
-    nC = im_min(Ck0 + pk, np - 1) - Clo + 1;
+    const int mid = mid_runs(ge), n_mid = (np - 1) * mid;
+    int height, cols;
+    if (set < n_mid) {
+      const int s = set / mid;
+      r0 = 8 * s + 4;
+      c0 = (set - s * mid) * 16;
+      height = 8;
+      cols = im_min(16, W - c0);
+      wcols = 4;
+    } else {
+      const int edge = edge_runs(ge), e = (set - n_mid) / edge;
+      r0 = e * (W - 4);
+      c0 = (set - n_mid - e * edge) * 32;
+      height = 4;
+      cols = im_min(32, W - c0);
+      wcols = 8;
+    }
+    kw = cols / wcols;
+    Rlo = first_patch(r0);
+    Clo = first_patch(c0);
+    nR = last_patch(r0 + height - 1, W) - Rlo + 1;
+    nC = last_patch(c0 + cols - 1, W) - Clo + 1;
   }
-  IM_HD int n_rows() const { return 64 * pk; }
+  IM_HD int n_rows() const { return 32 * kw; }
   IM_HD int n_cols() const { return 64 * nR * nC; }
   IM_HD int kpre() const { return 0; }
-  IM_HD int key_r(int t) const { return 8 * Rk + ((t >> 3) & 7); }
-  IM_HD int key_c(int t) const { return 8 * (Ck0 + (t >> 6)) + (t & 7); }
+  IM_HD int key_r(int t) const { return r0 + (t & 31) / wcols; }
+  IM_HD int key_c(int t) const { return c0 + (t >> 5) * wcols + (t & (wcols - 1)); }
   IM_HD int row_pos(int t) const { return T + key_r(t) * W + key_c(t); }
   IM_HD int col_pos(int c) const {
     const int pi = c >> 6, u = c & 63;
