@@ -2,8 +2,8 @@
 //
 // dQ: rows are the queries of a set and columns its keys - the forward index map as it is
 // (QueryRows).  dK / dV: rows are keys and columns the queries that see them.  For the patterns
-// whose sets number queries and keys alike, the query range of a key follows from the forward
-// map's monotone bounds by bisection (KeyRowsOf).  Block Scatter with a stripe offset and the
+// whose sets number queries and keys alike, the query range of a key starts at the key and ends
+// where the forward map says (KeyRowsOf).  Block Scatter with a stripe offset and the
 // per-token window have their own inverse maps.  Keys that are sinks are seen by every later
 // query of every set; they are left out of those maps' results (`store`) and get row blocks of
 // their own in the same launch (KeyRowsSinks), split over chunks of queries whose partial sums a
@@ -46,9 +46,11 @@ struct QueryRows {
   IM_HD bool sees(int, int) const { return true; }
 };
 
-// Keys of a set whose queries and keys carry the same numbering (LLM Scatter, Gather 1, window,
-// block Scatter without offset): key r is seen by the queries from the first one whose upper key
-// bound reaches r to the last one whose lower key bound does not exceed r; both are monotone in r.
+// Keys of a set whose queries and keys carry the same numbering and whose queries see keys up to
+// their own (LLM Scatter, Gather 1, window): key r is seen by the queries from r to the last one
+// whose lower key bound does not exceed r (last_query).  In closed form: a search for the two ends
+// in the forward map's bounds was six chains of a dozen dependent iterations in front of the first
+// request of every workgroup.
 template <class MAP>
 struct KeyRowsOf {
   MAP m;
@@ -60,25 +62,8 @@ struct KeyRowsOf {
   IM_HD int kpre() const { return 0; }
   IM_HD int row_pos(int t) const { return m.kpos(t); }
   IM_HD int col_pos(int c) const { return m.qpos(c); }
-  IM_HD int lo(int r) const {  // first tq with min(khi(tq), nk-1) >= r
-    int a = 0, b = m.nq();
-    const int kmax = m.nk() - 1;
-    while (a < b) {
-      const int mid = (a + b) >> 1;
-      if (im_min(m.khi(mid), kmax) >= r) b = mid;
-      else a = mid + 1;
-    }
-    return a;
-  }
-  IM_HD int hi(int r) const {  // last tq with klo(tq) <= r
-    int a = -1, b = m.nq() - 1;
-    while (a < b) {
-      const int mid = (a + b + 1) >> 1;
-      if (m.klo(mid) <= r) a = mid;
-      else b = mid - 1;
-    }
-    return a;
-  }
+  IM_HD int lo(int r) const { return r; }
+  IM_HD int hi(int r) const { return im_min(m.last_query(r), m.nq() - 1); }
   IM_HD int block_lo(int r0, int) const { return lo(r0); }
   IM_HD int block_hi(int, int r1) const { return hi(r1); }
   IM_HD bool store(int) const { return true; }

@@ -122,6 +122,7 @@ struct MapLlmScatter {
   IM_HD int kpos(int t) const { return t * G + g; }
   IM_HD int klo(int) const { return 0; }
   IM_HD int khi(int tq) const { return tq; }
+  IM_HD int last_query(int) const { return n - 1; }
 };
 
 // ------------------------------------- LLM gather1: segments of G tokens, segment s in group s % G
@@ -150,6 +151,7 @@ struct MapLlmGather1 {
   IM_HD int kpos(int t) const { return qpos(t); }
   IM_HD int klo(int) const { return 0; }
   IM_HD int khi(int tq) const { return tq; }
+  IM_HD int last_query(int) const { return n - 1; }
 };
 
 // -------------------------- LLM window: 64-query blocks see themselves plus window-64 earlier tokens
@@ -169,6 +171,8 @@ struct MapLlmWindow {
   IM_HD int kpos(int t) const { return t; }
   IM_HD int klo(int tq) const { return im_max((tq & ~63) - lookback, 0); }
   IM_HD int khi(int tq) const { return tq; }
+  // last query whose klo does not exceed key
+  IM_HD int last_query(int key) const { return (int)im_min64((((int64_t)key + lookback) & ~(int64_t)63) + 63, S - 1); }
 };
 
 // ------------- image scatter: 8 groups, grid token (r, c) in group (r%2)*4 + c%4, text chunk j rides
