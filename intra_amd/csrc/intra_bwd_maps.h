@@ -223,8 +223,9 @@ struct KeyRowsImgGroup {
 //  * the 4 upper and the 4 lower grid rows, 32 columns of the grid at a time: one patch row of columns.
 // Cutting along patches instead (2 patches of keys, 3 x 4 patches of columns, 6 of them a
 // wavefront's own) streams a quarter more columns, runs of 4 patches half as many again.
+// No division by a variable past the constructor: col_pos and sees run several times per step.
 struct KeyRowsImgWindow {
-  int W, T, np, r0, c0, kw, wcols, Rlo, Clo, nR, nC;
+  int W, T, np, r0, c0, kw, wshift, Rlo, Clo, nR, nC, inv_nC;
   static IM_HD int mid_runs(const IntraGeom& ge) { return (ge.width + 15) / 16; }
   static IM_HD int edge_runs(const IntraGeom& ge) { return (ge.width + 31) / 32; }
   static IM_HD int num_sets(const IntraGeom& ge) { return (ge.width / 8 - 1) * mid_runs(ge) + 2 * edge_runs(ge); }
@@ -244,30 +245,32 @@ struct KeyRowsImgWindow {
       c0 = (set - s * mid) * 16;
       height = 8;
       cols = im_min(16, W - c0);
-      wcols = 4;
+      wshift = 2;  // 4 columns of keys per wavefront
     } else {
       const int edge = edge_runs(ge), e = (set - n_mid) / edge;
       r0 = e * (W - 4);
       c0 = (set - n_mid - e * edge) * 32;
       height = 4;
       cols = im_min(32, W - c0);
-      wcols = 8;
+      wshift = 3;
     }
-    kw = cols / wcols;
+    kw = cols >> wshift;
     Rlo = first_patch(r0);
     Clo = first_patch(c0);
     nR = last_patch(r0 + height - 1, W) - Rlo + 1;
     nC = last_patch(c0 + cols - 1, W) - Clo + 1;
+    inv_nC = 65535 / nC + 1;
   }
   IM_HD int n_rows() const { return 32 * kw; }
   IM_HD int n_cols() const { return 64 * nR * nC; }
   IM_HD int kpre() const { return 0; }
-  IM_HD int key_r(int t) const { return r0 + (t & 31) / wcols; }
-  IM_HD int key_c(int t) const { return c0 + (t >> 5) * wcols + (t & (wcols - 1)); }
+  IM_HD int patch_row(int pi) const { return (pi * inv_nC) >> 16; }  // pi / nC (exact: pi * nC < 2^16)
+  IM_HD int key_r(int t) const { return r0 + ((t & 31) >> wshift); }
+  IM_HD int key_c(int t) const { return c0 + ((t >> 5) << wshift) + (t & ((1 << wshift) - 1)); }
   IM_HD int row_pos(int t) const { return T + key_r(t) * W + key_c(t); }
   IM_HD int col_pos(int c) const {
     const int pi = c >> 6, u = c & 63;
-    const int ri = pi / nC;
+    const int ri = patch_row(pi);
     return T + (8 * (Rlo + ri) + (u >> 3)) * W + 8 * (Clo + pi - ri * nC) + (u & 7);
   }
   IM_HD int lo(int) const { return 0; }
@@ -277,7 +280,7 @@ struct KeyRowsImgWindow {
   IM_HD bool store(int) const { return true; }
   static constexpr bool kBlockPredicate = true, kAccumulate = false;
   IM_HD bool sees(int t, int c) const {
-    const int pi = c >> 6, ri = pi / nC;
+    const int pi = c >> 6, ri = patch_row(pi);
     const int wr = MapImgPatch::win_start(Rlo + ri, np), wc = MapImgPatch::win_start(Clo + pi - ri * nC, np);
     const int r = key_r(t), cc = key_c(t);
     return r >= wr && r < wr + 16 && cc >= wc && cc < wc + 16;
