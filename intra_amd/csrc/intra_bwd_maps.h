@@ -213,22 +213,29 @@ struct KeyRowsImgGroup {
 // Grid keys of image Gather 0 against the grid queries.  Query patch (R, C) sees the grid rows
 // win(R) .. win(R)+15 and columns win(C) .. win(C)+15, so key (r, c) is seen by whole 8x8 query
 // patches: those with win(R) <= r < win(R)+16 and win(C) <= c < win(C)+16 - 2 x 2 of them away from
-// the borders, and the same ones along 8 grid rows that start half a patch (4 rows) above a patch.
+// the borders, and the same ones for all keys of an 8 x 8 square that starts half a patch (4 rows and
+// 4 columns) from the patch grid.
 // A set is one row block of up to 128 keys, its columns are the query patches that see any of them,
 // 64 queries each, so a block of 32 columns lies inside one patch and a row meets all of it or
-// nothing.  Sets, in this order:
-//  * for every s = 1 .. W/8 - 1 and every 16 columns: the 8 grid rows from 8s - 4 on, 32 rows of
-//    the set (a wavefront) being 8 x 4 keys, which all see the same 2 x 2 patches: 2 x 4 patches of
-//    columns, of which a wavefront works on its 4;
+// nothing.  32 rows of the set (a wavefront) are a cell of 8 x 4 keys, half such a square, or of 4 x 8.
+// Sets, in this order:
+//  * for every s = 1 .. W/8 - 1 the 8 grid rows from 8s - 4 on: the 12 leftmost columns (a border cell
+//    and a square), then 16 columns at a time (two squares: 2 x 3 patches of columns, of which a
+//    wavefront works on its 4), up to the last 4 columns;
+//  * the last 4 columns of these rows, 4 cells below each other at a time;
 //  * the 4 upper and the 4 lower grid rows, 32 columns of the grid at a time: one patch row of columns.
-// Cutting along patches instead (2 patches of keys, 3 x 4 patches of columns, 6 of them a
-// wavefront's own) streams a quarter more columns, runs of 4 patches half as many again.
+// (Where W is an odd number of patches the runs of 16 columns end with one of 12 that holds the last 4.)
+// Runs of 16 columns from 0 on stream 2 x 4 patches instead of 2 x 3, cells cut along the patches of
+// the rows as well 3 x 4.
 // No division by a variable past the constructor: col_pos and sees run several times per step.
 struct KeyRowsImgWindow {
-  int W, T, np, r0, c0, kw, wshift, Rlo, Clo, nR, nC, inv_nC;
-  static IM_HD int mid_runs(const IntraGeom& ge) { return (ge.width + 15) / 16; }
+  int W, T, np, r0, c0, kw, wshift, wrows, wcols, Rlo, Clo, nR, nC, inv_nC;
+  static IM_HD int mid_runs(const IntraGeom& ge) { return (ge.width + 8) / 16; }
+  static IM_HD int side_runs(const IntraGeom& ge) { return ge.width % 16 == 0 ? (ge.width / 8 + 2) / 4 : 0; }
   static IM_HD int edge_runs(const IntraGeom& ge) { return (ge.width + 31) / 32; }
-  static IM_HD int num_sets(const IntraGeom& ge) { return (ge.width / 8 - 1) * mid_runs(ge) + 2 * edge_runs(ge); }
+  static IM_HD int num_sets(const IntraGeom& ge) {
+    return (ge.width / 8 - 1) * mid_runs(ge) + side_runs(ge) + 2 * edge_runs(ge);
+  }
   static IM_HD int max_rows(const IntraGeom&) { return 128; }
   // first and last patch (along either axis) whose window covers grid row / column x
   static IM_HD int first_patch(int x) { return x <= 15 ? 0 : (x - 4) >> 3; }
@@ -237,24 +244,39 @@ struct KeyRowsImgWindow {
     W = ge.width;
     T = ge.text_len;
     np = W / 8;
-    const int mid = mid_runs(ge), n_mid = (np - 1) * mid;
+    const int mid = mid_runs(ge), n_mid = (np - 1) * mid, side = side_runs(ge);
     int height, cols;
     if (set < n_mid) {
-      const int s = set / mid;
+      const int s = set / mid, run = set - s * mid;
       r0 = 8 * s + 4;
-      c0 = (set - s * mid) * 16;
+      c0 = run == 0 ? 0 : 16 * run - 4;
       height = 8;
-      cols = im_min(16, W - c0);
-      wshift = 2;  // 4 columns of keys per wavefront
+      cols = run == 0 ? 12 : im_min(16, W - c0);
+      kw = cols >> 2;
+      wshift = 2;
+      wrows = 0;
+      wcols = 4;
+    } else if (set < n_mid + side) {
+      const int s = 4 * (set - n_mid);
+      r0 = 8 * s + 4;
+      c0 = W - 4;
+      kw = im_min(4, np - 1 - s);
+      height = 8 * kw;
+      cols = 4;
+      wshift = 2;
+      wrows = 8;
+      wcols = 0;
     } else {
-      const int edge = edge_runs(ge), e = (set - n_mid) / edge;
+      const int edge = edge_runs(ge), i = set - n_mid - side, e = i >= edge ? 1 : 0;
       r0 = e * (W - 4);
-      c0 = (set - n_mid - e * edge) * 32;
+      c0 = (i - e * edge) * 32;
       height = 4;
       cols = im_min(32, W - c0);
+      kw = cols >> 3;
       wshift = 3;
+      wrows = 0;
+      wcols = 8;
     }
-    kw = cols >> wshift;
     Rlo = first_patch(r0);
     Clo = first_patch(c0);
     nR = last_patch(r0 + height - 1, W) - Rlo + 1;
@@ -265,8 +287,8 @@ struct KeyRowsImgWindow {
   IM_HD int n_cols() const { return 64 * nR * nC; }
   IM_HD int kpre() const { return 0; }
   IM_HD int patch_row(int pi) const { return (pi * inv_nC) >> 16; }  // pi / nC (exact: pi * nC < 2^16)
-  IM_HD int key_r(int t) const { return r0 + ((t & 31) >> wshift); }
-  IM_HD int key_c(int t) const { return c0 + ((t >> 5) << wshift) + (t & ((1 << wshift) - 1)); }
+  IM_HD int key_r(int t) const { return r0 + (t >> 5) * wrows + ((t & 31) >> wshift); }
+  IM_HD int key_c(int t) const { return c0 + (t >> 5) * wcols + (t & ((1 << wshift) - 1)); }
   IM_HD int row_pos(int t) const { return T + key_r(t) * W + key_c(t); }
   IM_HD int col_pos(int c) const {
     const int pi = c >> 6, u = c & 63;
