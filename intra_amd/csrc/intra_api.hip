@@ -616,8 +616,17 @@ template <class R, class LEAD>
 int run_bwd_keys_lead(intra::BParams p, int64_t longest, hipStream_t stream) {
   p.grid = bwd_grid<R>(p, KEY_ROWS, 1);
   p.lead = bwd_grid<LEAD>(p, KEY_ROWS, 1);
-  p.lead_first = p.geom.sink_chunk > longest;
+  // (their work counts half where both halves of a workgroup share the columns)
+  p.lead_first = p.geom.sink_chunk / (intra::alternates<LEAD> ? 2 : 1) > longest;
   return launch_bwd<R, intra::BWD_DKV, 1, LEAD>(p, stream);
+}
+
+// The same with the sinks as leading keys.  Up to 64 of them fill two of a workgroup's four wavefronts:
+// the other two then take every other block of columns.
+template <class R>
+int run_bwd_keys_sinks(const intra::BParams& p, int64_t longest, hipStream_t stream) {
+  return p.geom.ns <= 64 ? run_bwd_keys_lead<R, intra::KeyRowsFewSinks>(p, longest, stream)
+                         : run_bwd_keys_lead<R, intra::KeyRowsSinks>(p, longest, stream);
 }
 
 // The leading keys' rows of dk and dv from their partial sums (one chunk: written by the launch itself)
@@ -734,12 +743,12 @@ int run_bwd(int domain, const void* q, const void* k, const void* v, const void*
     case MAP_LLM_BLOCK_SCATTER:
       if ((rc = run_bwd_dq<MapLlmBlockScatter>(p, sh.hp, st))) return rc;
       if (ns == 0) return run_bwd_keys<intra::KeyRowsBlockScatter>(p, st);
-      rc = run_bwd_keys_lead<intra::KeyRowsBlockScatter, intra::KeyRowsSinks>(p, intra::KeyRowsBlockScatter::max_rows(p.geom), st);
+      rc = run_bwd_keys_sinks<intra::KeyRowsBlockScatter>(p, intra::KeyRowsBlockScatter::max_rows(p.geom), st);
       return rc ? rc : run_bwd_lead_reduce(p, ns, st);
     case MAP_LLM_WINDOW_SINK:
       if ((rc = run_bwd_dq<MapLlmWindowSink>(p, sh.hp, st))) return rc;
       if (ns == 0) return run_bwd_keys<intra::KeyRowsWindowSink>(p, st);
-      rc = run_bwd_keys_lead<intra::KeyRowsWindowSink, intra::KeyRowsSinks>(p, (int64_t)p.geom.window + KEY_ROWS, st);
+      rc = run_bwd_keys_sinks<intra::KeyRowsWindowSink>(p, (int64_t)p.geom.window + KEY_ROWS, st);
       return rc ? rc : run_bwd_lead_reduce(p, ns, st);
     case MAP_IMG_SCATTER:  // grid keys against their group's queries, text keys against all queries
       if ((rc = run_bwd_dq<MapImgScatter>(p, sh.hp, st))) return rc;
@@ -782,6 +791,11 @@ float* noalloc_scratch() {
 // Host walk of the backward decomposition: count[q * S + k] += 1 for every (query, key) pair that
 // the dK / dV launches (key-row maps with their `store` rule, then the sink pass) multiply.
 template <class R>
+bool row_is_real(const R& m, int t) {
+  if constexpr (intra::alternates<R>) return m.real(t);
+  else return true;
+}
+template <class R>
 void bwd_walk(const IntraGeom& ge, uint8_t* count) {
   const int S = ge.S, rows = KEY_ROWS;
   for (int set = 0; set < R::num_sets(ge); ++set)
@@ -790,11 +804,12 @@ void bwd_walk(const IntraGeom& ge, uint8_t* count) {
       const int r1 = std::min(r0 + rows, m.n_rows()) - 1;
       for (int t = r0; t <= r1; ++t) {
         const int kp = m.row_pos(t);
-        if (!m.store(kp)) continue;
+        if (!m.store(kp) || !row_is_real(m, t)) continue;
         const int lo = std::max(m.lo(t), m.block_lo(r0, r1));
         const int hi = std::min(std::min(m.hi(t), m.n_cols() - 1), m.block_hi(r0, r1));
         for (int c = lo; c <= hi; ++c)
-          if (!R::kBlockPredicate || m.sees(t, c & ~31)) ++count[(size_t)m.col_pos(c) * S + kp];
+          if ((!R::kBlockPredicate || m.sees(t, c & ~31)) && (!intra::alternates<R> || ((c - m.block_lo(r0, r1)) >> 5 & 1) == (t >> 6)))
+            ++count[(size_t)m.col_pos(c) * S + kp];
       }
     }
 }
@@ -813,7 +828,8 @@ int model_mask_bwd(const Request& r, uint8_t* count) {
   }
   if (leading_keys(r) > 0) {
     set_leading_chunks(sh.geom, r.S, 1, 1, leading_keys(r));
-    bwd_walk<intra::KeyRowsSinks>(sh.geom, count);
+    if (sh.geom.ns <= 64) bwd_walk<intra::KeyRowsFewSinks>(sh.geom, count);
+    else bwd_walk<intra::KeyRowsSinks>(sh.geom, count);
   }
   return INTRA_OK;
 }

@@ -98,6 +98,7 @@ __device__ __forceinline__ void bwd_rows(const BParams& p, const BwdGrid& g, con
   // its ring is one slot deeper and a tile has two steps to land; the column scalars travel the same
   // way (every wavefront requests those of 16 columns) instead of through registers.
   constexpr bool DEEP = MODE == BWD_DKV;
+  constexpr bool ALT = alternates<RMAP>;  // wavefronts 0, 1 and 2, 3 share rows and take turns at the 32-column blocks
   const uint32_t lds_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)smem;
 
   const int tid = threadIdx.x;
@@ -155,6 +156,7 @@ __device__ __forceinline__ void bwd_rows(const BParams& p, const BwdGrid& g, con
     row[rt] = im_min(wr0 + 16 * rt + l16, r1);
     lo_l[rt] = map.lo(row[rt]);
     hi_l[rt] = map.hi(row[rt]);
+    if constexpr (ALT) row_valid[rt] = row_valid[rt] && map.real(row[rt]);
     rpos[rt] = map.row_pos(row[rt]);
   }
   // union and intersection of the ranges of the wavefront's rows
@@ -407,6 +409,7 @@ __device__ __forceinline__ void bwd_rows(const BParams& p, const BwdGrid& g, con
     }
 #pragma unroll
     for (int blk = 0; blk < 2; ++blk) {
+      if (ALT && blk != wave >> 1) continue;  // (the block that follows is the same one of the next tile)
       const int jb = 2 * cur.tile + blk;
       if (jb < jb_lo || jb > jb_hi) {
         have = false;
@@ -436,6 +439,7 @@ __device__ __forceinline__ void bwd_rows(const BParams& p, const BwdGrid& g, con
         const int here = blk * FBLOCK32;  // the block inside the step's slot
         // rows of the block that follows in this order, at tile `which` of its slot
         auto next_rows = [&](int which, int ff) {
+          if (ALT) return kread_b(kb1, here + which * FTILE, ff);
           return blk == 0 ? kread_b(kb0, FBLOCK32 + which * FTILE, ff) : kread_b(kb1, which * FTILE, ff);
         };
         if (MODE == BWD_DKV) {
@@ -452,7 +456,7 @@ __device__ __forceinline__ void bwd_rows(const BParams& p, const BwdGrid& g, con
       };
       const float* sc = reinterpret_cast<const float*>(smem + (sb0 + 128 * blk));
       // scalars of the block that follows in this order
-      const float* scn = blk == 0 ? sc + 32 : reinterpret_cast<const float*>(smem + sb1);
+      const float* scn = ALT ? reinterpret_cast<const float*>(smem + (sb1 + 128 * blk)) : blk == 0 ? sc + 32 : reinterpret_cast<const float*>(smem + sb1);
       if (!have) {  // first block of a run: nothing was prepared by a previous block
         if (MODE == BWD_DKV) {
           l4_keep[0] = *reinterpret_cast<const floatx4*>(sc);
@@ -582,13 +586,37 @@ __device__ __forceinline__ void bwd_rows(const BParams& p, const BwdGrid& g, con
 
   // ---------------------------------------------------------------- scale, round, store
   if (!wave_active) return;
+  if constexpr (ALT) {  // wavefronts 2, 3 hand their sums to 0, 1 through the ring, which nobody reads any more
+    static_assert(MODE == BWD_DKV && NW == 4 && 2 * 32 * 64 * 16 <= bwd_ring_slots(MODE) * BWD_SLOT, "64 KB");
+    floatx4* const hand = reinterpret_cast<floatx4*>(smem) + (wave & 1) * 32 * 64 + lane;
+    __syncthreads();
+    if (wave >= 2)
+#pragma unroll
+      for (int dt = 0; dt < 8; ++dt)
+#pragma unroll
+        for (int rt = 0; rt < 2; ++rt) {
+          hand[(2 * dt + rt) * 64] = acc[dt][rt];
+          hand[(16 + 2 * dt + rt) * 64] = acc_v[dt][rt];
+        }
+    __syncthreads();
+    if (wave >= 2) return;
+#pragma unroll
+    for (int dt = 0; dt < 8; ++dt)
+#pragma unroll
+      for (int rt = 0; rt < 2; ++rt) {
+        acc[dt][rt] += hand[(2 * dt + rt) * 64];
+        acc_v[dt][rt] += hand[(16 + 2 * dt + rt) * 64];
+      }
+  }
   if (PARTIAL && RMAP::num_sets(p.geom) > 1) {
-    // fp32 partial sums: part[((set * B + batch) * Hkv + kvh) * n_rows + row][128] of dk, behind all of them those of dv
-    const int64_t all = (int64_t)RMAP::num_sets(p.geom) * nbh * n_rows * 128;
+    // fp32 partial sums: part[((set * B + batch) * Hkv + kvh) * keys + row][128] of dk, behind all of them those of dv
+    int keys = n_rows;
+    if constexpr (ALT) keys = map.ns;
+    const int64_t all = (int64_t)RMAP::num_sets(p.geom) * nbh * keys * 128;
 #pragma unroll
     for (int rt = 0; rt < 2; ++rt)
       if (row_valid[rt]) {
-        float* prow = p.part + ((((int64_t)set * p.B + batch) * p.Hkv + kvh) * n_rows + row[rt]) * 128 + 4 * g4;
+        float* prow = p.part + ((((int64_t)set * p.B + batch) * p.Hkv + kvh) * keys + row[rt]) * 128 + 4 * g4;
 #pragma unroll
         for (int dt = 0; dt < 8; ++dt) {
           *reinterpret_cast<floatx4*>(prow + 16 * dt) = acc[dt][rt] * p.scale;

@@ -21,10 +21,16 @@
 //                                          row and 32-column block (first column c) whether the row
 //                                          meets the block - all of it or nothing
 //   kAccumulate                            the results are added to rows another pass has written
+//   alternates<RowMap>                     rows 0..63 and 64..127 are the same keys twice over: the
+//                                          first meet the even blocks of 32 columns, the second the odd
+//                                          ones, and the results of the two are added
 #pragma once
 #include "intra_maps.h"
 
 namespace intra {
+
+template <class RMAP>
+constexpr bool alternates = false;
 
 template <class MAP>
 struct QueryRows {
@@ -159,32 +165,39 @@ struct KeyRowsWindowSink {
 // The first ge.ns keys (LLM sinks; the text keys of the image patterns) against the queries of the
 // whole sequence: every later query (CAUSAL) or every query.  set = chunk of ge.sink_chunk queries
 // (leading_chunk on the host).  With several chunks the results are partial sums over the chunk.
-template <bool CAUSAL>
+// TWICE: for 64 leading keys at most, where a row block's second two wavefronts would have no rows.
+// A step of such a workgroup then takes the time of one block instead of two: training steps with 64
+// sinks, 32 / 8 heads, 504 -> 488 us (window 575, S = 8192), 830 -> 820 us (block Scatter G = 2, S = 6000).
+template <bool CAUSAL, bool TWICE = false>
 struct KeyRowsLeading {
   int S, ns, c0, c1;
   static IM_HD int num_sets(const IntraGeom& ge) { return (ge.S + ge.sink_chunk - 1) / ge.sink_chunk; }
-  static IM_HD int max_rows(const IntraGeom& ge) { return im_min(ge.ns, ge.S); }
+  static IM_HD int max_rows(const IntraGeom& ge) { return TWICE ? 128 : im_min(ge.ns, ge.S); }
   IM_HD KeyRowsLeading(const IntraGeom& ge, int set, int) {
     S = ge.S;
     ns = im_min(ge.ns, ge.S);
     c0 = set * ge.sink_chunk;
     c1 = im_min(c0 + ge.sink_chunk, S);
   }
-  IM_HD int n_rows() const { return ns; }
+  IM_HD int n_rows() const { return TWICE ? 128 : ns; }
   IM_HD int n_cols() const { return S; }
   IM_HD int kpre() const { return 0; }
-  IM_HD int row_pos(int t) const { return t; }
+  IM_HD int row_pos(int t) const { return TWICE ? im_min(t & 63, ns - 1) : t; }  // (rows past the last key repeat it)
+  IM_HD bool real(int t) const { return !TWICE || (t & 63) < ns; }
   IM_HD int col_pos(int c) const { return c; }
-  IM_HD int lo(int t) const { return CAUSAL ? im_max(t, c0) : c0; }
+  IM_HD int lo(int t) const { return CAUSAL ? im_max(row_pos(t), c0) : c0; }
   IM_HD int hi(int) const { return c1 - 1; }
-  IM_HD int block_lo(int r0, int) const { return CAUSAL ? im_max(r0, c0) : c0; }
+  IM_HD int block_lo(int r0, int) const { return lo(r0); }
   IM_HD int block_hi(int, int) const { return c1 - 1; }
   IM_HD bool store(int) const { return true; }
   static constexpr bool kBlockPredicate = false, kAccumulate = false;
   IM_HD bool sees(int, int) const { return true; }
 };
 using KeyRowsSinks = KeyRowsLeading<true>;
+using KeyRowsFewSinks = KeyRowsLeading<true, true>;
 using KeyRowsText = KeyRowsLeading<false>;
+template <bool CAUSAL>
+constexpr bool alternates<KeyRowsLeading<CAUSAL, true>> = true;
 
 // Grid keys of group g of the image patterns (grid token (r, c) in group (r%2)*4 + c%4), against
 // the queries of Scatter set g: its text chunk, then (unless TEXT_COLS_ONLY) its grid tokens; every

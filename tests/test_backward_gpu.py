@@ -171,6 +171,14 @@ def test_sink_chunks_grads(B, S, H, Hkv, n_sink):
     run_case("llm/window_sink", "window_sink", B, S, H, Hkv, window=70, n_sink=n_sink)
 
 
+@pytest.mark.parametrize("S", [65, 190, 2100])  # one chunk of queries, a ragged one, several
+@pytest.mark.parametrize("n_sink", [1, 32, 33, 63, 64, 65])
+def test_sinks_of_half_a_row_block_grads(S, n_sink):
+    """Up to 64 sinks: two pairs of wavefronts share the keys and take turns at the blocks of 32 queries."""
+    run_case("llm/window_sink", "window_sink", 1, S, 4, 2, window=40, n_sink=n_sink)
+    run_case("llm/block_scatter", "block_scatter", 1, S, 2, 1, group_num=2, block=256, offset=1, n_sink=n_sink)
+
+
 def test_model_setting_at_16k():
     run_case("llm/block_scatter", "block_scatter", 1, 16384, 8, 2, group_num=2, block=256, offset=1, n_sink=64)
     run_case("llm/window_sink", "window_sink", 1, 16384, 8, 2, window=575, n_sink=64)
