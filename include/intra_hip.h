@@ -160,8 +160,8 @@ int intra_get_softmax_mode(void);
  *              entry do not matter
  * Patterns: all five of intra_llm_fwd_ex; INTRA_LLM_BLOCK_SCATTER with offset != 0 needs
  * block % 256 == 0, softmax_scale must not be 0; otherwise INTRA_ERR_UNSUPPORTED.  Launches on
- * hip_stream: dq, dk, dv, and with sinks four more for the sink rows of dk and dv; nothing is
- * allocated.  Accuracy: weights are rounded to bf16 before the second product, as in the forward
+ * hip_stream: dq, then dk and dv in one pass, and with sinks one more that adds up the partial sums
+ * of the sink rows; nothing is allocated.  Accuracy: weights are rounded to bf16 before the second product, as in the forward
  * pass, accumulation is fp32. */
 int intra_llm_bwd(const void* q, const void* k, const void* v, const void* o, const float* lse,
                   const void* dout, void* dq, void* dk, void* dv, float* workspace, int B, int S,

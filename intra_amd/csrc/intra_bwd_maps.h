@@ -164,7 +164,7 @@ struct KeyRowsWindowSink {
 
 // The first ge.ns keys (LLM sinks; the text keys of the image patterns) against the queries of the
 // whole sequence: every later query (CAUSAL) or every query.  set = chunk of ge.sink_chunk queries
-// (leading_chunk on the host).  With several chunks the results are partial sums over the chunk.
+// (set_leading_chunks on the host).  With several chunks the results are partial sums over the chunk.
 // TWICE: for 64 leading keys at most, where a row block's second two wavefronts would have no rows.
 // A step of such a workgroup then takes the time of one block instead of two: training steps with 64
 // sinks, 32 / 8 heads, 504 -> 488 us (window 575, S = 8192), 830 -> 820 us (block Scatter G = 2, S = 6000).
