@@ -47,7 +47,7 @@ int make_request(int domain, int pattern, int B, int S, int H, int Hkv, int arg0
   r->H = H;
   r->Hkv = Hkv;
   r->geom = IntraGeom{S, 1, 64, 16, 8, 0, 1, 1, 64, 0, 0};  // derived fields: geom_finish() in shape_for()
-  r->geom.sink_chunk = 1024;  // backward: set by set_leading_chunks() once the number of leading keys is known
+  r->geom.sink_chunk = 1024;  // backward: set by set_leading_chunk() once the number of leading keys is known
   if (domain == 0) {
     if (!extended && (pattern == INTRA_LLM_BLOCK_SCATTER || pattern == INTRA_LLM_WINDOW_SINK))
       return fail(INTRA_ERR_INVALID, "unknown LLM pattern id %d (0 scatter, 1 gather1, 4 window)", pattern);
@@ -584,30 +584,11 @@ int run_bwd_dq(intra::BParams p, int hp, hipStream_t stream) {
 
 // dK and dV over a key-row map: row blocks of 128 keys of one kv head, all query heads of its group
 // streamed past.
-constexpr int KEY_ROWS = intra::bwd_waves(intra::BWD_DKV) * 32;
+using intra::KEY_ROWS;
 template <class R>
 int run_bwd_keys(intra::BParams p, hipStream_t stream) {
   p.grid = bwd_grid<R>(p, KEY_ROWS, 1);
   return launch_bwd<R, intra::BWD_DKV, 1>(p, stream);
-}
-
-// Chunks of queries that the pass over the `ns` leading keys (LLM sinks, image text keys) is cut into,
-// and their length, a multiple of 64 and at least 128 (except for the last).  The workspace holds
-// fp32 sums of one result for about one 256-key row block per CU of a device of WS_CUS CUs; dk and
-// dv share that room, so half as many chunks have both.  (Twice the chunks would even out sinks
-// better and cost the text keys of an image twice the partial sums.)
-constexpr int WS_CUS = 320;
-int workspace_chunks(int S, int B, int Hkv, int ns) {
-  const int64_t row_wgs = (int64_t)B * Hkv * ((ns + 255) / 256);
-  int64_t chunks = std::max<int64_t>(1, WS_CUS / row_wgs);
-  chunks = std::min<int64_t>(chunks, std::max(1, S / 128));
-  const int64_t chunk = 64 * ((S + 64 * chunks - 1) / (64 * chunks));
-  return (int)((S + chunk - 1) / chunk);
-}
-void set_leading_chunks(IntraGeom& ge, int S, int B, int Hkv, int ns) {
-  const int64_t chunks = std::max(1, workspace_chunks(S, B, Hkv, ns) / 2);
-  ge.ns = ns;
-  ge.sink_chunk = (int)(64 * ((S + 64 * chunks - 1) / (64 * chunks)));
 }
 
 // dK and dV over a key-row map and, in the same launch, over the leading keys LEAD.
@@ -648,13 +629,19 @@ int leading_keys(const Request& r) {
   return 0;
 }
 
+void set_leading_chunk(IntraGeom& ge, int S, int B, int Hkv, int ns, int cus) {
+  ge.ns = ns;
+  ge.sink_chunk = intra::leading_chunk(S, B, Hkv, ns, cus);
+}
+constexpr int MODEL_CUS = 256;  // host-only walks of the decomposition: any value gives a valid split
+
 // floats of workspace: -D = -rowsum(dO o O) and lse * log2(e) per (batch, head, token), then the partial
 // sums of the leading keys
 int64_t bwd_dsum_floats(int B, int S, int H) { return ((int64_t)B * H * S + 3) & ~(int64_t)3; }
 int64_t bwd_workspace_floats(const Request& r) {
   int64_t n = 2 * bwd_dsum_floats(r.B, r.S, r.H);
   const int ns = leading_keys(r);
-  if (ns > 0) n += (int64_t)workspace_chunks(r.S, r.B, r.Hkv, ns) * r.B * r.Hkv * ns * 128;
+  if (ns > 0) n += (int64_t)intra::workspace_chunks(r.S, r.B, r.Hkv, ns) * r.B * r.Hkv * ns * 128;
   return n;
 }
 
@@ -726,7 +713,11 @@ int run_bwd(int domain, const void* q, const void* k, const void* v, const void*
   if (!shape_for(r, default_hp(H / Hkv), &sh)) return fail(INTRA_ERR_UNSUPPORTED, "no kernel shape for this request");
   p.geom = sh.geom;
   const int ns = leading_keys(r);
-  if (ns > 0) set_leading_chunks(p.geom, S, B, Hkv, ns);
+  if (ns > 0) {
+    const int cus = cu_count();
+    if (cus <= 0) return fail(INTRA_ERR_HIP, "cannot query the current device: %s", hipGetErrorString(hipGetLastError()));
+    set_leading_chunk(p.geom, S, B, Hkv, ns, cus);
+  }
   p.lead = intra::BwdGrid{};
   p.lead_first = 0;
   hipStream_t st = static_cast<hipStream_t>(stream);
@@ -827,7 +818,7 @@ int model_mask_bwd(const Request& r, uint8_t* count) {
     default: return fail(INTRA_ERR_UNSUPPORTED, "backward: no kernels for this pattern");
   }
   if (leading_keys(r) > 0) {
-    set_leading_chunks(sh.geom, r.S, 1, 1, leading_keys(r));
+    set_leading_chunk(sh.geom, r.S, 1, 1, leading_keys(r), MODEL_CUS);
     if (sh.geom.ns <= 64) bwd_walk<intra::KeyRowsFewSinks>(sh.geom, count);
     else bwd_walk<intra::KeyRowsSinks>(sh.geom, count);
   }
@@ -849,7 +840,7 @@ int model_mask_image_bwd(const Request& r, uint8_t* count) {
   Shape sh;
   if (!shape_for(r, 1, &sh)) return fail(INTRA_ERR_UNSUPPORTED, "no kernel shape for this request");
   IntraGeom ge = sh.geom;
-  set_leading_chunks(ge, r.S, 1, 1, ge.text_len);  // the text keys are the leading keys every query sees
+  set_leading_chunk(ge, r.S, 1, 1, ge.text_len, MODEL_CUS);  // the text keys are the leading keys every query sees
   if (r.kind == KIND_IMG_SCATTER) {
     bwd_walk<intra::KeyRowsImgGroup<false>>(ge, count);
   } else {

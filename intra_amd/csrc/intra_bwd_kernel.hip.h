@@ -39,6 +39,7 @@ __device__ __forceinline__ void static_for(F&& f) {
 
 enum BwdMode : int { BWD_DQ = 0, BWD_DKV = 1 };
 constexpr int bwd_waves(int mode) { return mode == BWD_DKV ? 4 : 8; }
+static_assert(bwd_waves(BWD_DKV) * 32 == KEY_ROWS, "keys of a row block");
 
 // Workgroups of one row map in a launch
 struct BwdGrid {

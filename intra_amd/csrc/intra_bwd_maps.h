@@ -29,6 +29,8 @@
 
 namespace intra {
 
+constexpr int KEY_ROWS = 128;  // keys of a row block of the dK / dV launch
+
 template <class RMAP>
 constexpr bool alternates = false;
 
@@ -162,9 +164,36 @@ struct KeyRowsWindowSink {
   IM_HD bool sees(int, int) const { return true; }
 };
 
+// Chunks of queries that the row blocks of the `ns` leading keys (LLM sinks, image text keys) are cut
+// into, and their length, a multiple of 64 and at least 128 (except for the last).  The workspace has
+// room for the fp32 sums of workspace_chunks chunks of one result - about one block of 256 keys per CU
+// of a device of WS_CUS CUs, so that its size does not depend on the device; dk and dv share it, so a
+// launch has half as many chunks at most.  Nor does it have more workgroups on leading keys than the
+// device has CUs: a few too many are a second round of the longest kind on a few CUs, which everything
+// else waits for.  With 288 - 320 workgroups on 256 CUs against 192 - 256 (training steps, us): image
+// Scatter 2048^2 at 12 heads 1211 -> 1164, at 6 heads 691 -> 657; Gather 0 at 24 heads 384 -> 361
+// (1024^2) and 1234 -> 1174 (2048^2); 256 sinks, 32 / 8 heads, S = 16384: window 575 1202 -> 1124,
+// block Scatter 4750 -> 4660.  (Slower: 1000 sinks at S = 3000, 336 -> 348, where 5 short chunks
+// behind the window's row blocks fill the rounds better than 4.)
+constexpr int WS_CUS = 320;
+inline int workspace_chunks(int S, int B, int Hkv, int ns) {
+  const int64_t row_wgs = (int64_t)B * Hkv * ((ns + 255) / 256);
+  int64_t chunks = WS_CUS / row_wgs > 1 ? WS_CUS / row_wgs : 1;
+  if (chunks > S / 128) chunks = im_max(1, S / 128);
+  const int64_t chunk = 64 * ((S + 64 * chunks - 1) / (64 * chunks));
+  return (int)((S + chunk - 1) / chunk);
+}
+inline int leading_chunk(int S, int B, int Hkv, int ns, int cus) {
+  const int64_t row_wgs = (int64_t)B * Hkv * ((ns + KEY_ROWS - 1) / KEY_ROWS);
+  int64_t chunks = workspace_chunks(S, B, Hkv, ns) / 2;
+  if (chunks > cus / row_wgs) chunks = cus / row_wgs;
+  if (chunks < 1) chunks = 1;
+  return (int)(64 * ((S + 64 * chunks - 1) / (64 * chunks)));
+}
+
 // The first ge.ns keys (LLM sinks; the text keys of the image patterns) against the queries of the
 // whole sequence: every later query (CAUSAL) or every query.  set = chunk of ge.sink_chunk queries
-// (set_leading_chunks on the host).  With several chunks the results are partial sums over the chunk.
+// (leading_chunk on the host).  With several chunks the results are partial sums over the chunk.
 // TWICE: for 64 leading keys at most, where a row block's second two wavefronts would have no rows.
 // A step of such a workgroup then takes the time of one block instead of two: training steps with 64
 // sinks, 32 / 8 heads, 504 -> 488 us (window 575, S = 8192), 830 -> 820 us (block Scatter G = 2, S = 6000).
