@@ -86,7 +86,8 @@ struct KeyRowsOf {
 // block are numbered [own block][those blocks], which needs the row block inside one key block
 // (block size a multiple of 256).  Sinks (positions < n_sink) are not stored here.
 struct KeyRowsBlockScatter {
-  int G, blk, gk, off, n, S, skip, a, kb, own_len, qb0, ncols;
+  int G, blk, gk, off, n, skip, a, own, ncols;
+  uint32_t own_pos, far_pos, far_step;  // position of the own block, of the first column behind it; skipped per further block
   FastDiv dBlk;
   static IM_HD int num_sets(const IntraGeom& ge) { return ge.G; }
   static IM_HD int max_rows(const IntraGeom& ge) { return MapLlmBlockScatter::max_nq(ge); }
@@ -94,18 +95,19 @@ struct KeyRowsBlockScatter {
     G = ge.G;
     blk = ge.blk;
     off = ge.off;
-    S = ge.S;
     dBlk = ge.dBlk;
     gk = set;
     skip = im_min(ge.ns, ge.S);
     n = MapLlmBlockScatter::group_size(ge, gk);
     a = (int)fd_div(r0, dBlk);
-    kb = a * G + gk;
-    own_len = im_max(0, im_min(blk, S - kb * blk));
-    qb0 = kb + G - off;
+    far_step = (uint32_t)(G - 1) * (uint32_t)blk;
     if (off == 0) {
+      own = 0;
+      own_pos = 0;
+      far_pos = (uint32_t)gk * (uint32_t)blk;
       ncols = n;
     } else {
+      const int S = ge.S, kb = a * G + gk, qb0 = kb + G - off;
       const int nbt = (int)fd_div(S + blk - 1, dBlk);  // blocks in the sequence, the last one maybe short
       int later = 0;
       if (qb0 < nbt) {
@@ -113,7 +115,10 @@ struct KeyRowsBlockScatter {
         const int last = qb0 + (cnt - 1) * G;
         later = (cnt - 1) * blk + im_min(blk, S - last * blk);
       }
-      ncols = own_len + later;
+      own = im_max(0, im_min(blk, S - kb * blk));
+      own_pos = (uint32_t)kb * (uint32_t)blk;
+      far_pos = (uint32_t)qb0 * (uint32_t)blk;
+      ncols = own + later;
     }
   }
   IM_HD int n_rows() const { return n; }
@@ -123,12 +128,15 @@ struct KeyRowsBlockScatter {
     const int b = (int)fd_div(t, dBlk);
     return (b * G + gk) * blk + (t - b * blk);
   }
+  // Without a branch and from few scalars: it runs for every tile of the main loop, where a wavefront
+  // has its SIMD for itself.  A choice by `off` with both sides' scalars spilled them in the launch that
+  // more than 64 sinks share (19 lane reads and 36 branches per step, now 7 and 16), which cost 1 - 3 %
+  // where every tile is a new one (one query head per kv head): training steps with 128 sinks, G = 2,
+  // 32 / 32 heads, S = 8192, 1444 -> 1386 us (before the launch was shared 1438).
   IM_HD int col_pos(int c) const {
-    if (off == 0) return row_pos(c);
-    if (c < own_len) return kb * blk + c;
-    const int c2 = c - own_len;
-    const int m = (int)fd_div(c2, dBlk);
-    return (qb0 + m * G) * blk + (c2 - m * blk);
+    const uint32_t c2 = (uint32_t)im_max(c - own, 0);
+    const uint32_t far = far_pos + c2 + fd_div(c2, dBlk) * far_step;
+    return (int)(c < own ? own_pos + (uint32_t)c : far);
   }
   IM_HD int lo(int t) const { return off == 0 ? t : t - a * blk; }
   IM_HD int hi(int) const { return ncols - 1; }
