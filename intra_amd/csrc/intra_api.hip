@@ -591,23 +591,23 @@ int run_bwd_keys(intra::BParams p, hipStream_t stream) {
   return launch_bwd<R, intra::BWD_DKV, 1>(p, stream);
 }
 
-// dK and dV over a key-row map and, in the same launch, over the leading keys LEAD.
-// `longest`: columns of the longest row block of R.
+// dK and dV over a key-row map and, in the same launch, over the leading keys LEAD: first where they
+// meet more columns than the longest row block of R (the shorter workgroups then fill the last round).
 template <class R, class LEAD>
-int run_bwd_keys_lead(intra::BParams p, int64_t longest, hipStream_t stream) {
+int run_bwd_keys_lead(intra::BParams p, hipStream_t stream) {
   p.grid = bwd_grid<R>(p, KEY_ROWS, 1);
   p.lead = bwd_grid<LEAD>(p, KEY_ROWS, 1);
   // (their work counts half where both halves of a workgroup share the columns)
-  p.lead_first = p.geom.sink_chunk / (intra::alternates<LEAD> ? 2 : 1) > longest;
+  p.lead_first = std::min(p.geom.sink_chunk, p.geom.S) / (intra::alternates<LEAD> ? 2 : 1) > R::longest(p.geom);
   return launch_bwd<R, intra::BWD_DKV, 1, LEAD>(p, stream);
 }
 
 // The same with the sinks as leading keys.  Up to 64 of them fill two of a workgroup's four wavefronts:
 // the other two then take every other block of columns.
 template <class R>
-int run_bwd_keys_sinks(const intra::BParams& p, int64_t longest, hipStream_t stream) {
-  return p.geom.ns <= 64 ? run_bwd_keys_lead<R, intra::KeyRowsFewSinks>(p, longest, stream)
-                         : run_bwd_keys_lead<R, intra::KeyRowsSinks>(p, longest, stream);
+int run_bwd_keys_sinks(const intra::BParams& p, hipStream_t stream) {
+  return p.geom.ns <= 64 ? run_bwd_keys_lead<R, intra::KeyRowsFewSinks>(p, stream)
+                         : run_bwd_keys_lead<R, intra::KeyRowsSinks>(p, stream);
 }
 
 // The leading keys' rows of dk and dv from their partial sums (one chunk: written by the launch itself)
@@ -734,20 +734,20 @@ int run_bwd(int domain, const void* q, const void* k, const void* v, const void*
     case MAP_LLM_BLOCK_SCATTER:
       if ((rc = run_bwd_dq<MapLlmBlockScatter>(p, sh.hp, st))) return rc;
       if (ns == 0) return run_bwd_keys<intra::KeyRowsBlockScatter>(p, st);
-      rc = run_bwd_keys_sinks<intra::KeyRowsBlockScatter>(p, intra::KeyRowsBlockScatter::max_rows(p.geom), st);
+      rc = run_bwd_keys_sinks<intra::KeyRowsBlockScatter>(p, st);
       return rc ? rc : run_bwd_lead_reduce(p, ns, st);
     case MAP_LLM_WINDOW_SINK:
       if ((rc = run_bwd_dq<MapLlmWindowSink>(p, sh.hp, st))) return rc;
       if (ns == 0) return run_bwd_keys<intra::KeyRowsWindowSink>(p, st);
-      rc = run_bwd_keys_sinks<intra::KeyRowsWindowSink>(p, (int64_t)p.geom.window + KEY_ROWS, st);
+      rc = run_bwd_keys_sinks<intra::KeyRowsWindowSink>(p, st);
       return rc ? rc : run_bwd_lead_reduce(p, ns, st);
     case MAP_IMG_SCATTER:  // grid keys against their group's queries, text keys against all queries
       if ((rc = run_bwd_dq<MapImgScatter>(p, sh.hp, st))) return rc;
-      rc = run_bwd_keys_lead<intra::KeyRowsImgGroup<false>, intra::KeyRowsText>(p, S / 8, st);
+      rc = run_bwd_keys_lead<intra::KeyRowsImgGroup<false>, intra::KeyRowsText>(p, st);
       return rc ? rc : run_bwd_lead_reduce(p, ns, st);
     case MAP_IMG_GATHER0:  // grid keys against the grid queries around them, plus their group's text queries
       if ((rc = run_bwd_dq<MapImgGather0>(p, sh.hp, st))) return rc;
-      if ((rc = run_bwd_keys_lead<intra::KeyRowsImgWindow, intra::KeyRowsText>(p, 8 * 64, st))) return rc;
+      if ((rc = run_bwd_keys_lead<intra::KeyRowsImgWindow, intra::KeyRowsText>(p, st))) return rc;
       if ((rc = run_bwd_keys<intra::KeyRowsImgGroup<true>>(p, st))) return rc;
       return run_bwd_lead_reduce(p, ns, st);
     default: return fail(INTRA_ERR_UNSUPPORTED, "backward: no kernels for this pattern");

@@ -21,6 +21,7 @@
 //                                          row and 32-column block (first column c) whether the row
 //                                          meets the block - all of it or nothing
 //   kAccumulate                            the results are added to rows another pass has written
+//   static longest(ge)                     columns of the longest row block (maps that share a launch with leading keys)
 //   alternates<RowMap>                     rows 0..63 and 64..127 are the same keys twice over: the
 //                                          first meet the even blocks of 32 columns, the second the odd
 //                                          ones, and the results of the two are added
@@ -138,6 +139,7 @@ struct KeyRowsBlockScatter {
     const uint32_t far = far_pos + c2 + fd_div(c2, dBlk) * far_step;
     return (int)(c < own ? own_pos + (uint32_t)c : far);
   }
+  static int longest(const IntraGeom& ge) { return KeyRowsBlockScatter(ge, 0, 0).n_cols(); }  // (the first block's)
   IM_HD int lo(int t) const { return off == 0 ? t : t - a * blk; }
   IM_HD int hi(int) const { return ncols - 1; }
   IM_HD int block_lo(int r0, int) const { return lo(r0); }
@@ -153,6 +155,7 @@ struct KeyRowsWindowSink {
   int S, window, skip;
   static IM_HD int num_sets(const IntraGeom&) { return 1; }
   static IM_HD int max_rows(const IntraGeom& ge) { return ge.S; }
+  static int longest(const IntraGeom& ge) { return (int)im_min64((int64_t)ge.window + KEY_ROWS - 1, ge.S); }
   IM_HD KeyRowsWindowSink(const IntraGeom& ge, int, int) {
     S = ge.S;
     window = ge.window;
@@ -245,6 +248,7 @@ struct KeyRowsImgGroup {
   MapImgScatter sc;
   static IM_HD int num_sets(const IntraGeom&) { return 8; }
   static IM_HD int max_rows(const IntraGeom& ge) { return ge.width * ge.width / 8; }
+  static int longest(const IntraGeom& ge) { return KeyRowsImgGroup(ge, 0, 0).n_cols(); }  // (all row blocks of all groups)
   IM_HD KeyRowsImgGroup(const IntraGeom& ge, int set, int) : sc(ge, set, 0, 0) {}
   IM_HD int n_rows() const { return sc.nimg; }
   IM_HD int n_cols() const { return TEXT_COLS_ONLY ? sc.chunk : sc.chunk + sc.nimg; }
@@ -275,8 +279,11 @@ struct KeyRowsImgGroup {
 //  * the last 4 columns of these rows, 4 cells below each other at a time;
 //  * the 4 upper and the 4 lower grid rows, 32 columns of the grid at a time: one patch row of columns.
 // (Where W is an odd number of patches the runs of 16 columns end with one of 12 that holds the last 4.)
-// Runs of 16 columns from 0 on stream 2 x 4 patches instead of 2 x 3, cells cut along the patches of
-// the rows as well 3 x 4.
+// (Behind the border, whose 12 rows or columns share a patch, a run streams more: rows or columns 12 ..
+// 19 are seen by 3 patches, columns 12 .. 27 by 4, so that the longest row block has 3 x 4 of them - 3 x 5
+// on a grid of 40 x 40, 4 x 4 on 32 x 32, where the other border is as near - and the mean one 6.2 to 7.)
+// Runs of 16 columns from 0 on would stream 2 x 4 patches instead of 2 x 3, cells cut along the patches
+// of the rows as well 3 x 4.
 // No division by a variable past the constructor: col_pos and sees run several times per step.
 struct KeyRowsImgWindow {
   int W, T, np, r0, c0, kw, wshift, wrows, wcols, Rlo, Clo, nR, nC, inv_nC;
@@ -287,6 +294,8 @@ struct KeyRowsImgWindow {
     return (ge.width / 8 - 1) * mid_runs(ge) + side_runs(ge) + 2 * edge_runs(ge);
   }
   static IM_HD int max_rows(const IntraGeom&) { return 128; }
+  // (that of the rows and columns from 12 on, see above; two patches a side have one kind only)
+  static int longest(const IntraGeom& ge) { return KeyRowsImgWindow(ge, ge.width > 16 ? mid_runs(ge) + 1 : 0, 0).n_cols(); }
   // first and last patch (along either axis) whose window covers grid row / column x
   static IM_HD int first_patch(int x) { return x <= 15 ? 0 : (x - 4) >> 3; }
   static IM_HD int last_patch(int x, int W) { return x >= W - 16 ? W / 8 - 1 : (x + 4) >> 3; }

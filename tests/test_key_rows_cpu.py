@@ -1,6 +1,6 @@
 """The key-row maps of the dK / dV launch (intra_amd/csrc/intra_bwd_maps.h), compiled for the host: how
-the queries of the leading keys (LLM sinks, image text keys) are cut into chunks, and the columns of
-block Scatter's row blocks."""
+the queries of the leading keys (LLM sinks, image text keys) are cut into chunks, the columns of block
+Scatter's row blocks, and what the maps call their longest row block."""
 import os
 import shutil
 import subprocess
@@ -98,3 +98,49 @@ def test_columns_of_block_scatter_row_blocks(tmp_path, S, G, blk, off):
         own = [p for p in range(first, min(S, (kb + 1) * blk))]
         seen_by = [qb for qb in range(kb + 1, -(-S // blk)) if (qb + off) % G == kb % G]
         assert cols == own + [p for qb in seen_by for p in range(qb * blk, min(S, (qb + 1) * blk))], (S, G, blk, off, first)
+
+
+LONGEST = r"""
+#include <stdio.h>
+#include <string.h>
+#include <initializer_list>
+#include "intra_bwd_maps.h"
+using namespace intra;
+
+template <class R>
+static void check(const char* name, IntraGeom ge) {
+  geom_finish(ge);
+  int most = 0;
+  for (int set = 0; set < R::num_sets(ge); ++set)
+    for (int r0 = 0; r0 < R::max_rows(ge); r0 += KEY_ROWS) {
+      const R m(ge, set, r0);
+      if (r0 >= m.n_rows()) continue;
+      const int r1 = im_min(r0 + KEY_ROWS, m.n_rows()) - 1;
+      most = im_max(most, m.block_hi(r0, r1) - m.block_lo(r0, r1) + 1);
+    }
+  if (most != R::longest(ge)) printf("%s: S %d G %d block %d offset %d window %d width %d: %d columns, longest() says %d\n", name,
+                                     ge.S, ge.G, ge.blk, ge.off, ge.window, ge.width, most, R::longest(ge));
+}
+
+int main() {
+  IntraGeom ge0;
+  memset(&ge0, 0, sizeof ge0);
+  ge0.G = 1; ge0.window = 64; ge0.width = 16; ge0.text_len = 8; ge0.pg = 1; ge0.tm = 1; ge0.blk = 256; ge0.sink_chunk = 1024;
+  for (int S : {1, 100, 256, 300, 1000, 4096, 6000}) {
+    for (int G : {1, 2, 3, 8}) for (int off = 0; off < G; ++off) { IntraGeom ge = ge0; ge.S = S; ge.G = G; ge.off = off; check<KeyRowsBlockScatter>("block scatter", ge); }
+    for (int w : {1, 255, 575, 5000}) { IntraGeom ge = ge0; ge.S = S; ge.window = w; check<KeyRowsWindowSink>("window", ge); }
+  }
+  for (int width = 16; width <= 192; width += 8) for (int text : {8, 512}) {
+    IntraGeom ge = ge0;
+    ge.S = text + width * width; ge.width = width; ge.text_len = text;
+    check<KeyRowsImgWindow>("image gather 0", ge);
+    check<KeyRowsImgGroup<false>>("image scatter", ge);
+  }
+  return 0;
+}
+"""
+
+
+def test_longest_row_block(tmp_path):
+    """Which workgroups of the dK / dV launch come first is decided by it."""
+    assert compile_and_run(tmp_path, LONGEST) == ""
