@@ -161,8 +161,8 @@ int intra_get_softmax_mode(void);
  * Patterns: all five of intra_llm_fwd_ex; INTRA_LLM_BLOCK_SCATTER with offset != 0 needs
  * block % 256 == 0, softmax_scale must not be 0; otherwise INTRA_ERR_UNSUPPORTED.  Launches on
  * hip_stream: dq, then dk and dv in one pass, and with sinks one more that adds up the partial sums
- * of the sink rows; nothing is allocated.  Accuracy: weights are rounded to bf16 before the second product, as in the forward
- * pass, accumulation is fp32. */
+ * of the sink rows (none where the queries are one chunk); nothing is allocated.  Accuracy: weights
+ * are rounded to bf16 before the second product, as in the forward pass, accumulation is fp32. */
 int intra_llm_bwd(const void* q, const void* k, const void* v, const void* o, const float* lse,
                   const void* dout, void* dq, void* dk, void* dv, float* workspace, int B, int S,
                   int H, int Hkv, const int64_t q_strides[3], const int64_t k_strides[3],
@@ -171,10 +171,11 @@ int intra_llm_bwd(const void* q, const void* k, const void* v, const void* o, co
                   const int64_t dk_strides[3], const int64_t dv_strides[3],
                   const int64_t lse_strides[3], int pattern, int group_num, int window, int block,
                   int offset, int n_sink, float softmax_scale, void* hip_stream);
-/* Floats of workspace that intra_llm_bwd needs for such a call (twice B*H*S rounded up to 4, plus with
- * sinks chunks * B * Hkv * min(n_sink, S) * 128, the queries being cut into chunks so that the
- * sink pass has about one workgroup per CU; the size is the same on every device - it allows for
- * 320 CUs, and a launch never splits finer than that); -1 if the request is invalid or unsupported
+/* Floats of workspace that intra_llm_bwd needs for such a call: twice B*H*S rounded up to 4, plus,
+ * with sinks whose queries are cut into several chunks, 2 * chunks * B * Hkv * min(n_sink, S) * 128
+ * for the partial sums of their rows of dk and dv.  The size is the same on every device (a launch
+ * has at most half as many chunks as would give 320 CUs a block of 256 sinks each, and no more
+ * workgroups on sinks than the device has CUs); -1 if the request is invalid or unsupported
  * (intra_last_error() says why).  No counterpart in the reference. */
 int64_t intra_llm_bwd_workspace(int B, int S, int H, int Hkv, int pattern, int group_num,
                                 int window, int block, int offset, int n_sink);

@@ -641,7 +641,7 @@ int64_t bwd_dsum_floats(int B, int S, int H) { return ((int64_t)B * H * S + 3) &
 int64_t bwd_workspace_floats(const Request& r) {
   int64_t n = 2 * bwd_dsum_floats(r.B, r.S, r.H);
   const int ns = leading_keys(r);
-  if (ns > 0) n += (int64_t)intra::workspace_chunks(r.S, r.B, r.Hkv, ns) * r.B * r.Hkv * ns * 128;
+  if (ns > 0) n += intra::leading_floats(r.S, r.B, r.Hkv, ns);
   return n;
 }
 

@@ -176,10 +176,10 @@ struct KeyRowsWindowSink {
 };
 
 // Chunks of queries that the row blocks of the `ns` leading keys (LLM sinks, image text keys) are cut
-// into, and their length, a multiple of 64 and at least 128 (except for the last).  The workspace has
-// room for the fp32 sums of workspace_chunks chunks of one result - about one block of 256 keys per CU
-// of a device of WS_CUS CUs, so that its size does not depend on the device; dk and dv share it, so a
-// launch has half as many chunks at most.  Nor does it have more workgroups on leading keys than the
+// into, and their length, a multiple of 64 and at least 128 (except for the last).  Half as many as
+// would give every CU of a device of WS_CUS CUs one block of 256 keys, so that the fp32 partial sums of
+// dk and dv are as many as one such block per CU would have of one result, and their room
+// (leading_floats) does not depend on the device.  Nor are there more workgroups on leading keys than the
 // device has CUs: a few too many are a second round of the longest kind on a few CUs, which everything
 // else waits for.  With 288 - 320 workgroups on 256 CUs against 192 - 256 (training steps, us): image
 // Scatter 2048^2 at 12 heads 1211 -> 1164, at 6 heads 691 -> 657; Gather 0 at 24 heads 384 -> 361
@@ -187,19 +187,23 @@ struct KeyRowsWindowSink {
 // block Scatter 4750 -> 4660.  (Slower: 1000 sinks at S = 3000, 336 -> 348, where 5 short chunks
 // behind the window's row blocks fill the rounds better than 4.)
 constexpr int WS_CUS = 320;
-inline int workspace_chunks(int S, int B, int Hkv, int ns) {
-  const int64_t row_wgs = (int64_t)B * Hkv * ((ns + 255) / 256);
-  int64_t chunks = WS_CUS / row_wgs > 1 ? WS_CUS / row_wgs : 1;
-  if (chunks > S / 128) chunks = im_max(1, S / 128);
-  const int64_t chunk = 64 * ((S + 64 * chunks - 1) / (64 * chunks));
-  return (int)((S + chunk - 1) / chunk);
-}
-inline int leading_chunk(int S, int B, int Hkv, int ns, int cus) {
-  const int64_t row_wgs = (int64_t)B * Hkv * ((ns + KEY_ROWS - 1) / KEY_ROWS);
-  int64_t chunks = workspace_chunks(S, B, Hkv, ns) / 2;
-  if (chunks > cus / row_wgs) chunks = cus / row_wgs;
+inline int chunk_length(int S, int64_t chunks) {
   if (chunks < 1) chunks = 1;
   return (int)(64 * ((S + 64 * chunks - 1) / (64 * chunks)));
+}
+inline int chunk_count(int S, int chunk) { return (S + chunk - 1) / chunk; }
+inline int leading_chunk(int S, int B, int Hkv, int ns, int cus) {
+  int64_t chunks = WS_CUS / ((int64_t)B * Hkv * ((ns + 255) / 256));
+  if (chunks > S / 128) chunks = S / 128;
+  chunks = chunk_count(S, chunk_length(S, chunks)) / 2;
+  const int64_t one_round = cus / ((int64_t)B * Hkv * ((ns + KEY_ROWS - 1) / KEY_ROWS));
+  return chunk_length(S, chunks < one_round ? chunks : one_round);
+}
+// Floats of partial sums on any device: a smaller bound on the chunks never gives more of them, and a
+// single chunk writes its results at once.
+inline int64_t leading_floats(int S, int B, int Hkv, int ns) {
+  const int chunks = chunk_count(S, leading_chunk(S, B, Hkv, ns, INT32_MAX));
+  return chunks > 1 ? (int64_t)chunks * B * Hkv * ns * 2 * 128 : 0;
 }
 
 // The first ge.ns keys (LLM sinks; the text keys of the image patterns) against the queries of the

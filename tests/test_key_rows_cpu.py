@@ -19,7 +19,7 @@ int main() {  // every line of the input: S B Hkv ns cus
   int S, B, Hkv, ns, cus;
   while (scanf("%d %d %d %d %d", &S, &B, &Hkv, &ns, &cus) == 5) {
     const int chunk = leading_chunk(S, B, Hkv, ns, cus);
-    printf("%d %d %d\n", chunk, (S + chunk - 1) / chunk, workspace_chunks(S, B, Hkv, ns));
+    printf("%d %d %lld\n", chunk, (S + chunk - 1) / chunk, (long long)leading_floats(S, B, Hkv, ns));
   }
   return 0;
 }
@@ -37,7 +37,7 @@ def compile_and_run(tmp_path, source, text=""):
 
 
 def splits(tmp_path, shapes):
-    """(queries of a chunk, chunks, chunks of one result that the workspace holds) of every (S, B, Hkv, ns, cus)"""
+    """(queries of a chunk, chunks, floats of room for partial sums) of every (S, B, Hkv, ns, cus)"""
     out = compile_and_run(tmp_path, SRC, "\n".join(" ".join(map(str, s)) for s in shapes) + "\n")
     return [tuple(map(int, line.split())) for line in out.splitlines()]
 
@@ -52,7 +52,19 @@ def test_no_more_workgroups_on_leading_keys_than_cus(tmp_path):
         what = f"S={S} B={B} Hkv={Hkv} ns={ns} cus={cus}: {n} chunks of {chunk}"
         assert chunk % 64 == 0 and (n - 1) * chunk < S <= n * chunk, what
         assert n == 1 or n * B * Hkv * -(-ns // 128) <= cus, what
-        assert n == 1 or 2 * n <= room, what
+        assert n == 1 or 2 * n * B * Hkv * ns * 128 <= room, what
+
+
+def test_workspace_is_what_the_finest_split_writes(tmp_path, lib):
+    """No room that no launch uses: nothing for a single chunk, both results of the chunks otherwise."""
+    for S, B, Hkv, width in ((4608, 1, 3, 64), (4608, 1, 24, 64), (4608, 2, 24, 64), (16896, 1, 16, 128), (16896, 2, 24, 128)):
+        (_, n, _), = splits(tmp_path, [(S, B, Hkv, 512, 1 << 20)])
+        want = 2 * B * S * Hkv + (2 * n * B * Hkv * 512 * 128 if n > 1 else 0)
+        assert lib.intra_image_bwd_workspace(B, S, Hkv, Hkv, 0, width, 512) == want, (S, B, Hkv)
+    for S, B, Hkv, ns in ((64, 1, 1, 4), (390, 1, 2, 130), (1000, 3, 28, 64), (6000, 1, 8, 64), (320, 2, 82, 3)):
+        (_, n, _), = splits(tmp_path, [(S, B, Hkv, ns, 1 << 20)])
+        want = 2 * B * S * Hkv + (2 * n * B * Hkv * ns * 128 if n > 1 else 0)
+        assert lib.intra_llm_bwd_workspace(B, S, Hkv, Hkv, 9, 2, 575, 256, 0, ns) == want, (S, B, Hkv, ns)
 
 
 COLS = r"""
