@@ -165,8 +165,11 @@ def test_window_sink_grads(S, kw, B, H, Hkv):
 
 # The sinks' queries are cut into chunks whose partial sums are added up: one chunk (written without
 # partial sums, by few queries or by many kv heads), more sinks than a row block of 128, and more
-# chunks than the summation requests at once (8), with a remainder.
-@pytest.mark.parametrize("B,S,H,Hkv,n_sink", [(1, 130, 2, 1, 4), (1, 390, 4, 2, 130), (2, 320, 82, 82, 3), (1, 2700, 4, 1, 129)])
+# chunks than the summation requests at once (8), with a remainder (test_key_rows_cpu.py counts them).
+SINK_CHUNKS = [(1, 130, 2, 1, 4), (1, 390, 4, 2, 130), (2, 320, 82, 82, 3), (1, 2700, 4, 1, 129), (1, 4500, 4, 1, 129)]
+
+
+@pytest.mark.parametrize("B,S,H,Hkv,n_sink", SINK_CHUNKS)
 def test_sink_chunks_grads(B, S, H, Hkv, n_sink):
     run_case("llm/window_sink", "window_sink", B, S, H, Hkv, window=70, n_sink=n_sink)
 

@@ -55,6 +55,12 @@ def test_no_more_workgroups_on_leading_keys_than_cus(tmp_path):
         assert n == 1 or 2 * n * B * Hkv * ns * 128 <= room, what
 
 
+def test_the_gpu_tests_meet_every_kind_of_split(tmp_path):
+    from test_backward_gpu import SINK_CHUNKS
+    counts = {n for _, n, _ in splits(tmp_path, [(S, B, Hkv, ns, 256) for B, S, _, Hkv, ns in SINK_CHUNKS])}
+    assert 1 in counts and any(1 < n < 8 for n in counts) and any(n > 8 and n % 8 for n in counts), counts
+
+
 def test_workspace_is_what_the_finest_split_writes(tmp_path, lib):
     """No room that no launch uses: nothing for a single chunk, both results of the chunks otherwise."""
     for S, B, Hkv, width in ((4608, 1, 3, 64), (4608, 1, 24, 64), (4608, 2, 24, 64), (16896, 1, 16, 128), (16896, 2, 24, 128)):
