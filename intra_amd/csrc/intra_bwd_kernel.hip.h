@@ -71,7 +71,6 @@ struct BParams {
 };
 
 constexpr int BWD_SLOT = 2 * FTILE + 512;  // two tiles and 2 x 64 column scalars
-constexpr int BWD_LDS_BYTES = 3 * BWD_SLOT;
 constexpr int bwd_ring_slots(int mode) { return mode == BWD_DKV ? 4 : 3; }
 
 // 64 lanes x 4 bytes from per-lane global addresses to 256 consecutive LDS bytes at lds_addr (the
