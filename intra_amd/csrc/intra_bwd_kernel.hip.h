@@ -325,7 +325,11 @@ __device__ __forceinline__ void bwd_rows(const BParams& p, const BwdGrid& g, con
     c1hs = p.q_hs * 2;
     c2hs = p.do_hs * 2;
   }
-  auto col_pos = [&](int c) { return map.col_pos(c); };
+  int tile_shift = 0;  // (kTileShift) of the tile being requested
+  auto col_pos = [&](int c) {
+    if constexpr (RMAP::kTileShift) return c + tile_shift;
+    else return map.col_pos(c);
+  };
   // dK / dV take a tile once per query head of the group, head after head: the rows' positions are
   // worked out for the first head and kept for the others
   uint32_t pos_kept[16 / NW] = {};
@@ -339,6 +343,8 @@ __device__ __forceinline__ void bwd_rows(const BParams& p, const BwdGrid& g, con
               lds_base + slot_off + FTILE + grp * FGROUP_STRIDE);
   };
   auto load_tile = [&](const Cursor& cu, int slot_off) {
+    if constexpr (RMAP::kTileShift)
+      if (cu.head == 0) tile_shift = map.tile_shift(cb + cu.tile * BN);
 #pragma unroll
     for (int gi = 0; gi < 16 / NW; ++gi) load_group(cu, slot_off, gi);
   };

@@ -20,6 +20,8 @@
 //   kBlockPredicate / sees(t, c)           maps whose rows do not meet one range of columns say per
 //                                          row and 32-column block (first column c) whether the row
 //                                          meets the block - all of it or nothing
+//   kTileShift / tile_shift(c)             maps whose position - column is the same for all columns of a
+//                                          tile (64 from block_lo on) say it for the tile's first column
 //   kAccumulate                            the results are added to rows another pass has written
 //   static longest(ge)                     columns of the longest row block (maps that share a launch with leading keys)
 //   alternates<RowMap>                     rows 0..63 and 64..127 are the same keys twice over: the
@@ -51,7 +53,7 @@ struct QueryRows {
   IM_HD int block_lo(int r0, int) const { return m.kpre() > 0 ? 0 : m.klo(r0); }
   IM_HD int block_hi(int, int r1) const { return hi(r1); }
   IM_HD bool store(int) const { return true; }
-  static constexpr bool kBlockPredicate = false, kAccumulate = false;
+  static constexpr bool kBlockPredicate = false, kAccumulate = false, kTileShift = false;
   IM_HD bool sees(int, int) const { return true; }
 };
 
@@ -76,7 +78,7 @@ struct KeyRowsOf {
   IM_HD int block_lo(int r0, int) const { return lo(r0); }
   IM_HD int block_hi(int, int r1) const { return hi(r1); }
   IM_HD bool store(int) const { return true; }
-  static constexpr bool kBlockPredicate = false, kAccumulate = false;
+  static constexpr bool kBlockPredicate = false, kAccumulate = false, kTileShift = false;
   IM_HD bool sees(int, int) const { return true; }
 };
 
@@ -88,7 +90,7 @@ struct KeyRowsOf {
 // (block size a multiple of 256).  Sinks (positions < n_sink) are not stored here.
 struct KeyRowsBlockScatter {
   int G, blk, gk, off, n, skip, a, own, ncols;
-  uint32_t own_pos, far_pos, far_step;  // position of the own block, of the first column behind it; skipped per further block
+  uint32_t own_pos, far_pos, far_step;  // position minus column: in the own block, in the first one behind it; more per further block
   FastDiv dBlk;
   static IM_HD int num_sets(const IntraGeom& ge) { return ge.G; }
   static IM_HD int max_rows(const IntraGeom& ge) { return MapLlmBlockScatter::max_nq(ge); }
@@ -118,7 +120,7 @@ struct KeyRowsBlockScatter {
       }
       own = im_max(0, im_min(blk, S - kb * blk));
       own_pos = (uint32_t)kb * (uint32_t)blk;
-      far_pos = (uint32_t)qb0 * (uint32_t)blk;
+      far_pos = (uint32_t)qb0 * (uint32_t)blk - (uint32_t)own;
       ncols = own + later;
     }
   }
@@ -129,23 +131,23 @@ struct KeyRowsBlockScatter {
     const int b = (int)fd_div(t, dBlk);
     return (b * G + gk) * blk + (t - b * blk);
   }
-  // Without a branch and from few scalars: it runs for every tile of the main loop, where a wavefront
-  // has its SIMD for itself.  A choice by `off` with both sides' scalars spilled them in the launch that
-  // more than 64 sinks share (19 lane reads and 36 branches per step, now 7 and 16), which cost 1 - 3 %
-  // where every tile is a new one (one query head per kv head): training steps with 128 sinks, G = 2,
-  // 32 / 32 heads, S = 8192, 1444 -> 1386 us (before the launch was shared 1438).
-  IM_HD int col_pos(int c) const {
-    const uint32_t c2 = (uint32_t)im_max(c - own, 0);
-    const uint32_t far = far_pos + c2 + fd_div(c2, dBlk) * far_step;
-    return (int)(c < own ? own_pos + (uint32_t)c : far);
+  // Blocks start at multiples of 64 columns, so a tile lies inside one.  Worked out once per tile, in
+  // scalars: per lane and group of rows it was a chain of branches on `off` and on the own block, whose
+  // scalars were spilled and read back in the main loop of the launch that more than 64 sinks share
+  // (19 lane reads and 36 branches per step there, 27 branches elsewhere; now 2 and 13).  Training steps,
+  // G = 2, S = 8192: offset 1 and 128 sinks at 32 / 32 heads 1432 -> 1334 us, 64 sinks at 32 / 8 heads
+  // 1248 -> 1217, neither offset nor sinks 1121 -> 1107.
+  IM_HD int tile_shift(int c) const {
+    return (int)(c < own ? own_pos : far_pos + fd_div((uint32_t)(c - own), dBlk) * far_step);
   }
+  IM_HD int col_pos(int c) const { return c + tile_shift(c); }
   static int longest(const IntraGeom& ge) { return KeyRowsBlockScatter(ge, 0, 0).n_cols(); }  // (the first block's)
   IM_HD int lo(int t) const { return off == 0 ? t : t - a * blk; }
   IM_HD int hi(int) const { return ncols - 1; }
   IM_HD int block_lo(int r0, int) const { return lo(r0); }
   IM_HD int block_hi(int, int) const { return ncols - 1; }
   IM_HD bool store(int pos) const { return pos >= skip; }
-  static constexpr bool kBlockPredicate = false, kAccumulate = false;
+  static constexpr bool kBlockPredicate = false, kAccumulate = false, kTileShift = true;
   IM_HD bool sees(int, int) const { return true; }
 };
 
@@ -171,7 +173,7 @@ struct KeyRowsWindowSink {
   IM_HD int block_lo(int r0, int) const { return r0; }
   IM_HD int block_hi(int, int r1) const { return hi(r1); }
   IM_HD bool store(int pos) const { return pos >= skip; }
-  static constexpr bool kBlockPredicate = false, kAccumulate = false;
+  static constexpr bool kBlockPredicate = false, kAccumulate = false, kTileShift = false;
   IM_HD bool sees(int, int) const { return true; }
 };
 
@@ -234,7 +236,7 @@ struct KeyRowsLeading {
   IM_HD int block_lo(int r0, int) const { return lo(r0); }
   IM_HD int block_hi(int, int) const { return c1 - 1; }
   IM_HD bool store(int) const { return true; }
-  static constexpr bool kBlockPredicate = false, kAccumulate = false;
+  static constexpr bool kBlockPredicate = false, kAccumulate = false, kTileShift = false;
   IM_HD bool sees(int, int) const { return true; }
 };
 using KeyRowsSinks = KeyRowsLeading<true>;
@@ -264,7 +266,7 @@ struct KeyRowsImgGroup {
   IM_HD int block_lo(int, int) const { return 0; }
   IM_HD int block_hi(int, int) const { return n_cols() - 1; }
   IM_HD bool store(int) const { return true; }
-  static constexpr bool kBlockPredicate = false, kAccumulate = TEXT_COLS_ONLY;
+  static constexpr bool kBlockPredicate = false, kAccumulate = TEXT_COLS_ONLY, kTileShift = false;
   IM_HD bool sees(int, int) const { return true; }
 };
 
@@ -363,7 +365,7 @@ struct KeyRowsImgWindow {
   IM_HD int block_lo(int, int) const { return 0; }
   IM_HD int block_hi(int, int) const { return n_cols() - 1; }
   IM_HD bool store(int) const { return true; }
-  static constexpr bool kBlockPredicate = true, kAccumulate = false;
+  static constexpr bool kBlockPredicate = true, kAccumulate = false, kTileShift = false;
   IM_HD bool sees(int t, int c) const {
     const int pi = c >> 6, ri = patch_row(pi);
     const int wr = MapImgPatch::win_start(Rlo + ri, np), wc = MapImgPatch::win_start(Clo + pi - ri * nC, np);

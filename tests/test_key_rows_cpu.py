@@ -93,7 +93,11 @@ int main() {  // every line of the input: S G block offset; output: key block, t
         if (r0 >= m.n_rows()) continue;
         const int r1 = (r0 + KEY_ROWS < m.n_rows() ? r0 + KEY_ROWS : m.n_rows()) - 1;
         printf("%d", m.row_pos(r0));
-        for (int c = m.block_lo(r0, r1); c <= m.block_hi(r0, r1); ++c) printf(" %d", m.col_pos(c));
+        const int cb = m.block_lo(r0, r1);
+        for (int c = cb; c <= m.block_hi(r0, r1); ++c) {
+          printf(" %d", m.col_pos(c));
+          if (m.col_pos(c) - c != m.tile_shift(cb + ((c - cb) & ~63))) printf(" not the tile's shift");
+        }
         printf("\n");
       }
     printf("end\n");
