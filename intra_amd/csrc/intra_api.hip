@@ -707,6 +707,9 @@ int run_bwd(int domain, const void* q, const void* k, const void* v, const void*
   p.lse_bs = ls[0]; p.lse_hs = ls[1]; p.lse_ts = ls[2];
   p.ds_bs = (int64_t)H * S; p.ds_hs = S;
   p.B = B; p.H = H; p.Hkv = Hkv; p.ratio = H / Hkv;
+  p.far_rows = 0;
+  for (const int64_t* st : all)
+    if (((int64_t)S - 1) * st[1] * 2 + 256 > UINT32_MAX) p.far_rows = 1;
   p.scale = scale;
   p.scale_log2 = scale * 1.4426950408889634f;
   Shape sh;

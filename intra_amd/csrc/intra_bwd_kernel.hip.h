@@ -62,6 +62,7 @@ struct BParams {
   int64_t dq_bs, dq_rs, dq_hs, dk_bs, dk_rs, dk_hs, dv_bs, dv_rs, dv_hs;
   int64_t lse_bs, lse_hs, lse_ts, ds_bs, ds_hs;  // dsum is contiguous over tokens
   int B, H, Hkv, ratio;
+  int far_rows;      // some row of q, k, v or dout is 4 GiB or more behind the first of its head
   IntraGeom geom;
   float scale;       // softmax scale
   float scale_log2;  // scale * log2(e)
@@ -77,6 +78,18 @@ constexpr int bwd_ring_slots(int mode) { return mode == BWD_DKV ? 4 : 3; }
 // active lanes' parts of them), like dma_group
 __device__ __forceinline__ void dma_dwords(const void* gsrc, uint32_t lds_addr) {
   asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dword %0, off" : : "v"(gsrc), "s"(lds_addr) : "memory");
+}
+
+// The same two with a wave-uniform address and 32-bit per-lane byte offsets
+template <int LDS_OFFSET>
+__device__ __forceinline__ void dma_rows(const void* base, uint32_t offset, uint32_t lds_addr) {
+  asm volatile("s_add_u32 m0, %2, %3\n\tglobal_load_lds_dwordx4 %0, %1"
+               : : "v"(offset), "s"(base), "s"(lds_addr), "n"(LDS_OFFSET) : "memory", "scc");
+}
+template <int LDS_OFFSET>
+__device__ __forceinline__ void dma_scalars(const void* base, uint32_t offset, uint32_t lds_addr) {
+  asm volatile("s_add_u32 m0, %2, %3\n\tglobal_load_lds_dword %0, %1"
+               : : "v"(offset), "s"(base), "s"(lds_addr), "n"(LDS_OFFSET) : "memory", "scc");
 }
 
 // The work of one workgroup, number `block` of the grid `g`.  RMAP: row map (intra_bwd_maps.h).
@@ -96,7 +109,7 @@ __device__ __forceinline__ void bwd_rows(const BParams& p, const BwdGrid& g, con
 
   // BWD_DKV: a step of its single wavefront per SIMD is about as long as a tile takes to arrive, so
   // its ring is one slot deeper and a tile has two steps to land; the column scalars travel the same
-  // way (every wavefront requests those of 16 columns) instead of through registers.
+  // way instead of through registers.
   constexpr bool DEEP = MODE == BWD_DKV;
   constexpr bool ALT = alternates<RMAP>;  // wavefronts 0, 1 and 2, 3 share rows and take turns at the 32-column blocks
   const uint32_t lds_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)smem;
@@ -256,15 +269,17 @@ __device__ __forceinline__ void bwd_rows(const BParams& p, const BwdGrid& g, con
   // kread_b: row-per-lane operand 2 * ks + ct of a 32-row block (rows 16 * ct + l16, head dims of
   // k-step ks); vread_b: transposed operand (head dims 16 * dt .. + 15 of the block's 32 rows).
   // sb0, sb1: the same for the column scalars of the deep ring.
+  // (Wavefronts that take turns at the blocks work on one block of a tile; theirs is in the bases.)
+  const int half = ALT ? wave >> 1 : 0;
   int kb0[4], kb1[4], vb0[4], sb0 = 0, sb1 = 0;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    kb0[i] = kaddr[i];
-    kb1[i] = BWD_SLOT + kaddr[i];
-    vb0[i] = vaddr[i];
+    kb0[i] = half * FBLOCK32 + kaddr[i];
+    kb1[i] = half * FBLOCK32 + BWD_SLOT + kaddr[i];
+    vb0[i] = half * FBLOCK32 + vaddr[i];
   }
-  sb0 = 2 * FTILE + 16 * g4;
-  sb1 = BWD_SLOT + 2 * FTILE + 16 * g4;
+  sb0 = 2 * FTILE + 128 * half + 16 * g4;
+  sb1 = BWD_SLOT + 2 * FTILE + 128 * half + 16 * g4;
   auto kread_b = [&](const int (&kb)[4], int off, int f) {
     return *reinterpret_cast<const bf16x8*>(smem + (kb[f >> 1] + (off + (f & 1) * 4 * FGROUP_STRIDE)));
   };
@@ -325,39 +340,84 @@ __device__ __forceinline__ void bwd_rows(const BParams& p, const BwdGrid& g, con
     c1hs = p.q_hs * 2;
     c2hs = p.do_hs * 2;
   }
-  int tile_shift = 0;  // (kTileShift) of the tile being requested
-  auto col_pos = [&](int c) {
-    if constexpr (RMAP::kTileShift) return c + tile_shift;
-    else return map.col_pos(c);
-  };
-  // dK / dV take a tile once per query head of the group, head after head: the rows' positions are
-  // worked out for the first head and kept for the others
-  uint32_t pos_kept[16 / NW] = {};
-  int64_t spos_kept = 0;
-  auto load_group = [&](const Cursor& cu, int slot_off, int gi) {  // this wavefront's group gi of both tiles
-    const int grp = wave * (16 / NW) + gi;
-    if (ROWS_ARE_QUERIES || cu.head == 0) pos_kept[gi] = col_pos(im_min(cb + cu.tile * BN + 4 * grp + ld_row, n_cols - 1));
-    const uint32_t pos = pos_kept[gi];
-    dma_group(c1base + (cu.head * c1hs + (uint64_t)pos * c1rs + ld_col), lds_base + slot_off + grp * FGROUP_STRIDE);
-    dma_group(c2base + (cu.head * c2hs + (uint64_t)pos * c2rs + ld_col),
-              lds_base + slot_off + FTILE + grp * FGROUP_STRIDE);
-  };
-  auto load_tile = [&](const Cursor& cu, int slot_off) {
-    if constexpr (RMAP::kTileShift)
-      if (cu.head == 0) tile_shift = map.tile_shift(cb + cu.tile * BN);
+  // Requests.  A lane's rows of a tile are named by 32-bit byte offsets from a wave-uniform address.  For
+  // tiles whose positions follow one of the maps' patterns (tile_at) the offsets stay in registers from
+  // tile to tile and only that address moves; other tiles (cut by the end of the columns, or across two
+  // parts of them) get offsets of their own, from the tensor's start.  The query heads of a group share
+  // the offsets.  With the addresses worked out per lane and request (a 64-bit multiply-add each, behind a
+  // 64-bit product for the head's base) a step of dK / dV issued about 120 instructions for its requests,
+  // none of them behind an MFMA.  With these and the order of the block below (same box, training steps,
+  // us): Scatter G=8 S=32768 4385 -> 4189, its dK / dV launch 2395 -> 2090; image Scatter 2048^2 at 12
+  // heads 1166 -> 1076; window 575 with 64 sinks, S=8192, 486 -> 470; image Gather 0 1024^2 363 -> 344.
+  constexpr int GROUPS = 16 / NW;  // 4-row groups of either tile per wavefront
+  uint32_t vo1[GROUPS], vo2[GROUPS], vos = 0;
 #pragma unroll
-    for (int gi = 0; gi < 16 / NW; ++gi) load_group(cu, slot_off, gi);
+  for (int gi = 0; gi < GROUPS; ++gi) vo1[gi] = vo2[gi] = 0;
+  int vo_kind = -1;                     // what the offsets are for: a tile pattern, or -1
+  const char *a1 = c1base, *a2 = c2base, *as = nullptr;  // addresses of the step being requested
+  // the column scalars that this wavefront requests: lse * log2(e) (even wavefronts) or -D
+  const float* const sbase = (wave & 1 ? p.dsum : p.l2) + (batch * p.ds_bs + kvh * p.ratio * p.ds_hs);
+  auto aim = [&](int tile) {  // at the first head of a tile
+    const int c = cb + tile * BN;
+    TileAt at;
+    const bool pattern = c + BN <= n_cols && map.tile_at(c, at);
+    if (pattern && vo_kind != at.kind) {
+      vo_kind = at.kind;
+#pragma unroll
+      for (int gi = 0; gi < GROUPS; ++gi) {
+        const uint32_t rel = (uint32_t)map.tile_rel(at.kind, 4 * (wave * GROUPS + gi) + ld_row);
+        vo1[gi] = rel * c1rs + ld_col;
+        vo2[gi] = rel * c2rs + ld_col;
+      }
+      if (DEEP) vos = 4 * (uint32_t)map.tile_rel(at.kind, lane);
+    } else if (!pattern) {
+      vo_kind = -1;
+      at.base = 0;
+#pragma unroll
+      for (int gi = 0; gi < GROUPS; ++gi) {
+        const uint32_t pos = (uint32_t)map.col_pos(im_min(c + 4 * (wave * GROUPS + gi) + ld_row, n_cols - 1));
+        vo1[gi] = pos * c1rs + ld_col;
+        vo2[gi] = pos * c2rs + ld_col;
+      }
+      if (DEEP) vos = 4 * (uint32_t)map.col_pos(im_min(c + lane, n_cols - 1));
+    }
+    const uint32_t base = (uint32_t)__builtin_amdgcn_readfirstlane(at.base);
+    a1 = c1base + (uint64_t)base * c1rs;
+    a2 = c2base + (uint64_t)base * c2rs;
+    if (DEEP) as = reinterpret_cast<const char*>(sbase + base);
   };
-  // requests per wavefront for one step of the deep ring: its groups of both tiles and two for the scalars
-  constexpr int DEEP_REQUESTS = 2 * (16 / NW) + 2;
-  auto load_scalars = [&](const Cursor& cu, int slot_off) {  // (deep ring) lse * log2(e) and -D of the step's 64 columns
-    static_assert(!DEEP || NW == 4, "16 columns per wavefront");
-    if (cu.head == 0) spos_kept = col_pos(im_min(cb + cu.tile * BN + lane, n_cols - 1));
-    if ((lane >> 4) == wave) {
-      const int64_t pos = spos_kept;
-      const int hcol = kvh * p.ratio + cu.head;
-      dma_dwords(p.l2 + (batch * p.ds_bs + hcol * p.ds_hs + pos), lds_base + slot_off + 2 * FTILE);
-      dma_dwords(p.dsum + (batch * p.ds_bs + hcol * p.ds_hs + pos), lds_base + slot_off + 2 * FTILE + 256);
+  // tensors beyond the reach of 32-bit offsets: per-lane addresses
+  auto load_far = [&](const Cursor& cu, int slot_off) {
+#pragma unroll
+    for (int gi = 0; gi < GROUPS; ++gi) {
+      const int grp = wave * GROUPS + gi;
+      const uint64_t pos = (uint64_t)map.col_pos(im_min(cb + cu.tile * BN + 4 * grp + ld_row, n_cols - 1));
+      dma_group(c1base + (cu.head * c1hs + pos * c1rs + ld_col), lds_base + slot_off + grp * FGROUP_STRIDE);
+      dma_group(c2base + (cu.head * c2hs + pos * c2rs + ld_col), lds_base + slot_off + FTILE + grp * FGROUP_STRIDE);
+    }
+    if (DEEP)
+      dma_dwords(sbase + (cu.head * p.ds_hs + map.col_pos(im_min(cb + cu.tile * BN + lane, n_cols - 1))),
+                 lds_base + slot_off + 2 * FTILE + 256 * (wave & 1));
+  };
+  const uint32_t lds_rows = lds_base + wave * GROUPS * FGROUP_STRIDE;
+  const uint32_t lds_scalars = lds_base + 256 * (wave & 1);
+  constexpr int REQUESTS = 2 * GROUPS + (DEEP ? 1 : 0);  // per wavefront and step
+  auto load_step = [&](const Cursor& cu, int slot_off) {
+    if (p.far_rows) {
+      load_far(cu, slot_off);
+      return;
+    }
+    if (ROWS_ARE_QUERIES || cu.head == 0) aim(cu.tile);
+    static_for<0, GROUPS>([&](auto gi_c) {
+      constexpr int gi = decltype(gi_c)::value;
+      dma_rows<gi * FGROUP_STRIDE>(a1, vo1[gi], lds_rows + slot_off);
+      dma_rows<FTILE + gi * FGROUP_STRIDE>(a2, vo2[gi], lds_rows + slot_off);
+    });
+    if (DEEP) {  // (wavefronts 2, 3 repeat the scalars of 0, 1: every wavefront counts alike)
+      dma_scalars<2 * FTILE>(as, vos, lds_scalars + slot_off);
+      a1 += c1hs;  // from one head's addresses to the next one's
+      a2 += c2hs;
+      as += 4 * p.ds_hs;
     }
   };
   // Three tile slots: while step t works on its tile, the tile of step t+1 has landed (the scores
@@ -367,8 +427,7 @@ __device__ __forceinline__ void bwd_rows(const BParams& p, const BwdGrid& g, con
   // (Deep ring: one slot more, the tile of step t+3 is requested during step t, and the barrier of a
   // step leaves the most recent request in flight where one was made during the step before.)
   for (int t = 0; t < (DEEP ? 3 : 2) && t < n_steps; ++t) {
-    load_tile(ld, t * BWD_SLOT);
-    if (DEEP) load_scalars(ld, t * BWD_SLOT);
+    load_step(ld, t * BWD_SLOT);
     advance(ld);
   }
   // The deep ring's barriers leave requests in flight.  The row operands are ordinary loads the
@@ -380,18 +439,15 @@ __device__ __forceinline__ void bwd_rows(const BParams& p, const BwdGrid& g, con
     __builtin_amdgcn_s_waitcnt((0 & 15) | (7 << 4) | (15 << 8) | (0 << 14));  // vmcnt(0)
   }
   int slot0 = 0, slot1 = BWD_SLOT, slot2 = 2 * BWD_SLOT, slot3 = 3 * BWD_SLOT;
-  bool fresh = DEEP && n_steps >= 3;  // the most recent request is for the step after the next
+  bool fresh = n_steps >= 3;  // the most recent request is for the step after the next
   floatx4 s_cur[2][2];  // [ct][rt]
 #pragma unroll
   for (int t = 0; t < 4; ++t) s_cur[t >> 1][t & 1] = zero4;
   bool have = false;  // s_cur and fr hold what a previous block prepared for the one that comes next
   // One slot is one MFMA; an LDS operand serves two consecutive slots (the two row tiles).
   constexpr int NFRAG = MODE == BWD_DKV ? 32 : 24;  // LDS operands per block
-  constexpr int LA = MODE == BWD_DKV ? 8 : 6;       // operands between the request of one and its use
+  constexpr int LA = MODE == BWD_DKV ? 8 : 4;       // operands between the request of one and its use
   static_assert(NFRAG % LA == 0, "a block must leave the ring where the next block expects it");
-  // slot of the first dS stage and slots from one stage to the next (the P stages run while dP accumulates)
-  constexpr int WS = MODE == BWD_DKV ? 22 : 16;
-  constexpr int WSTEP = MODE == BWD_DKV ? 3 : 2;
   bf16x8 fr[LA];
 #pragma unroll
   for (int i = 0; i < LA; ++i) fr[i] = bf16x8{};
@@ -400,65 +456,57 @@ __device__ __forceinline__ void bwd_rows(const BParams& p, const BwdGrid& g, con
   const floatx4 nd_row[2] = {floatx4{-D_row[0], -D_row[0], -D_row[0], -D_row[0]}, floatx4{-D_row[1], -D_row[1], -D_row[1], -D_row[1]}};
   for (int t = 0; t < n_steps; ++t) {
     // the tiles of steps t and t+1 have landed for everybody; nobody reads that of t-1
-    if (DEEP && fresh) tile_barrier<DEEP_REQUESTS>();
+    if (DEEP && fresh) tile_barrier<REQUESTS>();
     else tile_barrier<0>();
-    if (DEEP) {
-      fresh = t + 3 < n_steps;
-      if (fresh) {
-        load_tile(ld, slot3);
-        load_scalars(ld, slot3);
-        advance(ld);
-      }
-    } else if (t + 2 < n_steps) {
-      load_tile(ld, slot2);
+    // the tile of step t + 3 (dQ: t + 2) into the slot of step t - 1
+    fresh = t + (DEEP ? 3 : 2) < n_steps;
+    if (fresh) {
+      load_step(ld, DEEP ? slot3 : slot2);
       advance(ld);
     }
-#pragma unroll
-    for (int blk = 0; blk < 2; ++blk) {
-      if (ALT && blk != wave >> 1) continue;  // (the block that follows is the same one of the next tile)
-      const int jb = 2 * cur.tile + blk;
-      if (jb < jb_lo || jb > jb_hi) {
-        have = false;
-        continue;
-      }
+    static_for<0, ALT ? 1 : 2>([&](auto blk_c) {
+      constexpr int blk = decltype(blk_c)::value;
+      const int jb = 2 * cur.tile + (ALT ? half : blk);
       const int sb_lo = cb + 32 * jb;  // first column of the block
-      // behind the prefix and in front of the wavefront's own range: nothing is visible (a run of 4 image
+      // (behind the prefix and in front of the wavefront's own range nothing is visible: a run of 4 image
       // patches streams 10 tiles of window keys, of which a patch sees 4: training steps of 24 heads
       // 397 -> 392 us at 1024^2, 1259 -> 1236 us at 2048^2)
-      if (kpre > 0 && !block_wanted(wb, kpre, sb_lo)) {
-        have = false;
-        continue;
-      }
+      bool wanted = jb >= jb_lo && jb <= jb_hi && (kpre == 0 || block_wanted(wb, kpre, sb_lo));
       // maps with a block predicate: a row meets the whole block or nothing of it
       bool lane_sees[2] = {true, true};
       bool masked;
-      if (RMAP::kBlockPredicate) {
+      if constexpr (RMAP::kBlockPredicate) {
         lane_sees[0] = map.sees(row[0], sb_lo);
         lane_sees[1] = map.sees(row[1], sb_lo);
-        if (__builtin_amdgcn_ballot_w64(lane_sees[0] || lane_sees[1]) == 0) {
-          have = false;
-          continue;
-        }
+        wanted = wanted && __builtin_amdgcn_ballot_w64(lane_sees[0] || lane_sees[1]) != 0;
         masked = __builtin_amdgcn_ballot_w64(lane_sees[0] && lane_sees[1]) != ~0ull;
       } else {
         masked = !block_unmasked(wb, kpre, sb_lo);
       }
-      // Hand-scheduled.  dQ: slots 0-15 dP of this block, 16-31 the scores of the next block, 32-47 the
-      // accumulation; dK / dV: dP, the dV accumulation, the next scores, the dK accumulation.  LDS
-      // operand f (slots 2f, 2f+1) is requested LA operands earlier into a ring of LA fragments,
-      // across block and step boundaries (both following blocks have landed); dS of element pair u is
-      // formed in slot WS + WSTEP * u, after dP has drained and before the accumulation needs it.  sched_barrier keeps the compiler from regrouping the slots.
+      if (!wanted) {
+        have = false;
+        return;
+      }
+      // Hand-scheduled.  Slots 0-15: dP of this block, 16-31: the scores of the next block, then the
+      // accumulation (dQ), or those of dV (32-47) and dK (48-63).  LDS operand f (slots 2f, 2f+1) is
+      // requested LA operands earlier into a ring of LA fragments, across block and step boundaries (both
+      // following blocks have landed).  What a slot may hold besides its MFMA was found with isolated
+      // loops on one SIMD: an MFMA keeps the vector port for 8 of its 16 cycles, so 8 cycles of vector
+      // work behind it (two plain instructions or one exponential) cost nothing and the rest does, and a
+      // request or a wait costs nothing directly behind the MFMA but some 10 cycles in front of one.
+      // Hence one exponential or two plain instructions per slot, and MFMA, wait, request, vector work in
+      // that order; sched_barrier keeps the compiler from regrouping.
       auto fetch = [&](int f) {
         const int here = blk * FBLOCK32;  // the block inside the step's slot
         // rows of the block that follows in this order, at tile `which` of its slot
         auto next_rows = [&](int which, int ff) {
-          if (ALT) return kread_b(kb1, here + which * FTILE, ff);
+          if (ALT) return kread_b(kb1, which * FTILE, ff);
           return blk == 0 ? kread_b(kb0, FBLOCK32 + which * FTILE, ff) : kread_b(kb1, which * FTILE, ff);
         };
         if (MODE == BWD_DKV) {
           if (f < 8) return kread_b(kb0, here + FTILE, f);   // dO rows: dP
-          if (f < 16) return vread_b(here + FTILE, f - 8);   // dO^T: dV accumulation
-          if (f < 24) return next_rows(0, f - 16);           // Q rows of the next block: its scores
+          if (f < 16) return next_rows(0, f - 8);            // Q rows of the next block: its scores
+          if (f < 24) return vread_b(here + FTILE, f - 16);  // dO^T: dV accumulation
           if (f < 32) return vread_b(here, f - 24);          // Q^T: dK accumulation
           return next_rows(1, f - 32);
         }
@@ -469,7 +517,7 @@ __device__ __forceinline__ void bwd_rows(const BParams& p, const BwdGrid& g, con
       };
       const float* sc = reinterpret_cast<const float*>(smem + (sb0 + 128 * blk));
       // scalars of the block that follows in this order
-      const float* scn = ALT ? reinterpret_cast<const float*>(smem + (sb1 + 128 * blk)) : blk == 0 ? sc + 32 : reinterpret_cast<const float*>(smem + sb1);
+      const float* scn = ALT ? reinterpret_cast<const float*>(smem + sb1) : blk == 0 ? sc + 32 : reinterpret_cast<const float*>(smem + sb1);
       if (!have) {  // first block of a run: nothing was prepared by a previous block
         if (MODE == BWD_DKV) {
           l4_keep[0] = *reinterpret_cast<const floatx4*>(sc);
@@ -503,72 +551,92 @@ __device__ __forceinline__ void bwd_rows(const BParams& p, const BwdGrid& g, con
       floatx4 dp[2][2], s_next[2][2];
       bf16x8 wp[2];
       bf16x8 wp_p[MODE == BWD_DKV ? 2 : 1];   // BWD_DKV: the weights P (wp holds dS)
-      floatx4 pf[2][2];                        // P before rounding, for dS
+      floatx4 pf[2][2];                        // exponents, then P before rounding, then dS
       // BWD_DKV: scalars of the lane's columns, per column tile (a block reads those of the next one in its last slots)
       floatx4 (&l4)[2] = l4_keep;
       floatx4 (&d4)[2] = d4_keep;
-      // P of pair u = 4 * rt + 2 * ct + h (columns 16 * ct + 4 * g4 + 2 * h, + 1 of row tile rt)
-      auto stage = [&](int u) {
+      // Pair u = 4 * rt + 2 * ct + h: columns 16 * ct + 4 * g4 + 2 * h, + 1 of row tile rt.  Exponents of P ...
+      auto p_fma = [&](int u) {
         const int rt = u >> 2, ct = (u >> 1) & 1, h = u & 1;
-        float w[2];
 #pragma unroll
-        for (int v = 0; v < 2; ++v) {
-          const int e = 2 * h + v;
-          const float l = ROWS_ARE_QUERIES ? L2_row[rt] : l4[ct][e];
-          w[v] = __builtin_amdgcn_exp2f(__builtin_fmaf(s_cur[ct][rt][e], c2, -l));
-        }
-        pf[ct][rt][2 * h] = w[0];  // (unrounded, for dS, which follows when dP is there)
-        pf[ct][rt][2 * h + 1] = w[1];
-        if (MODE == BWD_DKV) {
-          floatx2 f2 = {w[0], w[1]};
-          bf16x2 h2 = __builtin_convertvector(f2, bf16x2);
-          wp_p[rt][4 * ct + 2 * h] = h2[0];
-          wp_p[rt][4 * ct + 2 * h + 1] = h2[1];
-        }
+        for (int e = 2 * h; e < 2 * h + 2; ++e)
+          pf[ct][rt][e] = __builtin_fmaf(s_cur[ct][rt][e], c2, -(ROWS_ARE_QUERIES ? L2_row[rt] : l4[ct][e]));
       };
-      // dS = P * (dP - D) of pair u; the accumulators of dP start from -D
-      auto stage_ds = [&](int u) {
+      // ... P (one of the pair), unrounded for dS ...
+      auto p_exp = [&](int u, int v) {
+        const int rt = u >> 2, ct = (u >> 1) & 1, e = 2 * (u & 1) + v;
+        pf[ct][rt][e] = __builtin_amdgcn_exp2f(pf[ct][rt][e]);
+      };
+      auto pack = [&](bf16x8 (&to)[2], const floatx4 (&from)[2][2], int u) {
         const int rt = u >> 2, ct = (u >> 1) & 1, h = u & 1;
-        floatx2 f2 = {pf[ct][rt][2 * h] * dp[ct][rt][2 * h], pf[ct][rt][2 * h + 1] * dp[ct][rt][2 * h + 1]};  // (dP started from -D)
+        floatx2 f2 = {from[ct][rt][2 * h], from[ct][rt][2 * h + 1]};
         bf16x2 h2 = __builtin_convertvector(f2, bf16x2);
-        wp[rt][4 * ct + 2 * h] = h2[0];
-        wp[rt][4 * ct + 2 * h + 1] = h2[1];
+        to[rt][4 * ct + 2 * h] = h2[0];
+        to[rt][4 * ct + 2 * h + 1] = h2[1];
+      };
+      // ... and dS = P * (dP - D): the accumulators of dP start from -D
+      auto ds_mul = [&](int u) {
+        const int rt = u >> 2, ct = (u >> 1) & 1, h = u & 1;
+#pragma unroll
+        for (int e = 2 * h; e < 2 * h + 2; ++e) pf[ct][rt][e] *= dp[ct][rt][e];
       };
       constexpr int NSLOT = 2 * NFRAG;
+      // LDS instructions per operand, and those issued behind the request of operand f before its wait (in
+      // slot 2 * f - 1): the operands' and the next block's scalars'
+      constexpr auto reads_of = [](int f) { return f % NFRAG < 16 ? 1 : 2; };
+      constexpr auto scalar_slot = [](int i) { return MODE == BWD_DKV && i >= 50 && i <= 56 && i % 2 == 0; };
+      constexpr auto pending = [=](int f) {
+        int n = 0;
+        for (int x = f + 1; x < f + LA - 1; ++x) n += reads_of(x);
+        for (int i = 2 * (f - LA) + 2; i < 2 * f; ++i) n += scalar_slot((i + NSLOT) % NSLOT);
+        return n < 15 ? n : 15;
+      };
       // (compile-time slot numbers: a loop of this size is beyond what the compiler unrolls in full)
       static_for<0, NSLOT>([&](auto slot_c) {
         constexpr int i = decltype(slot_c)::value;
         constexpr int f = i >> 1, rt = i & 1;
         const bf16x8 a = fr[f % LA];
-        if constexpr (MODE == BWD_DKV) {
-          if constexpr (f < 8) dp[f & 1][rt] = mfma(a, r2f[rt][f >> 1], f < 2 ? d4[f & 1] : dp[f & 1][rt]);  // from -D of the tile's columns
-          else if constexpr (f < 16) acc_v[f - 8][rt] = mfma(a, wp_p[rt], acc_v[f - 8][rt]);
-          else if constexpr (f < 24) s_next[f & 1][rt] = mfma(a, r1f[rt][(f - 16) >> 1], f < 18 ? zero4 : s_next[f & 1][rt]);
-          else acc[f - 24][rt] = mfma(a, wp[rt], acc[f - 24][rt]);
-        } else {
-          if constexpr (f < 8) dp[f & 1][rt] = mfma(a, r2f[rt][f >> 1], f < 2 ? nd_row[rt] : dp[f & 1][rt]);  // from -D of the row
-          else if constexpr (f < 16) s_next[f & 1][rt] = mfma(a, r1f[rt][(f - 8) >> 1], f < 10 ? zero4 : s_next[f & 1][rt]);
-          else acc[f - 16][rt] = mfma(a, wp[rt], acc[f - 16][rt]);
+        if constexpr (f < 8) dp[f & 1][rt] = mfma(a, r2f[rt][f >> 1], f >= 2 ? dp[f & 1][rt] : MODE == BWD_DKV ? d4[f & 1] : nd_row[rt]);  // from -D
+        else if constexpr (f < 16) s_next[f & 1][rt] = mfma(a, r1f[rt][(f - 8) >> 1], f < 10 ? zero4 : s_next[f & 1][rt]);
+        else if constexpr (f < 24 && MODE == BWD_DKV) acc_v[f - 16][rt] = mfma(a, wp_p[rt], acc_v[f - 16][rt]);
+        else acc[f - (NFRAG - 8)][rt] = mfma(a, wp[rt], acc[f - (NFRAG - 8)][rt]);
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (rt == 1) {
+          __builtin_amdgcn_s_waitcnt(15 | (3 << 14) | (7 << 4) | (pending(f + 1) << 8));  // (LDS reads only)
+          fr[f % LA] = fetch(f + LA);
         }
-        if (rt == 1) fr[f % LA] = fetch(f + LA);
-        if (MODE == BWD_DKV) {  // P in front of the dV accumulation, dS behind dP
-          // the next block's scalars, when this block has used its own for the last time
+        if constexpr (MODE == BWD_DKV) {  // the next block's scalars, when this block has used its own for the last time
           if (i == 50) l4[0] = *reinterpret_cast<const floatx4*>(scn);
           if (i == 52) l4[1] = *reinterpret_cast<const floatx4*>(scn + 16);
           if (i == 54) d4[0] = *reinterpret_cast<const floatx4*>(scn + 64);
           if (i == 56) d4[1] = *reinterpret_cast<const floatx4*>(scn + 64 + 16);
-          if (i >= 5 && i < 16 && (i - 5) % 3 != 2) stage((i - 5) - (i - 5) / 3);  // slots 5, 6, 8, 9, 11, 12, 14, 15
-          if (i >= WS && (i - WS) % WSTEP == 0 && (i - WS) / WSTEP < 8) stage_ds((i - WS) / WSTEP);
-        } else {  // P while dP is formed (the scores are then free for those of the next block), dS behind it
-          if (i < 16 && i % 2 == 0) stage(i / 2);
-          if (i >= WS && (i - WS) % WSTEP == 0 && (i - WS) / WSTEP < 8) stage_ds((i - WS) / WSTEP);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (i >= 1 && i < 25) {
+          constexpr int u = (i - 1) / 3, part = (i - 1) % 3;
+          if (part == 0) p_fma(u);
+          else p_exp(u, part - 1);
+        }
+        if constexpr (MODE == BWD_DKV) {
+          if constexpr (i >= 25 && i < 29) {
+            pack(wp_p, pf, 2 * (i - 25));
+            pack(wp_p, pf, 2 * (i - 25) + 1);
+          }
+          if constexpr (i >= 29 && i < 37) ds_mul(i - 29);
+          if constexpr (i >= 37 && i < 41) {
+            pack(wp, pf, 2 * (i - 37));
+            pack(wp, pf, 2 * (i - 37) + 1);
+          }
+        } else if constexpr (i >= 24 && i < 32) {  // (two wavefronts per SIMD: three in a slot cost nothing)
+          ds_mul(i - 24);
+          pack(wp, pf, i - 24);
         }
         __builtin_amdgcn_sched_barrier(0);
       });
 #pragma unroll
       for (int t4 = 0; t4 < 4; ++t4) s_cur[t4 >> 1][t4 & 1] = s_next[t4 >> 1][t4 & 1];
       have = true;
-    }
+    });
     advance(cur);
     const int ts = slot0;
     slot0 = slot1;
@@ -621,6 +689,11 @@ __device__ __forceinline__ void bwd_rows(const BParams& p, const BwdGrid& g, con
         acc_v[dt][rt] += hand[(16 + 2 * dt + rt) * 64];
       }
   }
+  // (What the results' stores need is read from the kernel arguments here, not carried through the
+  // main loop in scalar registers, which it has too few of.)
+  typedef const __attribute__((address_space(4))) BParams* ArgsPtr;
+  ArgsPtr ka = (ArgsPtr)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(ka));
   if (PARTIAL && RMAP::num_sets(p.geom) > 1) {
     // fp32 partial sums: part[((set * B + batch) * Hkv + kvh) * keys + row][128] of dk, behind all of them those of dv
     int keys = n_rows;
@@ -629,10 +702,10 @@ __device__ __forceinline__ void bwd_rows(const BParams& p, const BwdGrid& g, con
 #pragma unroll
     for (int rt = 0; rt < 2; ++rt)
       if (row_valid[rt]) {
-        float* prow = p.part + ((((int64_t)set * p.B + batch) * p.Hkv + kvh) * keys + row[rt]) * 128 + 4 * g4;
+        float* prow = ka->part + ((((int64_t)set * ka->B + batch) * ka->Hkv + kvh) * keys + row[rt]) * 128 + 4 * g4;
 #pragma unroll
         for (int dt = 0; dt < 8; ++dt) {
-          *reinterpret_cast<floatx4*>(prow + 16 * dt) = acc[dt][rt] * p.scale;
+          *reinterpret_cast<floatx4*>(prow + 16 * dt) = acc[dt][rt] * ka->scale;
           *reinterpret_cast<floatx4*>(prow + all + 16 * dt) = acc_v[MODE == BWD_DKV ? dt : 0][rt];
         }
       }
@@ -647,9 +720,9 @@ __device__ __forceinline__ void bwd_rows(const BParams& p, const BwdGrid& g, con
     for (int rt = 0; rt < 2; ++rt) {
       const bool keep = row_valid[rt] && map.store((int)rpos[rt]);
       uint16_t* orow;
-      if (what == TO_DQ) orow = p.dq + (batch * p.dq_bs + rpos[rt] * p.dq_rs + hq * p.dq_hs + chunk_ofs);
-      else if (what == TO_DK) orow = p.dk + (batch * p.dk_bs + rpos[rt] * p.dk_rs + kvh * p.dk_hs + chunk_ofs);
-      else orow = p.dv + (batch * p.dv_bs + rpos[rt] * p.dv_rs + kvh * p.dv_hs + chunk_ofs);
+      if (what == TO_DQ) orow = ka->dq + (batch * ka->dq_bs + rpos[rt] * ka->dq_rs + hq * ka->dq_hs + chunk_ofs);
+      else if (what == TO_DK) orow = ka->dk + (batch * ka->dk_bs + rpos[rt] * ka->dk_rs + kvh * ka->dk_hs + chunk_ofs);
+      else orow = ka->dv + (batch * ka->dv_bs + rpos[rt] * ka->dv_rs + kvh * ka->dv_hs + chunk_ofs);
 #pragma unroll
       for (int m = 0; m < 4; ++m) {
         uint32_t w[2][2];
@@ -679,10 +752,10 @@ __device__ __forceinline__ void bwd_rows(const BParams& p, const BwdGrid& g, con
     }
   };
   if constexpr (MODE == BWD_DKV) {
-    store_rows(acc, TO_DK, p.scale);
+    store_rows(acc, TO_DK, ka->scale);
     store_rows(acc_v, TO_DV, 1.f);
   } else {
-    store_rows(acc, TO_DQ, p.scale);
+    store_rows(acc, TO_DQ, ka->scale);
   }
 }
 

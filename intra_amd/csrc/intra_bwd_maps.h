@@ -20,8 +20,8 @@
 //   kBlockPredicate / sees(t, c)           maps whose rows do not meet one range of columns say per
 //                                          row and 32-column block (first column c) whether the row
 //                                          meets the block - all of it or nothing
-//   kTileShift / tile_shift(c)             maps whose position - column is the same for all columns of a
-//                                          tile (64 from block_lo on) say it for the tile's first column
+//   tile_at(c, a), tile_rel(kind, i)       where the 64 columns from c on sit (TileAt in intra_maps.h), asked
+//                                          for tiles of 64 from block_lo on that lie inside the column list
 //   kAccumulate                            the results are added to rows another pass has written
 //   static longest(ge)                     columns of the longest row block (maps that share a launch with leading keys)
 //   alternates<RowMap>                     rows 0..63 and 64..127 are the same keys twice over: the
@@ -48,12 +48,14 @@ struct QueryRows {
   IM_HD int kpre() const { return m.kpre(); }
   IM_HD int row_pos(int t) const { return m.qpos(t); }
   IM_HD int col_pos(int c) const { return m.kpos(c); }
+  IM_HD bool tile_at(int c, TileAt& a) const { return m.tile_at(c, a); }
+  IM_HD int tile_rel(int kind, int i) const { return m.tile_rel(kind, i); }
   IM_HD int lo(int t) const { return m.klo(t); }
   IM_HD int hi(int t) const { return im_min(m.khi(t), m.nk() - 1); }
   IM_HD int block_lo(int r0, int) const { return m.kpre() > 0 ? 0 : m.klo(r0); }
   IM_HD int block_hi(int, int r1) const { return hi(r1); }
   IM_HD bool store(int) const { return true; }
-  static constexpr bool kBlockPredicate = false, kAccumulate = false, kTileShift = false;
+  static constexpr bool kBlockPredicate = false, kAccumulate = false;
   IM_HD bool sees(int, int) const { return true; }
 };
 
@@ -73,12 +75,14 @@ struct KeyRowsOf {
   IM_HD int kpre() const { return 0; }
   IM_HD int row_pos(int t) const { return m.kpos(t); }
   IM_HD int col_pos(int c) const { return m.qpos(c); }
+  IM_HD bool tile_at(int c, TileAt& a) const { return m.tile_at(c, a); }
+  IM_HD int tile_rel(int kind, int i) const { return m.tile_rel(kind, i); }
   IM_HD int lo(int r) const { return r; }
   IM_HD int hi(int r) const { return im_min(m.last_query(r), m.nq() - 1); }
   IM_HD int block_lo(int r0, int) const { return lo(r0); }
   IM_HD int block_hi(int, int r1) const { return hi(r1); }
   IM_HD bool store(int) const { return true; }
-  static constexpr bool kBlockPredicate = false, kAccumulate = false, kTileShift = false;
+  static constexpr bool kBlockPredicate = false, kAccumulate = false;
   IM_HD bool sees(int, int) const { return true; }
 };
 
@@ -141,13 +145,18 @@ struct KeyRowsBlockScatter {
     return (int)(c < own ? own_pos : far_pos + fd_div((uint32_t)(c - own), dBlk) * far_step);
   }
   IM_HD int col_pos(int c) const { return c + tile_shift(c); }
+  IM_HD bool tile_at(int c, TileAt& a) const {
+    a = TileAt{c + tile_shift(c), TILE_LINEAR};
+    return true;
+  }
+  IM_HD int tile_rel(int, int i) const { return i; }
   static int longest(const IntraGeom& ge) { return KeyRowsBlockScatter(ge, 0, 0).n_cols(); }  // (the first block's)
   IM_HD int lo(int t) const { return off == 0 ? t : t - a * blk; }
   IM_HD int hi(int) const { return ncols - 1; }
   IM_HD int block_lo(int r0, int) const { return lo(r0); }
   IM_HD int block_hi(int, int) const { return ncols - 1; }
   IM_HD bool store(int pos) const { return pos >= skip; }
-  static constexpr bool kBlockPredicate = false, kAccumulate = false, kTileShift = true;
+  static constexpr bool kBlockPredicate = false, kAccumulate = false;
   IM_HD bool sees(int, int) const { return true; }
 };
 
@@ -168,12 +177,17 @@ struct KeyRowsWindowSink {
   IM_HD int kpre() const { return 0; }
   IM_HD int row_pos(int t) const { return t; }
   IM_HD int col_pos(int c) const { return c; }
+  IM_HD bool tile_at(int c, TileAt& a) const {
+    a = TileAt{c, TILE_LINEAR};
+    return true;
+  }
+  IM_HD int tile_rel(int, int i) const { return i; }
   IM_HD int lo(int t) const { return t; }
   IM_HD int hi(int t) const { return (int)im_min64((int64_t)t + window - 1, S - 1); }
   IM_HD int block_lo(int r0, int) const { return r0; }
   IM_HD int block_hi(int, int r1) const { return hi(r1); }
   IM_HD bool store(int pos) const { return pos >= skip; }
-  static constexpr bool kBlockPredicate = false, kAccumulate = false, kTileShift = false;
+  static constexpr bool kBlockPredicate = false, kAccumulate = false;
   IM_HD bool sees(int, int) const { return true; }
 };
 
@@ -231,12 +245,17 @@ struct KeyRowsLeading {
   IM_HD int row_pos(int t) const { return TWICE ? im_min(t & 63, ns - 1) : t; }  // (rows past the last key repeat it)
   IM_HD bool real(int t) const { return !TWICE || (t & 63) < ns; }
   IM_HD int col_pos(int c) const { return c; }
+  IM_HD bool tile_at(int c, TileAt& a) const {
+    a = TileAt{c, TILE_LINEAR};
+    return true;
+  }
+  IM_HD int tile_rel(int, int i) const { return i; }
   IM_HD int lo(int t) const { return CAUSAL ? im_max(row_pos(t), c0) : c0; }
   IM_HD int hi(int) const { return c1 - 1; }
   IM_HD int block_lo(int r0, int) const { return lo(r0); }
   IM_HD int block_hi(int, int) const { return c1 - 1; }
   IM_HD bool store(int) const { return true; }
-  static constexpr bool kBlockPredicate = false, kAccumulate = false, kTileShift = false;
+  static constexpr bool kBlockPredicate = false, kAccumulate = false;
   IM_HD bool sees(int, int) const { return true; }
 };
 using KeyRowsSinks = KeyRowsLeading<true>;
@@ -261,12 +280,14 @@ struct KeyRowsImgGroup {
   IM_HD int kpre() const { return 0; }
   IM_HD int row_pos(int t) const { return sc.imgpos(t); }
   IM_HD int col_pos(int c) const { return sc.qpos(c); }
+  IM_HD bool tile_at(int c, TileAt& a) const { return sc.tile_in(c, sc.chunk, sc.chunk * sc.j, a); }
+  IM_HD int tile_rel(int kind, int i) const { return sc.tile_rel(kind, i); }
   IM_HD int lo(int) const { return 0; }
   IM_HD int hi(int) const { return n_cols() - 1; }
   IM_HD int block_lo(int, int) const { return 0; }
   IM_HD int block_hi(int, int) const { return n_cols() - 1; }
   IM_HD bool store(int) const { return true; }
-  static constexpr bool kBlockPredicate = false, kAccumulate = TEXT_COLS_ONLY, kTileShift = false;
+  static constexpr bool kBlockPredicate = false, kAccumulate = TEXT_COLS_ONLY;
   IM_HD bool sees(int, int) const { return true; }
 };
 
@@ -360,12 +381,17 @@ struct KeyRowsImgWindow {
     const int ri = patch_row(pi);
     return T + (8 * (Rlo + ri) + (u >> 3)) * W + 8 * (Clo + pi - ri * nC) + (u & 7);
   }
+  IM_HD bool tile_at(int c, TileAt& a) const {
+    a = TileAt{col_pos(c), TILE_PATCH};
+    return true;
+  }
+  IM_HD int tile_rel(int, int i) const { return (i >> 3) * W + (i & 7); }
   IM_HD int lo(int) const { return 0; }
   IM_HD int hi(int) const { return n_cols() - 1; }
   IM_HD int block_lo(int, int) const { return 0; }
   IM_HD int block_hi(int, int) const { return n_cols() - 1; }
   IM_HD bool store(int) const { return true; }
-  static constexpr bool kBlockPredicate = true, kAccumulate = false, kTileShift = false;
+  static constexpr bool kBlockPredicate = true, kAccumulate = false;
   IM_HD bool sees(int t, int c) const {
     const int pi = c >> 6, ri = patch_row(pi);
     const int wr = MapImgPatch::win_start(Rlo + ri, np), wc = MapImgPatch::win_start(Clo + pi - ri * nC, np);

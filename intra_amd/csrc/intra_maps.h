@@ -104,6 +104,23 @@ IM_HD int im_min(int a, int b) { return a < b ? a : b; }
 IM_HD int im_max(int a, int b) { return a > b ? a : b; }
 IM_HD int64_t im_min64(int64_t a, int64_t b) { return a < b ? a : b; }
 
+// Where the 64 keys of a tile sit when the pattern of their positions is one of a few that a loader can
+// keep in registers: key i of the tile is at position base + tile_rel(kind, i), and tile_rel depends on
+// nothing but the launch's geometry.  tile_at answers false for any other tile; it is asked for tiles
+// that lie inside the key list (t_first + 64 <= nk).
+struct TileAt {
+  int base, kind;
+};
+constexpr int TILE_LINEAR = 0;  // consecutive positions
+constexpr int TILE_STRIDED = 1; // every G-th position; the segments of a gather1 group; every fourth grid token of every second row
+constexpr int TILE_PATCH = 2;   // a strip of 4 columns by 16 rows of the grid; a patch of 8 x 8 of it
+// (for maps whose lists consist of runs of consecutive positions, in ascending order)
+template <class F>
+IM_HD bool tile_linear(F&& pos, int t_first, TileAt& a) {
+  a = TileAt{pos(t_first), TILE_LINEAR};
+  return pos(t_first + 63) == a.base + 63;
+}
+
 // ---------------------------------------------------------------- LLM scatter: token i in group i % G
 struct MapLlmScatter {
   static constexpr bool kHasPrefix = false;
@@ -120,6 +137,11 @@ struct MapLlmScatter {
   IM_HD int nk() const { return n; }
   IM_HD int qpos(int t) const { return t * G + g; }
   IM_HD int kpos(int t) const { return t * G + g; }
+  IM_HD bool tile_at(int t_first, TileAt& a) const {
+    a = TileAt{kpos(t_first), TILE_STRIDED};
+    return true;
+  }
+  IM_HD int tile_rel(int, int i) const { return i * G; }
   IM_HD int klo(int) const { return 0; }
   IM_HD int khi(int tq) const { return tq; }
   IM_HD int last_query(int) const { return n - 1; }
@@ -149,6 +171,14 @@ struct MapLlmGather1 {
     return (a * G + g) * G + (t - a * G);
   }
   IM_HD int kpos(int t) const { return qpos(t); }
+  IM_HD bool tile_at(int t_first, TileAt& a) const {  // (a tile that starts with a segment)
+    a = TileAt{qpos(t_first), TILE_STRIDED};
+    return t_first == (int)fd_div(t_first, dG) * G;
+  }
+  IM_HD int tile_rel(int, int i) const {
+    const int s = (int)fd_div(i, dG);
+    return s * G * G + (i - s * G);
+  }
   IM_HD int klo(int) const { return 0; }
   IM_HD int khi(int tq) const { return tq; }
   IM_HD int last_query(int) const { return n - 1; }
@@ -169,6 +199,11 @@ struct MapLlmWindow {
   IM_HD int nk() const { return S; }
   IM_HD int qpos(int t) const { return t; }
   IM_HD int kpos(int t) const { return t; }
+  IM_HD bool tile_at(int t_first, TileAt& a) const {
+    a = TileAt{t_first, TILE_LINEAR};
+    return true;
+  }
+  IM_HD int tile_rel(int, int i) const { return i; }
   IM_HD int klo(int tq) const { return im_max((tq & ~63) - lookback, 0); }
   IM_HD int khi(int tq) const { return tq; }
   // last query whose klo does not exceed key
@@ -206,6 +241,23 @@ struct MapImgScatter {
   IM_HD int nk() const { return T + nimg; }
   IM_HD int qpos(int t) const { return t < chunk ? chunk * j + t : imgpos(t - chunk); }
   IM_HD int kpos(int t) const { return t < T ? t : imgpos(t - T); }
+  // tile of a list of `lead` consecutive positions from `first` on and the group's grid tokens behind them
+  // (a grid tile has to start with a grid row)
+  IM_HD bool tile_in(int t_first, int lead, int first, TileAt& a) const {
+    if (t_first + 64 <= lead) {
+      a = TileAt{first + t_first, TILE_LINEAR};
+      return true;
+    }
+    const int u = t_first - lead;
+    if (u < 0) return false;
+    a = TileAt{imgpos(u), TILE_STRIDED};
+    return u == (int)fd_div(u, dWq) * wq;
+  }
+  IM_HD bool tile_at(int t_first, TileAt& a) const { return tile_in(t_first, T, 0, a); }
+  IM_HD int tile_rel(int kind, int i) const {
+    const int r = (int)fd_div(i, dWq);
+    return kind == TILE_LINEAR ? i : 2 * r * W + 4 * (i - r * wq);
+  }
   IM_HD int klo(int) const { return 0; }
   IM_HD int khi(int) const { return T + nimg - 1; }
 };
@@ -274,6 +326,17 @@ struct MapImgPatch {
     a = TileRows{T + r0 * W + cfirst + 4 * (u >> 6), W, 1};
     return true;
   }
+  IM_HD bool tile_at(int t_first, TileAt& a) const {
+    if (t_first + 64 <= T) {
+      a = TileAt{t_first, TILE_LINEAR};
+      return true;
+    }
+    const int u = t_first - T;
+    if (u < 0 || (u & 63) != 0) return false;
+    a = TileAt{T + r0 * W + cfirst + 4 * (u >> 6), TILE_PATCH};
+    return true;
+  }
+  IM_HD int tile_rel(int kind, int i) const { return kind == TILE_LINEAR ? i : (i >> 2) * W + (i & 3); }
 };
 
 // ---- image gather0, all rows: sets 0..7 are the text-only scatter sets (the longest work items,
@@ -294,6 +357,8 @@ struct MapImgGather0 {
   IM_HD int kpos(int t) const { return is_text ? sc.kpos(t) : pa.kpos(t); }
   IM_HD int klo(int tq) const { return is_text ? 0 : pa.klo(tq); }
   IM_HD int khi(int tq) const { return is_text ? sc.khi(tq) : pa.khi(tq); }
+  IM_HD bool tile_at(int t_first, TileAt& a) const { return is_text ? sc.tile_at(t_first, a) : pa.tile_at(t_first, a); }
+  IM_HD int tile_rel(int kind, int i) const { return kind == TILE_STRIDED ? sc.tile_rel(kind, i) : pa.tile_rel(kind, i); }
 };
 
 // ---- The forward launch of image gather0 deals the text queries like this.  A scatter group has
@@ -433,6 +498,8 @@ struct MapLlmBlockScatter {
     const int m = (int)fd_div(c, dBlk);
     return (m * G + gt) * blk + (c - m * blk);
   }
+  IM_HD bool tile_at(int t_first, TileAt& a) const { return tile_linear([&](int t) { return kpos(t); }, t_first, a); }
+  IM_HD int tile_rel(int, int i) const { return i; }
   IM_HD int klo(int) const { return 0; }
   IM_HD int khi(int tq) const {
     if (off == 0) return E + tq;
@@ -460,6 +527,8 @@ struct MapLlmWindowSink {
   IM_HD int kpre() const { return ns; }
   IM_HD int qpos(int t) const { return t; }
   IM_HD int kpos(int t) const { return t < ns ? t : wlo + (t - ns); }
+  IM_HD bool tile_at(int t_first, TileAt& a) const { return tile_linear([&](int t) { return kpos(t); }, t_first, a); }
+  IM_HD int tile_rel(int, int i) const { return i; }
   IM_HD int klo(int tq) const { return ns + im_max(tq - window + 1, wlo) - wlo; }
   IM_HD int khi(int tq) const { return tq < ns ? tq : ns + (tq - wlo); }
 };

@@ -68,6 +68,21 @@ def test_scatter_grads(S, G, B, H, Hkv):
     run_case("llm/scatter", "scatter", B, S, H, Hkv, group_num=G)
 
 
+@pytest.mark.parametrize("pattern,kw", [("scatter", dict(group_num=2)), ("window_sink", dict(window=64, n_sink=4))])
+def test_rows_beyond_the_reach_of_32_bit_offsets(pattern, kw):
+    """Token strides of 16 MB: the last rows of 300 are more than 4 GiB behind the first."""
+    S, stride = 300, 1 << 23
+    store = torch.empty(S * stride, dtype=torch.bfloat16, device=DEV)
+    views = [store.as_strided((1, S, 2, 128), (S * stride, stride, 128, 1), 256 * i) for i in range(4)]
+    plain = make(1, S, 2, 2, seed=5)
+    for view, x in zip(views, plain):
+        view.copy_(x)
+    q, k, v, dout = views
+    got = kernel_grads(q, k, v, dout, pattern, **kw)
+    for name, a, b in zip(("dq", "dk", "dv"), got, kernel_grads(*plain, pattern, **kw)):
+        assert torch.equal(a, b), name
+
+
 @pytest.mark.parametrize("S", [64, 1024, 2112])
 @pytest.mark.parametrize("B,H,Hkv", [(1, 8, 2), (2, 4, 4)])
 def test_gather1_grads(S, B, H, Hkv):
