@@ -271,6 +271,19 @@ IM_HD bool locate_item(const KParams& p, int xcd, int wgs_per_xcd, int wg_in_xcd
 template <int V>
 using ic = std::integral_constant<int, V>;
 
+// The kernel's arguments, read from the kernel argument segment anew.  A launch has about 120 dwords
+// of them and a wavefront 102 scalar registers: arguments that only the edges of a work item need
+// (dealing, strides, geometry) are read there, through an address the compiler cannot merge with
+// another read of them; carried through the tile loop they were moved between scalar registers and
+// lanes of vector registers, instruction by instruction.
+template <class P>
+__device__ __forceinline__ const P& args_again() {
+  typedef const __attribute__((address_space(4))) P* ArgsPtr;
+  ArgsPtr a = (ArgsPtr)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(a));
+  return *(const P*)a;
+}
+
 // One pass of a workgroup over its work items.  SM: softmax arithmetic, see the file comment.
 // REDO: visit only the items whose round is marked in `redo` (the SM_EXACT second pass of a kernel
 // whose first pass keeps no running maximum).
@@ -295,7 +308,7 @@ __device__ __forceinline__ void run_pass(const KParams& p, unsigned char* smem, 
   const int wgs_per_xcd = gridDim.x >> 3;
   const int wg_in_xcd = blockIdx.x >> 3;
   auto locate = [&](int round, Where& w) {
-    return locate_item<MAP, POS, REDO>(p, xcd, wgs_per_xcd, wg_in_xcd, redo, round, w);
+    return locate_item<MAP, POS, REDO>(args_again<KParams>(), xcd, wgs_per_xcd, wg_in_xcd, redo, round, w);
   };
   auto range_of = [&](const MAP& map, int mblk) { return range_of_block<MAP, POS>(map, mblk); };
 
@@ -313,7 +326,7 @@ __device__ __forceinline__ void run_pass(const KParams& p, unsigned char* smem, 
   static_assert((BN / 4) % NW == 0, "tile groups must split evenly over the wavefronts");
   const int ld_row = lane >> 4;                                  // row of the group this lane fetches
   const uint32_t ld_col = (((lane & 15) ^ (4 * ld_row)) << 4);   // byte column it fetches
-  const uint32_t k_rs_b = p.k_rs_bytes, v_rs_b = p.v_rs_bytes, q_rs_b = p.q_rs_bytes;
+  const uint32_t k_rs_b = p.k_rs_bytes, v_rs_b = p.v_rs_bytes;
   const uint32_t lds_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)smem;
   // The stream of a work item: slots -2 and -1 carry its 256 Q rows (wavefront w reads rows
   // 32 * (w % 2) .. of the K part (w / 2 even) or V part (w / 2 odd) of slot w / 4), slots 0 .. ntiles-1
@@ -330,6 +343,7 @@ __device__ __forceinline__ void run_pass(const KParams& p, unsigned char* smem, 
     int prev_round;    // round of the work item before it
   };
   auto feed_for = [&](const Where& w, int prev_round) {
+    const KParams& p = args_again<KParams>();
     const MAP map(p.geom, w.set, w.mblk * POS);
     return Feed{map, range_of(map, w.mblk), map.nk(), -2, true,
                 reinterpret_cast<const char*>(p.k + w.batch * p.k_bs + w.kvh * p.k_hs),
@@ -344,9 +358,11 @@ __device__ __forceinline__ void run_pass(const KParams& p, unsigned char* smem, 
   Feed fd = feed_for(cw, -1);
   // request the next slot of the stream into a ring slot (byte offset inside the K ring and the V ring)
   auto feed_tile = [&](int slot_off) {
-    if (fd.tile < 0) {  // 128 Q rows: rows of four wavefronts, two per part
+    if (__builtin_expect(fd.tile < 0, 0)) {  // 128 Q rows: rows of four wavefronts, two per part
 #pragma unroll
       for (int gi = 0; gi < GROUPS_PER_WAVE; ++gi) {
+        const KParams& p = args_again<KParams>();
+        const uint32_t q_rs_b = p.q_rs_bytes;
         const int grp = wave * GROUPS_PER_WAVE + gi;
         const int rho = 4 * grp + ld_row;  // row of the part
 #pragma unroll
@@ -385,7 +401,7 @@ __device__ __forceinline__ void run_pass(const KParams& p, unsigned char* smem, 
       }
     }
     ++fd.tile;
-    if (fd.tile == fd.rg.ntiles && fd.more) {
+    if (__builtin_expect(fd.tile == fd.rg.ntiles && fd.more, 0)) {
       Where w;
       if (locate(fd.w.round + 1, w)) fd = feed_for(w, fd.w.round);
       else fd.more = false;  // nothing left: keep requesting the (clamped) last row, nobody reads it
@@ -458,9 +474,10 @@ __device__ __forceinline__ void run_pass(const KParams& p, unsigned char* smem, 
 
   for (;;) {
   INTRA_DIAG(const long long t_a = wall_clock64();)
+  const KParams& pi = args_again<KParams>();
   const int set = cw.set, batch = cw.batch, kvh = cw.kvh, mblk = cw.mblk, hg = cw.hg;
   const int t0 = mblk * POS;
-  const MAP map(p.geom, set, t0);
+  const MAP map(pi.geom, set, t0);
   const int nq = map.nq();
   const int nk = map.nk();
   const int t1 = im_min(t0 + POS, nq) - 1;
@@ -505,7 +522,7 @@ __device__ __forceinline__ void run_pass(const KParams& p, unsigned char* smem, 
   wb.w_lo = __builtin_amdgcn_readfirstlane(wb.w_lo);
   wb.w_hi = __builtin_amdgcn_readfirstlane(wb.w_hi);
 
-  const int hq = kvh * p.ratio + hg * HP + hw;
+  const int hq = kvh * pi.ratio + hg * HP + hw;
 
   // ---------------------------------------------------------------- slot -2: the Q rows arrive
   INTRA_DIAG(const long long t_b = wall_clock64();)
@@ -527,7 +544,7 @@ __device__ __forceinline__ void run_pass(const KParams& p, unsigned char* smem, 
 #pragma unroll
       for (int ks = 0; ks < 4; ++ks) raw[4 * qt + ks] = __builtin_bit_cast(u32x4, kread_q(qa + qt * qstep + 64 * (ks ^ r)));
     if (SM == SM_FOLDED) {  // Q <- bf16(Q * softmax_scale * log2 e): the MFMA then yields exponents directly
-      const float cq = p.q_fold;
+      const float cq = pi.q_fold;
 #pragma unroll
       for (int f = 0; f < 8; ++f)
 #pragma unroll
@@ -536,7 +553,7 @@ __device__ __forceinline__ void run_pass(const KParams& p, unsigned char* smem, 
           floatx2 y = {__uint_as_float(x << 16) * cq, __uint_as_float(x & 0xffff0000u) * cq};
           raw[f][d] = __builtin_bit_cast(uint32_t, __builtin_convertvector(y, bf16x2));
         }
-    } else if (p.negate_q) {  // softmax_scale < 0: flip the sign of Q (exact) and use |scale| below
+    } else if (pi.negate_q) {  // softmax_scale < 0: flip the sign of Q (exact) and use |scale| below
 #pragma unroll
       for (int f = 0; f < 8; ++f) raw[f] ^= 0x80008000u;
     }
@@ -565,7 +582,7 @@ __device__ __forceinline__ void run_pass(const KParams& p, unsigned char* smem, 
   // exp2(score) with the scores already in exponent units).
   float mref[2] = {0.f, 0.f};
   float l_acc[2] = {0.f, 0.f};  // this lane's share of the two queries' weight sums
-  const float c = p.scale_log2;  // |softmax_scale| * log2(e)
+  const float c = pi.scale_log2;  // |softmax_scale| * log2(e)
 
   // operand reads: base register + compile-time byte offset
   auto kread_at = [&](int base, int off) { return *reinterpret_cast<const bf16x8*>(smem + (base + off)); };
@@ -822,6 +839,7 @@ __device__ __forceinline__ void run_pass(const KParams& p, unsigned char* smem, 
 
   // ---------------------------------------------------------------- normalise and store
   {
+  const KParams& po = args_again<KParams>();
   const float l_tot[2] = {lane_quad_sum(l_acc[0]), lane_quad_sum(l_acc[1])};
   if (FAST) {
     // Weights were formed without a reference: the result is good iff the weight sum stayed inside
@@ -835,17 +853,17 @@ __device__ __forceinline__ void run_pass(const KParams& p, unsigned char* smem, 
                             __HIP_MEMORY_SCOPE_WORKGROUP);
   }
   const float inv[2] = {l_tot[0] > 0.f ? 1.f / l_tot[0] : 0.f, l_tot[1] > 0.f ? 1.f / l_tot[1] : 0.f};
-  stored = wave_active ? (p.lse != nullptr ? 9 : 8) : 0;
+  stored = wave_active ? (po.lse != nullptr ? 9 : 8) : 0;
   if (wave_active) {
     // The four lanes of a query hold head dims 4 * g4 .. + 3 of every 16-dim tile.  For the tile pair
     // 2m, 2m+1 a lane quarter and its neighbour (g4 ^ 1) trade 8 bytes: the even one keeps its 4 dims
     // of tile 2m and receives the neighbour's (the next 4 dims), the odd one does the same for tile
     // 2m+1.  Each lane then owns one whole 16-byte chunk of the row, 4m + 2 * (g4 % 2) + g4 / 2, and
     // the four lanes of a query store 64 contiguous bytes per instruction.
-    const int64_t ohead = batch * p.o_bs + hq * p.o_hs + (2 * (g4 & 1) + (g4 >> 1)) * 8;
+    const int64_t ohead = batch * po.o_bs + hq * po.o_hs + (2 * (g4 & 1) + (g4 >> 1)) * 8;
 #pragma unroll
     for (int qt = 0; qt < 2; ++qt) {
-      uint16_t* orow = p.o + (ohead + qpos[qt] * p.o_rs);
+      uint16_t* orow = po.o + (ohead + qpos[qt] * po.o_rs);
 #pragma unroll
       for (int m = 0; m < 4; ++m) {
         uint32_t w[2][2];
@@ -863,9 +881,9 @@ __device__ __forceinline__ void run_pass(const KParams& p, unsigned char* smem, 
     }
     // ln sum_j exp(scale * q.k_j) = (mref + log2 l) * ln 2; the lane quarters g4 = 0, 1 store the values of
     // query tiles 0, 1, the other two (and lanes of clamped rows) repeat them
-    if (p.lse != nullptr) {
+    if (po.lse != nullptr) {
       const int qt = g4 & 1;
-      p.lse[batch * p.lse_bs + hq * p.lse_hs + (qt ? qpos[1] : qpos[0]) * p.lse_ts] =
+      po.lse[batch * po.lse_bs + hq * po.lse_hs + (qt ? qpos[1] : qpos[0]) * po.lse_ts] =
           ((qt ? mref[1] : mref[0]) + __builtin_amdgcn_logf(qt ? l_tot[1] : l_tot[0])) * 0.6931471805599453f;
     }
   }
@@ -894,7 +912,7 @@ __global__ __launch_bounds__(NW * 64) void intra_fwd_kernel(const KParams p) {
     const uint32_t mine = redo[threadIdx.x & (REDO_WORDS - 1)];
     if (__builtin_amdgcn_ballot_w64(mine != 0) == 0) return;  // the usual case
   }
-  run_pass<MAP, HP, NW, SM_EXACT, FAST>(p, smem, redo);
+  run_pass<MAP, HP, NW, SM_EXACT, FAST>(args_again<KParams>(), smem, redo);
 }
 
 }  // namespace intra

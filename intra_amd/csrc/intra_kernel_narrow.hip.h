@@ -53,7 +53,7 @@ __device__ __forceinline__ void run_pass_narrow(const KParams& p, unsigned char*
   const int wgs_per_xcd = gridDim.x >> 3;
   const int wg_in_xcd = blockIdx.x >> 3;
   auto locate = [&](int round, Where& w) {
-    return locate_item<MAP, POS, REDO>(p, xcd, wgs_per_xcd, wg_in_xcd, redo, round, w);
+    return locate_item<MAP, POS, REDO>(args_again<KParams>(), xcd, wgs_per_xcd, wg_in_xcd, redo, round, w);
   };
   auto range_of = [&](const MAP& map, int mblk) { return range_of_block<MAP, POS>(map, mblk); };
 
@@ -80,6 +80,7 @@ __device__ __forceinline__ void run_pass_narrow(const KParams& p, unsigned char*
     int prev_round;    // round of the work item before it
   };
   auto feed_for = [&](const Where& w, int prev_round) {
+    const KParams& p = args_again<KParams>();
     const MAP map(p.geom, w.set, w.mblk * POS);
     return Feed{map, range_of(map, w.mblk), map.nk(), 0, true,
                 reinterpret_cast<const char*>(p.k + w.batch * p.k_bs + w.kvh * p.k_hs),
@@ -127,7 +128,7 @@ __device__ __forceinline__ void run_pass_narrow(const KParams& p, unsigned char*
     }
     v_base = fd.vbase;
     ++fd.tile;
-    if (fd.tile == fd.rg.ntiles && fd.more) {
+    if (__builtin_expect(fd.tile == fd.rg.ntiles && fd.more, 0)) {
       Where w;
       if (locate(fd.w.round + 1, w)) fd = feed_for(w, fd.w.round);
       else fd.more = false;  // nothing left: keep requesting the (clamped) last row, nobody reads it
@@ -166,6 +167,7 @@ __device__ __forceinline__ void run_pass_narrow(const KParams& p, unsigned char*
   // through the hand-counted direct-to-LDS path between their issue and their first use.
   u32x4 qf[2][4];
   auto request_q = [&](const Where& w) {
+    const KParams& p = args_again<KParams>();
     const int t0 = w.mblk * POS;
     const MAP map(p.geom, w.set, t0);
     const int t1 = im_min(t0 + POS, map.nq()) - 1;
@@ -202,9 +204,10 @@ __device__ __forceinline__ void run_pass_narrow(const KParams& p, unsigned char*
 
   for (;;) {
   INTRA_DIAG(const long long t_a = wall_clock64();)
+  const KParams& pi = args_again<KParams>();
   const int set = cw.set, batch = cw.batch, kvh = cw.kvh, mblk = cw.mblk, hg = cw.hg;
   const int t0 = mblk * POS;
-  const MAP map(p.geom, set, t0);
+  const MAP map(pi.geom, set, t0);
   const int nq = map.nq();
   const int nk = map.nk();
   const int t1 = im_min(t0 + POS, nq) - 1;
@@ -249,11 +252,11 @@ __device__ __forceinline__ void run_pass_narrow(const KParams& p, unsigned char*
   wb.w_lo = __builtin_amdgcn_readfirstlane(wb.w_lo);
   wb.w_hi = __builtin_amdgcn_readfirstlane(wb.w_hi);
 
-  const int hq = kvh * p.ratio + hg * HP + hw;
+  const int hq = kvh * pi.ratio + hg * HP + hw;
 
   // ---------------------------------------------------------------- the Q rows have been requested
   if (SM == SM_FOLDED) {  // Q <- bf16(Q * softmax_scale * log2 e): the MFMA then yields exponents directly
-    const float cq = p.q_fold;
+    const float cq = pi.q_fold;
 #pragma unroll
     for (int f = 0; f < 8; ++f)
 #pragma unroll
@@ -262,7 +265,7 @@ __device__ __forceinline__ void run_pass_narrow(const KParams& p, unsigned char*
         floatx2 y = {__uint_as_float(x << 16) * cq, __uint_as_float(x & 0xffff0000u) * cq};
         qf[f >> 2][f & 3][d] = __builtin_bit_cast(uint32_t, __builtin_convertvector(y, bf16x2));
       }
-  } else if (p.negate_q) {  // softmax_scale < 0: flip the sign of Q (exact) and use |scale| below
+  } else if (pi.negate_q) {  // softmax_scale < 0: flip the sign of Q (exact) and use |scale| below
 #pragma unroll
     for (int f = 0; f < 8; ++f) qf[f >> 2][f & 3] ^= 0x80008000u;
   }
@@ -288,7 +291,7 @@ __device__ __forceinline__ void run_pass_narrow(const KParams& p, unsigned char*
   // exp2(score) with the scores already in exponent units).
   float mref[2] = {0.f, 0.f};
   float l_acc[2] = {0.f, 0.f};  // this lane's share of the two queries' weight sums
-  const float c = p.scale_log2;  // |softmax_scale| * log2(e)
+  const float c = pi.scale_log2;  // |softmax_scale| * log2(e)
 
   // operand reads: base register + compile-time byte offset
   auto kread_at = [&](int base, int off) { return *reinterpret_cast<const bf16x8*>(smem + (base + off)); };
@@ -532,6 +535,7 @@ __device__ __forceinline__ void run_pass_narrow(const KParams& p, unsigned char*
 
   // ---------------------------------------------------------------- normalise and store
   {
+  const KParams& po = args_again<KParams>();
   const float l_tot[2] = {lane_quad_sum(l_acc[0]), lane_quad_sum(l_acc[1])};
   if (FAST) {
     // Weights were formed without a reference: the result is good iff the weight sum stayed inside
@@ -551,10 +555,10 @@ __device__ __forceinline__ void run_pass_narrow(const KParams& p, unsigned char*
     // of tile 2m and receives the neighbour's (the next 4 dims), the odd one does the same for tile
     // 2m+1.  Each lane then owns one whole 16-byte chunk of the row, 4m + 2 * (g4 % 2) + g4 / 2, and
     // the four lanes of a query store 64 contiguous bytes per instruction.
-    const int64_t ohead = batch * p.o_bs + hq * p.o_hs + (2 * (g4 & 1) + (g4 >> 1)) * 8;
+    const int64_t ohead = batch * po.o_bs + hq * po.o_hs + (2 * (g4 & 1) + (g4 >> 1)) * 8;
 #pragma unroll
     for (int qt = 0; qt < 2; ++qt) {
-      uint16_t* orow = p.o + (ohead + qpos[qt] * p.o_rs);
+      uint16_t* orow = po.o + (ohead + qpos[qt] * po.o_rs);
 #pragma unroll
       for (int m = 0; m < 4; ++m) {
         uint32_t w[2][2];
@@ -572,9 +576,9 @@ __device__ __forceinline__ void run_pass_narrow(const KParams& p, unsigned char*
     }
     // ln sum_j exp(scale * q.k_j) = (mref + log2 l) * ln 2; the lane quarters g4 = 0, 1 store the values of
     // query tiles 0, 1, the other two (and lanes of clamped rows) repeat them
-    if (p.lse != nullptr) {
+    if (po.lse != nullptr) {
       const int qt = g4 & 1;
-      p.lse[batch * p.lse_bs + hq * p.lse_hs + (qt ? qpos[1] : qpos[0]) * p.lse_ts] =
+      po.lse[batch * po.lse_bs + hq * po.lse_hs + (qt ? qpos[1] : qpos[0]) * po.lse_ts] =
           ((qt ? mref[1] : mref[0]) + __builtin_amdgcn_logf(qt ? l_tot[1] : l_tot[0])) * 0.6931471805599453f;
     }
   }
@@ -611,7 +615,7 @@ __global__ __launch_bounds__(NARROW_WAVES * 64, 2) void intra_fwd_kernel_narrow(
     const uint32_t mine = redo[threadIdx.x & (REDO_WORDS - 1)];
     if (__builtin_amdgcn_ballot_w64(mine != 0) == 0) return;  // the usual case
   }
-  run_pass_narrow<MAP, HP, SM_EXACT, FAST>(p, smem, redo);
+  run_pass_narrow<MAP, HP, SM_EXACT, FAST>(args_again<KParams>(), smem, redo);
 }
 
 }  // namespace intra
