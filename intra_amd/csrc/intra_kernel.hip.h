@@ -494,12 +494,10 @@ __device__ __forceinline__ void run_pass(const KParams& p, unsigned char* smem, 
   const int wq0 = t0 + (wave / HP) * 32;
   const bool wave_active = wq0 <= t1;
   const int wq_last = im_min(wq0 + 31, t1);
-  bool row_valid[2];
   int lo_l[2], hi_l[2];
   int64_t qpos[2];
 #pragma unroll
   for (int qt = 0; qt < 2; ++qt) {
-    row_valid[qt] = wq0 + 16 * qt + l16 <= t1;
     const int tq = im_min(wq0 + 16 * qt + l16, t1);
     lo_l[qt] = map.klo(tq);
     hi_l[qt] = im_min(map.khi(tq), nk - 1);
@@ -673,7 +671,7 @@ __device__ __forceinline__ void run_pass(const KParams& p, unsigned char* smem, 
   bf16x8 ka[8];
   // HALF: which half of its tile the V reads (block j) and the K reads (block j + 2, one tile
   // further) address: the same for both.
-  auto steady = [&](const floatx4 (&s)[2][2], floatx4 (&n)[2][2], auto half_c, bool mask_next, int kb32_next) {
+  auto steady = [&](const floatx4 (&s)[2][2], floatx4 (&n)[2][2], auto half_c, bool next_wanted, bool mask_next, int kb32_next) {
     constexpr int HALF = decltype(half_c)::value;
     bf16x8 va[8], pb[2];
     float px[8][2];
@@ -755,14 +753,14 @@ __device__ __forceinline__ void run_pass(const KParams& p, unsigned char* smem, 
       m[0] = lane_quad_max(m[0]);
       m[1] = lane_quad_max(m[1]);
     }
-    finish_scores(n, m, mask_next, kb32_next);
+    if (next_wanted) finish_scores(n, m, mask_next, kb32_next);
   };
 
   // Step j: softmax + PV of key block j (scores in `cur`, V rows in the current tile) and QK^T of
   // key block j+1 into `nxt` (its K rows are in ka already; those of block j+2 are read meanwhile).
   // A wavefront runs the steps jq..jp for a run of blocks jq+1..jp it looks at: in step jq only the
   // QK^T half matters, so its scores are preset to -inf (weights 0); in step jp the QK^T half
-  // computes a block the wavefront does not look at, which the per-element mask turns into -inf.
+  // computes a block the wavefront does not look at, whose scores nobody reads (a run sets its own).
   // That keeps one code path through the accumulators.  Maps with a prefix have two such runs
   // (prefix blocks, own range); they are merged when they touch.
   int jq1 = bw_lo - 1, jp1 = bw_hi, jq2 = 1, jp2 = 0;
@@ -791,7 +789,7 @@ __device__ __forceinline__ void run_pass(const KParams& p, unsigned char* smem, 
       if (HALF == 0) load_ka(ka, k0 - k1, FBLOCK32);  // second half of the current tile
       else load_ka(ka, 0, 0);                         // first half of the next tile
     }
-    steady(cur, nxt, half_c, needs_mask(j + 1), kt_lo + 32 * (j + 1));
+    steady(cur, nxt, half_c, j != (in2 ? jp2 : jp1), needs_mask(j + 1), kt_lo + 32 * (j + 1));
   };
 
   // ---------------------------------------------------------------- main loop
@@ -846,8 +844,8 @@ __device__ __forceinline__ void run_pass(const KParams& p, unsigned char* smem, 
     // 2^-100 .. 2^60 (no weight overflowed, and the largest ones are far from underflow).  The
     // integer comparison of the bit patterns also catches a negative or NaN sum.
     const uint32_t lb0 = __float_as_uint(l_tot[0]), lb1 = __float_as_uint(l_tot[1]);
-    const bool bad = wave_active && ((row_valid[0] && !(lb0 >= 0x0d800000u && lb0 <= 0x5d800000u)) ||
-                                     (row_valid[1] && !(lb1 >= 0x0d800000u && lb1 <= 0x5d800000u)));
+    // (A clamped lane repeats the block's last row, and its sum.)
+    const bool bad = wave_active && (!(lb0 >= 0x0d800000u && lb0 <= 0x5d800000u) || !(lb1 >= 0x0d800000u && lb1 <= 0x5d800000u));
     if (INTRA_ABLATE == 0 && __builtin_amdgcn_ballot_w64(bad) != 0 && lane == 0)  // (an ablated pass is not run again)
       __hip_atomic_fetch_or(&redo[(cw.round >> 5) & (REDO_WORDS - 1)], 1u << (cw.round & 31), __ATOMIC_RELAXED,
                             __HIP_MEMORY_SCOPE_WORKGROUP);
