@@ -571,15 +571,31 @@ intra::BwdGrid bwd_grid(const intra::BParams& p, int rows, int hgroups) {
 }
 
 // dQ of a forward map: row blocks of 256 / hp queries of hp heads; also writes D = rowsum(dO o O)
+template <class R, class LEAD = intra::NoLeadingKeys>
+int launch_bwd_dq(const intra::BParams& p, int hp, hipStream_t stream) {
+  switch (hp) {
+    case 4: return launch_bwd<R, intra::BWD_DQ, 4, LEAD>(p, stream);
+    case 2: return launch_bwd<R, intra::BWD_DQ, 2, LEAD>(p, stream);
+    default: return launch_bwd<R, intra::BWD_DQ, 1, LEAD>(p, stream);
+  }
+}
 template <class MAP>
 int run_bwd_dq(intra::BParams p, int hp, hipStream_t stream) {
   using R = intra::QueryRows<MAP>;
   p.grid = bwd_grid<R>(p, 256 / hp, p.ratio / hp);
-  switch (hp) {
-    case 4: return launch_bwd<R, intra::BWD_DQ, 4>(p, stream);
-    case 2: return launch_bwd<R, intra::BWD_DQ, 2>(p, stream);
-    default: return launch_bwd<R, intra::BWD_DQ, 1>(p, stream);
-  }
+  return launch_bwd_dq<R>(p, hp, stream);
+}
+
+// dQ of image gather0: the patch runs, and in front of them (at large grids they meet the most columns)
+// the text rows, the chunks of two groups in one row block where that keeps it as short as a patch
+// run's (pick_text_merge).
+int run_bwd_dq_gather0(intra::BParams p, int hp, hipStream_t stream) {
+  using R = intra::QueryRows<MapImgPatch>;
+  using Text = intra::QueryRows<MapImgTextRows>;
+  p.grid = bwd_grid<R>(p, 256 / hp, p.ratio / hp);
+  p.lead = bwd_grid<Text>(p, 256 / hp, p.ratio / hp);
+  p.lead_first = 1;
+  return launch_bwd_dq<R, Text>(p, hp, stream);
 }
 
 // dK and dV over a key-row map: row blocks of 128 keys of one kv head, all query heads of its group
@@ -749,7 +765,7 @@ int run_bwd(int domain, const void* q, const void* k, const void* v, const void*
       rc = run_bwd_keys_lead<intra::KeyRowsImgGroup<false>, intra::KeyRowsText>(p, st);
       return rc ? rc : run_bwd_lead_reduce(p, ns, st);
     case MAP_IMG_GATHER0:  // grid keys against the grid queries around them, plus their group's text queries
-      if ((rc = run_bwd_dq<MapImgGather0>(p, sh.hp, st))) return rc;
+      if ((rc = run_bwd_dq_gather0(p, sh.hp, st))) return rc;
       if ((rc = run_bwd_keys_lead<intra::KeyRowsImgWindow, intra::KeyRowsText>(p, st))) return rc;
       if ((rc = run_bwd_keys<intra::KeyRowsImgGroup<true>>(p, st))) return rc;
       return run_bwd_lead_reduce(p, ns, st);

@@ -761,13 +761,16 @@ __device__ __forceinline__ void bwd_rows(const BParams& p, const BwdGrid& g, con
 
 struct NoLeadingKeys {};
 
-// One launch: the workgroups of RMAP and, with LEAD, those of the keys that every (later) query sees
-// (KeyRowsLeading).  The leading keys are few rows with very many columns, whose launch of its own
+// One launch: the workgroups of RMAP and, with LEAD, those of a second kind of rows - for dK / dV the keys
+// that every (later) query sees (KeyRowsLeading), for dQ of image Gather 0 the text queries (below).  The leading keys are few rows with very many columns, whose launch of its own
 // had one thin round of workgroups; here the rest of the GPU works on the other keys meanwhile.  The
 // longer kind of workgroup comes first, so that the short ones fill the last round.  Against two
 // launches of their own, dK (three products) and dV (two) with 8 wavefronts: a training step with 64
 // sinks 551 -> 505 us (window 575, S = 8192, 32 / 8 heads), 870 -> 817 us (block Scatter G = 2,
 // S = 6000), image Scatter 1024^2 at 24 heads 339 -> 327 us.
+// dQ of image Gather 0: the text rows and the patch runs have maps of their own.  One map for both
+// chose between their fields at every tile (383 scalar instructions per step of two blocks, 46 of
+// them and 2 more moving spilled scalars; the patch runs alone issue 291 and 18).
 template <class RMAP, int MODE, int HP, class LEAD = NoLeadingKeys>
 __global__ __launch_bounds__(bwd_waves(MODE) * 64) void intra_bwd_kernel(const BParams p) {
   __shared__ __attribute__((aligned(1024))) unsigned char smem[bwd_ring_slots(MODE) * BWD_SLOT];
@@ -775,7 +778,7 @@ __global__ __launch_bounds__(bwd_waves(MODE) * 64) void intra_bwd_kernel(const B
   if constexpr (!std::is_same_v<LEAD, NoLeadingKeys>) {
     const int lead_block = block - (p.lead_first ? 0 : p.grid.blocks);
     if (lead_block >= 0 && lead_block < p.lead.blocks) {
-      bwd_rows<LEAD, MODE, HP, true>(p, p.lead, lead_block, smem);
+      bwd_rows<LEAD, MODE, HP, MODE == BWD_DKV>(p, p.lead, lead_block, smem);
       return;
     }
     if (p.lead_first) block -= p.lead.blocks;

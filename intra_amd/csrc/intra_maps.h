@@ -277,8 +277,8 @@ struct TileRows {
 // row, so that the text keys (a prefix every query sees) and most of the window keys are shared.
 // The window keys of the set are the union of the patches' windows, cut into blocks of 4 grid
 // columns x 16 grid rows = 64 keys; window starts are multiples of 4, so a patch sees exactly 4
-// consecutive blocks.  The text queries of gather0 keep their scatter rows (MapImgScatter in
-// text_only mode); MapImgGather0 below puts both kinds of sets into one launch.
+// consecutive blocks.  The text queries of gather0 keep their scatter rows
+// (MapImgTextRows); MapImgGather0F below puts both kinds of sets into the forward launch.
 struct MapImgPatch {
   static constexpr bool kHasPrefix = true;
   int W, T, pg, np, R, C0, r0, cfirst, nblk;
@@ -339,29 +339,7 @@ struct MapImgPatch {
   IM_HD int tile_rel(int kind, int i) const { return kind == TILE_LINEAR ? i : (i >> 2) * W + (i & 3); }
 };
 
-// ---- image gather0, all rows: sets 0..7 are the text-only scatter sets (the longest work items,
-// so they come first), sets 8.. the patch runs.
-struct MapImgGather0 {
-  static constexpr bool kHasPrefix = true;
-  bool is_text;
-  MapImgScatter sc;
-  MapImgPatch pa;
-  static IM_HD int num_sets(const IntraGeom& ge) { return 8 + MapImgPatch::num_sets(ge); }
-  static IM_HD int max_nq(const IntraGeom& ge) { return im_max(ge.text_len / 8, MapImgPatch::max_nq(ge)); }
-  IM_HD MapImgGather0(const IntraGeom& ge, int set, int t0)
-      : is_text(set < 8), sc(ge, set < 8 ? set : 0, t0, 1), pa(ge, set < 8 ? 0 : set - 8, t0) {}
-  IM_HD int nq() const { return is_text ? sc.nq() : pa.nq(); }
-  IM_HD int nk() const { return is_text ? sc.nk() : pa.nk(); }
-  IM_HD int kpre() const { return is_text ? 0 : pa.kpre(); }
-  IM_HD int qpos(int t) const { return is_text ? sc.qpos(t) : pa.qpos(t); }
-  IM_HD int kpos(int t) const { return is_text ? sc.kpos(t) : pa.kpos(t); }
-  IM_HD int klo(int tq) const { return is_text ? 0 : pa.klo(tq); }
-  IM_HD int khi(int tq) const { return is_text ? sc.khi(tq) : pa.khi(tq); }
-  IM_HD bool tile_at(int t_first, TileAt& a) const { return is_text ? sc.tile_at(t_first, a) : pa.tile_at(t_first, a); }
-  IM_HD int tile_rel(int kind, int i) const { return kind == TILE_STRIDED ? sc.tile_rel(kind, i) : pa.tile_rel(kind, i); }
-};
-
-// ---- The forward launch of image gather0 deals the text queries like this.  A scatter group has
+// ---- The launches of image gather0 (forward and dQ) deal the text queries like this.  A scatter group has
 // only text_len / 8 text queries (64 at 512 text tokens), a quarter of a row block, and they see
 // the text keys and the group's grid keys; so the text chunks of tm = 1 or 2 groups share one row
 // block (8 / tm sets of text rows per head).  With two groups A, B the key list is
@@ -406,6 +384,18 @@ struct MapImgTextRows {
     const int p = grid(front ? cA : cB, front ? t : (int)tt - T);
     return tt < (unsigned)T ? (int)tt : p;
   }
+  // (a grid tile has to start with a grid row)
+  IM_HD bool tile_at(int t_first, TileAt& a) const {
+    const int tt = t_first - lead, u = tt < 0 ? t_first : tt - T;
+    if (tt >= 0 && tt + 64 <= T) {
+      a = TileAt{tt, TILE_LINEAR};
+      return true;
+    }
+    if (tt < 0 ? t_first + 64 > lead : u < 0) return false;  // across two parts
+    a = TileAt{grid(tt < 0 ? cA : cB, u), TILE_STRIDED};
+    return u == (int)fd_div(u, dWq) * (W / 4);
+  }
+  IM_HD int tile_rel(int kind, int i) const { return kind == TILE_LINEAR ? i : grid(0, i); }
   // with two groups the queries of the second chunk start behind the first group's grid keys
   IM_HD int klo(int tq) const { return 8 * tq >= T ? lead : 0; }
   IM_HD int khi(int tq) const { return klo(tq) + T + nimg - 1; }

@@ -81,7 +81,8 @@ int main() {
     IntraGeom ge = geom(text + width * width); ge.width = width; ge.text_len = text;
     keys<MapImgScatter>(ge, "image scatter"); columns<KeyRowsImgGroup<false>>(ge, "grid keys"); columns<KeyRowsImgGroup<true>>(ge, "grid keys, text columns");
     columns<KeyRowsImgWindow>(ge, "window keys");
-    for (int pg : {1, 2, 4}) { if ((width / 8) % pg) continue; ge.pg = pg; keys<MapImgGather0>(ge, "gather0"); }
+    for (int pg : {1, 2, 4}) { if ((width / 8) % pg) continue; ge.pg = pg; keys<MapImgPatch>(ge, "patch runs"); }
+    for (int tm : {1, 2}) { ge.tm = tm; keys<MapImgTextRows>(ge, "text rows"); }
   }
   report("image", p, o);
   return 0;
