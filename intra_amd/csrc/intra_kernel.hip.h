@@ -300,6 +300,19 @@ __device__ __forceinline__ void run_pass(const KParams& p, unsigned char* smem, 
   const int l16 = lane & 15;  // row or column of a 16x16 MFMA tile
   const int g4 = lane >> 4;   // which quarter of the wavefront
 
+  // (A kernel of one exact pass has scalar registers enough to keep the arguments: reading them again
+  // cost Gather 1 at S=7552 44.1 -> 45.3 us, image Gather 0 2048^2 at 6 heads 128.2 -> 130.4.)
+  // The look-up of the next work item, inside the tile loop: for the windows, whose items are about 9
+  // tiles, it reads the arguments again and is marked unlikely; for the longer items of the other maps
+  // it keeps them, as measured (read again / kept, us, same box: Scatter G=8 S=32768 981 / 974, G=2
+  // S=65536 14464 / 14167, Gather 1 S=8192 85.8 / 85.1; the mark, with / without: window 576 S=32768
+  // 332 / 337, S=3000 B=2 62.6 / 63.6, Scatter G=8 S=32768 995 / 988).
+  constexpr bool SWITCH_APART = std::is_same_v<MAP, MapLlmWindow> || std::is_same_v<MAP, MapLlmWindowSink>;
+  auto args = [&]() -> const KParams& {
+    if constexpr (FAST || REDO) return args_again<KParams>();
+    else return p;
+  };
+
   // ---------------------------------------------------------------- persistent loop over work items
   // The grid holds about one workgroup per CU and every workgroup walks through several work items
   // (row blocks), which saves the dispatch gap between consecutive workgroups on a CU; see
@@ -307,8 +320,12 @@ __device__ __forceinline__ void run_pass(const KParams& p, unsigned char* smem, 
   const int xcd = blockIdx.x & 7;
   const int wgs_per_xcd = gridDim.x >> 3;
   const int wg_in_xcd = blockIdx.x >> 3;
+  auto switch_args = [&]() -> const KParams& {
+    if constexpr (SWITCH_APART) return args();
+    else return p;
+  };
   auto locate = [&](int round, Where& w) {
-    return locate_item<MAP, POS, REDO>(args_again<KParams>(), xcd, wgs_per_xcd, wg_in_xcd, redo, round, w);
+    return locate_item<MAP, POS, REDO>(switch_args(), xcd, wgs_per_xcd, wg_in_xcd, redo, round, w);
   };
   auto range_of = [&](const MAP& map, int mblk) { return range_of_block<MAP, POS>(map, mblk); };
 
@@ -343,7 +360,7 @@ __device__ __forceinline__ void run_pass(const KParams& p, unsigned char* smem, 
     int prev_round;    // round of the work item before it
   };
   auto feed_for = [&](const Where& w, int prev_round) {
-    const KParams& p = args_again<KParams>();
+    const KParams& p = switch_args();
     const MAP map(p.geom, w.set, w.mblk * POS);
     return Feed{map, range_of(map, w.mblk), map.nk(), -2, true,
                 reinterpret_cast<const char*>(p.k + w.batch * p.k_bs + w.kvh * p.k_hs),
@@ -358,10 +375,10 @@ __device__ __forceinline__ void run_pass(const KParams& p, unsigned char* smem, 
   Feed fd = feed_for(cw, -1);
   // request the next slot of the stream into a ring slot (byte offset inside the K ring and the V ring)
   auto feed_tile = [&](int slot_off) {
-    if (__builtin_expect(fd.tile < 0, 0)) {  // 128 Q rows: rows of four wavefronts, two per part
+    if (SWITCH_APART ? __builtin_expect(fd.tile < 0, 0) : fd.tile < 0) {  // 128 Q rows: rows of four wavefronts, two per part
 #pragma unroll
       for (int gi = 0; gi < GROUPS_PER_WAVE; ++gi) {
-        const KParams& p = args_again<KParams>();
+        const KParams& p = args();
         const uint32_t q_rs_b = p.q_rs_bytes;
         const int grp = wave * GROUPS_PER_WAVE + gi;
         const int rho = 4 * grp + ld_row;  // row of the part
@@ -401,7 +418,7 @@ __device__ __forceinline__ void run_pass(const KParams& p, unsigned char* smem, 
       }
     }
     ++fd.tile;
-    if (__builtin_expect(fd.tile == fd.rg.ntiles && fd.more, 0)) {
+    if (SWITCH_APART ? __builtin_expect(fd.tile == fd.rg.ntiles && fd.more, 0) : fd.tile == fd.rg.ntiles && fd.more) {
       Where w;
       if (locate(fd.w.round + 1, w)) fd = feed_for(w, fd.w.round);
       else fd.more = false;  // nothing left: keep requesting the (clamped) last row, nobody reads it
@@ -474,7 +491,7 @@ __device__ __forceinline__ void run_pass(const KParams& p, unsigned char* smem, 
 
   for (;;) {
   INTRA_DIAG(const long long t_a = wall_clock64();)
-  const KParams& pi = args_again<KParams>();
+  const KParams& pi = args();
   const int set = cw.set, batch = cw.batch, kvh = cw.kvh, mblk = cw.mblk, hg = cw.hg;
   const int t0 = mblk * POS;
   const MAP map(pi.geom, set, t0);
@@ -837,7 +854,7 @@ __device__ __forceinline__ void run_pass(const KParams& p, unsigned char* smem, 
 
   // ---------------------------------------------------------------- normalise and store
   {
-  const KParams& po = args_again<KParams>();
+  const KParams& po = args();
   const float l_tot[2] = {lane_quad_sum(l_acc[0]), lane_quad_sum(l_acc[1])};
   if (FAST) {
     // Weights were formed without a reference: the result is good iff the weight sum stayed inside

@@ -47,13 +47,20 @@ __device__ __forceinline__ void run_pass_narrow(const KParams& p, unsigned char*
   const int l16 = lane & 15;  // row or column of a 16x16 MFMA tile
   const int g4 = lane >> 4;   // which quarter of the wavefront
 
+  // (A kernel of one exact pass has scalar registers enough to keep the arguments: reading them again
+  // cost Gather 1 at S=7552 44.1 -> 45.3 us, image Gather 0 2048^2 at 6 heads 128.2 -> 130.4.)
+  auto args = [&]() -> const KParams& {
+    if constexpr (FAST || REDO) return args_again<KParams>();
+    else return p;
+  };
+
   // ---------------------------------------------------------------- persistent loop over work items
   // Two workgroups per CU, each walking through its work items in the order of locate_item.
   const int xcd = blockIdx.x & 7;
   const int wgs_per_xcd = gridDim.x >> 3;
   const int wg_in_xcd = blockIdx.x >> 3;
   auto locate = [&](int round, Where& w) {
-    return locate_item<MAP, POS, REDO>(args_again<KParams>(), xcd, wgs_per_xcd, wg_in_xcd, redo, round, w);
+    return locate_item<MAP, POS, REDO>(args(), xcd, wgs_per_xcd, wg_in_xcd, redo, round, w);
   };
   auto range_of = [&](const MAP& map, int mblk) { return range_of_block<MAP, POS>(map, mblk); };
 
@@ -80,7 +87,7 @@ __device__ __forceinline__ void run_pass_narrow(const KParams& p, unsigned char*
     int prev_round;    // round of the work item before it
   };
   auto feed_for = [&](const Where& w, int prev_round) {
-    const KParams& p = args_again<KParams>();
+    const KParams& p = args();
     const MAP map(p.geom, w.set, w.mblk * POS);
     return Feed{map, range_of(map, w.mblk), map.nk(), 0, true,
                 reinterpret_cast<const char*>(p.k + w.batch * p.k_bs + w.kvh * p.k_hs),
@@ -167,7 +174,7 @@ __device__ __forceinline__ void run_pass_narrow(const KParams& p, unsigned char*
   // through the hand-counted direct-to-LDS path between their issue and their first use.
   u32x4 qf[2][4];
   auto request_q = [&](const Where& w) {
-    const KParams& p = args_again<KParams>();
+    const KParams& p = args();
     const int t0 = w.mblk * POS;
     const MAP map(p.geom, w.set, t0);
     const int t1 = im_min(t0 + POS, map.nq()) - 1;
@@ -204,7 +211,7 @@ __device__ __forceinline__ void run_pass_narrow(const KParams& p, unsigned char*
 
   for (;;) {
   INTRA_DIAG(const long long t_a = wall_clock64();)
-  const KParams& pi = args_again<KParams>();
+  const KParams& pi = args();
   const int set = cw.set, batch = cw.batch, kvh = cw.kvh, mblk = cw.mblk, hg = cw.hg;
   const int t0 = mblk * POS;
   const MAP map(pi.geom, set, t0);
@@ -533,7 +540,7 @@ __device__ __forceinline__ void run_pass_narrow(const KParams& p, unsigned char*
 
   // ---------------------------------------------------------------- normalise and store
   {
-  const KParams& po = args_again<KParams>();
+  const KParams& po = args();
   const float l_tot[2] = {lane_quad_sum(l_acc[0]), lane_quad_sum(l_acc[1])};
   if (FAST) {
     // Weights were formed without a reference: the result is good iff the weight sum stayed inside
