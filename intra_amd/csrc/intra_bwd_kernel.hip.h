@@ -77,18 +77,18 @@ constexpr int bwd_ring_slots(int mode) { return mode == BWD_DKV ? 4 : 3; }
 // 64 lanes x 4 bytes from per-lane global addresses to 256 consecutive LDS bytes at lds_addr (the
 // active lanes' parts of them), like dma_group
 __device__ __forceinline__ void dma_dwords(const void* gsrc, uint32_t lds_addr) {
-  asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dword %0, off" : : "v"(gsrc), "s"(lds_addr) : "memory");
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off" : : "v"(gsrc), "s"(lds_addr) : "memory");
 }
 
 // The same two with a wave-uniform address and 32-bit per-lane byte offsets
 template <int LDS_OFFSET>
 __device__ __forceinline__ void dma_rows(const void* base, uint32_t offset, uint32_t lds_addr) {
-  asm volatile("s_add_u32 m0, %2, %3\n\tglobal_load_lds_dwordx4 %0, %1"
+  asm volatile("s_add_u32 m0, %2, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
                : : "v"(offset), "s"(base), "s"(lds_addr), "n"(LDS_OFFSET) : "memory", "scc");
 }
 template <int LDS_OFFSET>
 __device__ __forceinline__ void dma_scalars(const void* base, uint32_t offset, uint32_t lds_addr) {
-  asm volatile("s_add_u32 m0, %2, %3\n\tglobal_load_lds_dword %0, %1"
+  asm volatile("s_add_u32 m0, %2, %3\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1"
                : : "v"(offset), "s"(base), "s"(lds_addr), "n"(LDS_OFFSET) : "memory", "scc");
 }
 

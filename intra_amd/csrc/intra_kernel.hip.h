@@ -164,8 +164,10 @@ constexpr int LDS_BYTES = RING_BYTES + REDO_WORDS * 4;
 // (wave-uniform).  Issued as inline assembly so that the compiler does not put a full vmcnt(0)
 // wait in front of every later LDS read; completion is tracked by hand with vmcnt (see the main
 // loop), and the "memory" clobber keeps LDS accesses from moving across it at compile time.
+// The LDS address travels in M0, and a scalar write of M0 needs one wait state before a load to LDS reads
+// it (s_nop); the compiler adds none inside inline assembly.
 __device__ __forceinline__ void dma_group(const void* gsrc, uint32_t lds_addr) {
-  asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off" : : "v"(gsrc), "s"(lds_addr) : "memory");
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" : : "v"(gsrc), "s"(lds_addr) : "memory");
 }
 
 // Workgroup barrier that leaves the `pending` most recent direct-to-LDS loads of this wavefront
