@@ -437,6 +437,12 @@ __device__ __forceinline__ void bwd_rows(const BParams& p, const BwdGrid& g, con
   if (DEEP) {
     load_rows();
     __builtin_amdgcn_s_waitcnt((0 & 15) | (7 << 4) | (15 << 8) | (0 << 14));  // vmcnt(0)
+    // They stay in the accumulation half of the register file, where an MFMA reads its B operand as well.  Of
+    // its own accord the compiler puts nothing but accumulators there, and copied them, or the V fragments,
+    // between the halves inside the blocks: of few sinks 44 moves and 13 waiting instructions per 64 MFMAs.
+    // With this no block holds a move (training step, window 575 with 64 sinks, S=8192, us: 471.3 -> 467.2).
+#pragma unroll
+    for (int i = 0; i < 8; ++i) asm volatile("" : "+a"(r1f[i >> 2][i & 3]), "+a"(r2f[i >> 2][i & 3]));
   }
   int slot0 = 0, slot1 = BWD_SLOT, slot2 = 2 * BWD_SLOT, slot3 = 3 * BWD_SLOT;
   bool fresh = n_steps >= 3;  // the most recent request is for the step after the next

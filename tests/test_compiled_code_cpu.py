@@ -1,6 +1,11 @@
-"""The direct-to-LDS requests in the compiled library.  They are inline assembly, for which the compiler inserts
-none of the wait states that the hardware asks for: one between a scalar write of M0 (the LDS address) and the
-load, five between a vector instruction that writes a scalar register and a load that takes its address from it."""
+"""What the kernels rely on in the compiled library, read from its disassembly.
+
+The direct-to-LDS requests are inline assembly, for which the compiler inserts none of the wait states that the
+hardware asks for: one between a scalar write of M0 (the LDS address) and the load, five between a vector
+instruction that writes a scalar register and a load that takes its address from it.
+
+The blocks of dK / dV keep 64 MFMAs and what stands between them in one order: nothing moves between the two
+halves of the register file there (one wavefront per SIMD, nothing hides such moves and the waits they bring)."""
 import os
 import re
 import shutil
@@ -79,9 +84,37 @@ def test_the_check_itself():
     assert request_faults(["\tv_readlane_b32 s3, v9, 1\n", "\ts_mov_b32 m0, s9\n", "\ts_nop 3\n", load])[1] == []
 
 
-def test_every_request_has_its_wait_states(code_object):
+def disassembly(code_object):
     with subprocess.Popen([llvm_tool("llvm-objdump"), "-d", "--no-show-raw-insn", code_object], text=True,
                           stdout=subprocess.PIPE) as dump:
-        n, faults = request_faults(dump.stdout)
-    assert dump.returncode == 0 and n > 1000
+        yield from dump.stdout
+    assert dump.returncode == 0
+
+
+def test_every_request_has_its_wait_states(code_object):
+    n, faults = request_faults(disassembly(code_object))
+    assert n > 1000
     assert not faults, (len(faults), faults[:4])
+
+
+def blocks(lines, kernel, mfmas):
+    """The instructions from the first to the last of the `mfmas` MFMAs in front of a branch, where there are as
+    many without a branch between them, in the kernels whose name contains `kernel`"""
+    inside, run = False, []
+    for line in lines:
+        if line.endswith(">:\n"):
+            inside, run = kernel in line, []
+        elif inside and line.startswith("\t"):
+            op = line.split()[0]
+            if not op.startswith(("s_cbranch", "s_branch", "s_endpgm")):
+                run.append(op)
+                continue
+            at = [i for i, o in enumerate(run) if o.startswith("v_mfma")]
+            if len(at) >= mfmas:
+                yield run[at[-mfmas]:at[-1] + 1]
+            run = []
+
+
+def test_no_moves_between_register_halves_in_the_blocks_of_dk_and_dv(code_object):
+    moves = [sum(op.startswith("v_accvgpr") for op in block) for block in blocks(disassembly(code_object), "intra_bwd_kernel", 64)]
+    assert len(moves) >= 30 and not any(moves), moves
