@@ -546,7 +546,8 @@ template <class RMAP, int MODE, int HP, class LEAD = intra::NoLeadingKeys>
 int launch_bwd(const intra::BParams& p, hipStream_t stream) {
   const int64_t grid = (int64_t)p.grid.blocks + p.lead.blocks;
   if (p.grid.blocks <= 0 || p.lead.blocks < 0 || grid > 0x7fffffff) return fail(INTRA_ERR_UNSUPPORTED, "backward needs more than 2^31 workgroups");
-  hipLaunchKernelGGL((intra::intra_bwd_kernel<RMAP, MODE, HP, LEAD>), dim3((unsigned)grid), dim3(intra::bwd_waves(MODE) * 64), 0, stream, p);
+  const auto kernel = p.far_rows ? intra::intra_bwd_kernel<RMAP, MODE, HP, LEAD, true> : intra::intra_bwd_kernel<RMAP, MODE, HP, LEAD, false>;
+  hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(intra::bwd_waves(MODE) * 64), 0, stream, p);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return fail(INTRA_ERR_HIP, "kernel launch failed: %s", hipGetErrorString(e));
   return INTRA_OK;
@@ -723,7 +724,7 @@ int run_bwd(int domain, const void* q, const void* k, const void* v, const void*
   p.lse_bs = ls[0]; p.lse_hs = ls[1]; p.lse_ts = ls[2];
   p.ds_bs = (int64_t)H * S; p.ds_hs = S;
   p.B = B; p.H = H; p.Hkv = Hkv; p.ratio = H / Hkv;
-  p.far_rows = 0;
+  p.far_rows = S >= 1 << 30;  // (four bytes a token of the workspace)
   for (const int64_t* st : all)
     if (((int64_t)S - 1) * st[1] * 2 + 256 > UINT32_MAX) p.far_rows = 1;
   p.scale = scale;

@@ -62,7 +62,7 @@ struct BParams {
   int64_t dq_bs, dq_rs, dq_hs, dk_bs, dk_rs, dk_hs, dv_bs, dv_rs, dv_hs;
   int64_t lse_bs, lse_hs, lse_ts, ds_bs, ds_hs;  // dsum is contiguous over tokens
   int B, H, Hkv, ratio;
-  int far_rows;      // some row of q, k, v or dout is 4 GiB or more behind the first of its head
+  int far_rows;      // some row of q, k, v or dout, or a token's workspace, is 4 GiB or more behind the first of its head
   IntraGeom geom;
   float scale;       // softmax scale
   float scale_log2;  // scale * log2(e)
@@ -94,14 +94,15 @@ __device__ __forceinline__ void dma_scalars(const void* base, uint32_t offset, u
 
 // The work of one workgroup, number `block` of the grid `g`.  RMAP: row map (intra_bwd_maps.h).
 // PARTIAL: where there are several sets, the results are partial sums over the set's columns, written
-// as fp32 to p.part instead of bf16 to dk / dv (leading keys).
+// as fp32 to p.part instead of bf16 to dk / dv (leading keys).  FAR: the columns are requested by 64-bit
+// addresses.
 //
 // MFMA layout (v_mfma_f32_16x16x32_bf16, as in the forward kernel): a block of 32 columns times the
 // wavefront's 32 rows is 2 x 2 tiles [ct][rt] with 4 k-steps; lane (l16 = lane % 16, g4 = lane / 16)
 // holds columns 16*ct + 4*g4 .. +3 of row 16*rt + l16.  The packed weights of a row tile are the B
 // operand of the accumulation, whose 32-column reduction is numbered slot s of lane quarter g4 =
 // column 16*(s/4) + 4*g4 + s%4; the transposing reads of the X tile follow that numbering.
-template <class RMAP, int MODE, int HP, bool PARTIAL>
+template <class RMAP, int MODE, int HP, bool PARTIAL, bool FAR>
 __device__ __forceinline__ void bwd_rows(const BParams& p, const BwdGrid& g, const int block, unsigned char* const smem) {
   constexpr int NW = bwd_waves(MODE);
   constexpr bool ROWS_ARE_QUERIES = MODE == BWD_DQ;
@@ -342,13 +343,20 @@ __device__ __forceinline__ void bwd_rows(const BParams& p, const BwdGrid& g, con
   }
   // Requests.  A lane's rows of a tile are named by 32-bit byte offsets from a wave-uniform address.  For
   // tiles whose positions follow one of the maps' patterns (tile_at) the offsets stay in registers from
-  // tile to tile and only that address moves; other tiles (cut by the end of the columns, or across two
-  // parts of them) get offsets of their own, from the tensor's start.  The query heads of a group share
-  // the offsets.  With the addresses worked out per lane and request (a 64-bit multiply-add each, behind a
-  // 64-bit product for the head's base) a step of dK / dV issued about 120 instructions for its requests,
-  // none of them behind an MFMA.  With these and the order of the block below (same box, training steps,
-  // us): Scatter G=8 S=32768 4385 -> 4189, its dK / dV launch 2395 -> 2090; image Scatter 2048^2 at 12
-  // heads 1166 -> 1076; window 575 with 64 sinks, S=8192, 486 -> 470; image Gather 0 1024^2 363 -> 344.
+  // tile to tile and only that address moves; a tile cut by the end of the columns (its last row repeated)
+  // and, in maps whose tiles do not all follow a pattern, the others get offsets of their own.  The query
+  // heads of a group share the offsets.  With the addresses worked out per lane and request (a 64-bit
+  // multiply-add each, behind a 64-bit product for the head's base) a step of dK / dV issued about 120
+  // instructions for its requests, none of them behind an MFMA.  With these and the order of the block below
+  // (same box, training steps, us): Scatter G=8 S=32768 4385 -> 4189, its dK / dV launch 2395 -> 2090; image
+  // Scatter 2048^2 at 12 heads 1166 -> 1076; window 575 with 64 sinks, S=8192, 486 -> 470; image Gather 0
+  // 1024^2 363 -> 344.
+  // What ordinary calls do not need stays out of the step, whose scalar registers are few: tensors beyond
+  // the reach of 32-bit offsets have kernels of their own (FAR; inlined here, their addresses kept 10 - 24
+  // scalars in lanes of vector registers), maps whose every tile follows a pattern (kEveryTile) hold no
+  // code for positions key by key, and the ring's slots follow from the present one.  Scalars moved to
+  // lanes and back on the ordinary path of a step: block Scatter 16 -> 1, Scatter 4 -> 0.  Training steps, us:
+  // block Scatter S=6000 780.5 -> 764.9, window 575 with 64 sinks, S=8192, 476.2 -> 468.9.
   constexpr int GROUPS = 16 / NW;  // 4-row groups of either tile per wavefront
   uint32_t vo1[GROUPS], vo2[GROUPS], vos = 0;
 #pragma unroll
@@ -359,18 +367,23 @@ __device__ __forceinline__ void bwd_rows(const BParams& p, const BwdGrid& g, con
   const float* const sbase = (wave & 1 ? p.dsum : p.l2) + (batch * p.ds_bs + kvh * p.ratio * p.ds_hs);
   auto aim = [&](int tile) {  // at the first head of a tile
     const int c = cb + tile * BN;
+    const int last = n_cols - 1 - c;
+    const bool cut = last < BN - 1;
     TileAt at;
-    const bool pattern = c + BN <= n_cols && map.tile_at(c, at);
-    if (pattern && vo_kind != at.kind) {
-      vo_kind = at.kind;
+    const bool pattern = (RMAP::kEveryTile || !cut) && map.tile_at(c, at);
+    if (RMAP::kEveryTile || pattern) {
+      if (vo_kind != at.kind || (RMAP::kEveryTile && cut)) {
+        vo_kind = RMAP::kEveryTile && cut ? -1 : at.kind;
+        auto row_of = [&](int i) { return (uint32_t)map.tile_rel(at.kind, RMAP::kEveryTile ? im_min(i, last) : i); };
 #pragma unroll
-      for (int gi = 0; gi < GROUPS; ++gi) {
-        const uint32_t rel = (uint32_t)map.tile_rel(at.kind, 4 * (wave * GROUPS + gi) + ld_row);
-        vo1[gi] = rel * c1rs + ld_col;
-        vo2[gi] = rel * c2rs + ld_col;
+        for (int gi = 0; gi < GROUPS; ++gi) {
+          const uint32_t rel = row_of(4 * (wave * GROUPS + gi) + ld_row);
+          vo1[gi] = rel * c1rs + ld_col;
+          vo2[gi] = rel * c2rs + ld_col;
+        }
+        if (DEEP) vos = 4 * row_of(lane);
       }
-      if (DEEP) vos = 4 * (uint32_t)map.tile_rel(at.kind, lane);
-    } else if (!pattern) {
+    } else {
       vo_kind = -1;
       at.base = 0;
 #pragma unroll
@@ -386,25 +399,21 @@ __device__ __forceinline__ void bwd_rows(const BParams& p, const BwdGrid& g, con
     a2 = c2base + (uint64_t)base * c2rs;
     if (DEEP) as = reinterpret_cast<const char*>(sbase + base);
   };
-  // tensors beyond the reach of 32-bit offsets: per-lane addresses
-  auto load_far = [&](const Cursor& cu, int slot_off) {
-#pragma unroll
-    for (int gi = 0; gi < GROUPS; ++gi) {
-      const int grp = wave * GROUPS + gi;
-      const uint64_t pos = (uint64_t)map.col_pos(im_min(cb + cu.tile * BN + 4 * grp + ld_row, n_cols - 1));
-      dma_group(c1base + (cu.head * c1hs + pos * c1rs + ld_col), lds_base + slot_off + grp * FGROUP_STRIDE);
-      dma_group(c2base + (cu.head * c2hs + pos * c2rs + ld_col), lds_base + slot_off + FTILE + grp * FGROUP_STRIDE);
-    }
-    if (DEEP)
-      dma_dwords(sbase + (cu.head * p.ds_hs + map.col_pos(im_min(cb + cu.tile * BN + lane, n_cols - 1))),
-                 lds_base + slot_off + 2 * FTILE + 256 * (wave & 1));
-  };
   const uint32_t lds_rows = lds_base + wave * GROUPS * FGROUP_STRIDE;
   const uint32_t lds_scalars = lds_base + 256 * (wave & 1);
   constexpr int REQUESTS = 2 * GROUPS + (DEEP ? 1 : 0);  // per wavefront and step
   auto load_step = [&](const Cursor& cu, int slot_off) {
-    if (p.far_rows) {
-      load_far(cu, slot_off);
+    if constexpr (FAR) {
+      const int c = cb + cu.tile * BN;
+#pragma unroll
+      for (int gi = 0; gi < GROUPS; ++gi) {
+        const uint64_t pos = (uint64_t)map.col_pos(im_min(c + 4 * (wave * GROUPS + gi) + ld_row, n_cols - 1));
+        dma_group(c1base + (cu.head * c1hs + pos * c1rs + ld_col), lds_rows + slot_off + gi * FGROUP_STRIDE);
+        dma_group(c2base + (cu.head * c2hs + pos * c2rs + ld_col), lds_rows + slot_off + FTILE + gi * FGROUP_STRIDE);
+      }
+      if (DEEP)
+        dma_dwords(sbase + (cu.head * p.ds_hs + map.col_pos(im_min(c + lane, n_cols - 1))),
+                   lds_scalars + slot_off + 2 * FTILE);
       return;
     }
     if (ROWS_ARE_QUERIES || cu.head == 0) aim(cu.tile);
@@ -417,7 +426,7 @@ __device__ __forceinline__ void bwd_rows(const BParams& p, const BwdGrid& g, con
       dma_scalars<2 * FTILE>(as, vos, lds_scalars + slot_off);
       a1 += c1hs;  // from one head's addresses to the next one's
       a2 += c2hs;
-      as += 4 * p.ds_hs;
+      as += 4 * (uint32_t)p.ds_hs;  // (S floats)
     }
   };
   // Three tile slots: while step t works on its tile, the tile of step t+1 has landed (the scores
@@ -444,7 +453,9 @@ __device__ __forceinline__ void bwd_rows(const BParams& p, const BwdGrid& g, con
 #pragma unroll
     for (int i = 0; i < 8; ++i) asm volatile("" : "+a"(r1f[i >> 2][i & 3]), "+a"(r2f[i >> 2][i & 3]));
   }
-  int slot0 = 0, slot1 = BWD_SLOT, slot2 = 2 * BWD_SLOT, slot3 = 3 * BWD_SLOT;
+  constexpr int LAST_SLOT = (bwd_ring_slots(MODE) - 1) * BWD_SLOT;
+  int ring = 0;  // slot of the step being computed
+  auto slot_after = [](int s) { return s == LAST_SLOT ? 0 : s + BWD_SLOT; };
   bool fresh = n_steps >= 3;  // the most recent request is for the step after the next
   floatx4 s_cur[2][2];  // [ct][rt]
 #pragma unroll
@@ -467,7 +478,7 @@ __device__ __forceinline__ void bwd_rows(const BParams& p, const BwdGrid& g, con
     // the tile of step t + 3 (dQ: t + 2) into the slot of step t - 1
     fresh = t + (DEEP ? 3 : 2) < n_steps;
     if (fresh) {
-      load_step(ld, DEEP ? slot3 : slot2);
+      load_step(ld, ring == 0 ? LAST_SLOT : ring - BWD_SLOT);
       advance(ld);
     }
     static_for<0, ALT ? 1 : 2>([&](auto blk_c) {
@@ -644,11 +655,10 @@ __device__ __forceinline__ void bwd_rows(const BParams& p, const BwdGrid& g, con
       have = true;
     });
     advance(cur);
-    const int ts = slot0;
-    slot0 = slot1;
-    slot1 = slot2;
     {
-      const int d0 = slot0 - ts, d1 = slot1 - slot0;  // (slot0 and slot1 are the new ones already; ts the old slot0)
+      const int next = slot_after(ring);
+      const int d0 = next - ring, d1 = slot_after(next) - next;
+      ring = next;
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         kb0[i] += d0;
@@ -662,12 +672,6 @@ __device__ __forceinline__ void bwd_rows(const BParams& p, const BwdGrid& g, con
         sb1 += d1;
         asm volatile("" : "+v"(sb0), "+v"(sb1));
       }
-    }
-    if (DEEP) {
-      slot2 = slot3;
-      slot3 = ts;
-    } else {
-      slot2 = ts;
     }
   }
 
@@ -779,19 +783,19 @@ struct NoLeadingKeys {};
 // them and 2 more moving spilled scalars; the patch runs alone issue 291 and 18).
 // With that and shared row blocks for the text rows, 1024^2 at 24 heads: the launch 115 -> 90 us (two
 // traces), the training step 345 -> 323.
-template <class RMAP, int MODE, int HP, class LEAD = NoLeadingKeys>
+template <class RMAP, int MODE, int HP, class LEAD, bool FAR>
 __global__ __launch_bounds__(bwd_waves(MODE) * 64) void intra_bwd_kernel(const BParams p) {
   __shared__ __attribute__((aligned(1024))) unsigned char smem[bwd_ring_slots(MODE) * BWD_SLOT];
   int block = blockIdx.x;
   if constexpr (!std::is_same_v<LEAD, NoLeadingKeys>) {
     const int lead_block = block - (p.lead_first ? 0 : p.grid.blocks);
     if (lead_block >= 0 && lead_block < p.lead.blocks) {
-      bwd_rows<LEAD, MODE, HP, MODE == BWD_DKV>(p, p.lead, lead_block, smem);
+      bwd_rows<LEAD, MODE, HP, MODE == BWD_DKV, FAR>(p, p.lead, lead_block, smem);
       return;
     }
     if (p.lead_first) block -= p.lead.blocks;
   }
-  bwd_rows<RMAP, MODE, HP, false>(p, p.grid, block, smem);
+  bwd_rows<RMAP, MODE, HP, false, FAR>(p, p.grid, block, smem);
 }
 
 // Adds up the partial sums of the leading keys over the chunks and writes their rows of dk

@@ -22,6 +22,7 @@
 //                                          meets the block - all of it or nothing
 //   tile_at(c, a), tile_rel(kind, i)       where the 64 columns from c on sit (TileAt in intra_maps.h), asked
 //                                          for tiles of 64 from block_lo on that lie inside the column list
+//   kEveryTile                             tile_at is true for each of them, and for one cut by the end of the list
 //   kAccumulate                            the results are added to rows another pass has written
 //   static longest(ge)                     columns of the longest row block (maps that share a launch with leading keys)
 //   alternates<RowMap>                     rows 0..63 and 64..127 are the same keys twice over: the
@@ -55,6 +56,7 @@ struct QueryRows {
   IM_HD int block_lo(int r0, int) const { return m.kpre() > 0 ? 0 : m.klo(r0); }
   IM_HD int block_hi(int, int r1) const { return hi(r1); }
   IM_HD bool store(int) const { return true; }
+  static constexpr bool kEveryTile = MAP::kEveryTile;
   static constexpr bool kBlockPredicate = false, kAccumulate = false;
   IM_HD bool sees(int, int) const { return true; }
 };
@@ -82,6 +84,7 @@ struct KeyRowsOf {
   IM_HD int block_lo(int r0, int) const { return lo(r0); }
   IM_HD int block_hi(int, int r1) const { return hi(r1); }
   IM_HD bool store(int) const { return true; }
+  static constexpr bool kEveryTile = MAP::kEveryTile;
   static constexpr bool kBlockPredicate = false, kAccumulate = false;
   IM_HD bool sees(int, int) const { return true; }
 };
@@ -156,6 +159,7 @@ struct KeyRowsBlockScatter {
   IM_HD int block_lo(int r0, int) const { return lo(r0); }
   IM_HD int block_hi(int, int) const { return ncols - 1; }
   IM_HD bool store(int pos) const { return pos >= skip; }
+  static constexpr bool kEveryTile = true;
   static constexpr bool kBlockPredicate = false, kAccumulate = false;
   IM_HD bool sees(int, int) const { return true; }
 };
@@ -187,6 +191,7 @@ struct KeyRowsWindowSink {
   IM_HD int block_lo(int r0, int) const { return r0; }
   IM_HD int block_hi(int, int r1) const { return hi(r1); }
   IM_HD bool store(int pos) const { return pos >= skip; }
+  static constexpr bool kEveryTile = true;
   static constexpr bool kBlockPredicate = false, kAccumulate = false;
   IM_HD bool sees(int, int) const { return true; }
 };
@@ -255,6 +260,7 @@ struct KeyRowsLeading {
   IM_HD int block_lo(int r0, int) const { return lo(r0); }
   IM_HD int block_hi(int, int) const { return c1 - 1; }
   IM_HD bool store(int) const { return true; }
+  static constexpr bool kEveryTile = true;
   static constexpr bool kBlockPredicate = false, kAccumulate = false;
   IM_HD bool sees(int, int) const { return true; }
 };
@@ -287,6 +293,7 @@ struct KeyRowsImgGroup {
   IM_HD int block_lo(int, int) const { return 0; }
   IM_HD int block_hi(int, int) const { return n_cols() - 1; }
   IM_HD bool store(int) const { return true; }
+  static constexpr bool kEveryTile = false;
   static constexpr bool kBlockPredicate = false, kAccumulate = TEXT_COLS_ONLY;
   IM_HD bool sees(int, int) const { return true; }
 };
@@ -391,6 +398,7 @@ struct KeyRowsImgWindow {
   IM_HD int block_lo(int, int) const { return 0; }
   IM_HD int block_hi(int, int) const { return n_cols() - 1; }
   IM_HD bool store(int) const { return true; }
+  static constexpr bool kEveryTile = false;
   static constexpr bool kBlockPredicate = true, kAccumulate = false;
   IM_HD bool sees(int t, int c) const {
     const int pi = c >> 6, ri = patch_row(pi);

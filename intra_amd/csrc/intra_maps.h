@@ -107,7 +107,8 @@ IM_HD int64_t im_min64(int64_t a, int64_t b) { return a < b ? a : b; }
 // Where the 64 keys of a tile sit when the pattern of their positions is one of a few that a loader can
 // keep in registers: key i of the tile is at position base + tile_rel(kind, i), and tile_rel depends on
 // nothing but the launch's geometry.  tile_at answers false for any other tile; it is asked for tiles
-// that lie inside the key list (t_first + 64 <= nk).
+// that lie inside the key list (t_first + 64 <= nk).  kEveryTile: the answer is never false, and it holds for
+// the keys of a tile that the end of the list cuts as well.
 struct TileAt {
   int base, kind;
 };
@@ -124,6 +125,7 @@ IM_HD bool tile_linear(F&& pos, int t_first, TileAt& a) {
 // ---------------------------------------------------------------- LLM scatter: token i in group i % G
 struct MapLlmScatter {
   static constexpr bool kHasPrefix = false;
+  static constexpr bool kEveryTile = true;
   IM_HD int kpre() const { return 0; }
   int G, g, n;
   static IM_HD int num_sets(const IntraGeom& ge) { return ge.G; }
@@ -152,6 +154,7 @@ struct MapLlmScatter {
 // in-set index, so causality in positions equals causality in in-set indices.
 struct MapLlmGather1 {
   static constexpr bool kHasPrefix = false;
+  static constexpr bool kEveryTile = false;
   IM_HD int kpre() const { return 0; }
   int G, g, n;
   FastDiv dG;
@@ -187,6 +190,7 @@ struct MapLlmGather1 {
 // -------------------------- LLM window: 64-query blocks see themselves plus window-64 earlier tokens
 struct MapLlmWindow {
   static constexpr bool kHasPrefix = false;
+  static constexpr bool kEveryTile = true;
   IM_HD int kpre() const { return 0; }
   int S, lookback;
   static IM_HD int num_sets(const IntraGeom&) { return 1; }
@@ -214,6 +218,7 @@ struct MapLlmWindow {
 // with group j; every query sees all text keys plus the grid keys of its own group.
 struct MapImgScatter {
   static constexpr bool kHasPrefix = false;
+  static constexpr bool kEveryTile = false;
   IM_HD int kpre() const { return 0; }
   int W, T, chunk, j, a, b, wq, nimg, text_only;
   FastDiv dWq;
@@ -281,6 +286,7 @@ struct TileRows {
 // (MapImgTextRows); MapImgGather0F below puts both kinds of sets into the forward launch.
 struct MapImgPatch {
   static constexpr bool kHasPrefix = true;
+  static constexpr bool kEveryTile = false;
   int W, T, pg, np, R, C0, r0, cfirst, nblk;
   static IM_HD int win_start(int idx, int np) {
     if (idx == np - 1) return idx * 8 - 8;
@@ -350,6 +356,7 @@ struct MapImgPatch {
 // MapImgScatter: its key bounds are compile-time constants that way, which its main loop needs.)
 struct MapImgTextRows {
   static constexpr bool kHasPrefix = false;
+  static constexpr bool kEveryTile = false;
   IM_HD int kpre() const { return 0; }
   // (few fields: two of these maps are live in the kernel's main loop, in scalar registers)
   int W, T, nimg, nq_, lead, cA, cB, q0;
@@ -440,6 +447,7 @@ IM_HD bool map_tile_rows(const MAP& map, int t_first, TileRows& a) { return map_
 // blocks must not straddle query blocks (the host picks the row-block size accordingly).
 struct MapLlmBlockScatter {
   static constexpr bool kHasPrefix = false;
+  static constexpr bool kEveryTile = false;
   IM_HD int kpre() const { return 0; }
   int G, blk, g, gt, off, n, E, own_base, own_len, qb;
   FastDiv dBlk;
@@ -503,6 +511,7 @@ struct MapLlmBlockScatter {
 // at the window and not at position 0.
 struct MapLlmWindowSink {
   static constexpr bool kHasPrefix = true;
+  static constexpr bool kEveryTile = false;
   int S, window, ns, wlo;
   static IM_HD int num_sets(const IntraGeom&) { return 1; }
   static IM_HD int max_nq(const IntraGeom& ge) { return ge.S; }

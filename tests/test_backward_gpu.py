@@ -68,17 +68,31 @@ def test_scatter_grads(S, G, B, H, Hkv):
     run_case("llm/scatter", "scatter", B, S, H, Hkv, group_num=G)
 
 
-@pytest.mark.parametrize("pattern,kw", [("scatter", dict(group_num=2)), ("window_sink", dict(window=64, n_sink=4))])
-def test_rows_beyond_the_reach_of_32_bit_offsets(pattern, kw):
-    """Token strides of 16 MB: the last rows of 300 are more than 4 GiB behind the first."""
-    S, stride = 300, 1 << 23
-    store = torch.empty(S * stride, dtype=torch.bfloat16, device=DEV)
-    views = [store.as_strided((1, S, 2, 128), (S * stride, stride, 128, 1), 256 * i) for i in range(4)]
-    plain = make(1, S, 2, 2, seed=5)
-    for view, x in zip(views, plain):
-        view.copy_(x)
-    q, k, v, dout = views
-    got = kernel_grads(q, k, v, dout, pattern, **kw)
+FAR_STRIDES = [1 << 23, 6 << 20]  # S = 300: rows beyond 32-bit byte offsets; offsets between 2^31 and 2^32
+
+
+def spread(tensors, stride):
+    """The same values, every token `stride` elements behind the one before it, all in one buffer"""
+    B, S = tensors[0].shape[:2]
+    store = torch.empty(B * S * stride, dtype=torch.bfloat16, device=DEV)
+    views, at = [], 0
+    for x in tensors:
+        views.append(store.as_strided(x.shape, (S * stride, stride, 128, 1), at))
+        views[-1].copy_(x)
+        at += 128 * x.shape[2]
+    return views
+
+
+@pytest.mark.parametrize("stride", FAR_STRIDES)
+@pytest.mark.parametrize("H,Hkv", [(2, 2), (4, 1)])
+@pytest.mark.parametrize("pattern,kw", [
+    ("scatter", dict(group_num=2)), ("gather1", dict(group_num=8)), ("window", dict(window=128)),
+    ("window_sink", dict(window=64, n_sink=4)), ("window_sink", dict(window=64, n_sink=100)),
+    ("block_scatter", dict(group_num=2, block=64)), ("block_scatter", dict(group_num=2, block=256, offset=1, n_sink=4))])
+def test_rows_at_and_beyond_the_reach_of_32_bit_offsets(pattern, kw, H, Hkv, stride):
+    """Tokens 16 MB apart (the last of 300 are more than 4 GiB behind the first) and 12 MB apart."""
+    plain = make(1, 320 if pattern == "gather1" else 300, H, Hkv, seed=5)
+    got = kernel_grads(*spread(plain, stride), pattern, **kw)
     for name, a, b in zip(("dq", "dk", "dv"), got, kernel_grads(*plain, pattern, **kw)):
         assert torch.equal(a, b), name
 

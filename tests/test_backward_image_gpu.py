@@ -8,7 +8,7 @@ import torch
 
 import oracle
 from intra_amd import _lib, intra_image_attn, intra_image_attn_bwd, intra_image_attn_func
-from test_backward_gpu import compare
+from test_backward_gpu import compare, spread
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
@@ -41,6 +41,20 @@ def test_flux_2048_grads(pattern):
         got = intra_image_attn_bwd(q, k, v, out, lse, dout, pattern, 128, softmax_scale=0.07)
     mask = oracle.mask_rows(f"image/{pattern}", S, device=DEV, width=128)
     compare(got, oracle.masked_attention_grads(q, k, v, dout, mask, softmax_scale=0.07), f"image/{pattern} 2048")
+
+
+@pytest.mark.parametrize("stride", [1 << 19, 3 << 17])
+@pytest.mark.parametrize("pattern", ["scatter", "gather0"])
+def test_rows_at_and_beyond_the_reach_of_32_bit_offsets(pattern, stride):
+    """4608 tokens 1 MB apart (the last are more than 4 GiB behind the first) and 768 KB apart."""
+    plain = make(1, 512 + 64 * 64, 2, 1, seed=5)
+    grads = []
+    for q, k, v, dout in (plain, spread(plain, stride)):
+        with torch.no_grad():
+            out, lse = intra_image_attn(q, k, v, pattern, 64, return_lse=True)
+            grads.append(intra_image_attn_bwd(q, k, v, out, lse, dout, pattern, 64))
+    for name, a, b in zip(("dq", "dk", "dv"), *grads):
+        assert torch.equal(a, b), name
 
 
 @pytest.mark.parametrize("width,text_len,H,Hkv", [(24, 72, 4, 4), (40, 8, 8, 2), (16, 200, 2, 1), (32, 96, 4, 1), (48, 64, 3, 3)])

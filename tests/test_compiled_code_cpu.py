@@ -118,3 +118,17 @@ def blocks(lines, kernel, mfmas):
 def test_no_moves_between_register_halves_in_the_blocks_of_dk_and_dv(code_object):
     moves = [sum(op.startswith("v_accvgpr") for op in block) for block in blocks(disassembly(code_object), "intra_bwd_kernel", 64)]
     assert len(moves) >= 30 and not any(moves), moves
+
+
+def test_ordinary_backward_kernels_keep_their_scalars(code_object):
+    """What only tensors beyond 32-bit offsets and single tiles need stays out of the other kernels' registers: more
+    scalars than this move to lanes of vector registers and back inside the tile loop."""
+    notes = subprocess.run([llvm_tool("llvm-readelf"), "--notes", code_object], check=True, capture_output=True, text=True).stdout
+    kernels = {}
+    for entry in notes.split("- .agpr_count:")[1:]:
+        fields = dict(re.findall(r"\.(name|sgpr_spill_count|vgpr_spill_count):\s+(\S+)", entry))
+        if "intra_bwd_kernel" in fields["name"]:
+            kernels[fields["name"]] = (int(fields["sgpr_spill_count"]), int(fields["vgpr_spill_count"]))
+    near = {name: n for name, n in kernels.items() if "Lb0EEEv" in name}
+    assert len(near) >= 30 and len(kernels) == 2 * len(near), (len(near), len(kernels))
+    assert all(vector == 0 and scalar <= 40 for scalar, vector in near.values()), near
