@@ -280,7 +280,7 @@ struct KeyRowsImgGroup {
   static IM_HD int num_sets(const IntraGeom&) { return 8; }
   static IM_HD int max_rows(const IntraGeom& ge) { return ge.width * ge.width / 8; }
   static int longest(const IntraGeom& ge) { return KeyRowsImgGroup(ge, 0, 0).n_cols(); }  // (all row blocks of all groups)
-  IM_HD KeyRowsImgGroup(const IntraGeom& ge, int set, int) : sc(ge, set, 0, 0) {}
+  IM_HD KeyRowsImgGroup(const IntraGeom& ge, int set, int) : sc(ge, set, 0) {}
   IM_HD int n_rows() const { return sc.nimg; }
   IM_HD int n_cols() const { return TEXT_COLS_ONLY ? sc.chunk : sc.chunk + sc.nimg; }
   IM_HD int kpre() const { return 0; }

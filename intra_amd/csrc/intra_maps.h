@@ -74,9 +74,8 @@ struct IntraGeom {
   int window;    // LLM window width in keys (>= 64)
   int width;     // image latent grid side (tokens)
   int text_len;  // image: text tokens in front of the grid
-  int text_only; // image scatter: only the text queries of each group (the text rows of gather0)
   int pg;        // image gather0: 8x8 patches per set (a run of pg patches in one patch row)
-  int tm;        // image gather0, forward: text chunks (scatter groups) per set of text rows: 1 or 2
+  int tm;        // image gather0, forward and dQ: text chunks (scatter groups) per set of text rows: 1 or 2
   int blk;       // LLM block scatter: tokens per block
   int off;       // LLM block scatter: stripe offset, 0 <= off < G
   int ns;        // LLM block scatter / window with sinks: leading tokens every query sees
@@ -220,13 +219,11 @@ struct MapImgScatter {
   static constexpr bool kHasPrefix = false;
   static constexpr bool kEveryTile = false;
   IM_HD int kpre() const { return 0; }
-  int W, T, chunk, j, a, b, wq, nimg, text_only;
+  int W, T, chunk, j, a, b, wq, nimg;
   FastDiv dWq;
   static IM_HD int num_sets(const IntraGeom&) { return 8; }
-  static IM_HD int max_nq(const IntraGeom& ge) {
-    return ge.text_only ? ge.text_len / 8 : ge.text_len / 8 + ge.width * ge.width / 8;
-  }
-  IM_HD MapImgScatter(const IntraGeom& ge, int set, int /*t0*/, int only_text = -1) {
+  static IM_HD int max_nq(const IntraGeom& ge) { return ge.text_len / 8 + ge.width * ge.width / 8; }
+  IM_HD MapImgScatter(const IntraGeom& ge, int set, int /*t0*/) {
     W = ge.width;
     T = ge.text_len;
     chunk = T / 8;
@@ -235,14 +232,13 @@ struct MapImgScatter {
     b = set & 3;
     wq = W / 4;
     nimg = W * W / 8;
-    text_only = only_text < 0 ? ge.text_only : only_text;
     dWq = ge.dWq;
   }
   IM_HD int imgpos(int u) const {
     const int r = (int)fd_div(u, dWq);
     return T + (a + 2 * r) * W + b + 4 * (u - r * wq);
   }
-  IM_HD int nq() const { return text_only ? chunk : chunk + nimg; }
+  IM_HD int nq() const { return chunk + nimg; }
   IM_HD int nk() const { return T + nimg; }
   IM_HD int qpos(int t) const { return t < chunk ? chunk * j + t : imgpos(t - chunk); }
   IM_HD int kpos(int t) const { return t < T ? t : imgpos(t - T); }
