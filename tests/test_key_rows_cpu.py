@@ -26,14 +26,14 @@ int main() {  // every line of the input: S B Hkv ns cus
 """
 
 
-def compile_and_run(tmp_path, source, text=""):
+def compile_and_run(tmp_path, source, text="", args=()):
     gxx = shutil.which("g++")
     if gxx is None:
         pytest.skip("g++ not available")
     src, exe = tmp_path / "probe.cpp", tmp_path / "probe"
     src.write_text(source)
     subprocess.run([gxx, "-std=c++17", "-O1", "-I", os.path.join(ROOT, "intra_amd", "csrc"), str(src), "-o", str(exe)], check=True)
-    return subprocess.run([str(exe)], input=text, check=True, capture_output=True, text=True).stdout
+    return subprocess.run([str(exe), *args], input=text, check=True, capture_output=True, text=True).stdout
 
 
 def splits(tmp_path, shapes):

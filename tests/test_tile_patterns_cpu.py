@@ -13,7 +13,7 @@ SRC = r"""
 #include "intra_bwd_maps.h"
 using namespace intra;
 
-static long n_pattern = 0, n_other = 0;
+static long n_pattern = 0, n_other = 0, n_whole = 0;
 static IntraGeom geom(int S) {
   IntraGeom ge;
   memset(&ge, 0, sizeof ge);
@@ -25,6 +25,7 @@ template <class M, class P>
 static void check(const M& m, int first, int n, P&& pos, const char* what) {
   for (int c = first; c < n; c += 64) {
     TileAt a;
+    if (c + 64 <= n) ++n_whole;
     const bool cut = c + 64 > n, every = std::decay_t<M>::kEveryTile;
     if (every && !m.tile_at(c, a)) { printf("%s: tile %d follows no pattern\n", what, c); exit(1); }
     if ((cut && !every) || !m.tile_at(c, a)) { ++n_other; continue; }
@@ -62,7 +63,48 @@ static void report(const char* what, long& p, long& o) {
   o = n_other;
 }
 
-int main() {
+// every whole tile since the last call followed a pattern, and there was one
+static void all_patterned(const char* what) {
+  static long p = 0, w = 0;
+  printf("%s %ld %ld\n", what, n_pattern - p, n_whole - w);
+  p = n_pattern;
+  w = n_whole;
+}
+
+static void aligned() {
+  all_patterned("-");
+  for (int S : {512, 4096}) {
+    { IntraGeom ge = geom(S); ge.G = 2; keys<MapLlmScatter>(ge, "scatter"); all_patterned("scatter"); }
+    { IntraGeom ge = geom(S); ge.G = 2; columns<KeyRowsOf<MapLlmScatter>>(ge, "scatter columns"); all_patterned("scatter_columns"); }
+    { IntraGeom ge = geom(S); ge.G = 8; if (S >= 4096) { keys<MapLlmGather1>(ge, "gather1"); all_patterned("gather1"); } }
+    { IntraGeom ge = geom(S); ge.G = 8; if (S >= 4096) { columns<KeyRowsOf<MapLlmGather1>>(ge, "gather1 columns"); all_patterned("gather1_columns"); } }
+    { IntraGeom ge = geom(S); ge.window = 576; keys<MapLlmWindow>(ge, "window"); all_patterned("window"); }
+    { IntraGeom ge = geom(S); ge.window = 576; columns<KeyRowsOf<MapLlmWindow>>(ge, "window columns"); all_patterned("window_columns"); }
+    for (int ns : {0, 64}) {
+      { IntraGeom ge = geom(S); ge.window = 575; ge.ns = ns; keys<MapLlmWindowSink>(ge, "window_sink"); all_patterned("window_sink"); }
+      { IntraGeom ge = geom(S); ge.window = 575; ge.ns = ns; columns<KeyRowsWindowSink>(ge, "window_sink columns"); all_patterned("window_sink_columns"); }
+      for (int off : {0, 1}) {
+        IntraGeom ge = geom(S); ge.G = 2; ge.blk = 256; ge.off = off; ge.ns = ns;
+        keys<MapLlmBlockScatter>(ge, "block_scatter"); all_patterned("block_scatter");
+        columns<KeyRowsBlockScatter>(ge, "block_scatter columns"); all_patterned("block_scatter_columns");
+      }
+    }
+    { IntraGeom ge = geom(S); ge.ns = 64; columns<KeyRowsFewSinks>(ge, "few sinks"); all_patterned("few_sinks"); }
+    { IntraGeom ge = geom(S); ge.ns = 512; columns<KeyRowsText>(ge, "text"); all_patterned("text"); }
+  }
+  for (int width : {32, 64, 128}) {
+    IntraGeom ge = geom(512 + width * width); ge.width = width; ge.text_len = 512;
+    keys<MapImgScatter>(ge, "image scatter"); all_patterned("image_scatter");
+    columns<KeyRowsImgGroup<false>>(ge, "grid keys"); all_patterned("grid_keys");
+    columns<KeyRowsImgGroup<true>>(ge, "grid keys, text columns"); all_patterned("grid_keys_text_columns");
+    columns<KeyRowsImgWindow>(ge, "window keys"); all_patterned("window_keys");
+    for (int pg : {1, 2, 4}) { ge.pg = pg; keys<MapImgPatch>(ge, "patch runs"); all_patterned("patch_runs"); }
+    for (int tm : {1, 2}) { ge.tm = tm; keys<MapImgTextRows>(ge, "text rows"); all_patterned("text_rows"); }
+  }
+}
+
+int main(int argc, char**) {
+  if (argc > 1) { aligned(); return 0; }
   long p = 0, o = 0;
   for (int S : {1, 63, 64, 65, 300, 777, 2048}) {
     for (int G : {1, 2, 3, 8, 13}) { IntraGeom ge = geom(S); ge.G = G; keys<MapLlmScatter>(ge, "scatter"); columns<KeyRowsOf<MapLlmScatter>>(ge, "scatter columns"); }
@@ -98,3 +140,11 @@ def test_patterned_tiles_sit_where_the_maps_put_their_keys(tmp_path):
     assert [line[0] for line in out] == ["llm", "image"], out
     for kind, pattern, other in out:  # both kinds of tiles occur
         assert int(pattern) > 1000 and int(other) > 100, (kind, pattern, other)
+
+
+def test_every_whole_tile_of_aligned_shapes_follows_a_pattern(tmp_path):
+    """Map by map: one that answers false there would leave its loader with positions row by row, unnoticed."""
+    lines = [line.split() for line in compile_and_run(tmp_path, SRC, args=["aligned"]).splitlines()][1:]
+    assert len({what for what, _, _ in lines}) == 18, lines
+    for what, pattern, whole in lines:
+        assert int(pattern) == int(whole) > 0, (what, pattern, whole)
