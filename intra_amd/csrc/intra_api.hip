@@ -46,7 +46,7 @@ int make_request(int domain, int pattern, int B, int S, int H, int Hkv, int arg0
   r->S = S;
   r->H = H;
   r->Hkv = Hkv;
-  r->geom = IntraGeom{S, 1, 64, 16, 8, 1, 1, 64, 0, 0};  // derived fields: geom_finish() in shape_for()
+  r->geom = IntraGeom{S, 1, 64, 16, 8, 0, 1, 1, 64, 0, 0};  // derived fields: geom_finish() in shape_for()
   r->geom.sink_chunk = 1024;  // backward: set by set_leading_chunk() once the number of leading keys is known
   if (domain == 0) {
     if (!extended && (pattern == INTRA_LLM_BLOCK_SCATTER || pattern == INTRA_LLM_WINDOW_SINK))

@@ -74,14 +74,16 @@ struct IntraGeom {
   int window;    // LLM window width in keys (>= 64)
   int width;     // image latent grid side (tokens)
   int text_len;  // image: text tokens in front of the grid
+  int sink_chunk;  // backward: queries per workgroup of the sink pass (a multiple of 64)
   int pg;        // image gather0: 8x8 patches per set (a run of pg patches in one patch row)
   int tm;        // image gather0, forward and dQ: text chunks (scatter groups) per set of text rows: 1 or 2
   int blk;       // LLM block scatter: tokens per block
   int off;       // LLM block scatter: stripe offset, 0 <= off < G
   int ns;        // LLM block scatter / window with sinks: leading tokens every query sees
-  int sink_chunk;  // backward: queries per workgroup of the sink pass (a multiple of 64)
   // derived by geom_finish()
-  FastDiv dG;        // / G
+  // (Where the fields lie decides how the compiler's loads of kernel arguments fall out: with all of them four
+  // bytes further in front the windows with sinks were 1.3 % slower, image Gather 0 forward 1.7 %.)
+  alignas(8) FastDiv dG;  // / G
   FastDiv dWq;       // / (width / 4)
   FastDiv dPerRow;   // / ((width / 8) / pg)
   FastDiv dBlk;      // / blk
