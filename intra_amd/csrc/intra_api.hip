@@ -127,6 +127,8 @@ int default_hp(int ratio) { return ratio % 4 == 0 ? 4 : (ratio % 2 == 0 ? 2 : 1)
 // quarter of the wavefronts busy, and the static dealing of work items wants items of about one
 // size: 2 if the estimated cost stays within 15 % of a patch item's, else 1.  A key tile with w of
 // 8 wavefronts busy is taken to cost 5/9 + w/18 of a full one (2/3 at w = 2, measured).
+// The forward launch decides for dQ too (24 heads, us, one chunk / two per row block: forward 1024^2 74.6 / 74.5,
+// 2048^2 261 / 302; dQ 122.7 / 101.8 and 377 / 372).
 int pick_text_merge(const IntraGeom& ge, int pos, int pg, int nw) {
   const int chunk = ge.text_len / 8, nimg = ge.width * ge.width / 8;
   if (chunk % 32 != 0 || 2 * chunk > pos) return 1;  // (more chunks than a row block holds share nothing)

@@ -141,7 +141,7 @@ struct KeyRowsBlockScatter {
   // Blocks start at multiples of 64 columns, so a tile lies inside one.  Worked out once per tile, in
   // scalars: per lane and group of rows it was a chain of branches on `off` and on the own block, whose
   // scalars were spilled and read back in the main loop of the launch that more than 64 sinks share
-  // (19 lane reads and 36 branches per step there, 27 branches elsewhere; now 2 and 13).  Training steps,
+  // (19 lane reads and 36 branches per step there, 27 branches elsewhere).  Training steps,
   // G = 2, S = 8192: offset 1 and 128 sinks at 32 / 32 heads 1432 -> 1334 us, 64 sinks at 32 / 8 heads
   // 1248 -> 1217, neither offset nor sinks 1121 -> 1107.
   IM_HD int tile_shift(int c) const {

@@ -165,7 +165,9 @@ constexpr int LDS_BYTES = RING_BYTES + REDO_WORDS * 4;
 // wait in front of every later LDS read; completion is tracked by hand with vmcnt (see the main
 // loop), and the "memory" clobber keeps LDS accesses from moving across it at compile time.
 // The LDS address travels in M0, and a scalar write of M0 needs one wait state before a load to LDS reads
-// it (s_nop); the compiler adds none inside inline assembly.
+// it (s_nop); the compiler adds none inside inline assembly.  (Its cost, before / after, us: Scatter G=8
+// S=32768 996 / 998, G=2 S=65536 15004 / 15102, image Gather 0 2048^2 234.4 / 235.7.  Neither the sum formed in M0
+// nor the address' last sum in place of the s_nop was better: window 1023 with 4 sinks 587 / 598 either way.)
 __device__ __forceinline__ void dma_group(const void* gsrc, uint32_t lds_addr) {
   asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" : : "v"(gsrc), "s"(lds_addr) : "memory");
 }
@@ -304,12 +306,16 @@ __device__ __forceinline__ void run_pass(const KParams& p, unsigned char* smem, 
 
   // (A kernel of one exact pass has scalar registers enough to keep the arguments: reading them again
   // cost Gather 1 at S=7552 44.1 -> 45.3 us, image Gather 0 2048^2 at 6 heads 128.2 -> 130.4.)
-  // The look-up of the next work item, inside the tile loop: for the windows, whose items are about 9
-  // tiles, it reads the arguments again and is marked unlikely; for the longer items of the other maps
-  // it keeps them, as measured (read again / kept, us, same box: Scatter G=8 S=32768 981 / 974, G=2
-  // S=65536 14464 / 14167, Gather 1 S=8192 85.8 / 85.1; the mark, with / without: window 576 S=32768
-  // 332 / 337, S=3000 B=2 62.6 / 63.6, Scatter G=8 S=32768 995 / 988).
-  constexpr bool SWITCH_APART = std::is_same_v<MAP, MapLlmWindow> || std::is_same_v<MAP, MapLlmWindowSink>;
+  // The look-up of the next work item, inside the tile loop: the kernels of the windows and of block Scatter
+  // read the arguments again there and mark it unlikely, those of the other maps keep them.  The line is drawn
+  // by what was measured, kept / read again and marked (same box, us), not by the length of the items:
+  // windows of 576 at S=32768 344.3 / 329.9, 1088 at S=16384 284.8 / 274.0, 2112 at S=32768 1023.2 / 976.9; 575
+  // with 64 sinks at S=8192 110.3 / 105.3, 1023 with 4 at S=32768 622.8 / 597.7; block Scatter G=2 S=6000
+  // 217.9 / 212.3, S=2000 41.4 / 40.1, S=32768 3904 / 3845, G=8 without sinks 1041 / 1025; image Scatter 2048^2
+  // 519.9 / 520.1, 1024^2 75.6 / 75.4; Scatter G=8 S=32768 974 / 981, G=2 S=65536 14167 / 14464, Gather 1 S=8192
+  // 85.1 / 85.8.
+  constexpr bool SWITCH_APART = std::is_same_v<MAP, MapLlmWindow> || std::is_same_v<MAP, MapLlmWindowSink> ||
+                                std::is_same_v<MAP, MapLlmBlockScatter>;
   auto args = [&]() -> const KParams& {
     if constexpr (FAST || REDO) return args_again<KParams>();
     else return p;
