@@ -12,8 +12,9 @@
 //    power limit): the A operand is a K tile row read from LDS (16 B per lane), the B operand is Q
 //    held in registers for a whole work item.  A 32-key block times the wavefront's 32 queries is
 //    2 x 2 tiles; in the accumulator layout a lane holds 4 keys per tile of ONE query per query
-//    tile, so the rescale factors are plain per-lane scalars and a query's maximum or sum is a
-//    reduction over four lanes (l, l ^ 16, l ^ 32, l ^ 48).
+//    tile, so the rescale factors are plain per-lane scalars and a query's maximum is a reduction
+//    over four lanes (l, l ^ 16, l ^ 32, l ^ 48).  Its weight sum comes out of one more MFMA per
+//    query tile, P^T behind a matrix of ones, so it is in every lane.
 //  * O^T = V^T P^T: P^T is the softmax output still in registers (packed to bf16, no LDS round
 //    trip): the lane's 8 weights of a query tile ARE its B operand, under a numbering of the 32-key
 //    reduction that the V^T operand follows; V^T comes from ds_read_b64_tr_b16 transposing reads of
@@ -604,7 +605,16 @@ __device__ __forceinline__ void run_pass(const KParams& p, unsigned char* smem, 
   // accumulated.  SM_SCALED and SM_FOLDED have no reference at all (weights exp2(score * c), or
   // exp2(score) with the scores already in exponent units).
   float mref[2] = {0.f, 0.f};
-  float l_acc[2] = {0.f, 0.f};  // this lane's share of the two queries' weight sums
+  // weight sums of the lane's two queries: a 16x16 tile whose 16 rows are all the same sum
+  floatx4 l_sum[2] = {floatx4{0.f, 0.f, 0.f, 0.f}, floatx4{0.f, 0.f, 0.f, 0.f}};
+  u32x4 ones_bits;  // (opaque: written once per work item, neither built anew at every use nor kept in memory)
+#pragma unroll
+  for (int d = 0; d < 4; ++d) {
+    uint32_t two;
+    asm volatile("v_mov_b32 %0, 0x3f803f80" : "=v"(two));
+    ones_bits[d] = two;
+  }
+  const bf16x8 ones = __builtin_bit_cast(bf16x8, ones_bits);
   const float c = pi.scale_log2;  // |softmax_scale| * log2(e)
 
   // operand reads: base register + compile-time byte offset
@@ -649,7 +659,7 @@ __device__ __forceinline__ void run_pass(const KParams& p, unsigned char* smem, 
   // EXACT mode: what can happen to a freshly computed block of raw scores q.k before it is
   // exponentiated as exp2(score * c - mref); all of it is rare.  `mx` are the block maxima of the
   // raw scores of the lane's two queries.  Four lanes hold a query (disjoint keys and head dims),
-  // so every decision here is taken per query: maximum and running sum are taken over the four.
+  // so every decision here is taken per query: the maximum is taken over the four.
   auto settle = [&](floatx4 (&nxt)[2][2], float (&mx)[2], bool masked, int kb32) {
     if (masked) {  // block cut by a bound: mask in place, then redo the maximum
       mask_block(nxt, kb32);
@@ -659,13 +669,13 @@ __device__ __forceinline__ void run_pass(const KParams& p, unsigned char* smem, 
     if (__builtin_amdgcn_ballot_w64(fmaxf(__builtin_fabsf(mxs[0]), __builtin_fabsf(mxs[1])) > 60.f) == 0) return;  // the usual case
 #pragma unroll
     for (int qt = 0; qt < 2; ++qt) {
-      const float l_run = lane_quad_sum(l_acc[qt]);  // of the query, not of this lane's keys
+      const float l_run = l_sum[qt][0];
       const bool need = mxs[qt] > 60.f || (l_run == 0.f && mxs[qt] < -60.f && mxs[qt] > -INFINITY);
       if (__builtin_amdgcn_ballot_w64(need) != 0) {
         const float delta = need ? mxs[qt] : 0.f;
         const float alpha = l_run == 0.f ? 1.f : __builtin_amdgcn_exp2f(-delta);
         mref[qt] += delta;
-        l_acc[qt] *= alpha;
+        l_sum[qt] *= alpha;
 #pragma unroll
         for (int dt = 0; dt < 8; ++dt) oacc[dt][qt] *= alpha;
       }
@@ -689,8 +699,8 @@ __device__ __forceinline__ void run_pass(const KParams& p, unsigned char* smem, 
   // B operand of PV as they stand: the lane's 8 weights of query tile qt, packed to bf16, are
   // keys 4*g4 .. +3 and 16 + 4*g4 .. +3 of the block, the numbering the V^T reads follow.  PV
   // runs query tile 0 first, so the weights of query tile 1 are only needed 8 slots later: the
-  // exponentials of the 8 bf16 pairs are spread over slots 0..20 of the 32, the packing and the row sums
-  // follow two slots behind, and in EXACT mode the maximum of the next block is taken in the last
+  // exponentials of the 8 bf16 pairs are spread over slots 0..20 of the 32, the packing follows two
+  // slots behind, and in EXACT mode the maximum of the next block is taken in the last
   // PV slots once its MFMA chain has drained.  sched_barrier keeps the compiler from regrouping
   // the slots.
   bf16x8 ka[8];
@@ -714,21 +724,11 @@ __device__ __forceinline__ void run_pass(const KParams& p, unsigned char* smem, 
         px[u][1] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[kt][qt][2 * h + 1], c, -mref[qt]));
       }
     };
-    uint32_t hx[8];
     auto stage_c = [&](int u) {
       floatx2 f = {px[u][0], px[u][1]};
       bf16x2 h2 = __builtin_convertvector(f, bf16x2);
-      hx[u] = __builtin_bit_cast(uint32_t, h2);
       pb[u >> 2][2 * (u & 3)] = h2[0];
       pb[u >> 2][2 * (u & 3) + 1] = h2[1];
-    };
-    // The row sum takes what PV multiplies: the two rounded weights of the pair, by one dot-product
-    // instruction with (1, 1).  (Widening them back to fp32 with a shift and a mask and adding
-    // twice - four plain instructions - measured 7 % slower: in this loop every instruction issued
-    // beside the MFMAs costs its cycles.)
-    auto stage_s = [&](int u) {
-      const bf16x2 ones2 = {(__bf16)1.0f, (__bf16)1.0f};
-      l_acc[u >> 2] = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, hx[u]), ones2, l_acc[u >> 2], false);
     };
     // slot (0..31, PV slots from 16) in which the exponentials of pair u are issued
     auto valu_slot = [&](int k) {
@@ -738,8 +738,7 @@ __device__ __forceinline__ void run_pass(const KParams& p, unsigned char* smem, 
         const int es = u < 4 ? 4 * u : 2 * u + 6;
         if (es == k) stage_e(u);
         if (es + 2 == k) stage_c(u);
-        if (es + 2 == k) stage_s(u);
-        if (INTRA_ABLATE == 5) {  // the same instructions once more (the sums count twice, the rest is rewritten)
+        if (INTRA_ABLATE == 5) {  // the same instructions once more (rewritten with the same values)
           if (es == k) {
             asm volatile("" : "+v"(px[u][0]), "+v"(px[u][1]));
             stage_e(u);
@@ -748,11 +747,14 @@ __device__ __forceinline__ void run_pass(const KParams& p, unsigned char* smem, 
             asm volatile("" : "+v"(px[u][0]), "+v"(px[u][1]));
             stage_c(u);
           }
-          if (es + 2 == k) stage_s(u);
         }
       }
     };
     if (INTRA_ABLATE == 4) pb[0] = qf[0][0], pb[1] = qf[1][0];
+    // The wavefront of a SIMD that is further in its tile gives way to the other one (priority 3 for the first
+    // quarter of a tile, 0 for the last): left to the hardware's order, one finishes its tile early, waits at the
+    // barrier and leaves the other's exponentials without MFMAs beside them.
+    __builtin_amdgcn_s_setprio(3 - 2 * HALF);
 #pragma unroll
     for (int k = 0; k < 16; ++k) {  // QK^T: k-step ks, key tile kt, query tile qt
       const int ks = k >> 2, kt = (k >> 1) & 1, qt = k & 1;
@@ -762,11 +764,18 @@ __device__ __forceinline__ void run_pass(const KParams& p, unsigned char* smem, 
       __builtin_amdgcn_sched_barrier(0);
     }
     float m[2] = {0.f, 0.f};
+    __builtin_amdgcn_s_setprio(2 - 2 * HALF);
 #pragma unroll
     for (int k = 0; k < 16; ++k) {  // PV: query tile qt, head-dim tile dt
       const int qt = k >> 3, dt = k & 7;
       if (k >= 8 && INTRA_ABLATE != 2) ka[k - 8] = kread_at(kb[(k - 8) >> 1], (k & 1) * 4 * FGROUP_STRIDE + HALF * FBLOCK32);
       oacc[dt][qt] = mfma(va[dt], pb[qt], oacc[dt][qt]);
+      // The row sums take what PV multiplies, the rounded weights, by one more MFMA per query tile with a matrix of
+      // ones. (One dot-product instruction with (1, 1) per pair, eight in all, holds the matrix pipe longer: 16 cycles
+      // each.  With these two and the priorities, us: Scatter G=8 S=32768 973 -> 955, Gather 1 S=8192 78.6 -> 77.3,
+      // window 576 S=32768 327 -> 324; with the sums alone 968 / 78.7 / 326, with the priorities alone 973 / 78.3 / 325.)
+      if (k == 3) l_sum[0] = mfma(ones, pb[0], l_sum[0]);
+      if (k == 15) l_sum[1] = mfma(ones, pb[1], l_sum[1]);
       valu_slot(16 + k);
       if (!FAST) {
         if (k == 12) m[0] = lane_max(n, 0);
@@ -863,7 +872,7 @@ __device__ __forceinline__ void run_pass(const KParams& p, unsigned char* smem, 
   // ---------------------------------------------------------------- normalise and store
   {
   const KParams& po = args();
-  const float l_tot[2] = {lane_quad_sum(l_acc[0]), lane_quad_sum(l_acc[1])};
+  const float l_tot[2] = {l_sum[0][0], l_sum[1][0]};
   if (FAST) {
     // Weights were formed without a reference: the result is good iff the weight sum stayed inside
     // 2^-100 .. 2^60 (no weight overflowed, and the largest ones are far from underflow).  The

@@ -406,24 +406,67 @@ struct MapImgTextRows {
   IM_HD int khi(int tq) const { return klo(tq) + T + nimg - 1; }
 };
 
-// image gather0, forward launch: the text rows, then the patch runs
+// image gather0, forward launch: the text rows, then the patch runs.  One set of fields for both kinds: a
+// wavefront carries the map of the work item that its loader is at through the tile loop, in scalar registers.
 struct MapImgGather0F {
   static constexpr bool kHasPrefix = true;
   bool is_text;
-  MapImgTextRows tx;
-  MapImgPatch pa;
+  int W, T, nq_, nk_;
+  int a, b, c;   // text rows: lead, cA, cB; patch run: positions of the window's and the queries' first grid token, first grid column
+  int q0;        // text rows: first query; patch run: first patch of the row (C0)
+  FastDiv dWq;
   static IM_HD int num_sets(const IntraGeom& ge) { return MapImgTextRows::num_sets(ge) + MapImgPatch::num_sets(ge); }
   static IM_HD int max_nq(const IntraGeom& ge) { return im_max(MapImgTextRows::max_nq(ge), MapImgPatch::max_nq(ge)); }
-  IM_HD MapImgGather0F(const IntraGeom& ge, int set, int t0)
-      : is_text(set < 8 / ge.tm), tx(ge, is_text ? set : 0, t0), pa(ge, is_text ? 0 : set - 8 / ge.tm, t0) {}
-  IM_HD int nq() const { return is_text ? tx.nq() : pa.nq(); }
-  IM_HD int nk() const { return is_text ? tx.nk() : pa.nk(); }
-  IM_HD int kpre() const { return is_text ? 0 : pa.kpre(); }
-  IM_HD int qpos(int t) const { return is_text ? tx.qpos(t) : pa.qpos(t); }
-  IM_HD int kpos(int t) const { return is_text ? tx.kpos(t) : pa.kpos(t); }
-  IM_HD int klo(int tq) const { return is_text ? tx.klo(tq) : pa.klo(tq); }
-  IM_HD int khi(int tq) const { return is_text ? tx.khi(tq) : pa.khi(tq); }
-  IM_HD bool tile_rows(int t_first, TileRows& a) const { return !is_text && pa.tile_rows(t_first, a); }
+  IM_HD MapImgGather0F(const IntraGeom& ge, int set, int t0) {
+    W = ge.width;
+    T = ge.text_len;
+    dWq = ge.dWq;
+    is_text = set < 8 / ge.tm;
+    if (is_text) {
+      const MapImgTextRows m(ge, set, t0);
+      nq_ = m.nq();
+      nk_ = m.nk();
+      a = m.lead;
+      b = m.cA;
+      c = m.cB;
+      q0 = m.q0;
+    } else {
+      const MapImgPatch m(ge, set - 8 / ge.tm, t0);
+      nq_ = m.nq();
+      nk_ = m.nk();
+      a = T + m.r0 * W + m.cfirst;
+      b = T + 8 * (m.R * W + m.C0);
+      c = m.cfirst;
+      q0 = m.C0;
+    }
+  }
+  IM_HD int nq() const { return nq_; }
+  IM_HD int nk() const { return nk_; }
+  IM_HD int kpre() const { return is_text ? 0 : T; }
+  IM_HD int qpos(int t) const { return is_text ? q0 + t : b + ((t & 63) >> 3) * W + 8 * (t >> 6) + (t & 7); }
+  // (text rows: MapImgTextRows::kpos; patch run: MapImgPatch::kpos)
+  IM_HD int kpos(int t) const {
+    if (is_text) {
+      const unsigned tt = (unsigned)(t - a);
+      const bool front = t < a;
+      const int u = front ? t : (int)tt - T;
+      const int p = (front ? b : c) + 4 * u + (int)fd_div(u, dWq) * W;
+      return tt < (unsigned)T ? (int)tt : p;
+    }
+    const int u = t - T;
+    return t < T ? t : a + ((u >> 2) & 15) * W + 4 * (u >> 6) + (u & 3);
+  }
+  IM_HD int klo(int tq) const {
+    if (is_text) return 8 * tq >= T ? a : 0;
+    return T + 16 * (MapImgPatch::win_start(q0 + (tq >> 6), W / 8) - c);
+  }
+  IM_HD int khi(int tq) const { return klo(tq) + (is_text ? T + W * W / 8 : 256) - 1; }
+  IM_HD bool tile_rows(int t_first, TileRows& r) const {
+    if (is_text) return false;
+    const int u = t_first - T;
+    r = u < 0 ? TileRows{t_first, 4, 1} : TileRows{a + 4 * (u >> 6), W, 1};
+    return t_first + 64 <= T || (u >= 0 && (u & 63) == 0 && t_first + 64 <= nk_);
+  }
 };
 
 // tile_rows of a map that has one, else false
