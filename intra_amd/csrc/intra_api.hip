@@ -406,6 +406,53 @@ int pick_softmax(float scale, unsigned flags) {
   }
 }
 
+// Cost of the row blocks of a set, first one first: its key tiles and what an item takes besides (set-up, first
+// key block and stores: 3.5 us where a tile takes 1.7).
+constexpr int ITEM_COST = 2;
+template <class MAP> struct RowBlockCosts {
+  static int go(const IntraGeom& ge, int pos, int n, int* cost) {
+    for (int m = 0; m < n; ++m) {
+      const MAP map(ge, 0, m * pos);
+      cost[m] = m * pos < map.nq() ? ITEM_COST + intra::range_of_block(map, m, pos).ntiles : 0;
+    }
+    return 0;
+  }
+};
+
+// Whether an XCD's items are dealt row block by row block (locate_item) and not pair by pair: the work of its longest
+// workgroup is added up for both.  Row block by row block is balanced where the row blocks of a pair do not fill
+// whole rounds, but all pairs are then worked on at once and share the L2 and each key tile less.  So it has to be
+// shorter by 3 % where at least four CUs come to a pair, by 12 % where at least two do, and is not taken with
+// fewer.  Pair by pair / row block by row block, us:
+//   four CUs and more  Scatter G=8 S=5000 49.9 / 40.1, 10000 136.6 / 115.0, 30000 982 / 843; G=3 S=20000 1013 / 946;
+//                      G=2 S=24000 2192 / 1956; block Scatter G=2 S=6000 209 / 163; window 2112 S=5000 b=2 257 / 248
+//                      (as long either way: Scatter G=8 S=32768 969 / 984, block Scatter G=8 S=20000 439 / 451)
+//   two                Scatter G=4 S=33472 of 32 kv heads 2680 / 2131, G=16 S=60000 1893 / 1727; 10 % shorter by this
+//                      count: block Scatter G=8 S=33472 of 16 kv heads 1111 / 1164
+//   one                Scatter G=8 S=33472 of 32 kv heads 1147 / 1249 (15 % shorter by this count)
+constexpr int MAX_COSTED_ROW_BLOCKS = 1024;  // (with more of them a pair's last, uneven round is a small share)
+constexpr int MAX_COSTED_WORKGROUPS = 128;
+bool row_order_pays(const int* cost, int n_mblocks, int pairs, int hgroups, int wgs) {
+  int longest[2];
+  for (int order = 0; order < 2; ++order) {
+    int load[MAX_COSTED_WORKGROUPS] = {}, col = 0, step = 1;
+    auto deal = [&](int c) {
+      load[col] += c;
+      col += step;
+      if (col < 0 || col == wgs) {  // next round, in the other direction
+        step = -step;
+        col += step;
+      }
+    };
+    const int outer = order ? n_mblocks : pairs, inner = order ? pairs : n_mblocks;
+    for (int a = 0; a < outer; ++a)
+      for (int b = 0; b < inner; ++b)
+        for (int h = 0; h < hgroups; ++h) deal(cost[n_mblocks - 1 - (order ? a : b)]);
+    longest[order] = *std::max_element(load, load + wgs);
+  }
+  return 100ll * longest[0] > (4 * pairs <= 32 ? 103ll : 112ll) * longest[1];
+}
+
 // Order of an XCD's work items (see KParams::Section).  One section - every pair, all row blocks -
 // except where a launch mixes kinds of items:
 //  * image scatter: a set has text_len / 8 + width^2 / 8 queries, so its last row block is partial
@@ -414,14 +461,22 @@ int pick_softmax(float scale, unsigned flags) {
 //  * image gather0: the text rows (the first sets; pairs are numbered set-major, so they are the
 //    first pair slots) and the patch runs can have different numbers of row blocks; each kind gets
 //    its section, so that no number goes to an empty item, text rows first.
-void set_sections(intra::KParams& p, const Request& r, const Shape& ph, const LaunchDims& d) {
+void set_sections(intra::KParams& p, const Request& r, const Shape& ph, const LaunchDims& d, int wgs_per_xcd) {
   const int pslots = (d.n_pairs + 7) / 8;
+  p.row_order = 0;
+  if (ph.map != MAP_IMG_SCATTER && ph.map != MAP_IMG_GATHER0 &&  // (has_sections: items of one length)
+      pslots > 1 && 2 * pslots <= 32 && pslots * d.n_mblocks * d.hgroups > wgs_per_xcd && wgs_per_xcd <= MAX_COSTED_WORKGROUPS &&
+      d.n_mblocks <= MAX_COSTED_ROW_BLOCKS) {
+    int cost[MAX_COSTED_ROW_BLOCKS];
+    by_map<RowBlockCosts>(ph.map, ph.geom, d.pos, d.n_mblocks, cost);
+    p.row_order = row_order_pays(cost, d.n_mblocks, pslots, d.hgroups, wgs_per_xcd);
+  }
   auto section = [&](int p_lo, int p_n, int mb_lo, int mb_hi) {
     intra::KParams::Section s;
     s.p_lo = p_lo;
     s.mb_hi = mb_hi;
     s.slots = p_n * (mb_hi - mb_lo) * d.hgroups;
-    s.d_ipp = make_fastdiv(std::max(1, (mb_hi - mb_lo) * d.hgroups));
+    s.d_items = make_fastdiv(std::max(1, (p.row_order ? p_n : mb_hi - mb_lo) * d.hgroups));
     return s;
   };
   p.sec[0] = section(0, pslots, 0, d.n_mblocks);
@@ -446,14 +501,14 @@ void set_sections(intra::KParams& p, const Request& r, const Shape& ph, const La
 }
 
 // what locate_item needs of a launch: geometry, item counts, sections, divisors
-void set_dealing(intra::KParams& p, const Request& r, const Shape& ph, const LaunchDims& dims) {
+void set_dealing(intra::KParams& p, const Request& r, const Shape& ph, const LaunchDims& dims, int grid) {
   p.B = r.B; p.H = r.H; p.Hkv = r.Hkv; p.ratio = r.H / r.Hkv;
   p.geom = ph.geom;
   p.n_sets = dims.n_sets;
   p.n_mblocks = dims.n_mblocks;
   p.hgroups = dims.hgroups;
   p.n_pairs = dims.n_pairs;
-  set_sections(p, r, ph, dims);
+  set_sections(p, r, ph, dims, grid / 8);
   p.d_nbh = make_fastdiv(r.B * r.Hkv);
   p.d_hkv = make_fastdiv(r.Hkv);
   p.d_hgroups = make_fastdiv(p.hgroups);
@@ -537,7 +592,7 @@ int run(int domain, const void* q, const void* k, const void* v, void* o, int B,
   const int grid = launch_grid(dims.work_items, ph.nw);
   if (grid <= 0)
     return fail(INTRA_ERR_HIP, "cannot query the current device: %s", hipGetErrorString(hipGetLastError()));
-  set_dealing(p, r, ph, dims);
+  set_dealing(p, r, ph, dims, grid);
   p.diag = (int64_t)grid * intra::DIAG_SLOTS <= g_diag_values.load() ? g_diag.load() : nullptr;
   return by_map<LaunchMap>(ph.map, p, ph.hp, ph.nw, pick_softmax(scale, flags), grid, static_cast<hipStream_t>(stream));
 }
@@ -1081,7 +1136,7 @@ int intra_model_deal(int domain, int pattern, int B, int S, int H, int Hkv, int 
     return fail(INTRA_ERR_INVALID, "grid must be a multiple of 8 in 8 .. work_items (%d)", dims.work_items);
   if (n_visits < dims.work_items) return fail(INTRA_ERR_INVALID, "visits holds %lld values, %d needed", (long long)n_visits, dims.work_items);
   intra::KParams p{};
-  set_dealing(p, r, ph, dims);
+  set_dealing(p, r, ph, dims, grid);
   return by_map<DealWalk>(ph.map, p, dims.pos, grid, dims.n_mblocks, visits);
 }
 

@@ -92,13 +92,15 @@ struct KParams {
   // The work items of an XCD are numbered section by section (costly kinds of items first, so
   // that the cheap ones fill the last, partial round of the workgroups; kinds of sets with
   // different numbers of row blocks apart, so that no number goes to an empty item): a section is
-  // a range of the XCD's pairs times a range of row blocks, taken pair by pair, last row block first.
+  // a range of the XCD's pairs times a range of row blocks, last row block first, taken pair by pair or
+  // (row_order) row block by row block, the same one of every pair in turn.
   struct Section {
     int p_lo;          // first pair slot (pair = 8 * pair slot + XCD)
     int mb_hi;         // one past its last row block
     int slots;         // pair slots * row blocks * hgroups
-    FastDiv d_ipp;     // division by its items per pair: row blocks * hgroups
+    FastDiv d_items;   // division by its items per pair, row blocks * hgroups, or (row_order) per row block, pair slots * hgroups
   } sec[2];
+  int row_order;
   FastDiv d_nbh, d_hkv, d_hgroups;  // divisions by B * Hkv, Hkv, hgroups
   long long* diag;     // INTRA_DIAG_TIMERS builds: DIAG_SLOTS counters per workgroup, or null
 };
@@ -230,44 +232,53 @@ struct Where {
 struct Range {
   int kt_lo, ntiles;
 };
-template <class MAP, int POS>
-IM_HD Range range_of_block(const MAP& map, int mblk) {
-  const int t0 = mblk * POS;
-  const int t1 = im_min(t0 + POS, map.nq()) - 1;
+template <class MAP>
+IM_HD Range range_of_block(const MAP& map, int mblk, int pos) {
+  const int t0 = mblk * pos;
+  const int t1 = im_min(t0 + pos, map.nq()) - 1;
   const int kt_lo = MAP::kHasPrefix ? 0 : map.klo(t0);  // first key the row block looks at
   const int kt_hi = im_min(map.khi(t1), map.nk() - 1);
   return Range{kt_lo, (kt_hi - kt_lo + BN) / BN};
 }
 
 // Dealing of work items.  Workgroups are handed to the 8 XCDs round-robin by id, so workgroup
-// id % 8 names the XCD.  All row blocks of one (batch, kv head, set) "pair" go to one XCD, one pair
-// after the other, longest row block first, so that the pair's K/V stays in that XCD's L2 while its
-// row blocks run.  Inside an XCD the slots are dealt to its workgroups in boustrophedon order
-// (0..w-1, w-1..0, ...), which balances the triangular causal workloads.
+// id % 8 names the XCD.  All row blocks of one (batch, kv head, set) "pair" go to one XCD, longest row
+// block first.  Inside an XCD the slots are dealt to its workgroups in boustrophedon order (0..w-1, w-1..0,
+// ...), which balances a sequence of descending lengths.  Taken pair by pair, so that a pair's K/V stays in
+// the XCD's L2 while its row blocks run, the lengths jump from 1 back to the longest at every new pair: balanced
+// where the pairs' ends fall together with those of the rounds, and up to half more than the mean for the
+// unluckiest workgroup elsewhere.  Taken row block by row block (KParams::row_order) they descend throughout.
+// The host decides (row_order_pays).
 // locate_item: the first non-empty work item of workgroup `wg_in_xcd` (of `wgs_per_xcd`) of XCD `xcd`
 // at or after `round`; false when there is none.  `redo` (device, second pass only): bitmap of the
 // rounds to visit.  Also runs on the host, where tests enumerate what every workgroup is dealt.
+// (Scalars are few: the image maps have two sections and one order, the others one section and two orders.  With
+// both for all of them Scatter spilled 32 more, S=65536 G=2 14199 -> 14324 us.)
+template <class MAP>
+constexpr bool has_sections = std::is_same_v<MAP, MapImgScatter> || std::is_same_v<MAP, MapImgGather0F>;
 template <class MAP, int POS, bool REDO>
 IM_HD bool locate_item(const KParams& p, int xcd, int wgs_per_xcd, int wg_in_xcd, const uint32_t* redo, int round, Where& w) {
   for (;; ++round) {
     const int slot = round * wgs_per_xcd + ((round & 1) ? wgs_per_xcd - 1 - wg_in_xcd : wg_in_xcd);
     if (slot >= p.n_slots) return false;
     if (REDO && !((redo[(round >> 5) & (REDO_WORDS - 1)] >> (round & 31)) & 1u)) continue;
-    const bool second = slot >= p.sec[0].slots;
+    const bool second = has_sections<MAP> && slot >= p.sec[0].slots;
     const int sslot = second ? slot - p.sec[0].slots : slot;
     const KParams::Section& sc = p.sec[second ? 1 : 0];
-    const int pq = (int)fd_div(sslot, sc.d_ipp);
-    const int pair = (sc.p_lo + pq) * 8 + xcd;
+    const int q1 = (int)fd_div(sslot, sc.d_items);
+    const int rem = sslot - q1 * (int)sc.d_items.d;
+    const int q2 = (int)fd_div(rem, p.d_hgroups);
+    const bool rows = !has_sections<MAP> && p.row_order;
+    const int pq = rows ? q2 : q1, rblk = rows ? q1 : q2;
+    const int pair = ((has_sections<MAP> ? sc.p_lo : 0) + pq) * 8 + xcd;
     if (pair >= p.n_pairs) continue;
-    const int rem = sslot - pq * (int)sc.d_ipp.d;
-    const int rblk = (int)fd_div(rem, p.d_hgroups);
     w.round = round;
     w.set = (int)fd_div(pair, p.d_nbh);
     const int bh = pair - w.set * (int)p.d_nbh.d;
     w.batch = (int)fd_div(bh, p.d_hkv);
     w.kvh = bh - w.batch * p.Hkv;
     w.mblk = sc.mb_hi - 1 - rblk;
-    w.hg = rem - rblk * p.hgroups;
+    w.hg = rem - q2 * p.hgroups;
     if (w.mblk * POS >= MAP(p.geom, w.set, w.mblk * POS).nq()) continue;
     return true;
   }
@@ -336,7 +347,7 @@ __device__ __forceinline__ void run_pass(const KParams& p, unsigned char* smem, 
   auto locate = [&](int round, Where& w) {
     return locate_item<MAP, POS, REDO>(switch_args(), xcd, wgs_per_xcd, wg_in_xcd, redo, round, w);
   };
-  auto range_of = [&](const MAP& map, int mblk) { return range_of_block<MAP, POS>(map, mblk); };
+  auto range_of = [&](const MAP& map, int mblk) { return range_of_block(map, mblk, POS); };
 
   // ---------------------------------------------------------------- loader: HBM rows -> LDS
   // One global_load_lds_dwordx4 moves a 4-row group: lane L fetches 16 bytes of row L/16 and the

@@ -66,7 +66,7 @@ __device__ __forceinline__ void run_pass_narrow(const KParams& p, unsigned char*
   auto locate = [&](int round, Where& w) {
     return locate_item<MAP, POS, REDO>(args(), xcd, wgs_per_xcd, wg_in_xcd, redo, round, w);
   };
-  auto range_of = [&](const MAP& map, int mblk) { return range_of_block<MAP, POS>(map, mblk); };
+  auto range_of = [&](const MAP& map, int mblk) { return range_of_block(map, mblk, POS); };
 
   // ---------------------------------------------------------------- loader: HBM rows -> LDS
   // One global_load_lds_dwordx4 moves a 4-row group (see the wide kernel's loader): 16 groups per

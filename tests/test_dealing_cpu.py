@@ -57,6 +57,25 @@ def test_other_patterns_every_row_block_once(lib, waves):
             assert np.array_equal(visits, base), (case, waves, grid)
 
 
+# Sizes whose pairs do not end with a round of the workgroups: dealt row block by row block where that is
+# better balanced (which depends on the grid)
+@pytest.mark.parametrize("waves", [8, 4])
+@pytest.mark.parametrize("case", [
+    (LLM, SCATTER, 1, 30000, 32, 8, 8, 0), (LLM, SCATTER, 1, 5000, 32, 8, 8, 0), (LLM, SCATTER, 1, 20000, 28, 4, 3, 0),
+    (LLM, SCATTER, 3, 3000, 32, 8, 4, 0), (LLM, GATHER1, 1, 20032, 16, 8, 8, 0), (LLM, WINDOW, 2, 5000, 32, 8, 8, 2112),
+    (LLM, SCATTER, 1, 2100, 8, 1, 9, 0)])
+def test_uneven_sizes_every_row_block_once(lib, case, waves):
+    rc, base = deal(lib, *case, waves, 8)
+    assert rc == 0, _lib.last_error()
+    assert base.max() == 1 and base.sum() > 0
+    for grid in (16, 64, 256, 512):
+        rc, visits = deal(lib, *case, waves, grid)
+        if rc != 0:
+            assert "grid" in _lib.last_error()
+            continue
+        assert np.array_equal(visits, base), (case, waves, grid)
+
+
 def test_plan_names_the_half_size_workgroups_for_image_gather0(lib):
     plan = _lib.IntraPlan()
     assert lib.intra_plan(IMAGE, GATHER0, 1, 16896, 24, 24, 128, 512, plan) == 0
