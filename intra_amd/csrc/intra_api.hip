@@ -610,17 +610,17 @@ int launch_bwd(const intra::BParams& p, hipStream_t stream) {
   return INTRA_OK;
 }
 
-// Workgroups of a row map with `rows` rows each: per XCD, bundles of pairs x items of a pair (see the
-// kernel).  blocks = -1 if they are too many to number.
+// Workgroups of a row map with `rows` rows each, per_cu of which a CU holds at once: per XCD, bundles of pairs x
+// items of a pair (see the kernel).  blocks = -1 if they are too many to number.
 template <class R>
-intra::BwdGrid bwd_grid(const intra::BParams& p, int rows, int hgroups) {
+intra::BwdGrid bwd_grid(const intra::BParams& p, int rows, int hgroups, int per_cu = 1) {
   intra::BwdGrid g;
   const int64_t pairs = (int64_t)R::num_sets(p.geom) * p.B * p.Hkv;
   g.hgroups = hgroups;
   g.n_rblocks = (R::max_rows(p.geom) + rows - 1) / rows;
   g.items_per_pair = g.n_rblocks * hgroups;
   const int64_t pairs_per_xcd = (pairs + 7) / 8;
-  const int64_t want = (32 + g.items_per_pair - 1) / g.items_per_pair;  // pairs that fill an XCD's 32 CUs
+  const int64_t want = (32 * per_cu + g.items_per_pair - 1) / g.items_per_pair;  // pairs that fill an XCD's 32 CUs
   g.bundle = (int)std::max<int64_t>(1, std::min<int64_t>(want, pairs_per_xcd));
   const int64_t bundles = (pairs_per_xcd + g.bundle - 1) / g.bundle;
   const int64_t blocks = 8 * bundles * g.bundle * g.items_per_pair;
@@ -628,32 +628,55 @@ intra::BwdGrid bwd_grid(const intra::BParams& p, int rows, int hgroups) {
   return g;
 }
 
-// dQ of a forward map: row blocks of 256 / hp queries of hp heads; also writes D = rowsum(dO o O)
-template <class R, class LEAD = intra::NoLeadingKeys>
+// dQ of a forward map: row blocks of 256 / hp queries of hp heads, or of half as many; also writes
+// D = rowsum(dO o O)
+template <class R, int MODE, class LEAD = intra::NoLeadingKeys>
 int launch_bwd_dq(const intra::BParams& p, int hp, hipStream_t stream) {
   switch (hp) {
-    case 4: return launch_bwd<R, intra::BWD_DQ, 4, LEAD>(p, stream);
-    case 2: return launch_bwd<R, intra::BWD_DQ, 2, LEAD>(p, stream);
-    default: return launch_bwd<R, intra::BWD_DQ, 1, LEAD>(p, stream);
+    case 4: return launch_bwd<R, MODE, 4, LEAD>(p, stream);
+    case 2: return launch_bwd<R, MODE, 2, LEAD>(p, stream);
+    default: return launch_bwd<R, MODE, 1, LEAD>(p, stream);
   }
 }
 template <class MAP>
 int run_bwd_dq(intra::BParams p, int hp, hipStream_t stream) {
   using R = intra::QueryRows<MAP>;
   p.grid = bwd_grid<R>(p, 256 / hp, p.ratio / hp);
-  return launch_bwd_dq<R>(p, hp, stream);
+  return launch_bwd_dq<R, intra::BWD_DQ>(p, hp, stream);
 }
 
-// dQ of image gather0: the patch runs, and in front of them (at large grids they meet the most columns)
-// the text rows, the chunks of two groups in one row block where that keeps it as short as a patch
-// run's (pick_text_merge).
+// The same in half-size workgroups where a row block meets at most HALF_COLUMNS columns: two workgroups on a CU
+// fill each other's prologues and ends, a long row block pays for every column tile being loaded twice as often
+// instead.  Training steps, 8 wavefronts / 4, us: window 255 with 4 sinks S=16384 613 / 582; 575 with 64,
+// S=8192, 457 / 445; 576 S=32768 1467 / 1448; 1023 with 64, S=16384, 1337 / 1324; 2112 S=16384 2097 / 2109; image
+// Scatter 1024^2 (1024 columns) 303 / 298, 2048^2 (2560) at 12 heads 1108 / 1121.  (Scatter, Gather 1 and block
+// Scatter, whose row blocks are of every length up to the set's: 0 to 3 % slower at any size.)
+constexpr int HALF_COLUMNS = 1152;
+template <class MAP>
+int run_bwd_dq_short(const intra::BParams& p0, int hp, int columns, hipStream_t stream) {
+  if (columns > HALF_COLUMNS) return run_bwd_dq<MAP>(p0, hp, stream);
+  using R = intra::QueryRows<MAP>;
+  intra::BParams p = p0;
+  p.grid = bwd_grid<R>(p, 128 / hp, p.ratio / hp, 2);
+  return launch_bwd_dq<R, intra::BWD_DQ_HALF>(p, hp, stream);
+}
+
+// dQ of image gather0, in half-size workgroups: the patch runs, and in front of them (at large grids they meet the
+// most columns) the text rows, the chunks of two groups in one row block where that keeps it as short as a patch
+// run's (pick_text_merge).  A run of 2 patches streams 14 tiles, of which a wavefront uses 12; one of 4, in 8
+// wavefronts, 18: the launch 85.9 -> 81.7 us at 1024^2 and 24 heads, the training step 313.9 -> 311.0, at 2048^2
+// 1115 -> 1092.
 int run_bwd_dq_gather0(intra::BParams p, int hp, hipStream_t stream) {
   using R = intra::QueryRows<MapImgPatch>;
   using Text = intra::QueryRows<MapImgTextRows>;
-  p.grid = bwd_grid<R>(p, 256 / hp, p.ratio / hp);
-  p.lead = bwd_grid<Text>(p, 256 / hp, p.ratio / hp);
+  const int pos = 128 / hp;
+  p.geom.pg = pos >= 128 && p.geom.width / 8 % 2 == 0 ? 2 : 1;
+  p.geom.tm = pick_text_merge(p.geom, pos, p.geom.pg, 4);
+  geom_finish(p.geom);
+  p.grid = bwd_grid<R>(p, pos, p.ratio / hp, 2);
+  p.lead = bwd_grid<Text>(p, pos, p.ratio / hp, 2);
   p.lead_first = 1;
-  return launch_bwd_dq<R, Text>(p, hp, stream);
+  return launch_bwd_dq<R, intra::BWD_DQ_HALF, Text>(p, hp, stream);
 }
 
 // dK and dV over a key-row map: row blocks of 128 keys of one kv head, all query heads of its group
@@ -806,7 +829,7 @@ int run_bwd(int domain, const void* q, const void* k, const void* v, const void*
       if ((rc = run_bwd_dq<MapLlmGather1>(p, sh.hp, st))) return rc;
       return run_bwd_keys<intra::KeyRowsOf<MapLlmGather1>>(p, st);
     case MAP_LLM_WINDOW:
-      if ((rc = run_bwd_dq<MapLlmWindow>(p, sh.hp, st))) return rc;
+      if ((rc = run_bwd_dq_short<MapLlmWindow>(p, sh.hp, p.geom.window, st))) return rc;
       return run_bwd_keys<intra::KeyRowsOf<MapLlmWindow>>(p, st);
     case MAP_LLM_BLOCK_SCATTER:
       if ((rc = run_bwd_dq<MapLlmBlockScatter>(p, sh.hp, st))) return rc;
@@ -814,12 +837,12 @@ int run_bwd(int domain, const void* q, const void* k, const void* v, const void*
       rc = run_bwd_keys_sinks<intra::KeyRowsBlockScatter>(p, st);
       return rc ? rc : run_bwd_lead_reduce(p, ns, st);
     case MAP_LLM_WINDOW_SINK:
-      if ((rc = run_bwd_dq<MapLlmWindowSink>(p, sh.hp, st))) return rc;
+      if ((rc = run_bwd_dq_short<MapLlmWindowSink>(p, sh.hp, (int)std::min<int64_t>((int64_t)p.geom.window + ns, S), st))) return rc;
       if (ns == 0) return run_bwd_keys<intra::KeyRowsWindowSink>(p, st);
       rc = run_bwd_keys_sinks<intra::KeyRowsWindowSink>(p, st);
       return rc ? rc : run_bwd_lead_reduce(p, ns, st);
     case MAP_IMG_SCATTER:  // grid keys against their group's queries, text keys against all queries
-      if ((rc = run_bwd_dq<MapImgScatter>(p, sh.hp, st))) return rc;
+      if ((rc = run_bwd_dq_short<MapImgScatter>(p, sh.hp, p.geom.text_len + p.geom.width * p.geom.width / 8, st))) return rc;
       rc = run_bwd_keys_lead<intra::KeyRowsImgGroup<false>, intra::KeyRowsText>(p, st);
       return rc ? rc : run_bwd_lead_reduce(p, ns, st);
     case MAP_IMG_GATHER0:  // grid keys against the grid queries around them, plus their group's text queries

@@ -37,8 +37,10 @@ __device__ __forceinline__ void static_for(F&& f) {
   }
 }
 
-enum BwdMode : int { BWD_DQ = 0, BWD_DKV = 1 };
-constexpr int bwd_waves(int mode) { return mode == BWD_DKV ? 4 : 8; }
+// BWD_DQ_HALF: dQ in half-size workgroups, 4 wavefronts of 128 / HP queries, two workgroups per CU, in steps of
+// 32 columns (a ring of four half tiles).
+enum BwdMode : int { BWD_DQ = 0, BWD_DKV = 1, BWD_DQ_HALF = 2 };
+constexpr int bwd_waves(int mode) { return mode == BWD_DQ ? 8 : 4; }
 static_assert(bwd_waves(BWD_DKV) * 32 == KEY_ROWS, "keys of a row block");
 
 // Workgroups of one row map in a launch
@@ -71,8 +73,10 @@ struct BParams {
   int lead_first;    // their workgroups come before the others
 };
 
-constexpr int BWD_SLOT = 2 * FTILE + 512;  // two tiles and 2 x 64 column scalars
-constexpr int bwd_ring_slots(int mode) { return mode == BWD_DKV ? 4 : 3; }
+// two tiles and 2 x 64 column scalars, or two half tiles
+constexpr int bwd_slot(int mode) { return mode == BWD_DQ_HALF ? 2 * FBLOCK32 : 2 * FTILE + 512; }
+constexpr int bwd_ring_slots(int mode) { return mode == BWD_DQ ? 3 : 4; }
+static_assert(2 * bwd_ring_slots(BWD_DQ_HALF) * bwd_slot(BWD_DQ_HALF) <= 160 * 1024, "two workgroups per CU");
 
 // 64 lanes x 4 bytes from per-lane global addresses to 256 consecutive LDS bytes at lds_addr (the
 // active lanes' parts of them), like dma_group
@@ -105,13 +109,16 @@ __device__ __forceinline__ void dma_scalars(const void* base, uint32_t offset, u
 template <class RMAP, int MODE, int HP, bool PARTIAL, bool FAR>
 __device__ __forceinline__ void bwd_rows(const BParams& p, const BwdGrid& g, const int block, unsigned char* const smem) {
   constexpr int NW = bwd_waves(MODE);
-  constexpr bool ROWS_ARE_QUERIES = MODE == BWD_DQ;
+  constexpr bool ROWS_ARE_QUERIES = MODE != BWD_DKV;
+  constexpr bool HALF = MODE == BWD_DQ_HALF;  // a step is one block of 32 columns
+  constexpr int BWD_SLOT = bwd_slot(MODE);
+  constexpr int SECOND = HALF ? FBLOCK32 : FTILE;  // the second tile of a slot
   constexpr int POS = ROWS_ARE_QUERIES ? NW * 32 / HP : NW * 32;  // rows per row block (of one head)
 
   // BWD_DKV: a step of its single wavefront per SIMD is about as long as a tile takes to arrive, so
   // its ring is one slot deeper and a tile has two steps to land; the column scalars travel the same
-  // way instead of through registers.
-  constexpr bool DEEP = MODE == BWD_DKV;
+  // way instead of through registers.  BWD_DQ_HALF has the same ring of half tiles.
+  constexpr bool DEEP = MODE != BWD_DQ;
   constexpr bool ALT = alternates<RMAP>;  // wavefronts 0, 1 and 2, 3 share rows and take turns at the 32-column blocks
   const uint32_t lds_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)smem;
 
@@ -313,12 +320,12 @@ __device__ __forceinline__ void bwd_rows(const BParams& p, const BwdGrid& g, con
   // at the last tile together and stay in step, so that a tile fetched for one of them is in the
   // L2 for the others.  A step is one (tile, head).
   const int n_streams = ROWS_ARE_QUERIES ? 1 : p.ratio;
-  const int n_steps = ntiles * n_streams;
+  const int n_steps = HALF ? (ce >= cb ? (ce - cb + 32) >> 5 : 0) : ntiles * n_streams;
   struct Cursor {
     int tile, head;
   };
   auto advance = [&](Cursor& c) {
-    if (ROWS_ARE_QUERIES) {
+    if (ROWS_ARE_QUERIES) {  // (HALF: half tiles)
       ++c.tile;
     } else if (++c.head == n_streams) {
       c.head = 0;
@@ -358,6 +365,9 @@ __device__ __forceinline__ void bwd_rows(const BParams& p, const BwdGrid& g, con
   // lanes and back on the ordinary path of a step: block Scatter 16 -> 1, Scatter 4 -> 0.  Training steps, us:
   // block Scatter S=6000 780.5 -> 764.9, window 575 with 64 sinks, S=8192, 476.2 -> 468.9.
   constexpr int GROUPS = 16 / NW;  // 4-row groups of either tile per wavefront
+  constexpr int STEP_GROUPS = HALF ? GROUPS / 2 : GROUPS;  // those of a step (HALF: one half of the tile, then the other)
+  // first row of group gi of this wavefront in the tile
+  auto group_row = [&](int gi) { return 4 * (wave * STEP_GROUPS + gi % STEP_GROUPS) + 32 * (gi / STEP_GROUPS) + ld_row; };
   uint32_t vo1[GROUPS], vo2[GROUPS], vos = 0;
 #pragma unroll
   for (int gi = 0; gi < GROUPS; ++gi) vo1[gi] = vo2[gi] = 0;
@@ -377,52 +387,57 @@ __device__ __forceinline__ void bwd_rows(const BParams& p, const BwdGrid& g, con
         auto row_of = [&](int i) { return (uint32_t)map.tile_rel(at.kind, RMAP::kEveryTile ? im_min(i, last) : i); };
 #pragma unroll
         for (int gi = 0; gi < GROUPS; ++gi) {
-          const uint32_t rel = row_of(4 * (wave * GROUPS + gi) + ld_row);
+          const uint32_t rel = row_of(group_row(gi));
           vo1[gi] = rel * c1rs + ld_col;
           vo2[gi] = rel * c2rs + ld_col;
         }
-        if (DEEP) vos = 4 * row_of(lane);
+        if (!ROWS_ARE_QUERIES) vos = 4 * row_of(lane);
       }
     } else {
       vo_kind = -1;
       at.base = 0;
 #pragma unroll
       for (int gi = 0; gi < GROUPS; ++gi) {
-        const uint32_t pos = (uint32_t)map.col_pos(im_min(c + 4 * (wave * GROUPS + gi) + ld_row, n_cols - 1));
+        const uint32_t pos = (uint32_t)map.col_pos(im_min(c + group_row(gi), n_cols - 1));
         vo1[gi] = pos * c1rs + ld_col;
         vo2[gi] = pos * c2rs + ld_col;
       }
-      if (DEEP) vos = 4 * (uint32_t)map.col_pos(im_min(c + lane, n_cols - 1));
+      if (!ROWS_ARE_QUERIES) vos = 4 * (uint32_t)map.col_pos(im_min(c + lane, n_cols - 1));
     }
     const uint32_t base = (uint32_t)__builtin_amdgcn_readfirstlane(at.base);
     a1 = c1base + (uint64_t)base * c1rs;
     a2 = c2base + (uint64_t)base * c2rs;
-    if (DEEP) as = reinterpret_cast<const char*>(sbase + base);
+    if (!ROWS_ARE_QUERIES) as = reinterpret_cast<const char*>(sbase + base);
   };
-  const uint32_t lds_rows = lds_base + wave * GROUPS * FGROUP_STRIDE;
+  const uint32_t lds_rows = lds_base + wave * STEP_GROUPS * FGROUP_STRIDE;
   const uint32_t lds_scalars = lds_base + 256 * (wave & 1);
-  constexpr int REQUESTS = 2 * GROUPS + (DEEP ? 1 : 0);  // per wavefront and step
+  constexpr int REQUESTS = 2 * STEP_GROUPS + (ROWS_ARE_QUERIES ? 0 : 1);  // per wavefront and step
   auto load_step = [&](const Cursor& cu, int slot_off) {
+    const int tile = HALF ? cu.tile >> 1 : cu.tile;
     if constexpr (FAR) {
-      const int c = cb + cu.tile * BN;
+      const int c = cb + cu.tile * (HALF ? 32 : BN);
 #pragma unroll
-      for (int gi = 0; gi < GROUPS; ++gi) {
-        const uint64_t pos = (uint64_t)map.col_pos(im_min(c + 4 * (wave * GROUPS + gi) + ld_row, n_cols - 1));
+      for (int gi = 0; gi < STEP_GROUPS; ++gi) {
+        const uint64_t pos = (uint64_t)map.col_pos(im_min(c + group_row(gi), n_cols - 1));
         dma_group(c1base + (cu.head * c1hs + pos * c1rs + ld_col), lds_rows + slot_off + gi * FGROUP_STRIDE);
-        dma_group(c2base + (cu.head * c2hs + pos * c2rs + ld_col), lds_rows + slot_off + FTILE + gi * FGROUP_STRIDE);
+        dma_group(c2base + (cu.head * c2hs + pos * c2rs + ld_col), lds_rows + slot_off + SECOND + gi * FGROUP_STRIDE);
       }
-      if (DEEP)
+      if (!ROWS_ARE_QUERIES)
         dma_dwords(sbase + (cu.head * p.ds_hs + map.col_pos(im_min(c + lane, n_cols - 1))),
                    lds_scalars + slot_off + 2 * FTILE);
       return;
     }
-    if (ROWS_ARE_QUERIES || cu.head == 0) aim(cu.tile);
-    static_for<0, GROUPS>([&](auto gi_c) {
-      constexpr int gi = decltype(gi_c)::value;
-      dma_rows<gi * FGROUP_STRIDE>(a1, vo1[gi], lds_rows + slot_off);
-      dma_rows<FTILE + gi * FGROUP_STRIDE>(a2, vo2[gi], lds_rows + slot_off);
-    });
-    if (DEEP) {  // (wavefronts 2, 3 repeat the scalars of 0, 1: every wavefront counts alike)
+    if (HALF ? (cu.tile & 1) == 0 : ROWS_ARE_QUERIES || cu.head == 0) aim(tile);
+    auto request = [&](auto first_c) {  // the groups from `first` on
+      static_for<0, STEP_GROUPS>([&](auto gi_c) {
+        constexpr int gi = decltype(gi_c)::value, first = decltype(first_c)::value;
+        dma_rows<gi * FGROUP_STRIDE>(a1, vo1[first + gi], lds_rows + slot_off);
+        dma_rows<SECOND + gi * FGROUP_STRIDE>(a2, vo2[first + gi], lds_rows + slot_off);
+      });
+    };
+    if (HALF && (cu.tile & 1)) request(ic<HALF ? STEP_GROUPS : 0>{});
+    else request(ic<0>{});
+    if (!ROWS_ARE_QUERIES) {  // (wavefronts 2, 3 repeat the scalars of 0, 1: every wavefront counts alike)
       dma_scalars<2 * FTILE>(as, vos, lds_scalars + slot_off);
       a1 += c1hs;  // from one head's addresses to the next one's
       a2 += c2hs;
@@ -450,6 +465,7 @@ __device__ __forceinline__ void bwd_rows(const BParams& p, const BwdGrid& g, con
     // its own accord the compiler puts nothing but accumulators there, and copied them, or the V fragments,
     // between the halves inside the blocks: of few sinks 44 moves and 13 waiting instructions per 64 MFMAs.
     // With this no block holds a move (training step, window 575 with 64 sinks, S=8192, us: 471.3 -> 467.2).
+    if constexpr (!ROWS_ARE_QUERIES)
 #pragma unroll
     for (int i = 0; i < 8; ++i) asm volatile("" : "+a"(r1f[i >> 2][i & 3]), "+a"(r2f[i >> 2][i & 3]));
   }
@@ -475,15 +491,15 @@ __device__ __forceinline__ void bwd_rows(const BParams& p, const BwdGrid& g, con
     // the tiles of steps t and t+1 have landed for everybody; nobody reads that of t-1
     if (DEEP && fresh) tile_barrier<REQUESTS>();
     else tile_barrier<0>();
-    // the tile of step t + 3 (dQ: t + 2) into the slot of step t - 1
+    // the tile of step t + 3 (BWD_DQ: t + 2) into the slot of step t - 1
     fresh = t + (DEEP ? 3 : 2) < n_steps;
     if (fresh) {
       load_step(ld, ring == 0 ? LAST_SLOT : ring - BWD_SLOT);
       advance(ld);
     }
-    static_for<0, ALT ? 1 : 2>([&](auto blk_c) {
+    static_for<0, ALT || HALF ? 1 : 2>([&](auto blk_c) {
       constexpr int blk = decltype(blk_c)::value;
-      const int jb = 2 * cur.tile + (ALT ? half : blk);
+      const int jb = HALF ? cur.tile : 2 * cur.tile + (ALT ? half : blk);
       const int sb_lo = cb + 32 * jb;  // first column of the block
       // (behind the prefix and in front of the wavefront's own range nothing is visible: a run of 4 image
       // patches streams 10 tiles of window keys, of which a patch sees 4: training steps of 24 heads
@@ -517,8 +533,8 @@ __device__ __forceinline__ void bwd_rows(const BParams& p, const BwdGrid& g, con
         const int here = blk * FBLOCK32;  // the block inside the step's slot
         // rows of the block that follows in this order, at tile `which` of its slot
         auto next_rows = [&](int which, int ff) {
-          if (ALT) return kread_b(kb1, which * FTILE, ff);
-          return blk == 0 ? kread_b(kb0, FBLOCK32 + which * FTILE, ff) : kread_b(kb1, which * FTILE, ff);
+          if (ALT || HALF) return kread_b(kb1, which * SECOND, ff);
+          return blk == 0 ? kread_b(kb0, FBLOCK32 + which * SECOND, ff) : kread_b(kb1, which * SECOND, ff);
         };
         if (MODE == BWD_DKV) {
           if (f < 8) return kread_b(kb0, here + FTILE, f);   // dO rows: dP
@@ -527,7 +543,7 @@ __device__ __forceinline__ void bwd_rows(const BParams& p, const BwdGrid& g, con
           if (f < 32) return vread_b(here, f - 24);          // Q^T: dK accumulation
           return next_rows(1, f - 32);
         }
-        if (f < 8) return kread_b(kb0, here + FTILE, f);
+        if (f < 8) return kread_b(kb0, here + SECOND, f);
         if (f < 16) return next_rows(0, f - 8);
         if (f < 24) return vread_b(here, f - 16);
         return next_rows(1, f - 24);
@@ -667,7 +683,7 @@ __device__ __forceinline__ void bwd_rows(const BParams& p, const BwdGrid& g, con
         // (opaque to the compiler, which would otherwise keep the lane parts and add the slot at every read)
         asm volatile("" : "+v"(kb0[i]), "+v"(vb0[i]), "+v"(kb1[i]));
       }
-      if (DEEP) {
+      if (!ROWS_ARE_QUERIES) {
         sb0 += d0;
         sb1 += d1;
         asm volatile("" : "+v"(sb0), "+v"(sb1));
@@ -678,7 +694,7 @@ __device__ __forceinline__ void bwd_rows(const BParams& p, const BwdGrid& g, con
   // ---------------------------------------------------------------- scale, round, store
   if (!wave_active) return;
   if constexpr (ALT) {  // wavefronts 2, 3 hand their sums to 0, 1 through the ring, which nobody reads any more
-    static_assert(MODE == BWD_DKV && NW == 4 && 2 * 32 * 64 * 16 <= bwd_ring_slots(MODE) * BWD_SLOT, "64 KB");
+    static_assert(MODE == BWD_DKV && NW == 4 && 2 * 32 * 64 * 16 <= bwd_ring_slots(MODE) * bwd_slot(MODE), "64 KB");
     floatx4* const hand = reinterpret_cast<floatx4*>(smem) + (wave & 1) * 32 * 64 + lane;
     __syncthreads();
     if (wave >= 2)
@@ -784,8 +800,8 @@ struct NoLeadingKeys {};
 // With that and shared row blocks for the text rows, 1024^2 at 24 heads: the launch 115 -> 90 us (two
 // traces), the training step 345 -> 323.
 template <class RMAP, int MODE, int HP, class LEAD, bool FAR>
-__global__ __launch_bounds__(bwd_waves(MODE) * 64) void intra_bwd_kernel(const BParams p) {
-  __shared__ __attribute__((aligned(1024))) unsigned char smem[bwd_ring_slots(MODE) * BWD_SLOT];
+__global__ __launch_bounds__(bwd_waves(MODE) * 64, MODE == BWD_DKV ? 1 : 2) void intra_bwd_kernel(const BParams p) {
+  __shared__ __attribute__((aligned(1024))) unsigned char smem[bwd_ring_slots(MODE) * bwd_slot(MODE)];
   int block = blockIdx.x;
   if constexpr (!std::is_same_v<LEAD, NoLeadingKeys>) {
     const int lead_block = block - (p.lead_first ? 0 : p.grid.blocks);
