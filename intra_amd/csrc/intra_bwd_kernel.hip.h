@@ -119,6 +119,14 @@ __device__ __forceinline__ void bwd_rows(const BParams& p, const BwdGrid& g, con
   // its ring is one slot deeper and a tile has two steps to land; the column scalars travel the same
   // way instead of through registers.  BWD_DQ_HALF has the same ring of half tiles.
   constexpr bool DEEP = MODE != BWD_DQ;
+  // BWD_DKV's wavefront is alone on its SIMD: nothing covers what it issues between its blocks.  So the requests of a
+  // step (three instructions each, nine of them) go behind MFMAs of its first block, and which blocks of a tile it
+  // needs and whether any of their pairs are hidden is worked out once per tile, not per head.  Training steps, in
+  // one piece in front of the blocks / so, us: Scatter G=8 S=32768 4339 / 4243, window 575 with 64 sinks S=8192 448 / 436,
+  // block Scatter S=6000 with 64 sinks 712 / 687, image Gather 0 1024^2 309 / 309.  (Left out altogether, the requests
+  // are worth 1 % of the Scatter step, all exponentials 2 %, all transposing reads 2 %, all vector
+  // instructions 4 %: what remains is the MFMAs, at the clock that the board's power allows.)
+  constexpr bool SPREAD = MODE == BWD_DKV && !FAR;
   constexpr bool ALT = alternates<RMAP>;  // wavefronts 0, 1 and 2, 3 share rows and take turns at the 32-column blocks
   const uint32_t lds_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)smem;
 
@@ -412,6 +420,14 @@ __device__ __forceinline__ void bwd_rows(const BParams& p, const BwdGrid& g, con
   const uint32_t lds_rows = lds_base + wave * STEP_GROUPS * FGROUP_STRIDE;
   const uint32_t lds_scalars = lds_base + 256 * (wave & 1);
   constexpr int REQUESTS = 2 * STEP_GROUPS + (ROWS_ARE_QUERIES ? 0 : 1);  // per wavefront and step
+  // request n of a step of dK / dV: the groups of either tile in turns, then the scalars (wavefronts 2, 3 repeat
+  // those of 0, 1: every wavefront counts alike)
+  auto request_one = [&](auto n_c, int slot_off) {
+    constexpr int n = decltype(n_c)::value;
+    if constexpr (n == 2 * GROUPS) dma_scalars<2 * FTILE>(as, vos, lds_scalars + slot_off);
+    else if constexpr (n % 2 == 0) dma_rows<n / 2 * FGROUP_STRIDE>(a1, vo1[n / 2], lds_rows + slot_off);
+    else dma_rows<FTILE + n / 2 * FGROUP_STRIDE>(a2, vo2[n / 2], lds_rows + slot_off);
+  };
   auto load_step = [&](const Cursor& cu, int slot_off) {
     const int tile = HALF ? cu.tile >> 1 : cu.tile;
     if constexpr (FAR) {
@@ -427,7 +443,18 @@ __device__ __forceinline__ void bwd_rows(const BParams& p, const BwdGrid& g, con
                    lds_scalars + slot_off + 2 * FTILE);
       return;
     }
-    if (HALF ? (cu.tile & 1) == 0 : ROWS_ARE_QUERIES || cu.head == 0) aim(tile);
+    if constexpr (SPREAD) {
+      if (cu.head == 0) {
+        aim(tile);
+      } else {  // from one head's addresses to the next one's
+        a1 += c1hs;
+        a2 += c2hs;
+        as += 4 * (uint32_t)p.ds_hs;  // (S floats)
+      }
+      if (slot_off >= 0) static_for<0, REQUESTS>([&](auto n_c) { request_one(n_c, slot_off); });
+      return;
+    }
+    if (HALF ? (cu.tile & 1) == 0 : true) aim(tile);
     auto request = [&](auto first_c) {  // the groups from `first` on
       static_for<0, STEP_GROUPS>([&](auto gi_c) {
         constexpr int gi = decltype(gi_c)::value, first = decltype(first_c)::value;
@@ -437,12 +464,6 @@ __device__ __forceinline__ void bwd_rows(const BParams& p, const BwdGrid& g, con
     };
     if (HALF && (cu.tile & 1)) request(ic<HALF ? STEP_GROUPS : 0>{});
     else request(ic<0>{});
-    if (!ROWS_ARE_QUERIES) {  // (wavefronts 2, 3 repeat the scalars of 0, 1: every wavefront counts alike)
-      dma_scalars<2 * FTILE>(as, vos, lds_scalars + slot_off);
-      a1 += c1hs;  // from one head's addresses to the next one's
-      a2 += c2hs;
-      as += 4 * (uint32_t)p.ds_hs;  // (S floats)
-    }
   };
   // Three tile slots: while step t works on its tile, the tile of step t+1 has landed (the scores
   // of its first block are formed at the end of step t) and the tile of step t+2 is in flight.
@@ -451,8 +472,9 @@ __device__ __forceinline__ void bwd_rows(const BParams& p, const BwdGrid& g, con
   // (Deep ring: one slot more, the tile of step t+3 is requested during step t, and the barrier of a
   // step leaves the most recent request in flight where one was made during the step before.)
   for (int t = 0; t < (DEEP ? 3 : 2) && t < n_steps; ++t) {
+    if (SPREAD && t > 0) advance(ld);  // (SPREAD: ld is the step requested last)
     load_step(ld, t * BWD_SLOT);
-    advance(ld);
+    if (!SPREAD) advance(ld);
   }
   // The deep ring's barriers leave requests in flight.  The row operands are ordinary loads the
   // compiler waits for at their first use, inside the main loop, with a count that knows nothing of
@@ -487,15 +509,38 @@ __device__ __forceinline__ void bwd_rows(const BParams& p, const BwdGrid& g, con
   floatx4 l4_keep[2] = {zero4, zero4}, d4_keep[2] = {zero4, zero4};
   // dQ: -D of the lane's two rows, as the accumulators of dP start from it
   const floatx4 nd_row[2] = {floatx4{-D_row[0], -D_row[0], -D_row[0], -D_row[0]}, floatx4{-D_row[1], -D_row[1], -D_row[1], -D_row[1]}};
+  // (dK / dV without a block predicate: what the wavefront does with the blocks of a tile, worked out once for all heads)
+  constexpr bool PER_TILE = SPREAD && !RMAP::kBlockPredicate;
+  int todo = 0;  // bits 2 * blk: the block is wanted, 2 * blk + 1: none of it is hidden
   for (int t = 0; t < n_steps; ++t) {
     // the tiles of steps t and t+1 have landed for everybody; nobody reads that of t-1
-    if (DEEP && fresh) tile_barrier<REQUESTS>();
+    if (SPREAD || (DEEP && fresh)) tile_barrier<REQUESTS>();
     else tile_barrier<0>();
     // the tile of step t + 3 (BWD_DQ: t + 2) into the slot of step t - 1
-    fresh = t + (DEEP ? 3 : 2) < n_steps;
-    if (fresh) {
-      load_step(ld, ring == 0 ? LAST_SLOT : ring - BWD_SLOT);
-      advance(ld);
+    const int free_slot = ring == 0 ? LAST_SLOT : ring - BWD_SLOT;
+    if constexpr (SPREAD) {
+      // Behind the last steps the last tile is requested again, which nobody reads: every step leaves the same number
+      // of requests in flight.
+      if (t + 3 < n_steps) {
+        advance(ld);
+        load_step(ld, -1);
+      }
+    } else {
+      fresh = t + (DEEP ? 3 : 2) < n_steps;
+      if (fresh) {
+        load_step(ld, free_slot);
+        advance(ld);
+      }
+    }
+    if (PER_TILE && cur.head == 0) {
+      todo = 0;
+#pragma unroll
+      for (int blk = 0; blk < (ALT ? 1 : 2); ++blk) {
+        const int jb = 2 * cur.tile + (ALT ? half : blk);
+        const int sb_lo = cb + 32 * jb;
+        if (jb >= jb_lo && jb <= jb_hi && (kpre == 0 || block_wanted(wb, kpre, sb_lo))) todo |= 1 << (2 * blk);
+        if (block_unmasked(wb, kpre, sb_lo)) todo |= 2 << (2 * blk);
+      }
     }
     static_for<0, ALT || HALF ? 1 : 2>([&](auto blk_c) {
       constexpr int blk = decltype(blk_c)::value;
@@ -504,7 +549,7 @@ __device__ __forceinline__ void bwd_rows(const BParams& p, const BwdGrid& g, con
       // (behind the prefix and in front of the wavefront's own range nothing is visible: a run of 4 image
       // patches streams 10 tiles of window keys, of which a patch sees 4: training steps of 24 heads
       // 397 -> 392 us at 1024^2, 1259 -> 1236 us at 2048^2)
-      bool wanted = jb >= jb_lo && jb <= jb_hi && (kpre == 0 || block_wanted(wb, kpre, sb_lo));
+      bool wanted = PER_TILE ? (todo >> (2 * blk)) & 1 : jb >= jb_lo && jb <= jb_hi && (kpre == 0 || block_wanted(wb, kpre, sb_lo));
       // maps with a block predicate: a row meets the whole block or nothing of it
       bool lane_sees[2] = {true, true};
       bool masked;
@@ -514,7 +559,17 @@ __device__ __forceinline__ void bwd_rows(const BParams& p, const BwdGrid& g, con
         wanted = wanted && __builtin_amdgcn_ballot_w64(lane_sees[0] || lane_sees[1]) != 0;
         masked = __builtin_amdgcn_ballot_w64(lane_sees[0] && lane_sees[1]) != ~0ull;
       } else {
-        masked = !block_unmasked(wb, kpre, sb_lo);
+        masked = PER_TILE ? !((todo >> (2 * blk + 1)) & 1) : !block_unmasked(wb, kpre, sb_lo);
+      }
+      constexpr bool REQUEST = SPREAD && blk == 0;
+      if constexpr (REQUEST) {
+        // (A branch of its own: with this code in the way around the block the compiler gives the accumulators other
+        // registers and moves them in and out of the block.)
+        int w = __builtin_amdgcn_readfirstlane((int)wanted);
+        asm volatile("" : "+s"(w));
+        if (!w) static_for<0, REQUESTS>([&](auto n_c) { request_one(n_c, free_slot); });
+        asm volatile("" : "+s"(w));
+        wanted = w;
       }
       if (!wanted) {
         have = false;
@@ -624,6 +679,9 @@ __device__ __forceinline__ void bwd_rows(const BParams& p, const BwdGrid& g, con
         for (int i = 2 * (f - LA) + 2; i < 2 * f; ++i) n += scalar_slot((i + NSLOT) % NSLOT);
         return n < 15 ? n : 15;
       };
+      // slots 26, 30, .. 58 (every 2nd, 4th or 7th from 0, 2, 26 or 42 on: the same within 0.2 %)
+      constexpr auto request_at = [](int i) { return i >= 26 && i % 4 == 2 ? (i - 26) / 4 : REQUESTS; };
+      static_assert(!REQUEST || request_at(58) == REQUESTS - 1, "every request has its slot");
       // (compile-time slot numbers: a loop of this size is beyond what the compiler unrolls in full)
       static_for<0, NSLOT>([&](auto slot_c) {
         constexpr int i = decltype(slot_c)::value;
@@ -644,6 +702,7 @@ __device__ __forceinline__ void bwd_rows(const BParams& p, const BwdGrid& g, con
           if (i == 54) d4[0] = *reinterpret_cast<const floatx4*>(scn + 64);
           if (i == 56) d4[1] = *reinterpret_cast<const floatx4*>(scn + 64 + 16);
         }
+        if constexpr (REQUEST && request_at(i) < REQUESTS) request_one(ic<request_at(i)>{}, free_slot);
         __builtin_amdgcn_sched_barrier(0);
         if constexpr (i >= 1 && i < 25) {
           constexpr int u = (i - 1) / 3, part = (i - 1) % 3;
@@ -690,6 +749,7 @@ __device__ __forceinline__ void bwd_rows(const BParams& p, const BwdGrid& g, con
       }
     }
   }
+  if (SPREAD) __builtin_amdgcn_s_waitcnt((0 & 15) | (7 << 4) | (15 << 8) | (0 << 14));  // vmcnt(0): the repeated requests
 
   // ---------------------------------------------------------------- scale, round, store
   if (!wave_active) return;
