@@ -8,6 +8,7 @@
 
 #include <algorithm>
 #include <atomic>
+#include <functional>
 #include <type_traits>
 
 #include "../../include/intra_hip.h"
@@ -127,8 +128,8 @@ int default_hp(int ratio) { return ratio % 4 == 0 ? 4 : (ratio % 2 == 0 ? 2 : 1)
 // quarter of the wavefronts busy, and the static dealing of work items wants items of about one
 // size: 2 if the estimated cost stays within 15 % of a patch item's, else 1.  A key tile with w of
 // 8 wavefronts busy is taken to cost 5/9 + w/18 of a full one (2/3 at w = 2, measured).
-// The forward launch decides for dQ too (24 heads, us, one chunk / two per row block: forward 1024^2 74.6 / 74.5,
-// 2048^2 261 / 302; dQ 122.7 / 101.8 and 377 / 372).
+// dQ asks with its own row blocks (24 heads, us, one chunk / two per row block: forward 1024^2 74.6 / 74.5,
+// 2048^2 261 / 302; dQ in 8 wavefronts 122.7 / 101.8 and 377 / 372).
 int pick_text_merge(const IntraGeom& ge, int pos, int pg, int nw) {
   const int chunk = ge.text_len / 8, nimg = ge.width * ge.width / 8;
   if (chunk % 32 != 0 || 2 * chunk > pos) return 1;  // (more chunks than a row block holds share nothing)
@@ -610,18 +611,62 @@ int launch_bwd(const intra::BParams& p, hipStream_t stream) {
   return INTRA_OK;
 }
 
+// When the last workgroup of an XCD ends if its pairs are taken in bundles of `bundle`: they start in order, each
+// where the first of `places` is free.
+int bundled_end(const int* cost, const intra::BwdGrid& g, int pairs, int bundle, int places) {
+  int ends[MAX_COSTED_WORKGROUPS] = {};  // (a heap: the earliest end in front)
+  for (int b0 = 0; b0 < pairs; b0 += bundle)
+    for (int item = 0; item < g.items_per_pair; ++item)
+      for (int pr = b0; pr < std::min(b0 + bundle, pairs); ++pr) {
+        std::pop_heap(ends, ends + places, std::greater<int>());
+        ends[places - 1] += cost[item / g.hgroups];
+        std::push_heap(ends, ends + places, std::greater<int>());
+      }
+  return *std::max_element(ends, ends + places);
+}
+
+// Whether a launch is more than 8 % shorter if all pairs of an XCD are one bundle: the longest row blocks of the last
+// bundle otherwise start only when those of the bundles before it have.  cost: of the row blocks, in the order in
+// which they start; pair: of all items of a pair.  Training steps, bundles as small as fill the CUs / one bundle, us:
+// Scatter G=3 S=7000 611 / 542 (dK / dV 35 % shorter by this count), G=8 S=5000 182 / 165 (24 %), G=2 S=3000 of 32 kv heads
+// 217 / 188 (dQ 38 %), G=2 S=6000 of 32 655 / 628 (dQ 22 %), Gather 1 S=4992 185 / 167, block Scatter G=2 S=6000 of 16
+// 376 / 347 (dQ 28 %).  With less to gain the pairs of one bundle only share the XCD's L2 with more others: block
+// Scatter G=8 S=20000 1875 / 1903 (4 %), of 16 kv heads 955 / 962 (4 %), Scatter G=8 S=20000 1733 / 1734 (4 %).
+constexpr int MAX_COSTED_BWD_ITEMS = 512;  // per XCD (with more of them the last bundle is a small share)
+bool one_bundle_pays(const int* cost, int64_t pair, const intra::BwdGrid& g, int pairs, int places) {
+  const int64_t longest = *std::max_element(cost, cost + g.n_rblocks), before = (pairs - 1) / g.bundle * g.bundle * pair;
+  if (100 * (before + places * longest) <= 108 * pairs * pair) return false;  // (too short a last row block to matter)
+  return 100ll * bundled_end(cost, g, pairs, g.bundle, places) > 108ll * bundled_end(cost, g, pairs, pairs, places);
+}
+
 // Workgroups of a row map with `rows` rows each, per_cu of which a CU holds at once: per XCD, bundles of pairs x
 // items of a pair (see the kernel).  blocks = -1 if they are too many to number.
 template <class R>
 intra::BwdGrid bwd_grid(const intra::BParams& p, int rows, int hgroups, int per_cu = 1) {
   intra::BwdGrid g;
   const int64_t pairs = (int64_t)R::num_sets(p.geom) * p.B * p.Hkv;
-  g.hgroups = hgroups;
+  g.hgroups = std::max(1, hgroups);
   g.n_rblocks = (R::max_rows(p.geom) + rows - 1) / rows;
-  g.items_per_pair = g.n_rblocks * hgroups;
+  g.items_per_pair = g.n_rblocks * g.hgroups;
   const int64_t pairs_per_xcd = (pairs + 7) / 8;
   const int64_t want = (32 * per_cu + g.items_per_pair - 1) / g.items_per_pair;  // pairs that fill an XCD's 32 CUs
   g.bundle = (int)std::max<int64_t>(1, std::min<int64_t>(want, pairs_per_xcd));
+  if (g.bundle < pairs_per_xcd && g.n_rblocks > 1 && pairs_per_xcd * g.items_per_pair <= MAX_COSTED_BWD_ITEMS) {
+    int cost[MAX_COSTED_BWD_ITEMS];
+    int64_t pair = 0;
+    bool one_range = true;
+    for (int b = 0; b < g.n_rblocks; ++b) {  // in the order in which they start: the longest first
+      const int r0 = (hgroups > 0 ? g.n_rblocks - 1 - b : b) * rows;
+      const R map(p.geom, 0, r0);
+      const int r1 = std::min(r0 + rows, map.n_rows()) - 1;
+      const int columns = r1 < r0 ? 0 : map.block_hi(r0, r1) - map.block_lo(r0, r1) + 1;
+      cost[b] = r1 < r0 ? 0 : ITEM_COST + (std::max(0, columns) + 63) / 64 * (hgroups > 0 ? 1 : p.ratio);
+      pair += (int64_t)cost[b] * g.hgroups;
+      one_range = one_range && map.kpre() == 0;
+    }
+    // (row blocks of about one length take as long either way)
+    if (one_range && 2 * cost[g.n_rblocks - 1] < cost[0] && one_bundle_pays(cost, pair, g, (int)pairs_per_xcd, 32 * per_cu)) g.bundle = (int)pairs_per_xcd;
+  }
   const int64_t bundles = (pairs_per_xcd + g.bundle - 1) / g.bundle;
   const int64_t blocks = 8 * bundles * g.bundle * g.items_per_pair;
   g.blocks = blocks > 0x7fffffff ? -1 : (int)blocks;
@@ -684,7 +729,7 @@ int run_bwd_dq_gather0(intra::BParams p, int hp, hipStream_t stream) {
 using intra::KEY_ROWS;
 template <class R>
 int run_bwd_keys(intra::BParams p, hipStream_t stream) {
-  p.grid = bwd_grid<R>(p, KEY_ROWS, 1);
+  p.grid = bwd_grid<R>(p, KEY_ROWS, 0);
   return launch_bwd<R, intra::BWD_DKV, 1>(p, stream);
 }
 
@@ -692,8 +737,8 @@ int run_bwd_keys(intra::BParams p, hipStream_t stream) {
 // meet more columns than the longest row block of R (the shorter workgroups then fill the last round).
 template <class R, class LEAD>
 int run_bwd_keys_lead(intra::BParams p, hipStream_t stream) {
-  p.grid = bwd_grid<R>(p, KEY_ROWS, 1);
-  p.lead = bwd_grid<LEAD>(p, KEY_ROWS, 1);
+  p.grid = bwd_grid<R>(p, KEY_ROWS, 0);
+  p.lead = bwd_grid<LEAD>(p, KEY_ROWS, 0);
   // (their work counts half where both halves of a workgroup share the columns)
   p.lead_first = std::min(p.geom.sink_chunk, p.geom.S) / (intra::alternates<LEAD> ? 2 : 1) > R::longest(p.geom);
   return launch_bwd<R, intra::BWD_DKV, 1, LEAD>(p, stream);
