@@ -454,6 +454,23 @@ bool row_order_pays(const int* cost, int n_mblocks, int pairs, int hgroups, int 
   return 100ll * longest[0] > (4 * pairs <= 32 ? 103ll : 112ll) * longest[1];
 }
 
+// log2 of the parts that the row blocks of a pair are split into, the parts dealt like pairs: the fewest after which
+// the XCD with the most work has at least a tenth fewer rounds.  A whole pair on one XCD loads its keys into one L2
+// only, but a call with few kv heads then leaves XCDs idle.  per_xcd: workgroups of an XCD at a time.  Whole / split, us:
+// window 255 with 4 sinks S=13568, 4 / 1 heads 103 / 20 (training step 422 / 158); window 2112 S=30000, 8 / 1 heads
+// 1469 / 229 (6416 / 971); window 1023 with 64 sinks S=11671, 28 / 4 heads 368 / 191 (1463 / 852); window 576 S=3000,
+// 16 / 4 heads 35.0 / 21.8; Scatter G=3 S=20000, 28 / 4 heads 1098 / 893 (4608 / 3625).  With as many rounds either way:
+// window 575 with 64 sinks S=6000, 12 / 12 heads 46.8 / 51.4.
+int xcd_split(int64_t pairs, int n_rblocks, int hgroups, int per_xcd) {
+  auto rounds = [&](int s) {
+    return (((pairs << s) + 7) / 8 * ((n_rblocks + (1 << s) - 1) >> s) * hgroups + per_xcd - 1) / per_xcd;
+  };
+  int split = 0;
+  for (int s = 1; s <= 3; ++s)
+    if (10 * rounds(split) > 11 * rounds(s)) split = s;
+  return split;
+}
+
 // Order of an XCD's work items (see KParams::Section).  One section - every pair, all row blocks -
 // except where a launch mixes kinds of items:
 //  * image scatter: a set has text_len / 8 + width^2 / 8 queries, so its last row block is partial
@@ -463,24 +480,29 @@ bool row_order_pays(const int* cost, int n_mblocks, int pairs, int hgroups, int 
 //    first pair slots) and the patch runs can have different numbers of row blocks; each kind gets
 //    its section, so that no number goes to an empty item, text rows first.
 void set_sections(intra::KParams& p, const Request& r, const Shape& ph, const LaunchDims& d, int wgs_per_xcd) {
-  const int pslots = (d.n_pairs + 7) / 8;
-  p.row_order = 0;
-  if (ph.map != MAP_IMG_SCATTER && ph.map != MAP_IMG_GATHER0 &&  // (has_sections: items of one length)
-      pslots > 1 && 2 * pslots <= 32 && pslots * d.n_mblocks * d.hgroups > wgs_per_xcd && wgs_per_xcd <= MAX_COSTED_WORKGROUPS &&
-      d.n_mblocks <= MAX_COSTED_ROW_BLOCKS) {
+  const bool llm = ph.map != MAP_IMG_SCATTER && ph.map != MAP_IMG_GATHER0;  // (the others: has_sections, items of one length)
+  const int split = llm ? xcd_split(d.n_pairs, d.n_mblocks, d.hgroups, wgs_per_xcd) : 0;
+  const int n_mblocks = (d.n_mblocks + (1 << split) - 1) >> split;  // of a part
+  p.n_pairs = d.n_pairs << split;
+  const int pslots = (p.n_pairs + 7) / 8;
+  bool row_order = false;
+  if (llm && pslots > 1 && 2 * pslots <= 32 && pslots * n_mblocks * d.hgroups > wgs_per_xcd &&
+      wgs_per_xcd <= MAX_COSTED_WORKGROUPS && d.n_mblocks <= MAX_COSTED_ROW_BLOCKS) {
     int cost[MAX_COSTED_ROW_BLOCKS];
     by_map<RowBlockCosts>(ph.map, ph.geom, d.pos, d.n_mblocks, cost);
-    p.row_order = row_order_pays(cost, d.n_mblocks, pslots, d.hgroups, wgs_per_xcd);
+    for (int m = 0; m < n_mblocks; ++m) cost[m] = cost[m << split];
+    row_order = row_order_pays(cost, n_mblocks, pslots, d.hgroups, wgs_per_xcd);
   }
+  p.order = 2 * split + row_order;
   auto section = [&](int p_lo, int p_n, int mb_lo, int mb_hi) {
     intra::KParams::Section s;
     s.p_lo = p_lo;
     s.mb_hi = mb_hi;
     s.slots = p_n * (mb_hi - mb_lo) * d.hgroups;
-    s.d_items = make_fastdiv(std::max(1, (p.row_order ? p_n : mb_hi - mb_lo) * d.hgroups));
+    s.d_items = make_fastdiv(std::max(1, (row_order ? p_n : mb_hi - mb_lo) * d.hgroups));
     return s;
   };
-  p.sec[0] = section(0, pslots, 0, d.n_mblocks);
+  p.sec[0] = section(0, pslots, 0, n_mblocks);
   p.sec[1] = section(0, 0, 0, 1);
   if (ph.map == MAP_IMG_SCATTER) {
     const int nq = r.geom.text_len / 8 + r.geom.width * r.geom.width / 8;
@@ -508,7 +530,6 @@ void set_dealing(intra::KParams& p, const Request& r, const Shape& ph, const Lau
   p.n_sets = dims.n_sets;
   p.n_mblocks = dims.n_mblocks;
   p.hgroups = dims.hgroups;
-  p.n_pairs = dims.n_pairs;
   set_sections(p, r, ph, dims, grid / 8);
   p.d_nbh = make_fastdiv(r.B * r.Hkv);
   p.d_hkv = make_fastdiv(r.Hkv);
@@ -644,9 +665,12 @@ bool one_bundle_pays(const int* cost, int64_t pair, const intra::BwdGrid& g, int
 template <class R>
 intra::BwdGrid bwd_grid(const intra::BParams& p, int rows, int hgroups, int per_cu = 1) {
   intra::BwdGrid g;
-  const int64_t pairs = (int64_t)R::num_sets(p.geom) * p.B * p.Hkv;
   g.hgroups = std::max(1, hgroups);
   g.n_rblocks = (R::max_rows(p.geom) + rows - 1) / rows;
+  int64_t pairs = (int64_t)R::num_sets(p.geom) * p.B * p.Hkv;
+  g.split = xcd_split(pairs, g.n_rblocks, g.hgroups, 32 * per_cu);
+  pairs <<= g.split;  // (parts of pairs from here on)
+  g.n_rblocks = (g.n_rblocks + (1 << g.split) - 1) >> g.split;
   g.items_per_pair = g.n_rblocks * g.hgroups;
   const int64_t pairs_per_xcd = (pairs + 7) / 8;
   const int64_t want = (32 * per_cu + g.items_per_pair - 1) / g.items_per_pair;  // pairs that fill an XCD's 32 CUs
@@ -656,7 +680,7 @@ intra::BwdGrid bwd_grid(const intra::BParams& p, int rows, int hgroups, int per_
     int64_t pair = 0;
     bool one_range = true;
     for (int b = 0; b < g.n_rblocks; ++b) {  // in the order in which they start: the longest first
-      const int r0 = (hgroups > 0 ? g.n_rblocks - 1 - b : b) * rows;
+      const int r0 = ((hgroups > 0 ? g.n_rblocks - 1 - b : b) << g.split) * rows;
       const R map(p.geom, 0, r0);
       const int r1 = std::min(r0 + rows, map.n_rows()) - 1;
       const int columns = r1 < r0 ? 0 : map.block_hi(r0, r1) - map.block_lo(r0, r1) + 1;

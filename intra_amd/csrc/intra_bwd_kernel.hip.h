@@ -45,11 +45,12 @@ static_assert(bwd_waves(BWD_DKV) * 32 == KEY_ROWS, "keys of a row block");
 
 // Workgroups of one row map in a launch
 struct BwdGrid {
-  int n_rblocks;       // row blocks per set
+  int n_rblocks;       // row blocks per set, or per part of one
   int hgroups;         // ratio / HP (dQ only)
   int items_per_pair;  // n_rblocks * hgroups
   int bundle;          // pairs of one XCD that are worked on together
   int blocks;          // workgroups, a multiple of 8
+  int split;           // log2 of the parts that a pair's row blocks are split into (row block m: part m % 2^split), taken as pairs
 };
 
 struct BParams {
@@ -147,13 +148,15 @@ __device__ __forceinline__ void bwd_rows(const BParams& p, const BwdGrid& g, con
   const int bun = slot / per_bundle, rem = slot - bun * per_bundle;
   const int heavy = rem / g.bundle;
   const int nbh = p.B * p.Hkv;
-  const int pair = (bun * g.bundle + (rem - heavy * g.bundle)) * 8 + xcd;
+  const int part = (bun * g.bundle + (rem - heavy * g.bundle)) * 8 + xcd;
+  const int pair = part >> g.split;
   if (pair >= RMAP::num_sets(p.geom) * nbh) return;
   int hg = 0, rblk = heavy;
   if (ROWS_ARE_QUERIES) {
     hg = heavy % g.hgroups;
     rblk = g.n_rblocks - 1 - heavy / g.hgroups;
   }
+  rblk = (rblk << g.split) + (part - (pair << g.split));
   const int set = pair / nbh;
   const int bh = pair % nbh;
   const int batch = bh / p.Hkv;

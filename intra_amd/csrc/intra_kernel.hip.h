@@ -87,20 +87,21 @@ struct KParams {
   int n_sets;          // sets per (batch, kv head)
   int n_mblocks;       // row blocks of the largest set
   int hgroups;         // ratio / HP
-  int n_pairs;         // B * Hkv * n_sets
+  int n_pairs;         // B * Hkv * n_sets, times the parts of a pair
   int n_slots;         // work items per XCD: sum of the sections' slots
   // The work items of an XCD are numbered section by section (costly kinds of items first, so
   // that the cheap ones fill the last, partial round of the workgroups; kinds of sets with
   // different numbers of row blocks apart, so that no number goes to an empty item): a section is
   // a range of the XCD's pairs times a range of row blocks, last row block first, taken pair by pair or
-  // (row_order) row block by row block, the same one of every pair in turn.
+  // (row_order) row block by row block, the same one of every pair in turn.  Where a pair's row blocks are split into
+  // 2^n parts, row block m belongs to part m % 2^n and the parts take the places of pairs.
   struct Section {
     int p_lo;          // first pair slot (pair = 8 * pair slot + XCD)
     int mb_hi;         // one past its last row block
     int slots;         // pair slots * row blocks * hgroups
     FastDiv d_items;   // division by its items per pair, row blocks * hgroups, or (row_order) per row block, pair slots * hgroups
   } sec[2];
-  int row_order;
+  int order;  // bit 0 (row_order): see above; from bit 1 on: log2 of the parts that a pair's row blocks are split into
   FastDiv d_nbh, d_hkv, d_hgroups;  // divisions by B * Hkv, Hkv, hgroups
   long long* diag;     // INTRA_DIAG_TIMERS builds: DIAG_SLOTS counters per workgroup, or null
 };
@@ -243,11 +244,12 @@ IM_HD Range range_of_block(const MAP& map, int mblk, int pos) {
 
 // Dealing of work items.  Workgroups are handed to the 8 XCDs round-robin by id, so workgroup
 // id % 8 names the XCD.  All row blocks of one (batch, kv head, set) "pair" go to one XCD, longest row
-// block first.  Inside an XCD the slots are dealt to its workgroups in boustrophedon order (0..w-1, w-1..0,
+// block first, or, where the pairs do not come out even over the XCDs, to 2, 4 or 8 of them in turn
+// (xcd_split).  Inside an XCD the slots are dealt to its workgroups in boustrophedon order (0..w-1, w-1..0,
 // ...), which balances a sequence of descending lengths.  Taken pair by pair, so that a pair's K/V stays in
 // the XCD's L2 while its row blocks run, the lengths jump from 1 back to the longest at every new pair: balanced
 // where the pairs' ends fall together with those of the rounds, and up to half more than the mean for the
-// unluckiest workgroup elsewhere.  Taken row block by row block (KParams::row_order) they descend throughout.
+// unluckiest workgroup elsewhere.  Taken row block by row block (KParams::order) they descend throughout.
 // The host decides (row_order_pays).
 // locate_item: the first non-empty work item of workgroup `wg_in_xcd` (of `wgs_per_xcd`) of XCD `xcd`
 // at or after `round`; false when there is none.  `redo` (device, second pass only): bitmap of the
@@ -268,16 +270,18 @@ IM_HD bool locate_item(const KParams& p, int xcd, int wgs_per_xcd, int wg_in_xcd
     const int q1 = (int)fd_div(sslot, sc.d_items);
     const int rem = sslot - q1 * (int)sc.d_items.d;
     const int q2 = (int)fd_div(rem, p.d_hgroups);
-    const bool rows = !has_sections<MAP> && p.row_order;
+    const int order = has_sections<MAP> ? 0 : p.order, split = order >> 1;
+    const bool rows = order & 1;
     const int pq = rows ? q2 : q1, rblk = rows ? q1 : q2;
-    const int pair = ((has_sections<MAP> ? sc.p_lo : 0) + pq) * 8 + xcd;
-    if (pair >= p.n_pairs) continue;
+    const int part = ((has_sections<MAP> ? sc.p_lo : 0) + pq) * 8 + xcd;
+    if (part >= p.n_pairs) continue;
+    const int pair = part >> split;
     w.round = round;
     w.set = (int)fd_div(pair, p.d_nbh);
     const int bh = pair - w.set * (int)p.d_nbh.d;
     w.batch = (int)fd_div(bh, p.d_hkv);
     w.kvh = bh - w.batch * p.Hkv;
-    w.mblk = sc.mb_hi - 1 - rblk;
+    w.mblk = ((sc.mb_hi - 1 - rblk) << split) + (part - (pair << split));
     w.hg = rem - q2 * p.hgroups;
     if (w.mblk * POS >= MAP(p.geom, w.set, w.mblk * POS).nq()) continue;
     return true;

@@ -76,6 +76,22 @@ def test_uneven_sizes_every_row_block_once(lib, case, waves):
         assert np.array_equal(visits, base), (case, waves, grid)
 
 
+@pytest.mark.parametrize("waves", [8, 4])
+@pytest.mark.parametrize("pattern,arg0,arg1", [(SCATTER, 1, 0), (SCATTER, 3, 0), (WINDOW, 8, 576)])
+@pytest.mark.parametrize("B,S,H,Hkv", [(1, 13568, 4, 1), (1, 5000, 28, 4), (3, 4099, 8, 1), (1, 9000, 6, 6), (3, 2500, 12, 3), (1, 700, 2, 1)])
+def test_few_pairs_every_row_block_once(lib, B, S, H, Hkv, pattern, arg0, arg1, waves):
+    """Pairs that do not come out even over the XCDs: their row blocks are split."""
+    rc, base = deal(lib, LLM, pattern, B, S, H, Hkv, arg0, arg1, waves, 8)
+    assert rc == 0, _lib.last_error()
+    assert base.max() == 1 and base.sum() > 0
+    for grid in (16, 64, 256, 512):
+        rc, visits = deal(lib, LLM, pattern, B, S, H, Hkv, arg0, arg1, waves, grid)
+        if rc != 0:
+            assert "grid" in _lib.last_error()
+            continue
+        assert np.array_equal(visits, base), (waves, grid)
+
+
 def test_plan_names_the_half_size_workgroups_for_image_gather0(lib):
     plan = _lib.IntraPlan()
     assert lib.intra_plan(IMAGE, GATHER0, 1, 16896, 24, 24, 128, 512, plan) == 0
