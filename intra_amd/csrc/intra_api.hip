@@ -230,6 +230,25 @@ int cu_count() {
   return n;
 }
 
+// log2 of the parts that the row blocks of a pair are split into, the parts dealt like pairs: the fewest after which
+// the XCD with the most work has at least a tenth fewer rounds.  A whole pair on one XCD loads its keys into one L2
+// only, but a call with few kv heads then leaves XCDs idle.  per_xcd: workgroups of an XCD at a time (half-size ones count one per CU: two on a CU take
+// turns, so they are spread first).  Whole / split, us:
+// window 255 with 4 sinks S=13568, 4 / 1 heads 103 / 20 (training step 422 / 158); window 2112 S=30000, 8 / 1 heads
+// 1469 / 229 (6416 / 971); window 1023 with 64 sinks S=11671, 28 / 4 heads 368 / 191 (1463 / 852); window 576 S=3000,
+// 16 / 4 heads 35.0 / 21.8; Scatter G=3 S=20000, 28 / 4 heads 1098 / 893 (4608 / 3625).  With as many rounds either way:
+// window 575 with 64 sinks S=6000, 12 / 12 heads 46.8 / 51.4.
+int64_t xcd_rounds(int64_t pairs, int n_rblocks, int hgroups, int per_xcd, int split) {
+  return (((pairs << split) + 7) / 8 * ((n_rblocks + (1 << split) - 1) >> split) * hgroups + per_xcd - 1) / per_xcd;
+}
+int xcd_split(int64_t pairs, int n_rblocks, int hgroups, int per_xcd) {
+  auto rounds = [&](int s) { return xcd_rounds(pairs, n_rblocks, hgroups, per_xcd, s); };
+  int split = 0;
+  for (int s = 1; s <= 3; ++s)
+    if (10 * rounds(split) > 11 * rounds(s)) split = s;
+  return split;
+}
+
 // Wavefronts per workgroup of a forward launch.  Half-size workgroups, two per CU, pay for every key
 // tile twice as often per query (measured: 7 % on the long rows of LLM Scatter), and gain where the
 // work items are short or few:
@@ -237,7 +256,9 @@ int cu_count() {
 //    workgroups of a CU fill each other's waits): 0.0775 -> 0.0694 ms at 1024^2, 0.266 -> 0.235 at 2048^2;
 //  * launches with so few row blocks that the CU with the most work gets at least a fifth less of it
 //    when the blocks are half as large (8 kv heads at S <= 1024: 22 -> 18 us; image scatter at
-//    1024^2, whose 576 row blocks of 256 queries are 2.25 per CU).
+//    1024^2, whose 576 row blocks of 256 queries are 2.25 per CU; where the row blocks of few kv heads are split over
+//    XCDs, 8 wavefronts / 4, us: window 1088 S=2000, 8 / 2 heads 31.9 / 24.1; Scatter G=2 S=8000, 4 / 1 heads 92.8 / 68.7; and
+//    where it is not taken, window 1088 S=8000, 8 / 1 heads 36.4 / 38.3).
 // The environment variable INTRA_WAVES (4 or 8) overrides the choice for measurements, where the
 // shape exists.
 int pick_waves(const Request& r, int hp) {
@@ -251,9 +272,14 @@ int pick_waves(const Request& r, int hp) {
   if (r.kind == KIND_IMG_GATHER0) return intra::NARROW_WAVES;
   int cus = cu_count();
   if (cus <= 0) cus = 256;  // (planning without a device)
-  const int64_t items8 = by_map<DimsOf>(wide.map, r, wide).work_items, items4 = by_map<DimsOf>(narrow.map, r, narrow).work_items;
-  if (items8 <= 0 || items4 <= 0) return 8;
-  const int64_t share8 = 2 * ((items8 + cus - 1) / cus), share4 = (items4 + cus - 1) / cus;  // in half-size items
+  const LaunchDims d8 = by_map<DimsOf>(wide.map, r, wide), d4 = by_map<DimsOf>(narrow.map, r, narrow);
+  if (d8.work_items <= 0 || d4.work_items <= 0) return 8;
+  auto share = [&](const LaunchDims& d) {  // items of the CU with the most of them
+    const int per_xcd = std::max(1, cus / 8);
+    const int split = r.kind == KIND_IMG_SCATTER ? 0 : xcd_split(d.n_pairs, d.n_mblocks, d.hgroups, per_xcd);
+    return xcd_rounds(d.n_pairs, d.n_mblocks, d.hgroups, per_xcd, split);
+  };
+  const int64_t share8 = 2 * share(d8), share4 = share(d4);  // in half-size items
   return 5 * share4 <= 4 * share8 ? intra::NARROW_WAVES : 8;
 }
 
@@ -454,23 +480,6 @@ bool row_order_pays(const int* cost, int n_mblocks, int pairs, int hgroups, int 
   return 100ll * longest[0] > (4 * pairs <= 32 ? 103ll : 112ll) * longest[1];
 }
 
-// log2 of the parts that the row blocks of a pair are split into, the parts dealt like pairs: the fewest after which
-// the XCD with the most work has at least a tenth fewer rounds.  A whole pair on one XCD loads its keys into one L2
-// only, but a call with few kv heads then leaves XCDs idle.  per_xcd: workgroups of an XCD at a time.  Whole / split, us:
-// window 255 with 4 sinks S=13568, 4 / 1 heads 103 / 20 (training step 422 / 158); window 2112 S=30000, 8 / 1 heads
-// 1469 / 229 (6416 / 971); window 1023 with 64 sinks S=11671, 28 / 4 heads 368 / 191 (1463 / 852); window 576 S=3000,
-// 16 / 4 heads 35.0 / 21.8; Scatter G=3 S=20000, 28 / 4 heads 1098 / 893 (4608 / 3625).  With as many rounds either way:
-// window 575 with 64 sinks S=6000, 12 / 12 heads 46.8 / 51.4.
-int xcd_split(int64_t pairs, int n_rblocks, int hgroups, int per_xcd) {
-  auto rounds = [&](int s) {
-    return (((pairs << s) + 7) / 8 * ((n_rblocks + (1 << s) - 1) >> s) * hgroups + per_xcd - 1) / per_xcd;
-  };
-  int split = 0;
-  for (int s = 1; s <= 3; ++s)
-    if (10 * rounds(split) > 11 * rounds(s)) split = s;
-  return split;
-}
-
 // Order of an XCD's work items (see KParams::Section).  One section - every pair, all row blocks -
 // except where a launch mixes kinds of items:
 //  * image scatter: a set has text_len / 8 + width^2 / 8 queries, so its last row block is partial
@@ -481,7 +490,7 @@ int xcd_split(int64_t pairs, int n_rblocks, int hgroups, int per_xcd) {
 //    its section, so that no number goes to an empty item, text rows first.
 void set_sections(intra::KParams& p, const Request& r, const Shape& ph, const LaunchDims& d, int wgs_per_xcd) {
   const bool llm = ph.map != MAP_IMG_SCATTER && ph.map != MAP_IMG_GATHER0;  // (the others: has_sections, items of one length)
-  const int split = llm ? xcd_split(d.n_pairs, d.n_mblocks, d.hgroups, wgs_per_xcd) : 0;
+  const int split = llm ? xcd_split(d.n_pairs, d.n_mblocks, d.hgroups, std::max(1, wgs_per_xcd * ph.nw / 8)) : 0;
   const int n_mblocks = (d.n_mblocks + (1 << split) - 1) >> split;  // of a part
   p.n_pairs = d.n_pairs << split;
   const int pslots = (p.n_pairs + 7) / 8;

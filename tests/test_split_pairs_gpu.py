@@ -11,6 +11,7 @@ from test_backward_gpu import make
 pytestmark = pytest.mark.gpu
 
 
+@pytest.mark.parametrize("waves", ["8", "4"])
 @pytest.mark.parametrize("pattern,S,r,kw", [
     ("window", 4997, 1, dict(window=1000)),                # 40 key blocks, 20 query blocks
     ("window", 5000, 4, dict(window=300)),                 # the forward's and dQ's row blocks are of 64 queries
@@ -19,8 +20,8 @@ pytestmark = pytest.mark.gpu
     ("scatter", 13001, 4, dict(group_num=3)),
     ("block_scatter", 9001, 4, dict(group_num=2, block=256, offset=1, n_sink=64)),
 ])
-def test_same_bits_for_few_kv_heads(monkeypatch, pattern, S, r, kw):
-    monkeypatch.setitem(os.environ, "INTRA_WAVES", "8")
+def test_same_bits_for_few_kv_heads(monkeypatch, waves, pattern, S, r, kw):
+    monkeypatch.setitem(os.environ, "INTRA_WAVES", waves)
     q, k, v, dout = make(1, S, 8 * r, 8, seed=S)
 
     def run(*tensors):
