@@ -242,6 +242,7 @@ int64_t xcd_rounds(int64_t pairs, int n_rblocks, int hgroups, int per_xcd, int s
   return (((pairs << split) + 7) / 8 * ((n_rblocks + (1 << split) - 1) >> split) * hgroups + per_xcd - 1) / per_xcd;
 }
 int xcd_split(int64_t pairs, int n_rblocks, int hgroups, int per_xcd) {
+  if (pairs % 8 == 0) return 0;  // (even: the usual case, and small calls are bound by the host)
   auto rounds = [&](int s) { return xcd_rounds(pairs, n_rblocks, hgroups, per_xcd, s); };
   int split = 0;
   for (int s = 1; s <= 3; ++s)
