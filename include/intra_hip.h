@@ -243,6 +243,24 @@ typedef struct IntraPlan {
 int intra_plan(int domain, int pattern, int B, int S, int H, int Hkv, int arg0, int arg1,
                IntraPlan* plan);
 
+/* What a backward call would launch: one entry per kind of rows, in launch order (the leading keys, or
+ * image Gather 0's text queries in dq, share the launch of the entry in front of them).  arg0, arg1 as in
+ * intra_plan.  rows holds max_rows entries; *n_rows is set to the number there are (at most 5).  Counted for
+ * 256 CUs, whatever the device.  No counterpart in the reference. */
+typedef struct IntraBwdRows {
+  int keys;           /* 0: rows are queries (dq), 1: keys (dk and dv) */
+  int leading;        /* 1: leading keys, or text queries in dq of image Gather 0 */
+  int waves;          /* wavefronts per workgroup */
+  int rows_per_block; /* rows of a row block, of one head */
+  int row_blocks;     /* per set, or per part of one */
+  int head_groups;    /* workgroups per row block */
+  int parts;          /* parts that the row blocks of a (set, batch, kv head) are split into, dealt over the XCDs */
+  int bundle;         /* parts that an XCD works on together */
+  int workgroups;
+} IntraBwdRows;
+int intra_plan_bwd(int domain, int pattern, int B, int S, int H, int Hkv, int arg0, int arg1, int block,
+                   int offset, int n_sink, IntraBwdRows* rows, int max_rows, int* n_rows);
+
 /* Walks the exact set / row-block / wavefront / 32-key-block decomposition the kernel uses
  * (same index maps and block classification, compiled for the host) and adds 1 to
  * count[q_pos * S + k_pos] for every score the kernel would compute and keep.  `count` is an

@@ -20,6 +20,11 @@ class IntraPlan(ctypes.Structure):
                 ("pairs_per_head", ctypes.c_int64)]
 
 
+class IntraBwdRows(ctypes.Structure):
+    _fields_ = [(n, ctypes.c_int) for n in ("keys", "leading", "waves", "rows_per_block", "row_blocks", "head_groups",
+                                            "parts", "bundle", "workgroups")]
+
+
 _FWD_ARGS = [ctypes.c_void_p] * 4 + [ctypes.c_int] * 4 + [ctypes.POINTER(ctypes.c_int64)] * 4 + \
     [ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_float, ctypes.c_void_p]
 
@@ -52,6 +57,8 @@ SYMBOLS = {
     "intra_diag_ablation": (ctypes.c_int, []),
     "intra_diag_mfma_ceiling": (ctypes.c_int, [ctypes.c_void_p] * 3 + [ctypes.c_int] * 3 + [ctypes.c_void_p]),
     "intra_plan": (ctypes.c_int, [ctypes.c_int] * 8 + [ctypes.POINTER(IntraPlan)]),
+    "intra_plan_bwd": (ctypes.c_int, [ctypes.c_int] * 11 + [ctypes.POINTER(IntraBwdRows), ctypes.c_int,
+                                                            ctypes.POINTER(ctypes.c_int)]),
     "intra_model_mask": (ctypes.c_int, [ctypes.c_int] * 7 + [ctypes.c_void_p]),
     "intra_model_deal": (ctypes.c_int, [ctypes.c_int] * 10 + [ctypes.c_void_p, ctypes.c_int64]),
 }

@@ -230,17 +230,21 @@ int cu_count() {
   return n;
 }
 
-// log2 of the parts that the row blocks of a pair are split into, the parts dealt like pairs: the fewest after which
-// the XCD with the most work has at least a tenth fewer rounds.  A whole pair on one XCD loads its keys into one L2
-// only, but a call with few kv heads then leaves XCDs idle.  per_xcd: workgroups of an XCD at a time (half-size ones count one per CU: two on a CU take
-// turns, so they are spread first).  Whole / split, us:
+// Rounds of the XCD with the most work, per_xcd workgroups at a time, if the row blocks of every pair are split into
+// 2^split parts that are dealt like pairs.
+int64_t xcd_rounds(int64_t pairs, int n_rblocks, int hgroups, int per_xcd, int split) {
+  return (((pairs << split) + 7) / 8 * ((n_rblocks + (1 << split) - 1) >> split) * hgroups + per_xcd - 1) / per_xcd;
+}
+// log2 of the parts: the fewest after which there is at least a tenth fewer rounds.  A whole pair on one XCD loads its
+// keys into one L2 only, but a call with few kv heads then leaves XCDs idle.  per_xcd: the CUs of an XCD, for half-size
+// workgroups too: two on a CU take turns, so they are spread first.  Whole / split, us:
 // window 255 with 4 sinks S=13568, 4 / 1 heads 103 / 20 (training step 422 / 158); window 2112 S=30000, 8 / 1 heads
 // 1469 / 229 (6416 / 971); window 1023 with 64 sinks S=11671, 28 / 4 heads 368 / 191 (1463 / 852); window 576 S=3000,
 // 16 / 4 heads 35.0 / 21.8; Scatter G=3 S=20000, 28 / 4 heads 1098 / 893 (4608 / 3625).  With as many rounds either way:
 // window 575 with 64 sinks S=6000, 12 / 12 heads 46.8 / 51.4.
-int64_t xcd_rounds(int64_t pairs, int n_rblocks, int hgroups, int per_xcd, int split) {
-  return (((pairs << split) + 7) / 8 * ((n_rblocks + (1 << split) - 1) >> split) * hgroups + per_xcd - 1) / per_xcd;
-}
+// dQ in half-size workgroups counted two / one per CU, forward and backward in a graph, us: window 576 S=2000, 4 / 1
+// heads 111 / 103; S=8000 119 / 109; S=3000, 8 / 2 heads 115 / 104; S=4096, 8 / 1 heads 177 / 163; with 64 sinks S=4096,
+// 8 / 2 heads 142 / 130; the same within 0.4 % where both spread them alike.
 int xcd_split(int64_t pairs, int n_rblocks, int hgroups, int per_xcd) {
   if (pairs % 8 == 0) return 0;  // (even: the usual case, and small calls are bound by the host)
   auto rounds = [&](int s) { return xcd_rounds(pairs, n_rblocks, hgroups, per_xcd, s); };
@@ -631,12 +635,31 @@ int run(int domain, const void* q, const void* k, const void* v, void* o, int B,
 
 
 // ------------------------------------------------------------------------------------ backward
+// Where the launches of a backward call go: to a stream, or into a list (intra_plan_bwd), and then no device is touched.
+struct BwdTarget {
+  hipStream_t stream;
+  IntraBwdRows* rows;  // null: launch
+  int max, n;
+};
+
+void note_rows(BwdTarget& to, int mode, int hp, int leading, const intra::BwdGrid& g) {
+  if (to.n < to.max)
+    to.rows[to.n] = IntraBwdRows{mode == intra::BWD_DKV, leading, intra::bwd_waves(mode), intra::bwd_waves(mode) * 32 / hp,
+                                 g.n_rblocks, g.hgroups, 1 << g.split, g.bundle, g.blocks};
+  ++to.n;
+}
+
 template <class RMAP, int MODE, int HP, class LEAD = intra::NoLeadingKeys>
-int launch_bwd(const intra::BParams& p, hipStream_t stream) {
+int launch_bwd(const intra::BParams& p, BwdTarget& to) {
   const int64_t grid = (int64_t)p.grid.blocks + p.lead.blocks;
   if (p.grid.blocks <= 0 || p.lead.blocks < 0 || grid > 0x7fffffff) return fail(INTRA_ERR_UNSUPPORTED, "backward needs more than 2^31 workgroups");
+  if (to.rows != nullptr) {
+    note_rows(to, MODE, HP, 0, p.grid);
+    if (p.lead.blocks > 0) note_rows(to, MODE, HP, 1, p.lead);
+    return INTRA_OK;
+  }
   const auto kernel = p.far_rows ? intra::intra_bwd_kernel<RMAP, MODE, HP, LEAD, true> : intra::intra_bwd_kernel<RMAP, MODE, HP, LEAD, false>;
-  hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(intra::bwd_waves(MODE) * 64), 0, stream, p);
+  hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(intra::bwd_waves(MODE) * 64), 0, to.stream, p);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return fail(INTRA_ERR_HIP, "kernel launch failed: %s", hipGetErrorString(e));
   return INTRA_OK;
@@ -678,7 +701,7 @@ intra::BwdGrid bwd_grid(const intra::BParams& p, int rows, int hgroups, int per_
   g.hgroups = std::max(1, hgroups);
   g.n_rblocks = (R::max_rows(p.geom) + rows - 1) / rows;
   int64_t pairs = (int64_t)R::num_sets(p.geom) * p.B * p.Hkv;
-  g.split = xcd_split(pairs, g.n_rblocks, g.hgroups, 32 * per_cu);
+  g.split = xcd_split(pairs, g.n_rblocks, g.hgroups, 32);
   pairs <<= g.split;  // (parts of pairs from here on)
   g.n_rblocks = (g.n_rblocks + (1 << g.split) - 1) >> g.split;
   g.items_per_pair = g.n_rblocks * g.hgroups;
@@ -710,18 +733,18 @@ intra::BwdGrid bwd_grid(const intra::BParams& p, int rows, int hgroups, int per_
 // dQ of a forward map: row blocks of 256 / hp queries of hp heads, or of half as many; also writes
 // D = rowsum(dO o O)
 template <class R, int MODE, class LEAD = intra::NoLeadingKeys>
-int launch_bwd_dq(const intra::BParams& p, int hp, hipStream_t stream) {
+int launch_bwd_dq(const intra::BParams& p, int hp, BwdTarget& to) {
   switch (hp) {
-    case 4: return launch_bwd<R, MODE, 4, LEAD>(p, stream);
-    case 2: return launch_bwd<R, MODE, 2, LEAD>(p, stream);
-    default: return launch_bwd<R, MODE, 1, LEAD>(p, stream);
+    case 4: return launch_bwd<R, MODE, 4, LEAD>(p, to);
+    case 2: return launch_bwd<R, MODE, 2, LEAD>(p, to);
+    default: return launch_bwd<R, MODE, 1, LEAD>(p, to);
   }
 }
 template <class MAP>
-int run_bwd_dq(intra::BParams p, int hp, hipStream_t stream) {
+int run_bwd_dq(intra::BParams p, int hp, BwdTarget& to) {
   using R = intra::QueryRows<MAP>;
   p.grid = bwd_grid<R>(p, 256 / hp, p.ratio / hp);
-  return launch_bwd_dq<R, intra::BWD_DQ>(p, hp, stream);
+  return launch_bwd_dq<R, intra::BWD_DQ>(p, hp, to);
 }
 
 // The same in half-size workgroups where a row block meets at most HALF_COLUMNS columns: two workgroups on a CU
@@ -732,12 +755,12 @@ int run_bwd_dq(intra::BParams p, int hp, hipStream_t stream) {
 // Scatter, whose row blocks are of every length up to the set's: 0 to 3 % slower at any size.)
 constexpr int HALF_COLUMNS = 1152;
 template <class MAP>
-int run_bwd_dq_short(const intra::BParams& p0, int hp, int columns, hipStream_t stream) {
-  if (columns > HALF_COLUMNS) return run_bwd_dq<MAP>(p0, hp, stream);
+int run_bwd_dq_short(const intra::BParams& p0, int hp, int columns, BwdTarget& to) {
+  if (columns > HALF_COLUMNS) return run_bwd_dq<MAP>(p0, hp, to);
   using R = intra::QueryRows<MAP>;
   intra::BParams p = p0;
   p.grid = bwd_grid<R>(p, 128 / hp, p.ratio / hp, 2);
-  return launch_bwd_dq<R, intra::BWD_DQ_HALF>(p, hp, stream);
+  return launch_bwd_dq<R, intra::BWD_DQ_HALF>(p, hp, to);
 }
 
 // dQ of image gather0, in half-size workgroups: the patch runs, and in front of them (at large grids they meet the
@@ -745,7 +768,7 @@ int run_bwd_dq_short(const intra::BParams& p0, int hp, int columns, hipStream_t 
 // run's (pick_text_merge).  A run of 2 patches streams 14 tiles, of which a wavefront uses 12; one of 4, in 8
 // wavefronts, 18: the launch 85.9 -> 81.7 us at 1024^2 and 24 heads, the training step 313.9 -> 311.0, at 2048^2
 // 1115 -> 1092.
-int run_bwd_dq_gather0(intra::BParams p, int hp, hipStream_t stream) {
+int run_bwd_dq_gather0(intra::BParams p, int hp, BwdTarget& to) {
   using R = intra::QueryRows<MapImgPatch>;
   using Text = intra::QueryRows<MapImgTextRows>;
   const int pos = 128 / hp;
@@ -755,43 +778,43 @@ int run_bwd_dq_gather0(intra::BParams p, int hp, hipStream_t stream) {
   p.grid = bwd_grid<R>(p, pos, p.ratio / hp, 2);
   p.lead = bwd_grid<Text>(p, pos, p.ratio / hp, 2);
   p.lead_first = 1;
-  return launch_bwd_dq<R, intra::BWD_DQ_HALF, Text>(p, hp, stream);
+  return launch_bwd_dq<R, intra::BWD_DQ_HALF, Text>(p, hp, to);
 }
 
 // dK and dV over a key-row map: row blocks of 128 keys of one kv head, all query heads of its group
 // streamed past.
 using intra::KEY_ROWS;
 template <class R>
-int run_bwd_keys(intra::BParams p, hipStream_t stream) {
+int run_bwd_keys(intra::BParams p, BwdTarget& to) {
   p.grid = bwd_grid<R>(p, KEY_ROWS, 0);
-  return launch_bwd<R, intra::BWD_DKV, 1>(p, stream);
+  return launch_bwd<R, intra::BWD_DKV, 1>(p, to);
 }
 
 // dK and dV over a key-row map and, in the same launch, over the leading keys LEAD: first where they
 // meet more columns than the longest row block of R (the shorter workgroups then fill the last round).
 template <class R, class LEAD>
-int run_bwd_keys_lead(intra::BParams p, hipStream_t stream) {
+int run_bwd_keys_lead(intra::BParams p, BwdTarget& to) {
   p.grid = bwd_grid<R>(p, KEY_ROWS, 0);
   p.lead = bwd_grid<LEAD>(p, KEY_ROWS, 0);
   // (their work counts half where both halves of a workgroup share the columns)
   p.lead_first = std::min(p.geom.sink_chunk, p.geom.S) / (intra::alternates<LEAD> ? 2 : 1) > R::longest(p.geom);
-  return launch_bwd<R, intra::BWD_DKV, 1, LEAD>(p, stream);
+  return launch_bwd<R, intra::BWD_DKV, 1, LEAD>(p, to);
 }
 
 // The same with the sinks as leading keys.  Up to 64 of them fill two of a workgroup's four wavefronts:
 // the other two then take every other block of columns.
 template <class R>
-int run_bwd_keys_sinks(const intra::BParams& p, hipStream_t stream) {
-  return p.geom.ns <= 64 ? run_bwd_keys_lead<R, intra::KeyRowsFewSinks>(p, stream)
-                         : run_bwd_keys_lead<R, intra::KeyRowsSinks>(p, stream);
+int run_bwd_keys_sinks(const intra::BParams& p, BwdTarget& to) {
+  return p.geom.ns <= 64 ? run_bwd_keys_lead<R, intra::KeyRowsFewSinks>(p, to)
+                         : run_bwd_keys_lead<R, intra::KeyRowsSinks>(p, to);
 }
 
 // The leading keys' rows of dk and dv from their partial sums (one chunk: written by the launch itself)
-int run_bwd_lead_reduce(const intra::BParams& p, int ns, hipStream_t stream) {
+int run_bwd_lead_reduce(const intra::BParams& p, int ns, BwdTarget& to) {
   const int chunks = intra::KeyRowsSinks::num_sets(p.geom);
-  if (chunks == 1) return INTRA_OK;
+  if (chunks == 1 || to.rows != nullptr) return INTRA_OK;
   const int64_t threads = (int64_t)p.B * p.Hkv * ns * 32;
-  hipLaunchKernelGGL(intra::intra_bwd_lead_reduce, dim3((unsigned)((threads + 255) / 256), 2), dim3(256), 0, stream, p,
+  hipLaunchKernelGGL(intra::intra_bwd_lead_reduce, dim3((unsigned)((threads + 255) / 256), 2), dim3(256), 0, to.stream, p,
                      chunks, ns);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return fail(INTRA_ERR_HIP, "kernel launch failed: %s", hipGetErrorString(e));
@@ -826,6 +849,45 @@ int bwd_supported(const Request& r) {
   if (r.kind == KIND_LLM_BLOCK_SCATTER && r.geom.off != 0 && r.geom.blk % 256 != 0)
     return fail(INTRA_ERR_UNSUPPORTED, "backward: block scatter with a stripe offset needs block % 256 == 0");
   return INTRA_OK;
+}
+
+// All launches of a backward call whose tensors, leading keys (ns) and geometry are in p
+int dispatch_bwd(const Shape& sh, intra::BParams& p, int ns, BwdTarget& to) {
+  int rc;
+  const int S = p.geom.S;
+  p.lead = intra::BwdGrid{};
+  p.lead_first = 0;
+  switch (sh.map) {
+    case MAP_LLM_SCATTER:
+      if ((rc = run_bwd_dq<MapLlmScatter>(p, sh.hp, to))) return rc;
+      return run_bwd_keys<intra::KeyRowsOf<MapLlmScatter>>(p, to);
+    case MAP_LLM_GATHER1:
+      if ((rc = run_bwd_dq<MapLlmGather1>(p, sh.hp, to))) return rc;
+      return run_bwd_keys<intra::KeyRowsOf<MapLlmGather1>>(p, to);
+    case MAP_LLM_WINDOW:
+      if ((rc = run_bwd_dq_short<MapLlmWindow>(p, sh.hp, p.geom.window, to))) return rc;
+      return run_bwd_keys<intra::KeyRowsOf<MapLlmWindow>>(p, to);
+    case MAP_LLM_BLOCK_SCATTER:
+      if ((rc = run_bwd_dq<MapLlmBlockScatter>(p, sh.hp, to))) return rc;
+      if (ns == 0) return run_bwd_keys<intra::KeyRowsBlockScatter>(p, to);
+      rc = run_bwd_keys_sinks<intra::KeyRowsBlockScatter>(p, to);
+      return rc ? rc : run_bwd_lead_reduce(p, ns, to);
+    case MAP_LLM_WINDOW_SINK:
+      if ((rc = run_bwd_dq_short<MapLlmWindowSink>(p, sh.hp, (int)std::min<int64_t>((int64_t)p.geom.window + ns, S), to))) return rc;
+      if (ns == 0) return run_bwd_keys<intra::KeyRowsWindowSink>(p, to);
+      rc = run_bwd_keys_sinks<intra::KeyRowsWindowSink>(p, to);
+      return rc ? rc : run_bwd_lead_reduce(p, ns, to);
+    case MAP_IMG_SCATTER:  // grid keys against their group's queries, text keys against all queries
+      if ((rc = run_bwd_dq_short<MapImgScatter>(p, sh.hp, p.geom.text_len + p.geom.width * p.geom.width / 8, to))) return rc;
+      rc = run_bwd_keys_lead<intra::KeyRowsImgGroup<false>, intra::KeyRowsText>(p, to);
+      return rc ? rc : run_bwd_lead_reduce(p, ns, to);
+    case MAP_IMG_GATHER0:  // grid keys against the grid queries around them, plus their group's text queries
+      if ((rc = run_bwd_dq_gather0(p, sh.hp, to))) return rc;
+      if ((rc = run_bwd_keys_lead<intra::KeyRowsImgWindow, intra::KeyRowsText>(p, to))) return rc;
+      if ((rc = run_bwd_keys<intra::KeyRowsImgGroup<true>>(p, to))) return rc;
+      return run_bwd_lead_reduce(p, ns, to);
+    default: return fail(INTRA_ERR_UNSUPPORTED, "backward: no kernels for this pattern");
+  }
 }
 
 int run_bwd(int domain, const void* q, const void* k, const void* v, const void* o, const float* lse, const void* dout,
@@ -897,40 +959,24 @@ int run_bwd(int domain, const void* q, const void* k, const void* v, const void*
     if (cus <= 0) return fail(INTRA_ERR_HIP, "cannot query the current device: %s", hipGetErrorString(hipGetLastError()));
     set_leading_chunk(p.geom, S, B, Hkv, ns, cus);
   }
-  p.lead = intra::BwdGrid{};
-  p.lead_first = 0;
-  hipStream_t st = static_cast<hipStream_t>(stream);
-  switch (sh.map) {
-    case MAP_LLM_SCATTER:
-      if ((rc = run_bwd_dq<MapLlmScatter>(p, sh.hp, st))) return rc;
-      return run_bwd_keys<intra::KeyRowsOf<MapLlmScatter>>(p, st);
-    case MAP_LLM_GATHER1:
-      if ((rc = run_bwd_dq<MapLlmGather1>(p, sh.hp, st))) return rc;
-      return run_bwd_keys<intra::KeyRowsOf<MapLlmGather1>>(p, st);
-    case MAP_LLM_WINDOW:
-      if ((rc = run_bwd_dq_short<MapLlmWindow>(p, sh.hp, p.geom.window, st))) return rc;
-      return run_bwd_keys<intra::KeyRowsOf<MapLlmWindow>>(p, st);
-    case MAP_LLM_BLOCK_SCATTER:
-      if ((rc = run_bwd_dq<MapLlmBlockScatter>(p, sh.hp, st))) return rc;
-      if (ns == 0) return run_bwd_keys<intra::KeyRowsBlockScatter>(p, st);
-      rc = run_bwd_keys_sinks<intra::KeyRowsBlockScatter>(p, st);
-      return rc ? rc : run_bwd_lead_reduce(p, ns, st);
-    case MAP_LLM_WINDOW_SINK:
-      if ((rc = run_bwd_dq_short<MapLlmWindowSink>(p, sh.hp, (int)std::min<int64_t>((int64_t)p.geom.window + ns, S), st))) return rc;
-      if (ns == 0) return run_bwd_keys<intra::KeyRowsWindowSink>(p, st);
-      rc = run_bwd_keys_sinks<intra::KeyRowsWindowSink>(p, st);
-      return rc ? rc : run_bwd_lead_reduce(p, ns, st);
-    case MAP_IMG_SCATTER:  // grid keys against their group's queries, text keys against all queries
-      if ((rc = run_bwd_dq_short<MapImgScatter>(p, sh.hp, p.geom.text_len + p.geom.width * p.geom.width / 8, st))) return rc;
-      rc = run_bwd_keys_lead<intra::KeyRowsImgGroup<false>, intra::KeyRowsText>(p, st);
-      return rc ? rc : run_bwd_lead_reduce(p, ns, st);
-    case MAP_IMG_GATHER0:  // grid keys against the grid queries around them, plus their group's text queries
-      if ((rc = run_bwd_dq_gather0(p, sh.hp, st))) return rc;
-      if ((rc = run_bwd_keys_lead<intra::KeyRowsImgWindow, intra::KeyRowsText>(p, st))) return rc;
-      if ((rc = run_bwd_keys<intra::KeyRowsImgGroup<true>>(p, st))) return rc;
-      return run_bwd_lead_reduce(p, ns, st);
-    default: return fail(INTRA_ERR_UNSUPPORTED, "backward: no kernels for this pattern");
-  }
+  BwdTarget to{static_cast<hipStream_t>(stream), nullptr, 0, 0};
+  return dispatch_bwd(sh, p, ns, to);
+}
+
+// The launches of a request without its tensors
+int plan_bwd(const Request& r, IntraBwdRows* rows, int max, int* n) {
+  if (int rc = bwd_supported(r)) return rc;
+  Shape sh;
+  if (!shape_for(r, default_hp(r.H / r.Hkv), &sh)) return fail(INTRA_ERR_UNSUPPORTED, "no kernel shape for this request");
+  intra::BParams p{};
+  p.B = r.B; p.H = r.H; p.Hkv = r.Hkv; p.ratio = r.H / r.Hkv;
+  p.geom = sh.geom;
+  const int ns = leading_keys(r);
+  if (ns > 0) set_leading_chunk(p.geom, r.S, r.B, r.Hkv, ns, MODEL_CUS);
+  BwdTarget to{nullptr, rows, max, 0};
+  const int rc = dispatch_bwd(sh, p, ns, to);
+  *n = to.n;
+  return rc;
 }
 
 // ------------------------------------------------------------------------------------ no-allocation backward
@@ -1208,6 +1254,16 @@ int intra_plan(int domain, int pattern, int B, int S, int H, int Hkv, int arg0, 
   int rc = make_request(domain, pattern, B, S, H, Hkv, arg0, arg1, &r);
   if (rc) return rc;
   return plan_for(r, default_hp(H / Hkv), plan);
+}
+
+int intra_plan_bwd(int domain, int pattern, int B, int S, int H, int Hkv, int arg0, int arg1, int block, int offset,
+                   int n_sink, IntraBwdRows* rows, int max_rows, int* n_rows) {
+  g_err[0] = 0;
+  if (!rows || max_rows < 1 || !n_rows) return fail(INTRA_ERR_INVALID, "rows and n_rows must be non-null, max_rows positive");
+  Request r;
+  int rc = make_request(domain, pattern, B, S, H, Hkv, arg0, arg1, &r, block, offset, n_sink, domain == 0);
+  if (rc) return rc;
+  return plan_bwd(r, rows, max_rows, n_rows);
 }
 
 int intra_model_mask(int domain, int pattern, int S, int arg0, int arg1, int heads_per_block,

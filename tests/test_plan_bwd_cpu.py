@@ -1,0 +1,54 @@
+"""Which workgroups a backward call launches (intra_plan_bwd, host only): the sizes of dQ's workgroups and the split
+of few pairs' row blocks over the XCDs."""
+import ctypes
+
+import pytest
+
+from intra_amd import _lib
+
+LLM, IMAGE = 0, 1
+SCATTER, WINDOW, GATHER0, BLOCK_SCATTER, WINDOW_SINK = 0, 4, 4, 8, 9
+XCDS, CUS = 8, 32
+
+
+def plan(domain, pattern, B, S, H, Hkv, arg0=0, arg1=0, block=64, offset=0, n_sink=0):
+    rows, n = (_lib.IntraBwdRows * 5)(), ctypes.c_int()
+    rc = _lib.load().intra_plan_bwd(domain, pattern, B, S, H, Hkv, arg0, arg1, block, offset, n_sink, rows, 5, ctypes.byref(n))
+    assert rc == 0, _lib.last_error()
+    return rows[:n.value]
+
+
+def window(B, S, H, Hkv, width, n_sink=None):
+    if n_sink is None:
+        return plan(LLM, WINDOW, B, S, H, Hkv, 8, width)
+    return plan(LLM, WINDOW_SINK, B, S, H, Hkv, 8, width, n_sink=n_sink)
+
+
+def test_entries_are_the_kinds_of_rows_of_a_call():
+    kinds = lambda rows: [(r.keys, r.leading) for r in rows]
+    assert kinds(plan(LLM, SCATTER, 1, 4096, 32, 8, 8)) == [(0, 0), (1, 0)]
+    assert kinds(window(1, 4096, 32, 8, 575, n_sink=64)) == [(0, 0), (1, 0), (1, 1)]
+    assert kinds(plan(IMAGE, GATHER0, 1, 4608, 24, 24, 64, 512)) == [(0, 0), (0, 1), (1, 0), (1, 1), (1, 0)]
+    rows, n = (_lib.IntraBwdRows * 1)(), ctypes.c_int()
+    lib = _lib.load()
+    assert lib.intra_plan_bwd(LLM, SCATTER, 1, 4096, 32, 8, 8, 0, 0, 0, 0, rows, 1, ctypes.byref(n)) == 0 and n.value == 2
+    assert lib.intra_plan_bwd(LLM, BLOCK_SCATTER, 1, 512, 4, 4, 2, 0, 64, 1, 0, rows, 1, ctypes.byref(n)) == _lib.INTRA_ERR_UNSUPPORTED
+    assert lib.intra_plan_bwd(LLM, SCATTER, 1, 4096, 32, 8, 8, 0, 0, 0, 0, None, 1, ctypes.byref(n)) == _lib.INTRA_ERR_INVALID
+
+
+@pytest.mark.parametrize("n_sink", [None, 64])
+@pytest.mark.parametrize("S,H,Hkv", [(8000, 4, 1), (2000, 8, 1), (4000, 4, 1), (4000, 8, 2), (3000, 8, 2), (2048, 4, 1)])
+def test_half_size_workgroups_take_a_cu_each_before_they_share_one(S, H, Hkv, n_sink):
+    """As many row blocks as the CUs of some XCDs hold one by one, or fewer: none of these XCDs gets a 33rd."""
+    dq = window(1, S, H, Hkv, 576, n_sink)[0]
+    assert dq.keys == 0 and dq.waves == 4
+    per_pair = -(-S // dq.rows_per_block) * dq.head_groups
+    assert per_pair * Hkv <= XCDS * CUS
+    fullest = -(-Hkv * dq.parts // XCDS) * dq.row_blocks * dq.head_groups
+    assert fullest <= CUS, (dq.parts, dq.row_blocks, fullest)
+
+
+@pytest.mark.parametrize("Hkv", [8, 16, 32])
+def test_pairs_that_come_out_even_stay_whole(Hkv):
+    for rows in (window(1, 5000, Hkv, Hkv, 576), plan(LLM, SCATTER, 1, 5000, Hkv, Hkv, 8)):
+        assert [r.parts for r in rows] == [1, 1]
