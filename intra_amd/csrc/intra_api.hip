@@ -254,6 +254,14 @@ int xcd_split(int64_t pairs, int n_rblocks, int hgroups, int per_xcd) {
   return split;
 }
 
+// The environment variable INTRA_WAVES (4 or 8) names the workgroup size for measurements and tests, of the forward
+// and of dQ, where the shape exists; 0: it names none.
+int named_waves() {
+  const char* e = getenv("INTRA_WAVES");
+  const int n = e ? atoi(e) : 0;
+  return n == 8 || n == intra::NARROW_WAVES ? n : 0;
+}
+
 // Wavefronts per workgroup of a forward launch.  Half-size workgroups, two per CU, pay for every key
 // tile twice as often per query (measured: 7 % on the long rows of LLM Scatter), and gain where the
 // work items are short or few:
@@ -264,16 +272,11 @@ int xcd_split(int64_t pairs, int n_rblocks, int hgroups, int per_xcd) {
 //    1024^2, whose 576 row blocks of 256 queries are 2.25 per CU; where the row blocks of few kv heads are split over
 //    XCDs, 8 wavefronts / 4, us: window 1088 S=2000, 8 / 2 heads 31.9 / 24.1; Scatter G=2 S=8000, 4 / 1 heads 92.8 / 68.7; and
 //    where it is not taken, window 1088 S=8000, 8 / 1 heads 36.4 / 38.3).
-// The environment variable INTRA_WAVES (4 or 8) overrides the choice for measurements, where the
-// shape exists.
 int pick_waves(const Request& r, int hp) {
   Shape narrow, wide;
   if (!shape_for(r, hp, &narrow, intra::NARROW_WAVES)) return 8;
   if (!shape_for(r, hp, &wide, 8)) return intra::NARROW_WAVES;  // (block scatter with an offset: smaller row blocks fit smaller blocks)
-  if (const char* e = getenv("INTRA_WAVES")) {
-    const int n = atoi(e);
-    if (n == 8 || n == intra::NARROW_WAVES) return n;
-  }
+  if (const int n = named_waves()) return n;
   if (r.kind == KIND_IMG_GATHER0) return intra::NARROW_WAVES;
   int cus = cu_count();
   if (cus <= 0) cus = 256;  // (planning without a device)
@@ -763,22 +766,42 @@ int run_bwd_dq_short(const intra::BParams& p0, int hp, int columns, BwdTarget& t
   return launch_bwd_dq<R, intra::BWD_DQ_HALF>(p, hp, to);
 }
 
-// dQ of image gather0, in half-size workgroups: the patch runs, and in front of them (at large grids they meet the
-// most columns) the text rows, the chunks of two groups in one row block where that keeps it as short as a patch
-// run's (pick_text_merge).  A run of 2 patches streams 14 tiles, of which a wavefront uses 12; one of 4, in 8
-// wavefronts, 18: the launch 85.9 -> 81.7 us at 1024^2 and 24 heads, the training step 313.9 -> 311.0, at 2048^2
-// 1115 -> 1092.
+// dQ of image gather0: the patch runs, and in front of them (at large grids they meet the most columns) the text rows,
+// the chunks of two groups in one row block where that keeps it as short as a patch run's (pick_text_merge).  In
+// half-size workgroups where the fullest CU then gets less to do, counted in half-size row blocks as the forward does;
+// where it gets as much, over several rounds and if a run then streams less than 4/5 of the tiles (with one head in a
+// workgroup: 14, of which a wavefront uses 12, not 18).  In a single round nothing covers the tiles that two on a CU load
+// twice.  Forward and backward in a graph, 8 wavefronts / 4 (fullest CU), us:
+//   less     1024^2  3 heads 120 / 114 (2 / 1), 6: 136 / 130, 16: 254 / 244 (4 / 3), 16 / 4: 237 / 230 (4 / 3)
+//            2048^2  12 heads 588 / 571 (8 / 7), 24: 1112 / 1086 (14 / 13), 8 / 4: 414 / 398 (6 / 5), 4 / 1: 286 / 270
+//   as much  1024^2  12 heads 188 / 190 (2 / 2), 24: 310.4 / 308.4 (4 / 4), 8 / 4: 142 / 147, 24 / 12: 290 / 292 (4 / 4),
+//                    24 / 6: 268 / 271 (4 / 4)
+//            2048^2  3 heads 232 / 244 (2 / 2), 6: 321 / 322 (4 / 4)
 int run_bwd_dq_gather0(intra::BParams p, int hp, BwdTarget& to) {
   using R = intra::QueryRows<MapImgPatch>;
   using Text = intra::QueryRows<MapImgTextRows>;
-  const int pos = 128 / hp;
-  p.geom.pg = pos >= 128 && p.geom.width / 8 % 2 == 0 ? 2 : 1;
-  p.geom.tm = pick_text_merge(p.geom, pos, p.geom.pg, 4);
-  geom_finish(p.geom);
-  p.grid = bwd_grid<R>(p, pos, p.ratio / hp, 2);
-  p.lead = bwd_grid<Text>(p, pos, p.ratio / hp, 2);
+  const int half_pos = 128 / hp;
+  IntraGeom half = p.geom;
+  half.pg = half_pos >= 128 && half.width / 8 % 2 == 0 ? 2 : 1;
+  half.tm = pick_text_merge(half, half_pos, half.pg, 4);
+  geom_finish(half);
+  auto rounds = [&](const IntraGeom& ge, int pos) {  // of the XCD with the most work
+    auto items = [&](int sets, int rows) {
+      return xcd_rounds((int64_t)sets * p.B * p.Hkv, (rows + pos - 1) / pos, p.ratio / hp, 1, 0);
+    };
+    return (items(R::num_sets(ge), R::max_rows(ge)) + items(Text::num_sets(ge), Text::max_rows(ge)) + 31) / 32;
+  };
+  auto run_tiles = [](const IntraGeom& ge) { return (ge.text_len + 16 * (16 + 8 * (ge.pg - 1))) / 64; };
+  const int64_t half_share = rounds(half, half_pos), share = 2 * rounds(p.geom, 2 * half_pos);
+  const int named = named_waves();
+  const bool is_half = named ? named == 4
+                             : half_share < share || (half_share == share && share > 2 && 5 * run_tiles(half) < 4 * run_tiles(p.geom));
+  if (is_half) p.geom = half;
+  const int pos = is_half ? half_pos : 2 * half_pos, per_cu = is_half ? 2 : 1;
+  p.grid = bwd_grid<R>(p, pos, p.ratio / hp, per_cu);
+  p.lead = bwd_grid<Text>(p, pos, p.ratio / hp, per_cu);
   p.lead_first = 1;
-  return launch_bwd_dq<R, intra::BWD_DQ_HALF, Text>(p, hp, to);
+  return is_half ? launch_bwd_dq<R, intra::BWD_DQ_HALF, Text>(p, hp, to) : launch_bwd_dq<R, intra::BWD_DQ, Text>(p, hp, to);
 }
 
 // dK and dV over a key-row map: row blocks of 128 keys of one kv head, all query heads of its group

@@ -48,6 +48,19 @@ def test_half_size_workgroups_take_a_cu_each_before_they_share_one(S, H, Hkv, n_
     assert fullest <= CUS, (dq.parts, dq.row_blocks, fullest)
 
 
+# dQ of image Gather 0: half-size workgroups where the fullest of the CUs then gets less to do (or as much, in more than
+# one round, and each less of the tiles)
+@pytest.mark.parametrize("width,B,H,Hkv,waves", [
+    (64, 1, 3, 3, 4), (64, 1, 6, 6, 4), (64, 1, 12, 12, 8), (64, 2, 6, 6, 8), (64, 1, 16, 16, 4), (64, 1, 24, 24, 4),
+    (64, 1, 8, 4, 8), (64, 1, 24, 6, 8), (64, 1, 16, 4, 4), (128, 1, 3, 3, 8), (128, 1, 6, 6, 4), (128, 1, 12, 12, 4),
+    (128, 1, 24, 24, 4), (128, 1, 8, 4, 4), (128, 1, 4, 1, 4)])
+def test_gather0_dq_workgroups_follow_the_rounds(width, B, H, Hkv, waves):
+    patches, text = plan(IMAGE, GATHER0, B, 512 + width * width, H, Hkv, width, 512)[:2]
+    assert (patches.keys, text.keys, text.leading) == (0, 0, 1)
+    assert patches.waves == text.waves == waves
+    assert patches.rows_per_block == text.rows_per_block == waves * 32 // (H // Hkv)
+
+
 @pytest.mark.parametrize("Hkv", [8, 16, 32])
 def test_pairs_that_come_out_even_stay_whole(Hkv):
     for rows in (window(1, 5000, Hkv, Hkv, 576), plan(LLM, SCATTER, 1, 5000, Hkv, Hkv, 8)):
