@@ -750,16 +750,19 @@ int run_bwd_dq(intra::BParams p, int hp, BwdTarget& to) {
   return launch_bwd_dq<R, intra::BWD_DQ>(p, hp, to);
 }
 
-// The same in half-size workgroups where a row block meets at most HALF_COLUMNS columns: two workgroups on a CU
-// fill each other's prologues and ends, a long row block pays for every column tile being loaded twice as often
-// instead.  Training steps, 8 wavefronts / 4, us: window 255 with 4 sinks S=16384 613 / 582; 575 with 64,
+// The same in half-size workgroups where a query sees at most HALF_COLUMNS keys (and its row block a few more): two
+// workgroups on a CU fill each other's prologues and ends, a long row block pays for every column tile being loaded
+// twice as often instead.  Training steps, 8 wavefronts / 4, us: window 255 with 4 sinks S=16384 613 / 582; 575 with 64,
 // S=8192, 457 / 445; 576 S=32768 1467 / 1448; 1023 with 64, S=16384, 1337 / 1324; 2112 S=16384 2097 / 2109; image
-// Scatter 1024^2 (1024 columns) 303 / 298, 2048^2 (2560) at 12 heads 1108 / 1121.  (Scatter, Gather 1 and block
-// Scatter, whose row blocks are of every length up to the set's: 0 to 3 % slower at any size.)
+// Scatter 1024^2 (1024 keys) 303 / 298, 2048^2 (2560) at 12 heads 1108 / 1121.  Between 1152 and 2000 keys there is no
+// difference to see, in a graph: window S=16384 1152 1194 / 1195, 1400 1433 / 1430, 1600 1591 / 1587, 1800 1793 / 1788, 2000
+// 1944 / 1972; S=8192 of 24 kv heads 1400 572 / 575, 2000 746 / 743.  (Scatter, Gather 1 and block Scatter, whose
+// row blocks are of every length up to the set's: 0 to 3 % slower at any size.)
 constexpr int HALF_COLUMNS = 1152;
 template <class MAP>
-int run_bwd_dq_short(const intra::BParams& p0, int hp, int columns, BwdTarget& to) {
-  if (columns > HALF_COLUMNS) return run_bwd_dq<MAP>(p0, hp, to);
+int run_bwd_dq_short(const intra::BParams& p0, int hp, int64_t keys, BwdTarget& to) {
+  const int named = named_waves();
+  if (named ? named == 8 : keys > HALF_COLUMNS) return run_bwd_dq<MAP>(p0, hp, to);
   using R = intra::QueryRows<MAP>;
   intra::BParams p = p0;
   p.grid = bwd_grid<R>(p, 128 / hp, p.ratio / hp, 2);
@@ -888,7 +891,7 @@ int dispatch_bwd(const Shape& sh, intra::BParams& p, int ns, BwdTarget& to) {
       if ((rc = run_bwd_dq<MapLlmGather1>(p, sh.hp, to))) return rc;
       return run_bwd_keys<intra::KeyRowsOf<MapLlmGather1>>(p, to);
     case MAP_LLM_WINDOW:
-      if ((rc = run_bwd_dq_short<MapLlmWindow>(p, sh.hp, p.geom.window, to))) return rc;
+      if ((rc = run_bwd_dq_short<MapLlmWindow>(p, sh.hp, std::min(p.geom.window, S), to))) return rc;
       return run_bwd_keys<intra::KeyRowsOf<MapLlmWindow>>(p, to);
     case MAP_LLM_BLOCK_SCATTER:
       if ((rc = run_bwd_dq<MapLlmBlockScatter>(p, sh.hp, to))) return rc;
@@ -896,7 +899,7 @@ int dispatch_bwd(const Shape& sh, intra::BParams& p, int ns, BwdTarget& to) {
       rc = run_bwd_keys_sinks<intra::KeyRowsBlockScatter>(p, to);
       return rc ? rc : run_bwd_lead_reduce(p, ns, to);
     case MAP_LLM_WINDOW_SINK:
-      if ((rc = run_bwd_dq_short<MapLlmWindowSink>(p, sh.hp, (int)std::min<int64_t>((int64_t)p.geom.window + ns, S), to))) return rc;
+      if ((rc = run_bwd_dq_short<MapLlmWindowSink>(p, sh.hp, std::min<int64_t>((int64_t)p.geom.window + ns, S), to))) return rc;
       if (ns == 0) return run_bwd_keys<intra::KeyRowsWindowSink>(p, to);
       rc = run_bwd_keys_sinks<intra::KeyRowsWindowSink>(p, to);
       return rc ? rc : run_bwd_lead_reduce(p, ns, to);

@@ -48,6 +48,16 @@ def test_half_size_workgroups_take_a_cu_each_before_they_share_one(S, H, Hkv, n_
     assert fullest <= CUS, (dq.parts, dq.row_blocks, fullest)
 
 
+@pytest.mark.parametrize("S,width,waves", [
+    (1000, 576, 4), (1000, 4096, 4), (1152, 4096, 4), (1153, 4096, 8), (3000, 1152, 4), (3000, 1153, 8), (700, 2 ** 31 - 1, 4)])
+def test_short_rows_are_those_of_queries_that_see_few_keys(S, width, waves):
+    """Up to 1152 keys, of those that there are: a window longer than the sequence is as long as the sequence."""
+    assert window(1, S, 8, 2, width)[0].waves == waves
+    assert window(1, S, 8, 2, width, n_sink=0)[0].waves == waves
+    if S >= 1153 and width >= 1152:
+        assert window(1, S, 8, 2, width - 33, n_sink=33)[0].waves == waves
+
+
 # dQ of image Gather 0: half-size workgroups where the fullest of the CUs then gets less to do (or as much, in more than
 # one round, and each less of the tiles)
 @pytest.mark.parametrize("width,B,H,Hkv,waves", [
