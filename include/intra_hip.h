@@ -12,8 +12,9 @@
  * of measurement builds (intra_diag_set_buffer), and per-device caches of the CU count.
  * Environment variables read by the library, both for experiments only: INTRA_SOFTMAX (the
  * starting value of that default) and INTRA_WAVES (8 or 4: the workgroup size of the forward
- * launches, where the named shape exists; otherwise the library picks - workgroups of 4 wavefronts,
- * two per CU, for image gather0 and for launches with few row blocks, 8 wavefronts for the rest).
+ * launches and of dq for the windows and the images, where the named shape exists; otherwise the
+ * library picks - forward: workgroups of 4 wavefronts, two per CU, for image gather0 and for launches
+ * with few row blocks, 8 wavefronts for the rest; dq: 4 where queries see few keys).
  *
  * Every function returns INTRA_OK or an error code; intra_last_error() then describes the failure
  * (thread-local string).  Argument validation happens before any HIP call, so it can be exercised
@@ -278,6 +279,17 @@ int intra_model_mask(int domain, int pattern, int S, int arg0, int arg1, int hea
  * counterpart in the reference: it launches one thread block per row block.) */
 int intra_model_deal(int domain, int pattern, int B, int S, int H, int Hkv, int arg0, int arg1,
                      int waves, int grid, uint8_t* visits, int64_t n_visits);
+
+/* In which order a forward launch deals them, on a device of 256 CUs (arguments as in intra_plan and, for the
+ * LLM patterns, intra_llm_fwd_ex). */
+typedef struct IntraDeal {
+  int waves;     /* wavefronts per workgroup */
+  int grid;      /* workgroups */
+  int parts;     /* parts that the row blocks of a (set, batch, kv head) are split into, dealt over the XCDs */
+  int row_order; /* 1: an XCD's items row block by row block, 0: pair by pair */
+} IntraDeal;
+int intra_plan_deal(int domain, int pattern, int B, int S, int H, int Hkv, int arg0, int arg1, int block,
+                    int offset, int n_sink, IntraDeal* deal);
 
 /* intra_plan / intra_model_mask for the arguments of intra_llm_fwd_ex (the walk: row blocks of 8
  * wavefronts). */

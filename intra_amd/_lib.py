@@ -25,6 +25,10 @@ class IntraBwdRows(ctypes.Structure):
                                             "parts", "bundle", "workgroups")]
 
 
+class IntraDeal(ctypes.Structure):
+    _fields_ = [(n, ctypes.c_int) for n in ("waves", "grid", "parts", "row_order")]
+
+
 _FWD_ARGS = [ctypes.c_void_p] * 4 + [ctypes.c_int] * 4 + [ctypes.POINTER(ctypes.c_int64)] * 4 + \
     [ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_float, ctypes.c_void_p]
 
@@ -57,6 +61,7 @@ SYMBOLS = {
     "intra_diag_ablation": (ctypes.c_int, []),
     "intra_diag_mfma_ceiling": (ctypes.c_int, [ctypes.c_void_p] * 3 + [ctypes.c_int] * 3 + [ctypes.c_void_p]),
     "intra_plan": (ctypes.c_int, [ctypes.c_int] * 8 + [ctypes.POINTER(IntraPlan)]),
+    "intra_plan_deal": (ctypes.c_int, [ctypes.c_int] * 11 + [ctypes.POINTER(IntraDeal)]),
     "intra_plan_bwd": (ctypes.c_int, [ctypes.c_int] * 11 + [ctypes.POINTER(IntraBwdRows), ctypes.c_int,
                                                             ctypes.POINTER(ctypes.c_int)]),
     "intra_model_mask": (ctypes.c_int, [ctypes.c_int] * 7 + [ctypes.c_void_p]),

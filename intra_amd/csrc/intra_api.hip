@@ -340,10 +340,9 @@ template <class MAP> struct DealWalk {
   }
 };
 
-// Persistent workgroups, as many as the CUs hold at once (LDS allows one of 8 wavefronts or two of
+// Persistent workgroups, as many as the n CUs hold at once (LDS allows one of 8 wavefronts or two of
 // 4 per CU), in multiples of the 8 XCDs.
-int launch_grid(int work_items, int nw) {
-  const int n = cu_count();
+int launch_grid(int work_items, int nw, int n) {
   if (n <= 0) return -1;
   int g = (n / 8) * 8;
   if (g < 8) g = 8;
@@ -628,7 +627,7 @@ int run(int domain, const void* q, const void* k, const void* v, void* o, int B,
   const LaunchDims dims = by_map<DimsOf>(ph.map, r, ph);
   if (dims.work_items <= 0 || dims.n_pairs <= 0)
     return fail(INTRA_ERR_UNSUPPORTED, "problem needs more than 2^31 work items");
-  const int grid = launch_grid(dims.work_items, ph.nw);
+  const int grid = launch_grid(dims.work_items, ph.nw, cu_count());
   if (grid <= 0)
     return fail(INTRA_ERR_HIP, "cannot query the current device: %s", hipGetErrorString(hipGetLastError()));
   set_dealing(p, r, ph, dims, grid);
@@ -1322,6 +1321,27 @@ int intra_model_deal(int domain, int pattern, int B, int S, int H, int Hkv, int 
   intra::KParams p{};
   set_dealing(p, r, ph, dims, grid);
   return by_map<DealWalk>(ph.map, p, dims.pos, grid, dims.n_mblocks, visits);
+}
+
+int intra_plan_deal(int domain, int pattern, int B, int S, int H, int Hkv, int arg0, int arg1, int block, int offset,
+                    int n_sink, IntraDeal* deal) {
+  g_err[0] = 0;
+  if (!deal) return fail(INTRA_ERR_INVALID, "deal pointer is null");
+  Request r;
+  int rc = make_request(domain, pattern, B, S, H, Hkv, arg0, arg1, &r, block, offset, n_sink, domain == 0);
+  if (rc) return rc;
+  const int hp = default_hp(H / Hkv);
+  Shape ph;
+  if (!shape_for(r, hp, &ph, pick_waves(r, hp)))
+    return fail(INTRA_ERR_UNSUPPORTED, "block size does not fit the row blocks of this head layout");
+  const LaunchDims dims = by_map<DimsOf>(ph.map, r, ph);
+  if (dims.work_items <= 0 || dims.n_pairs <= 0)
+    return fail(INTRA_ERR_UNSUPPORTED, "problem needs more than 2^31 work items");
+  intra::KParams p{};
+  const int grid = launch_grid(dims.work_items, ph.nw, MODEL_CUS);
+  set_dealing(p, r, ph, dims, grid);
+  *deal = IntraDeal{ph.nw, grid, 1 << (p.order >> 1), p.order & 1};
+  return INTRA_OK;
 }
 
 int intra_llm_fwd_ex(const void* q, const void* k, const void* v, void* o, int B, int S, int H,

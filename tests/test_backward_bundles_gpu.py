@@ -5,22 +5,26 @@ import pytest
 import torch
 
 from intra_amd import intra_llm_attn, intra_llm_attn_bwd
+from plan_util import backward, one_bundle
 from test_backward_gpu import make
 
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("pattern,B,S,H,Hkv,kw", [
-    ("scatter", 1, 7000, 32, 8, dict(group_num=3)),   # one bundle for dK / dV only
-    ("scatter", 1, 3000, 16, 16, dict(group_num=4)),  # for dQ too
-    ("scatter", 2, 2501, 8, 8, dict(group_num=4)),
-    ("gather1", 1, 4992, 16, 4, dict(group_num=8)),
-    ("block_scatter", 1, 6000, 16, 16, dict(group_num=2, block=256, offset=0, n_sink=0)),
-    ("window", 2, 1700, 8, 8, dict(window=1600)),
+# together: the launches (dQ, dK / dV) that take all pairs of an XCD as one bundle
+@pytest.mark.parametrize("pattern,B,S,H,Hkv,kw,sets,together", [
+    ("scatter", 1, 7000, 32, 8, dict(group_num=3), 3, [True, True]),
+    ("scatter", 1, 3000, 16, 16, dict(group_num=4), 4, [False, True]),
+    ("scatter", 2, 2501, 8, 8, dict(group_num=4), 4, [False, True]),
+    ("gather1", 1, 4992, 16, 8, dict(group_num=8), 8, [True, True]),
+    ("block_scatter", 1, 6000, 16, 16, dict(group_num=2, block=256, offset=0, n_sink=0), 2, [True, False]),
+    ("window", 4, 1700, 8, 8, dict(window=1600), 1, [False, True]),
 ])
-def test_same_bits_in_either_order(pattern, B, S, H, Hkv, kw):
+def test_same_bits_in_either_order(pattern, B, S, H, Hkv, kw, sets, together):
     q, k, v, dout = make(B, S, H, Hkv, seed=S)
     r = H // Hkv
+    assert [one_bundle(rows, B * Hkv * sets) for rows in backward(pattern, B, S, H, Hkv, **kw)] == together
+    assert not any(one_bundle(rows, sets) for rows in backward(pattern, 1, S, r, 1, **kw))
 
     def grads(*tensors):
         with torch.no_grad():

@@ -3,8 +3,8 @@ windows the same products in the same order as in the large ones, so the same bi
 import pytest
 import torch
 
+from plan_util import backward
 from test_backward_gpu import kernel_grads, make, run_case
-from test_plan_bwd_cpu import window
 
 pytestmark = pytest.mark.gpu
 LIMIT = 1152  # keys up to which a row is short
@@ -19,7 +19,7 @@ def test_same_bits_in_either_size(monkeypatch, S, H, Hkv):
     grads = {}
     for waves in (8, 4):
         monkeypatch.setenv("INTRA_WAVES", str(waves))
-        assert window(2, S, H, Hkv, 300)[0].waves == waves
+        assert backward("window", 2, S, H, Hkv, window=300)[0].waves == waves
         grads[waves] = kernel_grads(q, k, v, dout, "window", window=300)
     for name, a, b in zip(("dq", "dk", "dv"), grads[8], grads[4]):
         assert torch.equal(a, b), name
@@ -31,13 +31,13 @@ def test_same_bits_in_either_size(monkeypatch, S, H, Hkv):
 def test_windows_with_sinks_in_either_size(monkeypatch, waves, S, H, Hkv):
     """The columns of a row block start where its first query's window does, so the sizes share no blocks of 32."""
     monkeypatch.setenv("INTRA_WAVES", str(waves))
-    assert window(1, S, H, Hkv, 300, 33)[0].waves == waves
+    assert backward("window_sink", 1, S, H, Hkv, window=300, n_sink=33)[0].waves == waves
     run_case("llm/window_sink", "window_sink", 1, S, H, Hkv, window=300, n_sink=33)
 
 
 @pytest.mark.parametrize("H,Hkv", HEADS)
 @pytest.mark.parametrize("columns", [LIMIT - 1, LIMIT, LIMIT + 1])
 def test_grads_at_the_limit(columns, H, Hkv):
-    assert window(1, 2300, H, Hkv, columns)[0].waves == (4 if columns <= LIMIT else 8)
+    assert backward("window", 1, 2300, H, Hkv, window=columns)[0].waves == (4 if columns <= LIMIT else 8)
     run_case("llm/window", "window", 1, 2300, H, Hkv, window=columns)
     run_case("llm/window_sink", "window_sink", 1, 2300, H, Hkv, window=columns - 33, n_sink=33)

@@ -8,6 +8,7 @@ import torch
 
 from intra_amd import intra_llm_attn
 from parity_util import make_qkv
+from plan_util import forward
 
 pytestmark = pytest.mark.gpu
 
@@ -24,6 +25,7 @@ def test_same_bits_in_either_order(monkeypatch, waves, pattern, B, S, H, Hkv, kw
     monkeypatch.setitem(os.environ, "INTRA_WAVES", waves)
     q, k, v = make_qkv(B, S, H, Hkv, seed=S)
     r = H // Hkv
+    assert forward(pattern, B, S, H, Hkv, **kw).row_order == 1 and forward(pattern, 1, S, r, 1, **kw).row_order == 0
     with torch.no_grad():
         out = intra_llm_attn(q, k, v, pattern, **kw)
         for h in range(Hkv):

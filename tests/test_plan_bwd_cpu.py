@@ -5,6 +5,7 @@ import ctypes
 import pytest
 
 from intra_amd import _lib
+from plan_util import backward_of
 
 LLM, IMAGE = 0, 1
 SCATTER, WINDOW, GATHER0, BLOCK_SCATTER, WINDOW_SINK = 0, 4, 4, 8, 9
@@ -12,10 +13,7 @@ XCDS, CUS = 8, 32
 
 
 def plan(domain, pattern, B, S, H, Hkv, arg0=0, arg1=0, block=64, offset=0, n_sink=0):
-    rows, n = (_lib.IntraBwdRows * 5)(), ctypes.c_int()
-    rc = _lib.load().intra_plan_bwd(domain, pattern, B, S, H, Hkv, arg0, arg1, block, offset, n_sink, rows, 5, ctypes.byref(n))
-    assert rc == 0, _lib.last_error()
-    return rows[:n.value]
+    return backward_of(domain, pattern, B, S, H, Hkv, arg0, arg1, block, offset, n_sink)
 
 
 def window(B, S, H, Hkv, width, n_sink=None):
@@ -69,6 +67,16 @@ def test_gather0_dq_workgroups_follow_the_rounds(width, B, H, Hkv, waves):
     assert (patches.keys, text.keys, text.leading) == (0, 0, 1)
     assert patches.waves == text.waves == waves
     assert patches.rows_per_block == text.rows_per_block == waves * 32 // (H // Hkv)
+
+
+def test_text_keys_of_an_image_can_be_split_too():
+    """33 row blocks of text keys for 9 heads: more workgroups than CUs, so the queries are one chunk and the 9 pairs
+    leave XCDs with a third round; the public calls (512 text keys) always fit one round."""
+    for pattern in (SCATTER, GATHER0):
+        text = [r for r in plan(IMAGE, pattern, 1, 4224 + 256, 9, 9, 16, 4224) if r.keys and r.leading]
+        assert [r.parts for r in text] == [2]
+        for width, B, H in ((64, 1, 3), (64, 1, 24), (64, 3, 40), (128, 1, 5), (128, 2, 24)):
+            assert all(r.parts == 1 for r in plan(IMAGE, pattern, B, 512 + width * width, H, H, width, 512))
 
 
 @pytest.mark.parametrize("Hkv", [8, 16, 32])
