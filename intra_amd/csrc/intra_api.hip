@@ -269,9 +269,9 @@ int named_waves() {
 //    workgroups of a CU fill each other's waits): 0.0775 -> 0.0694 ms at 1024^2, 0.266 -> 0.235 at 2048^2;
 //  * launches with so few row blocks that the CU with the most work gets at least a fifth less of it
 //    when the blocks are half as large (8 kv heads at S <= 1024: 22 -> 18 us; image scatter at
-//    1024^2, whose 576 row blocks of 256 queries are 2.25 per CU; where the row blocks of few kv heads are split over
-//    XCDs, 8 wavefronts / 4, us: window 1088 S=2000, 8 / 2 heads 31.9 / 24.1; Scatter G=2 S=8000, 4 / 1 heads 92.8 / 68.7; and
-//    where it is not taken, window 1088 S=8000, 8 / 1 heads 36.4 / 38.3).
+//    1024^2, whose 576 row blocks of 256 queries are 2.25 per CU; where the row blocks of few kv heads are
+//    split over XCDs, 8 wavefronts / 4, us: window 1088 S=2000, 8 / 2 heads 31.9 / 24.1; Scatter G=2
+//    S=8000, 4 / 1 heads 92.8 / 68.7; and where it is not taken, window 1088 S=8000, 8 / 1 heads 36.4 / 38.3).
 int pick_waves(const Request& r, int hp) {
   Shape narrow, wide;
   if (!shape_for(r, hp, &narrow, intra::NARROW_WAVES)) return 8;
@@ -696,11 +696,12 @@ bool one_bundle_pays(const int* cost, int64_t pair, const intra::BwdGrid& g, int
 }
 
 // Workgroups of a row map with `rows` rows each, per_cu of which a CU holds at once: per XCD, bundles of pairs x
-// items of a pair (see the kernel).  blocks = -1 if they are too many to number.
-template <class R>
+// items of a pair (see the kernel).  Rows are queries (dQ: hgroups workgroups of heads per row block, the last row blocks
+// first) or KEYS (dK / dV: all heads in one workgroup, the first row blocks first).  blocks = -1 if they are too many to number.
+template <class R, bool KEYS = false>
 intra::BwdGrid bwd_grid(const intra::BParams& p, int rows, int hgroups, int per_cu = 1) {
   intra::BwdGrid g;
-  g.hgroups = std::max(1, hgroups);
+  g.hgroups = hgroups;
   g.n_rblocks = (R::max_rows(p.geom) + rows - 1) / rows;
   int64_t pairs = (int64_t)R::num_sets(p.geom) * p.B * p.Hkv;
   g.split = xcd_split(pairs, g.n_rblocks, g.hgroups, 32);
@@ -715,16 +716,17 @@ intra::BwdGrid bwd_grid(const intra::BParams& p, int rows, int hgroups, int per_
     int64_t pair = 0;
     bool one_range = true;
     for (int b = 0; b < g.n_rblocks; ++b) {  // in the order in which they start: the longest first
-      const int r0 = ((hgroups > 0 ? g.n_rblocks - 1 - b : b) << g.split) * rows;
+      const int r0 = ((KEYS ? b : g.n_rblocks - 1 - b) << g.split) * rows;
       const R map(p.geom, 0, r0);
       const int r1 = std::min(r0 + rows, map.n_rows()) - 1;
       const int columns = r1 < r0 ? 0 : map.block_hi(r0, r1) - map.block_lo(r0, r1) + 1;
-      cost[b] = r1 < r0 ? 0 : ITEM_COST + (std::max(0, columns) + 63) / 64 * (hgroups > 0 ? 1 : p.ratio);
+      cost[b] = r1 < r0 ? 0 : ITEM_COST + (std::max(0, columns) + 63) / 64 * (KEYS ? p.ratio : 1);
       pair += (int64_t)cost[b] * g.hgroups;
       one_range = one_range && map.kpre() == 0;
     }
     // (row blocks of about one length take as long either way)
-    if (one_range && 2 * cost[g.n_rblocks - 1] < cost[0] && one_bundle_pays(cost, pair, g, (int)pairs_per_xcd, 32 * per_cu)) g.bundle = (int)pairs_per_xcd;
+    if (one_range && 2 * cost[g.n_rblocks - 1] < cost[0] && one_bundle_pays(cost, pair, g, (int)pairs_per_xcd, 32 * per_cu))
+      g.bundle = (int)pairs_per_xcd;
   }
   const int64_t bundles = (pairs_per_xcd + g.bundle - 1) / g.bundle;
   const int64_t blocks = 8 * bundles * g.bundle * g.items_per_pair;
@@ -811,7 +813,7 @@ int run_bwd_dq_gather0(intra::BParams p, int hp, BwdTarget& to) {
 using intra::KEY_ROWS;
 template <class R>
 int run_bwd_keys(intra::BParams p, BwdTarget& to) {
-  p.grid = bwd_grid<R>(p, KEY_ROWS, 0);
+  p.grid = bwd_grid<R, true>(p, KEY_ROWS, 1);
   return launch_bwd<R, intra::BWD_DKV, 1>(p, to);
 }
 
@@ -819,8 +821,8 @@ int run_bwd_keys(intra::BParams p, BwdTarget& to) {
 // meet more columns than the longest row block of R (the shorter workgroups then fill the last round).
 template <class R, class LEAD>
 int run_bwd_keys_lead(intra::BParams p, BwdTarget& to) {
-  p.grid = bwd_grid<R>(p, KEY_ROWS, 0);
-  p.lead = bwd_grid<LEAD>(p, KEY_ROWS, 0);
+  p.grid = bwd_grid<R, true>(p, KEY_ROWS, 1);
+  p.lead = bwd_grid<LEAD, true>(p, KEY_ROWS, 1);
   // (their work counts half where both halves of a workgroup share the columns)
   p.lead_first = std::min(p.geom.sink_chunk, p.geom.S) / (intra::alternates<LEAD> ? 2 : 1) > R::longest(p.geom);
   return launch_bwd<R, intra::BWD_DKV, 1, LEAD>(p, to);

@@ -124,9 +124,9 @@ __device__ __forceinline__ void bwd_rows(const BParams& p, const BwdGrid& g, con
   // step (three instructions each, nine of them) go behind MFMAs of its first block, and which blocks of a tile it
   // needs and whether any of their pairs are hidden is worked out once per tile, not per head.  Training steps, in
   // one piece in front of the blocks / so, us: Scatter G=8 S=32768 4339 / 4243, window 575 with 64 sinks S=8192 448 / 436,
-  // block Scatter S=6000 with 64 sinks 712 / 687, image Gather 0 1024^2 309 / 309.  (Left out altogether, the requests
-  // are worth 1 % of the Scatter step, all exponentials 2 %, all transposing reads 2 %, all vector
-  // instructions 4 %: what remains is the MFMAs, at the clock that the board's power allows.)
+  // block Scatter S=6000 with 64 sinks 712 / 687, image Gather 0 1024^2 309 / 309.  (Left out altogether, of a
+  // Scatter step of 4265 us: without the requests 4233, the transposing reads 4231, all vector instructions 4168.  What
+  // remains is the MFMAs, at the clock that the board's power allows.)
   constexpr bool SPREAD = MODE == BWD_DKV && !FAR;
   constexpr bool ALT = alternates<RMAP>;  // wavefronts 0, 1 and 2, 3 share rows and take turns at the 32-column blocks
   const uint32_t lds_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)smem;
@@ -139,10 +139,12 @@ __device__ __forceinline__ void bwd_rows(const BParams& p, const BwdGrid& g, con
 
   // ---------------------------------------------------------------- work item
   // Workgroups start in blockIdx order, round-robin over the 8 XCDs, and a CU takes the next one
-  // when it has finished one.  Per XCD the (set, batch, kv head) pairs are taken in bundles of
-  // `bundle` pairs - as few as fill its 32 CUs - so that the workgroups running together stream the
-  // same few megabytes of columns through the XCD's L2; within a bundle the row blocks with the
-  // most columns come first (the last query blocks for dQ, the first key blocks for dK / dV).
+  // when it has finished one (half-size ones: when it has finished one of its two).  The unit is a part of a (set, batch,
+  // kv head) pair: all its row blocks, or every 2nd, 4th or 8th where whole pairs would leave XCDs idle (xcd_split).
+  // Per XCD the parts are taken in bundles of `bundle`, as few as fill its 32 CUs (64 places for half-size workgroups), so
+  // that the workgroups running together stream the same few megabytes of columns through the XCD's L2, or all as one
+  // bundle where the last one's long row blocks would end the launch late (one_bundle_pays).  Within a bundle the row
+  // blocks with the most columns come first (the last query blocks for dQ, the first key blocks for dK / dV).
   const int xcd = block & 7, slot = block >> 3;
   const int per_bundle = g.bundle * g.items_per_pair;
   const int bun = slot / per_bundle, rem = slot - bun * per_bundle;
@@ -472,8 +474,10 @@ __device__ __forceinline__ void bwd_rows(const BParams& p, const BwdGrid& g, con
   // of its first block are formed at the end of step t) and the tile of step t+2 is in flight.
   Cursor cur{ROWS_ARE_QUERIES ? 0 : ntiles - 1, 0};  // step being computed
   Cursor ld = cur;                                   // step being requested
-  // (Deep ring: one slot more, the tile of step t+3 is requested during step t, and the barrier of a
-  // step leaves the most recent request in flight where one was made during the step before.)
+  // (Deep ring: one slot more, the tile of step t+3 is requested during step t, and the barrier of a step leaves the
+  // requests of the step before in flight.  SPREAD: every step makes as many, the last three for a tile that nobody
+  // reads, and the wait behind the loop is for these.  Otherwise the last steps make none, and the barriers behind them
+  // wait for all.)
   for (int t = 0; t < (DEEP ? 3 : 2) && t < n_steps; ++t) {
     if (SPREAD && t > 0) advance(ld);  // (SPREAD: ld is the step requested last)
     load_step(ld, t * BWD_SLOT);
