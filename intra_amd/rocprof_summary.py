@@ -78,11 +78,15 @@ def counters(directories, only):
 
 
 def _reading(directory, counter, kernel_part, largest=False):
-    """Mean over the dispatches of the first kernel whose name contains kernel_part; largest=True
-    takes its largest dispatch instead (the 1 GiB calibration copies among smaller copies)."""
+    """Mean over the dispatches of the first kernel whose name contains kernel_part, which have to be of one size
+    (bench.py's CPU leg launches smaller problems too: --no-cpu); largest=True takes its largest dispatch
+    instead (the 1 GiB calibration copies among smaller copies)."""
     hits = [cs[counter] for name, cs in counter_values(directory).items() if kernel_part in name and counter in cs]
     if not hits:
         raise SystemExit(f"{counter} of a kernel matching {kernel_part!r} not found under {directory}")
+    if not largest and max(hits[0]) > 1.25 * min(hits[0]):
+        raise SystemExit(f"{counter} of {kernel_part!r} is {min(hits[0]):.0f} .. {max(hits[0]):.0f} KiB: launches of several "
+                         "sizes; profile bench.py with --no-cpu")
     return max(hits[0]) if largest else sum(hits[0]) / len(hits[0])
 
 
