@@ -129,7 +129,7 @@ int intra_version(void);
  *       arithmetic inside the same launch, so results stay finite and correct for any input.  Equal
  *       to EXACT up to the rounding of the weights; accuracy does not depend on the size of q, k.
  *   INTRA_SOFTMAX_FOLDED: multiplies softmax_scale * log2(e) into the bf16 query rows instead (one
- *       multiply per score less; about 2 % faster), then as SCALED.  Rounding the scaled query to
+ *       multiply per score less; about 3 % faster), then as SCALED.  Rounding the scaled query to
  *       bf16 perturbs a score by about 1.1e-3 * scale * sqrt(sum_d q_d^2 k_d^2) rms, i.e. in
  *       proportion to the magnitudes of q and k: as accurate as the other two for unit-variance
  *       inputs, outside the 1.6e-2 output bound once q and k are about twice as large.  Opt-in.
@@ -333,7 +333,7 @@ int intra_model_mask_image_bwd(int pattern, int S, int width, int text_len, uint
  * intra_diag_ablation: 0 for every library whose results are meant to be used.  Measurement builds can
  * be compiled with -DINTRA_ABLATE=<n> (python -m intra_amd.build --ablate <n>), which removes or doubles
  * one ingredient of the forward kernel's inner step (1: V^T operand reads, 2: K operand re-reads, 3: the
- * barrier between tiles, 4: exponentials, packing and row sums; 5: those issued twice; 6: the loader's
+ * barrier between tiles, 4: exponentials and packing; 5: those issued twice; 6: the loader's
  * rows: the same 64 for every tile, so no address arithmetic and only L2 hits) so that its cost shows
  * in the phase timers; such a library computes wrong results on purpose and reports <n> here. */
 int intra_diag_set_buffer(long long* counters, int64_t n_values);

@@ -43,7 +43,7 @@ def set_softmax_mode(mode):
     the fp32 scores after the first product and keeps a running reference like the reference
     (csrc/flash_attn/src/softmax.h:65-91); "scaled" scales them the same way but keeps no running
     maximum and recomputes, exactly, the queries whose weight sum leaves the safe exponent range;
-    "folded" multiplies the scale into the bf16 queries instead (about 2 % faster, error grows with
+    "folded" multiplies the scale into the bf16 queries instead (about 3 % faster, error grows with
     the magnitude of q and k); "auto" (default) is scaled up to four times the default
     softmax_scale, exact beyond.  Meant for experiments: pass `softmax=` per call otherwise."""
     if _C.intra_set_softmax_mode(SOFTMAX_MODES[mode]) != _lib.INTRA_OK:
