@@ -397,6 +397,10 @@ __device__ __forceinline__ void run_pass(const KParams& p, unsigned char* smem, 
   long long* dgw = nullptr;  // measurement builds: the barrier counters
   INTRA_DIAG(long long dg[DIAG_SLOTS] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0}; dgw = dg + 8;)
   Feed fd = feed_for(cw, -1);
+  // (Block Scatter only asks for it in half-size workgroups: here the other wavefront of the SIMD covers the positions, and
+  // 25 - 53 scalars more are spilled: S=6000 166.2 / 164.4 us without / with, 20000 G=8 442 / 435, exact arithmetic S=8000
+  // 281 / 284, the training step S=6000 698 / 696, runs of one side apart by 1 - 5 %.)
+  constexpr bool TILE_ROWS = !std::is_same_v<MAP, MapLlmBlockScatter>;
   // request the next slot of the stream into a ring slot (byte offset inside the K ring and the V ring)
   auto feed_tile = [&](int slot_off) {
     if (SWITCH_APART ? __builtin_expect(fd.tile < 0, 0) : fd.tile < 0) {  // 128 Q rows: rows of four wavefronts, two per part
@@ -415,7 +419,7 @@ __device__ __forceinline__ void run_pass(const KParams& p, unsigned char* smem, 
                     lds_base + part * VBASE + slot_off + grp * FGROUP_STRIDE);
         }
       }
-    } else if (TileRows tr; INTRA_ABLATE != 6 && map_tile_rows(fd.map, fd.rg.kt_lo + fd.tile * BN, tr)) {
+    } else if (TileRows tr; TILE_ROWS && INTRA_ABLATE != 6 && map_tile_rows(fd.map, fd.rg.kt_lo + fd.tile * BN, tr)) {
       // (wave-uniform) a tile whose key positions are affine: no per-key index arithmetic
       const uint32_t row = (uint32_t)(ld_row * tr.row_step);
 #pragma unroll

@@ -118,7 +118,11 @@ __device__ __forceinline__ void run_pass_narrow(const KParams& p, unsigned char*
                   lds_base + VBASE + v_off + (wave * GROUPS_PER_WAVE + gi) * FGROUP_STRIDE);
     }
     TileRows tr;
-    if (map_tile_rows(fd.map, fd.rg.kt_lo + fd.tile * BN, tr)) {  // (wave-uniform)
+    // (wave-uniform.  Block Scatter: where one workgroup comes to a CU nothing covers what a wavefront does between its
+    // blocks; its positions key by key, four times behind branches on the parts of the list, were a tenth of a tile.
+    // In a graph, us: S=300, 16 / 4 heads 12.2 -> 11.7; S=2000 28.3 -> 25.5, exact arithmetic 29.5 -> 28.0; S=3000, 4 / 1
+    // heads 38.0 -> 33.7, 32 / 8 48.2 -> 45.8; with more work on a CU, S=2000 of 32 / 8 heads 34.5 -> 34.4.)
+    if (map_tile_rows(fd.map, fd.rg.kt_lo + fd.tile * BN, tr)) {
       const uint32_t row = (uint32_t)(ld_row * tr.row_step);
 #pragma unroll
       for (int gi = 0; gi < GROUPS_PER_WAVE; ++gi) {

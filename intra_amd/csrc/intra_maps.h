@@ -538,6 +538,12 @@ struct MapLlmBlockScatter {
     return (m * G + gt) * blk + (c - m * blk);
   }
   IM_HD bool tile_at(int t_first, TileAt& a) const { return tile_linear([&](int t) { return kpos(t); }, t_first, a); }
+  IM_HD bool tile_rows(int t_first, TileRows& r) const {
+    TileAt a;
+    if (t_first + 64 > nk() || !tile_at(t_first, a)) return false;
+    r = TileRows{a.base, 4, 1};
+    return true;
+  }
   IM_HD int tile_rel(int, int i) const { return i; }
   IM_HD int klo(int) const { return 0; }
   IM_HD int khi(int tq) const {
